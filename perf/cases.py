@@ -249,3 +249,27 @@ def tolerance(case):
     if case["tin"] in F8_MAX:          # measured: rel up to 1.5e-5, max 8.4e-5
         return {"rel": 6e-5, "max": 3.5e-4}
     return {"rel": 4e-6, "max": 3e-5}  # measured: rel up to 8.0e-7, max 6.2e-6
+
+
+def exact(case, seed):
+    """The product in 64 bits, one batch at a time (a fresh C is zero, so beta adds nothing); None
+    where the outputs are bits."""
+    if case["path"] == "packing":
+        return None
+    state = prepare(case, seed)
+    planes = []
+    for x in (state["a"].cuda(), state["b"].cuda()):
+        x = x.movedim(3, 1) if case["axis_in"] == "interleaved" else x   # [B][2][rows][K]
+        planes.append(x * 2.0 - 1.0 if case["tin"] == "int1" else x)     # (a 1-bit sample is +1 or -1)
+    a, b = planes
+    alpha = complex(case["alpha_re"], case["alpha_im"])
+    c = torch.zeros(state["c"].shape, dtype=torch.float64, device="cuda")
+    for i in range(case["B"]):
+        (ar, ai), (br, bi) = a[i].double(), b[i].double()
+        brt, bit = br.t().contiguous(), bi.t().contiguous()
+        re, im = ar @ brt - ai @ bit, ar @ bit + ai @ brt
+        re, im = alpha.real * re - alpha.imag * im, alpha.real * im + alpha.imag * re
+        if case["order"] == "col":
+            re, im = re.t(), im.t()
+        c[i] = torch.stack([re, im], dim=2 if case["axis_out"] == "interleaved" else 0)
+    return {"c": c}
