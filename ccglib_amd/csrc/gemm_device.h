@@ -104,7 +104,6 @@ struct KernelArgs {
   size_t x_batch_bytes, y_batch_bytes;
   float alpha_re, alpha_im, beta_re, beta_im;
   int have_alpha, have_beta, c_interleaved;
-  int c_vector_ok;  // C base is 16-byte aligned: wide stores allowed
   // 1-bit samples on the MFMA: what the zero bits past K add to every imaginary sum
   unsigned im_excess;
 };
@@ -244,7 +243,6 @@ inline KernelArgs make_kernel_args(const GemmParams &p, int bx, int by) {
   a.have_alpha = p.have_alpha;
   a.have_beta = p.have_beta;
   a.c_interleaved = p.c_interleaved;
-  a.c_vector_ok = ((uintptr_t)p.c % 16 == 0);
   a.im_excess = (p.type_in == kInt1) ? 2u * (p.k_tiles * (unsigned)k_per_tile(kInt1) - p.k) : 0u;
   return a;
 }

@@ -860,6 +860,15 @@ __device__ __forceinline__ void mma_step32_interleaved(const char *slot, const i
 #undef CCGLIB_PIN
 }
 
+// Wide accesses to C at an address that is aligned to its elements only: rows of any
+// length start anywhere, and global memory takes any alignment on this target. Element
+// by element, every store instruction touches 64 lines for 4 bytes each: B=16 255x128x256
+// bf16 with beta and rows of 255 took 30.2 us instead of 17.2, B=16 300x3001x577 fp16 to
+// (re, im) rows of 3001 pairs 158.5 instead of 144.7 (with its transposes).
+typedef float4_t float4_any_t __attribute__((aligned(4)));
+typedef int4_t int4_any_t __attribute__((aligned(2)));
+typedef ushort4_t ushort4_any_t __attribute__((aligned(2)));
+
 // Epilogue of one wave: alpha * acc + beta * C, conversion, bounds-checked
 // store, piece by piece (four consecutive elements of the contiguous C axis).
 template <int TOUT, int TX, int TY, int MS = 16, int TILE0 = 0, typename Acc>
@@ -873,7 +882,6 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
   const bool have_alpha = args.have_alpha, have_beta = args.have_beta;
   const float ar = args.alpha_re, ai = args.alpha_im, br = args.beta_re, bi = args.beta_im;
   Tout *cbase = reinterpret_cast<Tout *>(args.c) + (size_t)b * 2 * nx * ny;
-  const bool vec_ok = (nx % 4 == 0) && args.c_vector_ok;
 #pragma unroll
   for (int j = 0; j < TY; ++j) {
 #pragma unroll
@@ -892,7 +900,7 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
           im[e] = alpha_times_im(ar, ai, r0, im[e]);
         }
       }
-      const bool full = vec_ok && (x + 4 <= nx);
+      const bool full = x + 4 <= nx;
       if (!args.c_interleaved) {
         Tout *pr = cbase + (size_t)y * nx + x;
         Tout *pi = pr + (size_t)nx * ny;
@@ -900,7 +908,8 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
           // (whole pieces: C comes in with one wide load per plane)
           Tout cr4[4], ci4[4];
           if (full) {
-            typedef Tout Piece __attribute__((ext_vector_type(4)));
+            typedef Tout Vec __attribute__((ext_vector_type(4)));
+            typedef Vec Piece __attribute__((aligned(sizeof(Tout))));
             const Piece vr = *reinterpret_cast<const Piece *>(pr), vi = *reinterpret_cast<const Piece *>(pi);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -920,13 +929,13 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
         }
         if (full) {
           if constexpr (TOUT == kFloat32) {
-            *reinterpret_cast<float4_t *>(pr) = float4_t{re[0], re[1], re[2], re[3]};
-            *reinterpret_cast<float4_t *>(pi) = float4_t{im[0], im[1], im[2], im[3]};
+            *reinterpret_cast<float4_any_t *>(pr) = float4_t{re[0], re[1], re[2], re[3]};
+            *reinterpret_cast<float4_any_t *>(pi) = float4_t{im[0], im[1], im[2], im[3]};
           } else {
             Tout r4[4] = {(Tout)re[0], (Tout)re[1], (Tout)re[2], (Tout)re[3]};
             Tout i4[4] = {(Tout)im[0], (Tout)im[1], (Tout)im[2], (Tout)im[3]};
-            *reinterpret_cast<ushort4_t *>(pr) = __builtin_bit_cast(ushort4_t, r4);
-            *reinterpret_cast<ushort4_t *>(pi) = __builtin_bit_cast(ushort4_t, i4);
+            *reinterpret_cast<ushort4_any_t *>(pr) = __builtin_bit_cast(ushort4_t, r4);
+            *reinterpret_cast<ushort4_any_t *>(pi) = __builtin_bit_cast(ushort4_t, i4);
           }
         } else {
 #pragma unroll
@@ -942,7 +951,8 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
         if (have_beta) {
           Tout c8[8];
           if (full) {
-            typedef Tout Piece __attribute__((ext_vector_type(8)));
+            typedef Tout Vec __attribute__((ext_vector_type(8)));
+            typedef Vec Piece __attribute__((aligned(sizeof(Tout))));
             const Piece v = *reinterpret_cast<const Piece *>(p);
 #pragma unroll
             for (int e = 0; e < 8; ++e) c8[e] = v[e];
@@ -959,12 +969,12 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
         }
         if (full) {
           if constexpr (TOUT == kFloat32) {
-            reinterpret_cast<float4_t *>(p)[0] = float4_t{re[0], im[0], re[1], im[1]};
-            reinterpret_cast<float4_t *>(p)[1] = float4_t{re[2], im[2], re[3], im[3]};
+            reinterpret_cast<float4_any_t *>(p)[0] = float4_t{re[0], im[0], re[1], im[1]};
+            reinterpret_cast<float4_any_t *>(p)[1] = float4_t{re[2], im[2], re[3], im[3]};
           } else {
             Tout v8[8] = {(Tout)re[0], (Tout)im[0], (Tout)re[1], (Tout)im[1],
                           (Tout)re[2], (Tout)im[2], (Tout)re[3], (Tout)im[3]};
-            *reinterpret_cast<int4_t *>(p) = __builtin_bit_cast(int4_t, v8);
+            *reinterpret_cast<int4_any_t *>(p) = __builtin_bit_cast(int4_t, v8);
           }
         } else {
 #pragma unroll
@@ -993,7 +1003,6 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
   const unsigned br = (unsigned)(int)args.beta_re, bi = (unsigned)(int)args.beta_im;
   const bool have_beta = args.have_beta;
   unsigned *cbase = reinterpret_cast<unsigned *>(args.c) + (size_t)b * 2 * nx * ny;
-  const bool vec_ok = (nx % 4 == 0) && args.c_vector_ok;
 #pragma unroll
   for (int j = 0; j < TY; ++j) {
 #pragma unroll
@@ -1009,7 +1018,7 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
         re[e] = ar * sr - ai * si;
         im[e] = ai * sr + ar * si;
       }
-      const bool full = vec_ok && (x + 4 <= nx);
+      const bool full = x + 4 <= nx;
       if (!args.c_interleaved) {
         unsigned *pr = cbase + (size_t)y * nx + x, *pi = pr + (size_t)nx * ny;
 #pragma unroll
@@ -1021,8 +1030,8 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
           }
         }
         if (full) {
-          *reinterpret_cast<int4_t *>(pr) = int4_t{(int)re[0], (int)re[1], (int)re[2], (int)re[3]};
-          *reinterpret_cast<int4_t *>(pi) = int4_t{(int)im[0], (int)im[1], (int)im[2], (int)im[3]};
+          *reinterpret_cast<int4_any_t *>(pr) = int4_t{(int)re[0], (int)re[1], (int)re[2], (int)re[3]};
+          *reinterpret_cast<int4_any_t *>(pi) = int4_t{(int)im[0], (int)im[1], (int)im[2], (int)im[3]};
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -1043,8 +1052,8 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
           }
         }
         if (full) {
-          reinterpret_cast<int4_t *>(p)[0] = int4_t{(int)re[0], (int)im[0], (int)re[1], (int)im[1]};
-          reinterpret_cast<int4_t *>(p)[1] = int4_t{(int)re[2], (int)im[2], (int)re[3], (int)im[3]};
+          reinterpret_cast<int4_any_t *>(p)[0] = int4_t{(int)re[0], (int)im[0], (int)re[1], (int)im[1]};
+          reinterpret_cast<int4_any_t *>(p)[1] = int4_t{(int)re[2], (int)im[2], (int)re[3], (int)im[3]};
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -1060,7 +1069,7 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
 }
 
 // Epilogue of the exchanged-roles layout (kAcc16T) for the common case (planar
-// C, beta = 0, wave tile entirely inside C, vector-aligned rows): register e of
+// C, beta = 0, wave tile entirely inside C): register e of
 // the four tiles of a tile row are four consecutive x, so a lane writes 16 bytes
 // (8 for fp16 / bf16 C) and a store instruction four whole 256-byte row segments,
 // straight from the accumulators.
@@ -1092,10 +1101,10 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
         if constexpr (kAblateStores) {
           if (v[0] == 12345.678f) *p = (Tout)v[1];   // (timing-only build)
         } else if constexpr (TOUT == kFloat32) {
-          *reinterpret_cast<float4_t *>(p) = float4_t{v[0], v[1], v[2], v[3]};
+          *reinterpret_cast<float4_any_t *>(p) = float4_t{v[0], v[1], v[2], v[3]};
         } else {
           Tout t[4] = {(Tout)v[0], (Tout)v[1], (Tout)v[2], (Tout)v[3]};
-          *reinterpret_cast<ushort4_t *>(p) = __builtin_bit_cast(ushort4_t, t);
+          *reinterpret_cast<ushort4_any_t *>(p) = __builtin_bit_cast(ushort4_t, t);
         }
       }
     }
@@ -1141,7 +1150,7 @@ __device__ __forceinline__ void store_wave_tile_staged(const KernelArgs &args, u
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float4_t v = *reinterpret_cast<const float4_t *>(rd + r * 4 * 272);
-        *reinterpret_cast<float4_t *>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 4) * nx) = v;
+        *reinterpret_cast<float4_any_t *>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 4) * nx) = v;
       }
     }
   }
@@ -1184,7 +1193,7 @@ __device__ __forceinline__ void store_wave_tile_staged_narrow(const KernelArgs &
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
         const int4_t v = *reinterpret_cast<const int4_t *>(rd + r * 8 * 144);
-        *reinterpret_cast<int4_t *>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 8) * nx) = v;
+        *reinterpret_cast<int4_any_t *>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 8) * nx) = v;
       }
     }
   }
@@ -1225,7 +1234,7 @@ __device__ __forceinline__ void store_wave_tile_staged_il(const KernelArgs &args
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float4_t v = *reinterpret_cast<const float4_t *>(rd + r * 4 * 272);
-        *reinterpret_cast<float4_t *>(out + ((size_t)(j * 16 + r * 4) * nx + h * 32) * 2) = v;
+        *reinterpret_cast<float4_any_t *>(out + ((size_t)(j * 16 + r * 4) * nx + h * 32) * 2) = v;
       }
     }
   }
@@ -1276,7 +1285,7 @@ __device__ __forceinline__ void store_wave_tile_staged32(const KernelArgs &args,
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const float4_t v = *reinterpret_cast<const float4_t *>(rd + q * 8 * 144);
-          *reinterpret_cast<float4_t *>(out + (size_t)plane * nx * ny +
+          *reinterpret_cast<float4_any_t *>(out + (size_t)plane * nx * ny +
                                         (size_t)(j * 32 + q * 8) * nx + i * 32) = v;
         }
       }
@@ -1723,10 +1732,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       yil32_off[h][u] = X_BYTES + (wy * WY) * 128 + off;
     }
   }
-  // wide stores through LDS: no beta term, vector-aligned rows (interleaved C
-  // only with the 16-row layout)
-  const bool staged_ok = (MS == 16 || !args.c_interleaved) && !args.have_beta &&
-                         args.c_vector_ok && (args.nx % 4 == 0);
+  // wide stores through LDS: no beta term (interleaved C only with the 16-row layout)
+  const bool staged_ok = (MS == 16 || !args.c_interleaved) && !args.have_beta;
 
   // ---- pipeline ----------------------------------------------------------
   point_x(xs.tile);
@@ -1880,7 +1887,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     }
     if constexpr (!XT && MS == 16 && (TOUT == kFloat16 || TOUT == kBfloat16) && TX == 4 &&
                   !SPLIT && NW * kStagePatchBytes <= SLOT_BYTES) {
-      if (staged_ok && !args.c_interleaved && args.nx % 8 == 0) {
+      if (staged_ok && !args.c_interleaved) {
         // ([X | Y] slots here: the rings are one)
         unsigned free_slot = y_slot + YLEAD;
         free_slot = free_slot >= SLOTS ? free_slot - SLOTS : free_slot;
