@@ -1617,6 +1617,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         unsigned tile = row0 / kTileRows;
         tile = tile < args.x_tiles ? tile : args.x_tiles - 1;   // rows past the end: never stored
         x_src[i] = op + (size_t)tile * args.k_tile_stride * kTileBytes;
+        // (a block lower than an operand tile starts inside it)
+        if constexpr (BX < kTileRows) x_src[i] += (tc.block_x * BX) % kTileRows * kTileRowBytes;
       } else {
         unsigned row = row0 + (XT ? xt_row : r);
         row = row < args.nx ? row : args.nx - 1;   // likewise
@@ -1637,6 +1639,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         unsigned tile = row0 / kTileRows;
         tile = tile < args.y_tiles ? tile : args.y_tiles - 1;
         y_src[i] = op + (size_t)tile * args.k_tile_stride * kTileBytes;
+        // (a block lower than an operand tile starts inside it)
+        if constexpr (BY < kTileRows) y_src[i] += (tc.block_y * BY) % kTileRows * kTileRowBytes;
       } else {
         unsigned row = row0 + r;
         row = row < args.ny ? row : args.ny - 1;
@@ -2075,20 +2079,48 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Whether 128 x 128 block tiles beat 256 x 128 ones for this problem: they do
-// when the larger tiles would leave compute units without work (fewer tiles
-// than units, or a last round that is mostly empty), although the smaller
-// block moves a third more bytes from L2 to LDS per flop (`penalty`: how much
-// slower per flop it measured once every unit is busy). Estimated from the
-// fraction of unit-rounds that hold a tile under either tiling.
-inline bool small_tiles_pay(const GemmParams &p, double penalty) {
-  if (p.block_tile == 1 || p.block_tile == 2) return p.block_tile == 2;
+// Which block shape of complex_gemm_mfma_dtl a problem gets: the one whose busiest compute
+// unit finishes first by
+//   rounds of tiles over the units * area of a tile * cost per element of C.
+// The smaller a block, the more of the chip a small problem fills and the less it
+// computes beyond the edges of C, but the more bytes it moves from L2 to LDS per flop; the
+// cost is what that measured once every unit is busy, relative to 256 x 128:
+//   16 bits, 4096x4096x512:  256x128 76 us, 128x128 91 us, 64x64 102 us;
+//            B=5 1024^3:     49, 65, 59 us;
+//            B=256 96x96x1024 (256 tiles of either larger shape):  70, 40, 52 us;
+//            B=16 255x128x256:  26, 17, 10 us;   256^3:  14.8, 12.5, 7.6 us
+//   32 bits (bound by the matrix cores at any of the shapes), 4096x4096x512:  493, 508,
+//            516 us;   B=2 1000^3:  483, 251, 145 us
+//   8 bits (with their transposes), 4096x4096x512:  57, 57, 76 us;   1024^3:  33, 29, 20 us.
+// Two 64 x 64 blocks share a unit. With 32-bit input they take turns on the matrix
+// cores and a unit's tiles simply add up; below that one block alone leaves them idle
+// half of the time, and an odd tile costs as much as two (B=3 1024^3 16 bits, three tiles a
+// unit: 38 us, 128x128 34 us).
+enum BlockShape { k256x128, k128x128, k64x64 };
+struct BlockChoice {
+  BlockShape shape;
+  double time;
+};
+inline BlockChoice block_choice(const GemmParams &p) {
   const size_t units = (size_t)compute_units();
-  auto busy = [&](size_t bx, size_t by) {
-    const size_t tiles = (size_t)p.batch * ceil_div((size_t)p.nx, bx) * ceil_div((size_t)p.ny, by);
-    return (double)tiles / (double)(units * ceil_div(tiles, units));
+  auto tiles = [&](size_t bx, size_t by) {
+    return (size_t)p.batch * ceil_div((size_t)p.nx, bx) * ceil_div((size_t)p.ny, by);
   };
-  return busy(128, 128) / penalty > busy(256, 128);
+  const bool bits8 = p.type_in == kFloat8e4m3 || p.type_in == kFloat8e5m2;
+  const double cost_128 = p.type_in == kInt1 ? 1.0 : bits8 || p.type_in == kFloat32 ? 1.05 : 1.25;
+  const double t256 = (double)ceil_div(tiles(256, 128), units) * (256 * 128);
+  const double t128 = (double)ceil_div(tiles(128, 128), units) * (128 * 128) * cost_128;
+  if (p.block_tile == 1) return {k256x128, t256};
+  if (p.block_tile == 2) return {k128x128, t128};
+  const BlockChoice larger = t128 < t256 ? BlockChoice{k128x128, t128} : BlockChoice{k256x128, t256};
+  // (interleaved 8-bit rows and 1-bit input have no 64 x 64 block: their steps are made for
+  // 2 x 2 tiles of the 32-row MFMA per wave)
+  if (p.type_in == kInt1 || (bits8 && p.input_interleaved)) return larger;
+  const size_t n = tiles(64, 64);
+  const bool adds_up = p.type_in == kFloat32 || n <= units;
+  const double rounds = adds_up ? (double)ceil_div(n, units) : 2.0 * (double)ceil_div(n, 2 * units);
+  const double t64 = rounds * (64 * 64) * (p.type_in == kFloat32 ? 1.06 : 1.5);
+  return t64 < larger.time ? BlockChoice{k64x64, t64} : larger;
 }
 
 // Whether the 192 x 256 block of gemm_mfma_wide.h can compute this problem (what
@@ -2114,18 +2146,7 @@ inline bool wide_tiles_apply(const GemmParams &p) {
 }
 inline bool wide_tiles_pay(const GemmParams &p) {
   if (p.block_tile != 0) return p.block_tile == 3;
-  const size_t units = (size_t)compute_units();
-  // fraction of the unit-rounds' tile area that holds elements of C
-  auto useful = [&](size_t bx, size_t by) {
-    const size_t cols = ceil_div((size_t)p.nx, bx), rows = ceil_div((size_t)p.ny, by);
-    const size_t tiles = (size_t)p.batch * cols * rows;
-    return (double)p.batch * p.nx * p.ny / (double)(units * ceil_div(tiles, units) * bx * by);
-  };
-  const double wide_useful =
-      (double)p.batch * p.nx * p.ny / ((double)units * wide_tiling(p).rounds * kWideBX * kWideBY);
-  const double other = useful(256, 128) > useful(128, 128) / 1.15 ? useful(256, 128)
-                                                                   : useful(128, 128) / 1.15;
-  return wide_useful * 1.075 > other;
+  return wide_tiling(p).rounds * (kWideBX * kWideBY) < 1.075 * block_choice(p).time;
 }
 
 template <int DT, int TOUT>
@@ -2136,6 +2157,7 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   // into LDS as well; anything else goes through the register-staged kernel
   const bool planar_direct = (p.variant == kBasic) && (k_bytes >= 16) && (k_bytes % 16 == 0) &&
                              ((uintptr_t)p.x % 16 == 0) && ((uintptr_t)p.y % 16 == 0);
+  const BlockShape shape = block_choice(p).shape;
   if (p.input_interleaved) {
     // raw (re, im) rows straight from the caller: the host side only takes this
     // path for 8- and 16-bit input whose rows are whole aligned 16-byte chunks
@@ -2145,12 +2167,13 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
       if constexpr (DtypeTraits<DT>::kElemBytes == 2) {
         if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT, true>(p, stream);
       }
-      if (small_tiles_pay(p, 1.15)) {
+      if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec>(p, stream);
+      if (shape == k128x128) {
         return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadInterleavedVec>(p, stream);
       }
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec>(p, stream);
     } else {
-      if (small_tiles_pay(p, 1.05)) {
+      if (shape == k128x128) {
         return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadInterleavedVec, 32>(p, stream);
       }
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec, 32>(p, stream);
@@ -2169,13 +2192,19 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
       // cache lines; the other layout regroups the tile through LDS into whole
       // rows of pairs (measured 5 % faster at B=64 512x4096x576).
       if constexpr (TOUT == kFloat32) {
-        if (p.variant == kOpt && p.c_interleaved) {
+        if (p.variant == kOpt && p.c_interleaved && shape == k256x128) {
           return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 16, false>(p, stream);
         }
       }
       // problems too small to give every compute unit a 256 x 128 tile: 128 x 128
-      // blocks, 8 waves of 64 x 32, 4-slot ring
-      if (small_tiles_pay(p, 1.15)) {
+      // blocks, 8 waves of 64 x 32, 4-slot ring, or 64 x 64 blocks, 4 waves of 32 x 32,
+      // 5-slot ring, two blocks a unit
+      if (shape == k64x64) {
+        return p.variant == kOpt
+                   ? launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadTiled, 16>(p, stream)
+                   : launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 16>(p, stream);
+      }
+      if (shape == k128x128) {
         return p.variant == kOpt
                    ? launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadTiled, 16>(p, stream)
                    : launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadPlanarVec, 16>(p, stream);
@@ -2186,8 +2215,14 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
     } else {
       // fp8: the 32x32x64 MFMA takes one K tile per instruction, which lets the
       // same block shape and ring as for 16-bit input fit into LDS
-      // (small problems: 128 x 128 blocks, 4 waves of 64 x 64, two blocks a unit)
-      if (small_tiles_pay(p, 1.05)) {
+      // (small problems: 128 x 128 blocks, 4 waves of 64 x 64, or 64 x 64 blocks, 4 waves
+      // of 32 x 32; two blocks a unit)
+      if (shape == k64x64) {
+        return p.variant == kOpt
+                   ? launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadTiled, 32>(p, stream)
+                   : launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 32>(p, stream);
+      }
+      if (shape == k128x128) {
         return p.variant == kOpt
                    ? launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadTiled, 32>(p, stream)
                    : launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadPlanarVec, 32>(p, stream);
@@ -2259,7 +2294,7 @@ hipError_t launch_gemm_mfma_int1(const GemmParams &p, hipStream_t stream) {
   // packed 1-bit samples expanded in registers; the caller has checked that
   // planar rows are whole aligned 16-byte chunks and that K fits fp32 sums
   if (p.type_out != kInt32 || p.input_interleaved) return hipErrorInvalidValue;
-  if (small_tiles_pay(p, 1.0)) {
+  if (block_choice(p).shape == k128x128) {
     return p.variant == kOpt
                ? launch_dtl<kInt1, kInt32, 128, 128, 64, 64, 2, 2, kLoadTiled, 32>(p, stream)
                : launch_dtl<kInt1, kInt32, 128, 128, 64, 64, 2, 2, kLoadPlanarVec, 32>(p, stream);
@@ -2280,24 +2315,30 @@ const char *describe_gemm_mfma(const GemmParams &p) {
   const size_t k_bytes = (size_t)p.k * bits_of(p.type_in) / 8;
   const bool planar_direct = (p.variant == kBasic) && (k_bytes >= 16) && (k_bytes % 16 == 0) &&
                              ((uintptr_t)p.x % 16 == 0) && ((uintptr_t)p.y % 16 == 0);
-  const double penalty = int1 ? 1.0 : bits8 ? 1.05 : 1.15;
+  const BlockShape shape = block_choice(p).shape;
+  auto name = [&](const char *large, const char *middle, const char *small) {
+    return shape == k256x128 ? large : shape == k128x128 ? middle : small;
+  };
   if (p.input_interleaved) {
     if (bits16 && wide_tiles_apply(p) && wide_tiles_pay(p)) {
       return "complex_gemm_mfma_wide, 192x256 block, one wave per SIMD, interleaved rows";
     }
-    return small_tiles_pay(p, penalty) ? "complex_gemm_mfma_dtl, 128x128 block, interleaved rows"
-                                       : "complex_gemm_mfma_dtl, 256x128 block, interleaved rows";
+    return name("complex_gemm_mfma_dtl, 256x128 block, interleaved rows",
+                "complex_gemm_mfma_dtl, 128x128 block, interleaved rows",
+                "complex_gemm_mfma_dtl, 64x64 block, interleaved rows");
   }
   if (p.variant == kOpt || planar_direct || int1) {
     if (bits16 && wide_tiles_apply(p) && wide_tiles_pay(p)) {
       return "complex_gemm_mfma_wide, 192x256 block, one wave per SIMD";
     }
     if (p.variant == kOpt) {
-      return small_tiles_pay(p, penalty) ? "complex_gemm_mfma_dtl, 128x128 block, tiled operands"
-                                         : "complex_gemm_mfma_dtl, 256x128 block, tiled operands";
+      return name("complex_gemm_mfma_dtl, 256x128 block, tiled operands",
+                  "complex_gemm_mfma_dtl, 128x128 block, tiled operands",
+                  "complex_gemm_mfma_dtl, 64x64 block, tiled operands");
     }
-    return small_tiles_pay(p, penalty) ? "complex_gemm_mfma_dtl, 128x128 block, planar rows"
-                                       : "complex_gemm_mfma_dtl, 256x128 block, planar rows";
+    return name("complex_gemm_mfma_dtl, 256x128 block, planar rows",
+                "complex_gemm_mfma_dtl, 128x128 block, planar rows",
+                "complex_gemm_mfma_dtl, 64x64 block, planar rows");
   }
   return "complex_gemm_mfma, 128x128 block, planar rows through registers";
 }

@@ -1,0 +1,87 @@
+"""Problems that leave compute units without work at the larger block shapes run on 64 x 64
+blocks: half an operand tile high, so blocks start in the middle of one."""
+import numpy as np
+import pytest
+
+import ccglib_amd as cc
+from gpu_util import stream
+from test_gemm_gpu import COL, INTERLEAVED, PLANAR, ROW, float_case, quantize, run_gemm
+
+pytestmark = pytest.mark.gpu
+
+VT = cc.ValueType
+TYPES = [(VT.float16, VT.float32), (VT.float16, VT.float16), (VT.bfloat16, VT.bfloat16),
+         (VT.float32, VT.float32), (VT.float8e4m3, VT.float32), (VT.float8e5m2, VT.float32)]
+
+
+def takes_64(B, M, N, K, tin, tout, variant):
+    gemm = cc.GEMM(B, M, N, K, 0, stream(), cc.Precision(tin, tout), variant)
+    return "64x64" in gemm.KernelName()
+
+
+@pytest.mark.parametrize("tin,tout", TYPES)
+@pytest.mark.parametrize("variant", [cc.Variant.basic, cc.Variant.opt])
+@pytest.mark.parametrize("B,M,N,K", [
+    (1, 1, 1, 16),         # one element, one K tile: the ring runs past the work
+    (2, 64, 64, 64),       # one block exactly
+    (2, 63, 65, 80),       # one short of a block, one more than one
+    (1, 129, 190, 1040),   # blocks in both halves of an operand tile, the last one partial
+    (3, 200, 320, 336),    # several blocks, more K tiles than ring slots
+])
+def test_64x64_blocks(B, M, N, K, tin, tout, variant):
+    assert takes_64(B, M, N, K, tin, tout, variant)
+    float_case(B, M, N, K, tin, tout, variant, PLANAR, ROW, seed=1)
+    float_case(B, M, N, K, tin, tout, variant, PLANAR, COL, alpha=0.5 - 1.5j, beta=0.25 + 0.5j, seed=2)
+    if variant == cc.Variant.opt:
+        float_case(B, M, N, K, tin, tout, variant, INTERLEAVED, ROW, alpha=1.5j, seed=3)
+        float_case(B, M, N, K, tin, tout, variant, INTERLEAVED, COL, beta=0.5, seed=4)
+
+
+@pytest.mark.parametrize("tin,B,M,N,K", [(VT.float32, 70, 180, 190, 48), (VT.float16, 256, 33, 130, 64),
+                                         (VT.float16, 256, 33, 130, 200), (VT.float8e4m3, 512, 60, 40, 64)])
+def test_64x64_blocks_several_tiles_each(tin, B, M, N, K):
+    """More tiles than resident blocks, among them K of one tile: the same bits as the
+    128 x 128 block, which adds up in the same order."""
+    rng = np.random.default_rng(5)
+    qa = quantize(rng.uniform(-1, 1, (B, 2, M, K)).astype(np.float32), tin).reshape(-1)
+    qb = quantize(rng.uniform(-1, 1, (B, 2, N, K)).astype(np.float32), tin).reshape(-1)
+    for variant in (cc.Variant.basic, cc.Variant.opt):
+        assert takes_64(B, M, N, K, tin, VT.float32, variant)
+        got = run_gemm(qa, qb, B, M, N, K, tin, VT.float32, variant, alpha=0.5 - 2j)
+        with cc.option(cc.Option.gemm_block_tile, 2):
+            want = run_gemm(qa, qb, B, M, N, K, tin, VT.float32, variant, alpha=0.5 - 2j)
+        assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("tin,tout", TYPES[:3])
+@pytest.mark.parametrize("B,M,N,K", [(1, 1, 3, 8), (2, 63, 65, 72), (200, 100, 40, 200), (256, 64, 130, 40)])
+def test_64x64_blocks_on_interleaved_rows(B, M, N, K, tin, tout):
+    """The pipeline's (re, im) rows of 16-bit samples, read in place."""
+    import torch
+    rng = np.random.default_rng(6)
+    a = rng.uniform(-1, 1, (B, M, K, 2)).astype(np.float32)
+    b = rng.uniform(-1, 1, (B, N, K, 2)).astype(np.float32)
+    tdt = torch.float16 if tin == VT.float16 else torch.bfloat16
+    d_a, d_b = torch.from_numpy(a).cuda().to(tdt), torch.from_numpy(b).cuda().to(tdt)
+    results = []
+    for block_tile in (0, 2):
+        c = torch.full((B, 2, M, N), float("nan"), device="cuda",
+                       dtype={VT.float32: torch.float32, VT.float16: torch.float16,
+                              VT.bfloat16: torch.bfloat16}[tout])
+        with cc.option(cc.Option.gemm_block_tile, block_tile):
+            pipe = cc.Pipeline(B, M, N, K, 0, stream(), INTERLEAVED, PLANAR, ROW, COL, ROW, tin, tout,
+                               cc.Variant.opt)
+        assert pipe.ReadsInPlace()
+        pipe.Run(d_a.data_ptr(), d_b.data_ptr(), c.data_ptr())
+        torch.cuda.synchronize()
+        results.append(c)
+    assert torch.equal(results[0], results[1])
+    ca = torch.view_as_complex(d_a.cpu().double()).numpy()
+    cb = torch.view_as_complex(d_b.cpu().double()).numpy()
+    want = np.einsum("bmk,bnk->bmn", ca, cb)
+    got = results[0].cpu().double().numpy()
+    got = got[:, 0] + 1j * got[:, 1]
+    # fp32 sums of 2 K products, then one rounding to the type of C
+    eps = {VT.float32: 0.0, VT.float16: 2.0 ** -11, VT.bfloat16: 2.0 ** -8}[tout]
+    sums = np.einsum("bmk,bnk->bmn", np.abs(ca), np.abs(cb))
+    assert (np.abs(got - want) <= 2 * K * 2.0 ** -23 * sums + 2 * eps * np.abs(want) + 1e-7).all()
