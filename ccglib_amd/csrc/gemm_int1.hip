@@ -214,11 +214,19 @@ __device__ __forceinline__ unsigned nonzero_bits_transposed(uint4_t v) {
   return (t & 0xffu) | ((t >> 8) & 0xff00u);
 }
 
+// The operands of one launch: blocks below first_blocks along y pack the first one, the
+// others the second. Only rows that exist are packed: what the rest of a row tile holds reaches
+// no element of C.
+struct PackOperands {
+  const unsigned char *src[2];
+  char *dst[2];
+  unsigned rows[2], row_tiles[2];
+  unsigned first_blocks;
+};
+
 constexpr int kPackLoads = 4;   // loads in flight per thread (two rows each per wave)
 template <bool VEC>
-__global__ __launch_bounds__(256) void pack_bytes_to_tiles(const unsigned char *__restrict__ src,
-                                                           char *__restrict__ dst, unsigned rows,
-                                                           unsigned row_tiles, unsigned k,
+__global__ __launch_bounds__(256) void pack_bytes_to_tiles(const PackOperands ops, unsigned k,
                                                            unsigned k1_tiles) {
   // blockIdx: x = four K tiles of 512 samples (one per wave: a block reads 2 KiB
   // contiguous of each of its rows), y = block of 2 kPackLoads rows, z = (batch, plane)
@@ -226,14 +234,19 @@ __global__ __launch_bounds__(256) void pack_bytes_to_tiles(const unsigned char *
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned p = lane & 31;                 // 16-byte piece of the 512 samples of a tile row
   constexpr unsigned RPW = 2 * kPackLoads, WPT = kTileRows / RPW;   // rows per wave, waves per tile
-  const unsigned rt = blockIdx.y / WPT;
+  const bool second = blockIdx.y >= ops.first_blocks;
+  const unsigned char *src = ops.src[second];
+  char *dst = ops.dst[second];
+  const unsigned rows = ops.rows[second], row_tiles = ops.row_tiles[second];
+  const unsigned block_y = blockIdx.y - (second ? ops.first_blocks : 0);
+  const unsigned rt = block_y / WPT;
   const size_t b = blockIdx.z >> 1;
   const unsigned plane = blockIdx.z & 1;
   const unsigned kt = blockIdx.x * 4 + wave;
   if (kt >= k1_tiles) return;
   const unsigned k0 = kt * 512 + p * 16;
-  const unsigned row0_in_tile = (blockIdx.y % WPT) * RPW + (lane >> 5);   // + 2 i
-  const unsigned block_row0 = rt * kTileRows + (blockIdx.y % WPT) * RPW;
+  const unsigned row0_in_tile = (block_y % WPT) * RPW + (lane >> 5);   // + 2 i
+  const unsigned block_row0 = rt * kTileRows + (block_y % WPT) * RPW;
   unsigned half[kPackLoads];
   // the same for all threads of a wave: all its rows and all 512 samples exist
   if (VEC && block_row0 + RPW <= rows && kt * 512 + 512 <= k) {
@@ -343,17 +356,20 @@ __device__ __forceinline__ unsigned pair_bits(uint4_t v) {
 
 constexpr unsigned kPairRowsPerWave = 8;
 template <bool VEC>
-__global__ __launch_bounds__(256) void pack_pairs_to_tiles(const unsigned char *__restrict__ src,
-                                                           char *__restrict__ dst, unsigned rows,
-                                                           unsigned row_tiles, unsigned k,
+__global__ __launch_bounds__(256) void pack_pairs_to_tiles(const PackOperands ops, unsigned k,
                                                            unsigned k1_tiles) {
   // blockIdx: x = four K tiles of 512 samples (one per wave: a block reads 4 KiB
   // contiguous of each of its rows), y = block of eight rows, z = batch
   const unsigned lane = threadIdx.x & 63;
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr unsigned RPW = kPairRowsPerWave, WPT = kTileRows / RPW;
-  const unsigned rt = blockIdx.y / WPT;
-  const unsigned row0_in_tile = (blockIdx.y % WPT) * RPW;
+  const bool second = blockIdx.y >= ops.first_blocks;
+  const unsigned char *src = ops.src[second];
+  char *dst = ops.dst[second];
+  const unsigned rows = ops.rows[second], row_tiles = ops.row_tiles[second];
+  const unsigned block_y = blockIdx.y - (second ? ops.first_blocks : 0);
+  const unsigned rt = block_y / WPT;
+  const unsigned row0_in_tile = (block_y % WPT) * RPW;
   const size_t b = blockIdx.z;
   const unsigned kt = blockIdx.x * 4 + wave;
   if (kt >= k1_tiles) return;
@@ -415,31 +431,40 @@ hipError_t launch_gemm_int1_from_bytes(const GemmParams &p, hipStream_t stream) 
   const unsigned k1_tiles = (unsigned)ceil_div(p.k, 512);
   const size_t x_bytes = (size_t)p.batch * p.x_tiles * k1_tiles * kTileBytes;
   char *ws_x = static_cast<char *>(p.workspace), *ws_y = ws_x + x_bytes;
-  for (int which = 0; which < 2; ++which) {
-    const unsigned rows = which ? p.ny : p.nx, row_tiles = which ? p.y_tiles : p.x_tiles;
-    const unsigned char *src = static_cast<const unsigned char *>(which ? p.y : p.x);
-    if (p.input_interleaved) {
-      // (re, im) byte pairs
-      const dim3 grid((unsigned)ceil_div(k1_tiles, 4), (kTileRows / kPairRowsPerWave) * row_tiles, p.batch);
-      const bool vec = (p.k % 8 == 0) && ((uintptr_t)src % 16 == 0);
-      if (vec) {
-        hipLaunchKernelGGL(pack_pairs_to_tiles<true>, grid, dim3(256), 0, stream, src,
-                           which ? ws_y : ws_x, rows, row_tiles, p.k, k1_tiles);
-      } else {
-        hipLaunchKernelGGL(pack_pairs_to_tiles<false>, grid, dim3(256), 0, stream, src,
-                           which ? ws_y : ws_x, rows, row_tiles, p.k, k1_tiles);
-      }
-      continue;
-    }
-    const dim3 grid((unsigned)ceil_div(k1_tiles, 4), (kTileRows / (2 * kPackLoads)) * row_tiles, 2 * p.batch);
-    const bool vec = (p.k % 16 == 0) && ((uintptr_t)src % 16 == 0);
-    if (vec) {
-      hipLaunchKernelGGL(pack_bytes_to_tiles<true>, grid, dim3(256), 0, stream, src,
-                         which ? ws_y : ws_x, rows, row_tiles, p.k, k1_tiles);
-    } else {
-      hipLaunchKernelGGL(pack_bytes_to_tiles<false>, grid, dim3(256), 0, stream, src,
-                         which ? ws_y : ws_x, rows, row_tiles, p.k, k1_tiles);
-    }
+  const unsigned rows_per_block = p.input_interleaved ? kPairRowsPerWave : 2 * kPackLoads;
+  PackOperands ops;
+  ops.src[0] = static_cast<const unsigned char *>(p.x);
+  ops.src[1] = static_cast<const unsigned char *>(p.y);
+  ops.dst[0] = ws_x;
+  ops.dst[1] = ws_y;
+  ops.rows[0] = p.nx;
+  ops.rows[1] = p.ny;
+  ops.row_tiles[0] = p.x_tiles;
+  ops.row_tiles[1] = p.y_tiles;
+  const unsigned blocks[2] = {(unsigned)ceil_div(p.nx, rows_per_block),
+                              (unsigned)ceil_div(p.ny, rows_per_block)};
+  // (whole 16-byte pieces: 16 samples, or 8 pairs)
+  const bool k_ok = p.k % (p.input_interleaved ? 8 : 16) == 0;
+  const bool vec[2] = {k_ok && (uintptr_t)p.x % 16 == 0, k_ok && (uintptr_t)p.y % 16 == 0};
+  auto launch = [&](unsigned grid_y, bool wide) {
+    const dim3 grid((unsigned)ceil_div(k1_tiles, 4), grid_y, (p.input_interleaved ? 1 : 2) * p.batch);
+    if (grid_y == 0) return;
+    auto kernel = p.input_interleaved ? (wide ? pack_pairs_to_tiles<true> : pack_pairs_to_tiles<false>)
+                                      : (wide ? pack_bytes_to_tiles<true> : pack_bytes_to_tiles<false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, ops, p.k, k1_tiles);
+  };
+  // Both operands in one launch (a small 1-bit product is mostly its launches: B=1 32x32x512,
+  // 128 x 128 blocks, 11.1 -> 9.1 us; B=256 32x700x640, where most of a row tile is padding
+  // that was written as well, 237 -> 203 us),
+  // unless only one of them can be read in 16-byte pieces or the grid would be too high.
+  if (vec[0] == vec[1] && blocks[0] + blocks[1] <= 65535) {
+    ops.first_blocks = blocks[0];
+    launch(blocks[0] + blocks[1], vec[0]);
+  } else {
+    ops.first_blocks = blocks[0];
+    launch(blocks[0], vec[0]);
+    ops.first_blocks = 0;
+    launch(blocks[1], vec[1]);
   }
   if (hipError_t e = hipGetLastError()) return e;
   GemmParams q = p;

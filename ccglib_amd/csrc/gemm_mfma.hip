@@ -631,6 +631,39 @@ __device__ __forceinline__ void mma_step32_bits(const char *slot, const int (&x_
 #undef CCGLIB_PIN
 }
 
+// The same for a wave with one 32 x 32 tile. Every word is expanded for a single tile
+// here, so the vector ALU has about as much to do as the matrix cores; the order of
+// the instructions is left to the compiler.
+template <int BX, int BY, typename Mid>
+__device__ __forceinline__ void mma_step32_bits_single(const char *slot, const int (&x_off)[2],
+                                                       const int (&y_off)[2],
+                                                       float16_t_ (&acc_re)[1][1],
+                                                       float16_t_ (&acc_im)[1][1], Mid &&mid) {
+  constexpr int XP = BX * kTileRowBytes, YP = BY * kTileRowBytes;
+  int4_t xr[2], xi[2], yr[2], yi[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    xr[u] = *reinterpret_cast<const int4_t *>(slot + x_off[u]);
+    yr[u] = *reinterpret_cast<const int4_t *>(slot + y_off[u]);
+    yi[u] = *reinterpret_cast<const int4_t *>(slot + y_off[u] + YP);
+    xi[u] = *reinterpret_cast<const int4_t *>(slot + x_off[u] + XP);
+  }
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int u = s >> 2, w = s & 3;
+    const int4_t x0 = expand_bits(xr[u][w]), x1 = expand_bits(xi[u][w]);
+    const int4_t y0 = expand_bits(yr[u][w]), y1 = expand_bits(yi[u][w]);
+    int4_t y1n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y1n[e] = y1[e] ^ (int)0x88888888u;
+    acc_re[0][0] = mfma_fp4(x0, y0, acc_re[0][0]);
+    acc_im[0][0] = mfma_fp4(x0, y1, acc_im[0][0]);
+    acc_re[0][0] = mfma_fp4(x1, y1n, acc_re[0][0]);
+    acc_im[0][0] = mfma_fp4(x1, y0, acc_im[0][0]);
+    if (s == 0) mid();
+  }
+}
+
 // The same for interleaved operands (rows of (re, im) pairs, as the caller's
 // buffers hold them). With K running over the 2K real numbers of a row,
 //   Re = sum X~ . Y1,  Y1 = (yr, -yi, ...)   and   Im = sum X~ . Y2,  Y2 = (yi, yr, ...)
@@ -858,6 +891,40 @@ __device__ __forceinline__ void mma_step32_interleaved(const char *slot, const i
     CCGLIB_PIN;
   }
 #undef CCGLIB_PIN
+}
+
+// The same for a wave with one 32 x 32 tile, in the order of the sums above.
+template <int DT, typename Mid>
+__device__ __forceinline__ void mma_step32_interleaved_single(const char *slot, const int (&x_off)[2][2],
+                                                              const int (&y_off)[2][2],
+                                                              float16_t_ (&acc_re)[1][1],
+                                                              float16_t_ (&acc_im)[1][1], Mid &&mid) {
+  static_assert(DtypeTraits<DT>::kElemBytes == 1, "8-bit input");
+  Fragment32 x[2], raw[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      x[h].v[u] = *reinterpret_cast<const int4_t *>(slot + x_off[h][u]);
+      raw[h].v[u] = *reinterpret_cast<const int4_t *>(slot + y_off[h][u]);
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    Fragment32 ya, yb;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const unsigned v = (unsigned)raw[h].v[u][w];
+        ya.v[u][w] = (int)(v ^ 0x80008000u);                               // (yr, -yi, ...)
+        yb.v[u][w] = (int)__builtin_amdgcn_perm(v, v, 0x02030001u);        // (yi, yr, ...)
+      }
+    }
+    acc_re[0][0] = mfma32<DT>(x[h], ya, acc_re[0][0]);
+    acc_im[0][0] = mfma32<DT>(x[h], yb, acc_im[0][0]);
+    if (h == 0) mid();
+  }
 }
 
 // Wide accesses to C at an address that is aligned to its elements only: rows of any
@@ -1823,7 +1890,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       } else {
         const char *slot_ptr = lds + x_slot_off(x_slot);
-        if constexpr (IL && MS == 32) {
+        if constexpr (IL && MS == 32 && TX == 1 && TY == 1) {
+          mma_step32_interleaved_single<DT>(slot_ptr, xil32_off, yil32_off, acc_re, acc_im,
+                                            refill_slots);
+        } else if constexpr (IL && MS == 32) {
           static_assert(TX == 2 && TY == 2, "2 x 2 tiles of 32 x 32 per wave");
           mma_step32_interleaved<DT, BX, BY>(slot_ptr, xil32_off, yil32_off, acc_re, acc_im,
                                              refill_slots);
@@ -1835,7 +1905,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
                                                    refill_slots);
         } else {
           const char *tile[KPM] = {slot_ptr};
-          if constexpr (DT == kInt1) {
+          if constexpr (DT == kInt1 && TX == 1 && TY == 1) {
+            mma_step32_bits_single<BX, BY>(tile[0], x32_off, y32_off, acc_re, acc_im, refill_slots);
+          } else if constexpr (DT == kInt1) {
             static_assert(MS == 32 && TX == 2 && TY == 2, "2 x 2 tiles of 32 x 32 per wave");
             mma_step32_bits<BX, BY>(tile[0], x32_off, y32_off, acc_re, acc_im, refill_slots);
           } else if constexpr (MS == 32 && TX == 2 && TY == 2) {
@@ -2092,8 +2164,10 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 //   32 bits (bound by the matrix cores at any of the shapes), 4096x4096x512:  493, 508,
 //            516 us;   B=2 1000^3:  483, 251, 145 us
 //   8 bits (with their transposes), 4096x4096x512:  57, 57, 76 us;   1024^3:  33, 29, 20 us.
-// Two 64 x 64 blocks share a unit. With 32-bit input they take turns on the matrix
-// cores and a unit's tiles simply add up; below that one block alone leaves them idle
+//   1 bit (with the packing), 64x64x65536:  534, 311, 122 us;   1024x1024x32768:  299, 185,
+//            95 us;   B=4 1024x1024x8192:  102, 77, 86 us;   B=5 1024x1024x16384:  206, 209, 194 us.
+// Two 64 x 64 blocks share a unit. With 32-bit and 1-bit input, where a K tile is long
+// work, they take turns on the matrix cores and a unit's tiles simply add up; elsewhere one block alone leaves them idle
 // half of the time, and an odd tile costs as much as two (B=3 1024^3 16 bits, three tiles a
 // unit: 38 us, 128x128 34 us).
 enum BlockShape { k256x128, k128x128, k64x64 };
@@ -2113,13 +2187,11 @@ inline BlockChoice block_choice(const GemmParams &p) {
   if (p.block_tile == 1) return {k256x128, t256};
   if (p.block_tile == 2) return {k128x128, t128};
   const BlockChoice larger = t128 < t256 ? BlockChoice{k128x128, t128} : BlockChoice{k256x128, t256};
-  // (interleaved 8-bit rows and 1-bit input have no 64 x 64 block: their steps are made for
-  // 2 x 2 tiles of the 32-row MFMA per wave)
-  if (p.type_in == kInt1 || (bits8 && p.input_interleaved)) return larger;
   const size_t n = tiles(64, 64);
-  const bool adds_up = p.type_in == kFloat32 || n <= units;
+  const bool adds_up = p.type_in == kFloat32 || p.type_in == kInt1 || n <= units;
   const double rounds = adds_up ? (double)ceil_div(n, units) : 2.0 * (double)ceil_div(n, 2 * units);
-  const double t64 = rounds * (64 * 64) * (p.type_in == kFloat32 ? 1.06 : 1.5);
+  const double cost_64 = p.type_in == kFloat32 ? 1.06 : p.type_in == kInt1 ? 1.25 : 1.5;
+  const double t64 = rounds * (64 * 64) * cost_64;
   return t64 < larger.time ? BlockChoice{k64x64, t64} : larger;
 }
 
@@ -2173,6 +2245,9 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
       }
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec>(p, stream);
     } else {
+      if (shape == k64x64) {
+        return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 32>(p, stream);
+      }
       if (shape == k128x128) {
         return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadInterleavedVec, 32>(p, stream);
       }
@@ -2294,7 +2369,13 @@ hipError_t launch_gemm_mfma_int1(const GemmParams &p, hipStream_t stream) {
   // packed 1-bit samples expanded in registers; the caller has checked that
   // planar rows are whole aligned 16-byte chunks and that K fits fp32 sums
   if (p.type_out != kInt32 || p.input_interleaved) return hipErrorInvalidValue;
-  if (block_choice(p).shape == k128x128) {
+  const BlockShape shape = block_choice(p).shape;
+  if (shape == k64x64) {
+    return p.variant == kOpt
+               ? launch_dtl<kInt1, kInt32, 64, 64, 32, 32, 5, 2, kLoadTiled, 32>(p, stream)
+               : launch_dtl<kInt1, kInt32, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 32>(p, stream);
+  }
+  if (shape == k128x128) {
     return p.variant == kOpt
                ? launch_dtl<kInt1, kInt32, 128, 128, 64, 64, 2, 2, kLoadTiled, 32>(p, stream)
                : launch_dtl<kInt1, kInt32, 128, 128, 64, 64, 2, 2, kLoadPlanarVec, 32>(p, stream);

@@ -87,8 +87,7 @@ CCGLIB_API const char *ccglib_version(void);
  *   GEMM_BLOCK_TILE  0 (default): GEMMs on tiled or whole-chunk planar
  *                    operands use 256 x 128 block tiles, 128 x 128 ones when
  *                    the larger would leave compute units idle (small
- *                    problems), 64 x 64 ones when those would too (8-, 16- and
- *                    32-bit input), or 192 x 256 ones (16-bit tiled input, planar C
+ *                    problems), 64 x 64 ones when those would too, or 192 x 256 ones (16-bit tiled input, planar C
  *                    without beta, M and N multiples of 64, K of more
  *                    than 32) when those fill the compute units well enough;
  *                    1: always 256 x 128; 2: always 128 x 128; 3: 192 x 256

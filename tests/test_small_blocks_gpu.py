@@ -5,7 +5,7 @@ import pytest
 
 import ccglib_amd as cc
 from gpu_util import stream
-from test_gemm_gpu import COL, INTERLEAVED, PLANAR, ROW, float_case, quantize, run_gemm
+from test_gemm_gpu import COL, INTERLEAVED, PLANAR, ROW, float_case, int1_case, quantize, run_gemm
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +85,63 @@ def test_64x64_blocks_on_interleaved_rows(B, M, N, K, tin, tout):
     eps = {VT.float32: 0.0, VT.float16: 2.0 ** -11, VT.bfloat16: 2.0 ** -8}[tout]
     sums = np.einsum("bmk,bnk->bmn", np.abs(ca), np.abs(cb))
     assert (np.abs(got - want) <= 2 * K * 2.0 ** -23 * sums + 2 * eps * np.abs(want) + 1e-7).all()
+
+
+@pytest.mark.parametrize("variant", [cc.Variant.basic, cc.Variant.opt])
+@pytest.mark.parametrize("B,M,N,K", [(1, 1, 1, 128), (2, 64, 64, 512), (2, 63, 65, 1152), (1, 129, 190, 4224),
+                                     (70, 180, 190, 640)])   # (the last: several tiles a block)
+def test_64x64_blocks_int1(B, M, N, K, variant):
+    assert takes_64(B, M, N, K, VT.int1, VT.int32, variant)
+    int1_case(B, M, N, K, variant, seed=1)
+    int1_case(B, M, N, K, variant, c_order=COL, alpha=2 - 1j, beta=1 + 3j, seed=2)
+    if variant == cc.Variant.opt:
+        int1_case(B, M, N, K, variant, c_axis=INTERLEAVED, seed=3)
+
+
+@pytest.mark.parametrize("axis", [PLANAR, INTERLEAVED])
+@pytest.mark.parametrize("offsets", [(0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("B,M,N,K", [(1, 1, 7, 32), (3, 129, 40, 544), (2, 8, 300, 1024)])
+def test_packing_of_both_operands(B, M, N, K, offsets, axis):
+    """Raw samples at any address: both operands in one launch, or one each where only one of them
+    is aligned; row counts below, at and above a block of rows and a row tile."""
+    import torch
+    rng = np.random.default_rng(7)
+    planes, device = [], []
+    for rows, offset in ((M, offsets[0]), (N, offsets[1])):
+        x = rng.integers(0, 2, (B, 2, rows, K), dtype=np.uint8)
+        planes.append(2 * x.astype(np.int64) - 1)
+        raw = np.ascontiguousarray(x if axis == PLANAR else x.transpose(0, 2, 3, 1)).reshape(-1)
+        buffer = torch.zeros(raw.size + 16, dtype=torch.uint8, device="cuda")
+        buffer[offset:offset + raw.size] = torch.from_numpy(raw).cuda()
+        device.append(buffer)
+    c = torch.zeros((B, 2, M, N), dtype=torch.int32, device="cuda")
+    pipe = cc.Pipeline(B, M, N, K, 0, stream(), axis, PLANAR, ROW, COL, ROW, VT.int1, VT.int32,
+                       cc.Variant.opt)
+    pipe.Run(device[0].data_ptr() + offsets[0], device[1].data_ptr() + offsets[1], c.data_ptr())
+    torch.cuda.synchronize()
+    (ar, ai), (br, bi) = [(p[:, 0], p[:, 1]) for p in planes]
+    brt, bit = br.transpose(0, 2, 1), bi.transpose(0, 2, 1)
+    want = np.stack([ar @ brt - ai @ bit, ar @ bit + ai @ brt], axis=1)
+    assert np.array_equal(c.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("tin", [VT.float8e4m3, VT.float8e5m2])
+@pytest.mark.parametrize("B,M,N,K", [(1, 1, 3, 8), (2, 63, 65, 200), (200, 100, 40, 136), (256, 64, 64, 512)])
+def test_64x64_blocks_on_interleaved_bytes(B, M, N, K, tin):
+    """The pipeline's (re, im) rows of 8-bit samples: the same bits as the 128 x 128 block."""
+    import torch
+    tdt = torch.float8_e4m3fn if tin == VT.float8e4m3 else torch.float8_e5m2
+    gen = torch.Generator().manual_seed(8)
+    a = torch.randn((B, M, K, 2), generator=gen).to(tdt).cuda()
+    b = torch.randn((B, N, K, 2), generator=gen).to(tdt).cuda()
+    results = []
+    for block_tile in (0, 2):
+        c = torch.full((B, 2, M, N), float("nan"), device="cuda")
+        with cc.option(cc.Option.gemm_block_tile, block_tile):
+            pipe = cc.Pipeline(B, M, N, K, 0, stream(), INTERLEAVED, PLANAR, ROW, COL, ROW, tin, VT.float32,
+                               cc.Variant.opt)
+        assert pipe.ReadsInPlace()
+        pipe.Run(a.data_ptr(), b.data_ptr(), c.data_ptr())
+        torch.cuda.synchronize()
+        results.append(c)
+    assert torch.isfinite(results[0]).all() and torch.equal(results[0], results[1])
