@@ -2192,6 +2192,7 @@ inline BlockChoice block_choice(const GemmParams &p) {
   const double rounds = adds_up ? (double)ceil_div(n, units) : 2.0 * (double)ceil_div(n, 2 * units);
   const double cost_64 = p.type_in == kFloat32 ? 1.06 : p.type_in == kInt1 ? 1.25 : 1.5;
   const double t64 = rounds * (64 * 64) * cost_64;
+  if (p.block_tile == 4) return {k64x64, t64};
   return t64 < larger.time ? BlockChoice{k64x64, t64} : larger;
 }
 

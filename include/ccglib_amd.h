@@ -87,13 +87,15 @@ CCGLIB_API const char *ccglib_version(void);
  *   GEMM_BLOCK_TILE  0 (default): GEMMs on tiled or whole-chunk planar
  *                    operands use 256 x 128 block tiles, 128 x 128 ones when
  *                    the larger would leave compute units idle (small
- *                    problems), 64 x 64 ones when those would too, or 192 x 256 ones (16-bit tiled input, planar C
- *                    without beta, M and N multiples of 64, K of more
- *                    than 32) when those fill the compute units well enough;
+ *                    problems), 64 x 64 ones when those would too, or
+ *                    192 x 256 ones (16-bit tiled input, planar C without
+ *                    beta, M and N multiples of 64, K of more than 32) when
+ *                    those fill the compute units well enough;
  *                    1: always 256 x 128; 2: always 128 x 128; 3: 192 x 256
- *                    wherever that kernel applies, else as 0. The 192 x 256
- *                    block also serves 16-bit interleaved rows read in place
- *                    (the pipeline) when K is a multiple of 32.
+ *                    wherever that kernel applies, else as 0; 4: always
+ *                    64 x 64. The 192 x 256 block also serves 16-bit
+ *                    interleaved rows read in place (the pipeline) when K is a
+ *                    multiple of 32.
  *   EXPECT_UNALIGNED 0 (default): a basic-variant GEMM that meets operands that
  *                    are not 16-byte aligned allocates its tiled copies at that
  *                    Run, and a pipeline that reads rows in place creates the

@@ -489,14 +489,13 @@ def test_int1_alpha_beta(variant, int1_kernel):
     int1_case(16, 256, 128, 256, variant, alpha=2 - 3j, beta=3 - 2j)
 
 
-# ---- both block tiles of the MFMA kernels ------------------------------------------------
+# ---- the block tiles of the MFMA kernels -------------------------------------------------
 
-@pytest.mark.parametrize("block_tile", [1, 2])
-@pytest.mark.parametrize("tin,tout", [(VT.float16, VT.float32), (VT.bfloat16, VT.bfloat16),
-                                      (VT.float32, VT.float16), (VT.float8e4m3, VT.float32)])
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("tin,tout", FLOAT_PAIRS)
 @pytest.mark.parametrize("variant", [cc.Variant.basic, cc.Variant.opt])
 def test_block_tiles(block_tile, tin, tout, variant):
-    """The dispatch picks 256 x 128 or 128 x 128 block tiles by problem size (option
+    """The dispatch picks 256 x 128, 128 x 128 or 64 x 64 block tiles by problem size (option
     GEMM_BLOCK_TILE = 0); here each is forced in turn on the same problems: one
     partial tile, many tiles with ragged edges, a long K, alpha / beta, column-major
     and (opt) interleaved C."""
@@ -509,7 +508,7 @@ def test_block_tiles(block_tile, tin, tout, variant):
             float_case(3, 257, 129, 72, tin, tout, variant, INTERLEAVED, ROW, alpha=2j, seed=4)
 
 
-@pytest.mark.parametrize("block_tile", [1, 2])
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
 @pytest.mark.parametrize("variant", [cc.Variant.basic, cc.Variant.opt])
 def test_block_tiles_int1(block_tile, variant):
     with cc.option(cc.Option.gemm_block_tile, block_tile):
@@ -574,7 +573,7 @@ def test_block_tile_choice_is_invisible(B, M, N, K, alpha):
     qa = quantize(rng.standard_normal((B, 2, M, K)).astype(np.float32), VT.float16).reshape(-1)
     qb = quantize(rng.standard_normal((B, 2, N, K)).astype(np.float32), VT.float16).reshape(-1)
     results = []
-    for block_tile in (0, 1, 2, 3):
+    for block_tile in (0, 1, 2, 3, 4):
         with cc.option(cc.Option.gemm_block_tile, block_tile):
             results.append(run_gemm(qa, qb, B, M, N, K, VT.float16, VT.float32, cc.Variant.opt, alpha=alpha))
     for r in results[1:]:

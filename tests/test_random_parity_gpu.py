@@ -26,8 +26,12 @@ def interleave(q, B, rows, K):
     return np.ascontiguousarray(q.reshape(B, 2, rows, K).transpose(0, 2, 3, 1)).reshape(-1)
 
 
-@pytest.mark.parametrize("seed", [11, 12, 13, 14])
-def test_random_cases(seed):
+@pytest.mark.parametrize("seed,block_tile", [(11, 0), (12, 0), (13, 0), (14, 0), (11, 1), (12, 2), (13, 1),
+                                             (14, 2), (12, 4)])
+def test_random_cases(seed, block_tile):
+    """By default nearly all of these small problems run on 64 x 64 blocks; the same problems
+    with each of the block shapes forced."""
+    cc.set_option(cc.Option.gemm_block_tile, block_tile)   # (every test starts from the defaults)
     rng = np.random.default_rng(seed)
     for case in range(40):
         tin, tout = PAIRS[rng.integers(len(PAIRS))]
@@ -89,10 +93,12 @@ def _pack_rows(bits, B, rows, K):
     return np.packbits(padded, axis=1, bitorder="little").view(np.uint32).reshape(-1)
 
 
-@pytest.mark.parametrize("seed", [21, 22])
-def test_random_int1_cases(seed):
+@pytest.mark.parametrize("seed,block_tile", [(21, 0), (22, 0), (21, 1), (22, 2)])
+def test_random_int1_cases(seed, block_tile):
     """1-bit GEMM and pipeline, bit-exact: both variants, ragged shapes, integer alpha / beta,
-    and the option that selects the popcount kernel."""
+    the option that selects the popcount kernel, and the block shapes that these small problems
+    do not get by themselves."""
+    cc.set_option(cc.Option.gemm_block_tile, block_tile)
     rng = np.random.default_rng(seed)
     for case in range(40):
         B = int(rng.integers(1, 6))

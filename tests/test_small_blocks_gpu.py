@@ -64,7 +64,7 @@ def test_64x64_blocks_on_interleaved_rows(B, M, N, K, tin, tout):
     tdt = torch.float16 if tin == VT.float16 else torch.bfloat16
     d_a, d_b = torch.from_numpy(a).cuda().to(tdt), torch.from_numpy(b).cuda().to(tdt)
     results = []
-    for block_tile in (0, 2):
+    for block_tile in (4, 2):
         c = torch.full((B, 2, M, N), float("nan"), device="cuda",
                        dtype={VT.float32: torch.float32, VT.float16: torch.float16,
                               VT.bfloat16: torch.bfloat16}[tout])
@@ -128,14 +128,17 @@ def test_packing_of_both_operands(B, M, N, K, offsets, axis):
 @pytest.mark.parametrize("tin", [VT.float8e4m3, VT.float8e5m2])
 @pytest.mark.parametrize("B,M,N,K", [(1, 1, 3, 8), (2, 63, 65, 200), (200, 100, 40, 136), (256, 64, 64, 512)])
 def test_64x64_blocks_on_interleaved_bytes(B, M, N, K, tin):
-    """The pipeline's (re, im) rows of 8-bit samples: the same bits as the 128 x 128 block."""
+    """The pipeline's (re, im) rows of 8-bit samples: the same bits as the 128 x 128 block, and the
+    product in 64 bits within what the matrix instruction's sums of 64 lose (four times the largest
+    relative error, 1.5e-5, and the largest difference, 8.4e-5 of the root mean square, measured on
+    8-bit products of K up to 8192)."""
     import torch
     tdt = torch.float8_e4m3fn if tin == VT.float8e4m3 else torch.float8_e5m2
     gen = torch.Generator().manual_seed(8)
     a = torch.randn((B, M, K, 2), generator=gen).to(tdt).cuda()
     b = torch.randn((B, N, K, 2), generator=gen).to(tdt).cuda()
     results = []
-    for block_tile in (0, 2):
+    for block_tile in (4, 2):
         c = torch.full((B, 2, M, N), float("nan"), device="cuda")
         with cc.option(cc.Option.gemm_block_tile, block_tile):
             pipe = cc.Pipeline(B, M, N, K, 0, stream(), INTERLEAVED, PLANAR, ROW, COL, ROW, tin, VT.float32,
@@ -144,4 +147,12 @@ def test_64x64_blocks_on_interleaved_bytes(B, M, N, K, tin):
         pipe.Run(a.data_ptr(), b.data_ptr(), c.data_ptr())
         torch.cuda.synchronize()
         results.append(c)
-    assert torch.isfinite(results[0]).all() and torch.equal(results[0], results[1])
+    assert torch.equal(results[0], results[1])
+    ca = torch.view_as_complex(a.cpu().double()).numpy()
+    cb = torch.view_as_complex(b.cpu().double()).numpy()
+    got = results[0].cpu().double().numpy()
+    got = got[:, 0] + 1j * got[:, 1]
+    want = np.einsum("bmk,bnk->bmn", ca, cb)
+    rms = np.sqrt(np.mean(np.abs(want) ** 2))
+    assert np.linalg.norm(got - want) <= 6e-5 * np.linalg.norm(want)
+    assert (np.abs(got - want) <= 3.5e-4 * np.maximum(rms, np.abs(want))).all()
