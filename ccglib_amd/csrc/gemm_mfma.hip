@@ -2152,48 +2152,69 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 }
 
 // Which block shape of complex_gemm_mfma_dtl a problem gets: the one whose busiest compute
-// unit finishes first by
-//   rounds of tiles over the units * area of a tile * cost per element of C.
-// The smaller a block, the more of the chip a small problem fills and the less it
-// computes beyond the edges of C, but the more bytes it moves from L2 to LDS per flop; the
-// cost is what that measured once every unit is busy, relative to 256 x 128:
-//   16 bits, 4096x4096x512:  256x128 76 us, 128x128 91 us, 64x64 102 us;
-//            B=5 1024^3:     49, 65, 59 us;
-//            B=256 96x96x1024 (256 tiles of either larger shape):  70, 40, 52 us;
-//            B=16 255x128x256:  26, 17, 10 us;   256^3:  14.8, 12.5, 7.6 us
-//   32 bits (bound by the matrix cores at any of the shapes), 4096x4096x512:  493, 508,
-//            516 us;   B=2 1000^3:  483, 251, 145 us
-//   8 bits (with their transposes), 4096x4096x512:  57, 57, 76 us;   1024^3:  33, 29, 20 us.
-//   1 bit (with the packing), 64x64x65536:  534, 311, 122 us;   1024x1024x32768:  299, 185,
-//            95 us;   B=4 1024x1024x8192:  102, 77, 86 us;   B=5 1024x1024x16384:  206, 209, 194 us.
-// Two 64 x 64 blocks share a unit. With 32-bit and 1-bit input, where a K tile is long
-// work, they take turns on the matrix cores and a unit's tiles simply add up; elsewhere one block alone leaves them idle
-// half of the time, and an odd tile costs as much as two (B=3 1024^3 16 bits, three tiles a
-// unit: 38 us, 128x128 34 us).
+// unit finishes first, by
+//   tiles of a unit * area of a tile * cost * (64-byte pieces of K + what a tile costs besides),
+// with the costs relative to 256 x 128, where a tile costs as much as 10 pieces of K besides
+// its K loop (ring fill, stores). The smaller a block, the more of the chip a small
+// problem fills and the less it computes beyond the edges of C, but the more bytes it
+// moves per flop. From where they move them decides by how much: contiguous tiles cost a 64 x 64
+// block 1.7 times as much per flop with 8- and 16-bit input, half cache lines of planar rows
+// 2.5 times (fp16 on planar rows, B=157 192x604x3680: 256x128 742 us, 128x128 905, 64x64 1026;
+// B=167 800x184x2064: 584, 674, 884), while 32-bit input is bound by the matrix cores at any shape
+// (4096x4096x512: 493, 508, 516 us) and 1-bit input by the expansion of its words, of which a wave
+// with one tile makes less use (3452x1504x32256: 271, 286, 311).
+//   Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles of 8- and 1-bit input, and
+// a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
+//   With beta the epilogue first reads C, from all its registers' addresses at once, which costs
+// the larger tiles more (fp8 on planar rows, B=11 456x1542x192: 96, 85, 47 us).
+// The constants are fitted, for each type and operand layout, to times of all three shapes over
+// 30000 problems of random sizes, half of them on operands that no cache held
+// (python -m ccglib_amd.tuning.block_choice times such problems): the choice is then on average
+// 0.2 % behind the fastest of the three shapes, and more than 8 % behind in 0.7 % of the problems.
 enum BlockShape { k256x128, k128x128, k64x64 };
 struct BlockChoice {
   BlockShape shape;
-  double time;
+  double time;   // in units of one element of C in a 256 x 128 tile
 };
+struct BlockCosts {
+  double cost_128, cost_64;   // per element of C and piece of K, of 256 x 128's
+  double tile_128, tile_64;   // what a tile costs besides its K loop, in pieces of K
+  double lone_128, lone_64;   // what a tile without a neighbour costs more, of a tile
+  double beta_256, beta_128, beta_64;   // added to the tile's cost with beta
+};
+inline BlockCosts block_costs(const GemmParams &p) {
+  if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0};
+  if (p.type_in == kFloat32) return {1.04, 1.04, 10.3, 10.9, 0.0, 0.0, 0.0, 0.0, 0.0};
+  const bool planar = p.variant == kBasic && !p.input_interleaved;
+  if (bits_of(p.type_in) == 8) {
+    if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0};
+    if (planar) return {1.30, 2.54, 7.6, 7.9, 0.3, 0.1, 13.0, 10.0, 1.0};
+    return {1.05, 1.49, 9.2, 13.6, 0.3, 0.1, 13.0, 10.0, 1.0};
+  }
+  if (p.input_interleaved) return {1.19, 1.90, 11.7, 8.8, 0.0, 0.25, 12.0, 8.0, 6.0};
+  if (planar) return {1.24, 2.58, 12.6, 6.8, 0.0, 0.25, 12.0, 8.0, 6.0};
+  return {1.30, 1.71, 11.0, 10.1, 0.0, 0.25, 12.0, 8.0, 6.0};
+}
 inline BlockChoice block_choice(const GemmParams &p) {
   const size_t units = (size_t)compute_units();
-  auto tiles = [&](size_t bx, size_t by) {
-    return (size_t)p.batch * ceil_div((size_t)p.nx, bx) * ceil_div((size_t)p.ny, by);
+  const BlockCosts costs = block_costs(p);
+  // (pieces of a plane's row: an interleaved row holds both planes)
+  const double pieces = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
+  const double large = pieces + 10.0 + (p.have_beta ? costs.beta_256 : 0.0);
+  auto time = [&](size_t bx, size_t by, double cost, double tile, double lone, double beta) {
+    const size_t tiles = (size_t)p.batch * ceil_div((size_t)p.nx, bx) * ceil_div((size_t)p.ny, by);
+    const size_t mine = ceil_div(tiles, units);
+    return ((double)mine + (mine % 2 ? lone : 0.0)) * (double)(bx * by) * cost *
+           (pieces + tile + (p.have_beta ? beta : 0.0)) / large;
   };
-  const bool bits8 = p.type_in == kFloat8e4m3 || p.type_in == kFloat8e5m2;
-  const double cost_128 = p.type_in == kInt1 ? 1.0 : bits8 || p.type_in == kFloat32 ? 1.05 : 1.25;
-  const double t256 = (double)ceil_div(tiles(256, 128), units) * (256 * 128);
-  const double t128 = (double)ceil_div(tiles(128, 128), units) * (128 * 128) * cost_128;
+  const double t256 = time(256, 128, 1.0, 10.0, 0.0, costs.beta_256);
+  const double t128 = time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
+  const double t64 = time(64, 64, costs.cost_64, costs.tile_64, costs.lone_64, costs.beta_64);
   if (p.block_tile == 1) return {k256x128, t256};
   if (p.block_tile == 2) return {k128x128, t128};
-  const BlockChoice larger = t128 < t256 ? BlockChoice{k128x128, t128} : BlockChoice{k256x128, t256};
-  const size_t n = tiles(64, 64);
-  const bool adds_up = p.type_in == kFloat32 || p.type_in == kInt1 || n <= units;
-  const double rounds = adds_up ? (double)ceil_div(n, units) : 2.0 * (double)ceil_div(n, 2 * units);
-  const double cost_64 = p.type_in == kFloat32 ? 1.06 : p.type_in == kInt1 ? 1.25 : 1.5;
-  const double t64 = rounds * (64 * 64) * cost_64;
   if (p.block_tile == 4) return {k64x64, t64};
-  return t64 < larger.time ? BlockChoice{k64x64, t64} : larger;
+  if (t256 <= t128 && t256 <= t64) return {k256x128, t256};
+  return t128 <= t64 ? BlockChoice{k128x128, t128} : BlockChoice{k64x64, t64};
 }
 
 // Whether the 192 x 256 block of gemm_mfma_wide.h can compute this problem (what
