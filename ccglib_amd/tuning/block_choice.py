@@ -56,16 +56,35 @@ def problem(rng):
         beta = 0 if rng.random() < 0.8 or tin == VT.int1 else 0.25 + 0.5j
         B, M, N = log_size(rng, 1, 256), extent(rng), extent(rng)
         K = (128 if tin == VT.int1 else 16) * log_size(rng, 4, 256)
-        rows = [M, N]
-        k = K
-        if layout == "tiled":
-            mb, nb, kc = cc.GEMM.GetDimensions(cc.Precision(tin, tout))
-            rows = [cc.ceildiv(M, mb) * mb, cc.ceildiv(N, nb) * nb]
-            k = cc.ceildiv(K, kc) * kc
-        sizes = [B * 2 * r * k * BITS[tin] // 8 for r in rows] + [B * 2 * M * N * BITS[tout] // 8]
+        sizes = bytes_of(tin, tout, layout, B, M, N, K)
         if (8 * B * M * N * K / RATE[tin] <= 1.5e-3 and max(sizes) <= POOL_BYTES and
                 B * cc.ceildiv(M, 128) * cc.ceildiv(N, 256) <= 1536):
             return (tin, tout, layout, c_axis, alpha, beta, B, M, N, K), sizes
+
+
+def bytes_of(tin, tout, layout, B, M, N, K):
+    """Bytes of A, B and C as the GEMM reads and writes them."""
+    rows, k = [M, N], K
+    if layout == "tiled":
+        mb, nb, kc = cc.GEMM.GetDimensions(cc.Precision(tin, tout))
+        rows, k = [cc.ceildiv(M, mb) * mb, cc.ceildiv(N, nb) * nb], cc.ceildiv(K, kc) * kc
+    return [B * 2 * r * k * BITS[tin] // 8 for r in rows] + [B * 2 * M * N * BITS[tout] // 8]
+
+
+# the problems that the comment of block_choice quotes
+NAMED = [(VT.float16, VT.float32, "tiled", 0, 1, 4096, 4096, 512),
+         (VT.float16, VT.float32, "tiled", 0, 5, 1024, 1024, 1024),
+         (VT.float16, VT.float32, "tiled", 0, 256, 96, 96, 1024),
+         (VT.float16, VT.float32, "tiled", 0, 1, 256, 256, 256),
+         (VT.float16, VT.float16, "planar", 0, 167, 800, 184, 2064),
+         (VT.float16, VT.float32, "planar", 0, 157, 192, 604, 3680),
+         (VT.float32, VT.float32, "tiled", 0, 1, 4096, 4096, 512),
+         (VT.float32, VT.float32, "tiled", 0, 2, 1000, 1000, 1000),
+         (VT.float8e4m3, VT.float32, "tiled", 0, 1, 4096, 4096, 512),
+         (VT.float8e4m3, VT.float32, "tiled", 0, 1, 1024, 1024, 1024),
+         (VT.float8e4m3, VT.float32, "planar", 0.25 + 0.5j, 11, 456, 1542, 192),
+         (VT.int1, VT.int32, "tiled", 0, 1, 3452, 1504, 32256),
+         (VT.int1, VT.int32, "tiled", 0, 1, 64, 64, 65536)]
 
 
 _pools = {}
@@ -137,6 +156,13 @@ def main():
     ap.add_argument("--warm", action="store_true")
     ap.add_argument("--csv")
     args = ap.parse_args()
+    print("us: 256x128, 128x128, 64x64 on cold operands; on warm ones; default (warm)")
+    for tin, tout, layout, beta, B, M, N, K in NAMED:
+        case = (tin, tout, layout, AX.complex_planar, 1, beta, B, M, N, K)
+        cold, warm = (measure(case, bytes_of(tin, tout, layout, B, M, N, K), w) for w in (False, True))
+        print("%-52s %8.1f %8.1f %8.1f   %8.1f %8.1f %8.1f   %8.1f" % (
+            "%s->%s %s%s B=%d %dx%dx%d" % (tin.name, tout.name, layout, " beta" if beta else "", B, M, N, K),
+            cold[1], cold[2], cold[4], warm[1], warm[2], warm[4], warm[0]), flush=True)
     rng = random.Random(args.seed)
     groups, worst = collections.defaultdict(list), []
     csv = open(args.csv, "w") if args.csv else None

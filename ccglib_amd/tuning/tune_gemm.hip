@@ -32,10 +32,16 @@
 // kernels one works on most - for a build of under a minute.
 #ifdef TUNE_GEMM_SMALL
 #define CCGLIB_GEMM_MFMA_PART 99   // none of the library's own instantiations
+#else
+#define CCGLIB_GEMM_MFMA_PART 5    // of the library's own instantiations those behind gemm_int1.hip
 #endif
 #include "../csrc/gemm_mfma.hip"
 #ifndef TUNE_GEMM_SMALL
 #include "../csrc/gemm_int1.hip"
+// (the dispatch over all input types, which only the 1-bit launcher calls here)
+hipError_t ccglib_amd::launch_gemm_mfma(const GemmParams &p, hipStream_t stream) {
+  return p.type_in == kInt1 ? launch_gemm_mfma_int1(p, stream) : hipErrorInvalidValue;
+}
 #endif
 
 #include <hip/hip_fp8.h>
@@ -104,6 +110,13 @@ static const std::vector<Config> kConfigs = {
     {"f16 256x128 w64x64 s3 m32", launch_dtl<kFloat16, kFloat32, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>, kFloat16, kFloat32},
     {"f16 128x128 w64x64 s2 m16", launch_dtl<kFloat16, kFloat32, 128, 128, 64, 64, 2, 2, kLoadTiled, 16>, kFloat16, kFloat32},
     {"f16 128x128 w64x32 s4 m16", launch_dtl<kFloat16, kFloat32, 128, 128, 64, 32, 4, 2, kLoadTiled, 16>, kFloat16, kFloat32},
+    {"f16 64x64 w32x32 s5 m16", launch_dtl<kFloat16, kFloat32, 64, 64, 32, 32, 5, 2, kLoadTiled, 16>, kFloat16, kFloat32},
+    {"f32 64x64 w32x32 s5 m16", launch_dtl<kFloat32, kFloat32, 64, 64, 32, 32, 5, 2, kLoadTiled, 16>, kFloat32, kFloat32},
+    {"fp8 64x64 w32x32 s5 m32", launch_dtl<kFloat8e4m3, kFloat32, 64, 64, 32, 32, 5, 2, kLoadTiled, 32>, kFloat8e4m3, kFloat32},
+    {"int1 64x64 w32x32 s5 m32", launch_dtl<kInt1, kInt32, 64, 64, 32, 32, 5, 2, kLoadTiled, 32>, kInt1, kInt32},
+    {"f16 planar 64x64 w32x32 s5 m16", launch_dtl<kFloat16, kFloat32, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 16>, kFloat16, kFloat32, kLoadPlanarVec},
+    {"f16 interleaved 64x64 w32x32 s5 m16", launch_dtl<kFloat16, kFloat32, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 16>, kFloat16, kFloat32, kLoadInterleavedVec},
+    {"fp8 interleaved 64x64 w32x32 s5 m32", launch_dtl<kFloat8e4m3, kFloat32, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 32>, kFloat8e4m3, kFloat32, kLoadInterleavedVec},
     {"f32 256x128 w64x64 s3 m16", launch_dtl<kFloat32, kFloat32, 256, 128, 64, 64, 3, 2, kLoadTiled, 16>, kFloat32, kFloat32},
     {"fp8 256x128 w64x64 s3 m32", launch_dtl<kFloat8e4m3, kFloat32, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>, kFloat8e4m3, kFloat32},
     {"fp8 128x128 w64x64 s2 m32", launch_dtl<kFloat8e4m3, kFloat32, 128, 128, 64, 64, 2, 2, kLoadTiled, 32>, kFloat8e4m3, kFloat32},
@@ -287,6 +300,39 @@ __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void probe_mfma(const int4_t
   out[blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
 
+// The same for the 32x32x64 instruction on 8-bit (e4m3) operands and on the +-1 fp4 values
+// that 1-bit samples become.
+template <bool FP4, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES / 4) void probe_mfma_narrow(const int4_t *in, float *out, int iters) {
+  Fragment32 a[4], b[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      a[i].v[u] = in[(threadIdx.x % 64) * 16 + 2 * i + u];
+      b[i].v[u] = in[(threadIdx.x % 64) * 16 + 8 + 2 * i + u];
+    }
+    if (FP4) {
+      a[i].v[0] = expand_bits((unsigned)a[i].v[0][0]);
+      b[i].v[0] = expand_bits((unsigned)b[i].v[0][0]);
+    }
+  }
+  float16_t_ acc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+  for (int it = 0; it < iters; ++it) {
+#pragma unroll
+    for (int n = 0; n < 64; ++n) {
+      const int i = n % 4, j = (n / 4) % 4;
+      acc[n % 8] = FP4 ? mfma_fp4(a[i].v[0], b[j].v[0], acc[n % 8]) : mfma32<kFloat8e4m3>(a[i], b[j], acc[n % 8]);
+    }
+  }
+  float s = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s += acc[i][0] + acc[i][3];
+  out[blockIdx.x * blockDim.x + threadIdx.x] = s;
+}
+
 // What an instruction between two 16x16x32 MFMAs costs one wave per SIMD. MODE 0:
 // none; 1 / 2: one / two vector-ALU instructions behind every MFMA; 3: four in a row
 // behind every fourth; 4: a ds_read_b128 behind every eighth; 5: a 1 KiB global ->
@@ -394,6 +440,17 @@ static int run_probe(const std::string &probe, const std::string &fill) {
     run("16x16x32, 2 waves per SIMD", probe_mfma<16, 8>, 8, 2.0 * 16 * 16 * 32);
     run("32x32x16, 1 wave per SIMD", probe_mfma<32, 4>, 4, 2.0 * 32 * 32 * 16);
     run("32x32x16, 2 waves per SIMD", probe_mfma<32, 8>, 8, 2.0 * 32 * 32 * 16);
+    auto run_narrow = [&](const char *name, auto kernel, int waves, double peak) {
+      const float ms = time_launches([&] { hipLaunchKernelGGL(kernel, dim3(256), dim3(64 * waves), 0, 0, in, out, iters); }, 10);
+      const double tflops = 64.0 * 2.0 * 32 * 32 * 64 * iters * waves * 256 / (ms * 1e-3) / 1e12;
+      std::printf("%-32s %8.3f ms %8.1f TFLOP/s  %5.1f%% of %.1f\n", name, ms, tflops, 100 * tflops / peak, peak);
+    };
+    if (fill != "zero") fill_baseline(in, 1 << 20, kFloat8e4m3, kLoadInterleavedVec, 1, false, 7);
+    run_narrow("fp8 32x32x64, 1 wave per SIMD", probe_mfma_narrow<false, 4>, 4, 5033.2);
+    run_narrow("fp8 32x32x64, 2 waves per SIMD", probe_mfma_narrow<false, 8>, 8, 5033.2);
+    if (fill != "zero") fill_baseline(in, 1 << 20, kInt1, kLoadInterleavedVec, 1, false, 7);
+    run_narrow("+-1 fp4 32x32x64, 1 wave/SIMD", probe_mfma_narrow<true, 4>, 4, 10066.3);
+    run_narrow("+-1 fp4 32x32x64, 2 waves/SIMD", probe_mfma_narrow<true, 8>, 8, 10066.3);
   } else if (probe == "mix") {
     std::printf("one wave per SIMD issuing 16x16x32 MFMAs and, between them (%s operands):\n", fill.c_str());
     auto run = [&](const char *name, auto kernel) {
