@@ -931,7 +931,8 @@ __device__ __forceinline__ void mma_step32_interleaved_single(const char *slot, 
 // length start anywhere, and global memory takes any alignment on this target. Element
 // by element, every store instruction touches 64 lines for 4 bytes each: B=16 255x128x256
 // bf16 with beta and rows of 255 took 30.2 us instead of 17.2, B=16 300x3001x577 fp16 to
-// (re, im) rows of 3001 pairs 158.5 instead of 144.7 (with its transposes).
+// (re, im) rows of 3001 pairs 158.5 instead of 144.7 (with its transposes). (1-bit C is
+// stored like this, but with beta still read element by element.)
 typedef float4_t float4_any_t __attribute__((aligned(4)));
 typedef int4_t int4_any_t __attribute__((aligned(2)));
 typedef ushort4_t ushort4_any_t __attribute__((aligned(2)));
@@ -2157,18 +2158,25 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // with the costs relative to 256 x 128, where a tile costs as much as 10 pieces of K besides
 // its K loop (ring fill, stores). The smaller a block, the more of the chip a small
 // problem fills and the less it computes beyond the edges of C, but the more bytes it
-// moves per flop. From where they move them decides by how much: contiguous tiles cost a 64 x 64
-// block 1.7 times as much per flop with 8- and 16-bit input, half cache lines of planar rows
-// 2.5 times (fp16 on planar rows, B=157 192x604x3680: 256x128 742 us, 128x128 905, 64x64 1026;
-// B=167 800x184x2064: 584, 674, 884), while 32-bit input is bound by the matrix cores at any shape
-// (4096x4096x512: 493, 508, 516 us) and 1-bit input by the expansion of its words, of which a wave
-// with one tile makes less use (3452x1504x32256: 271, 286, 311).
-//   Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles of 8- and 1-bit input, and
+// moves per flop. Times with 256 x 128, 128 x 128 and 64 x 64 blocks in us, on operands that no cache
+// held (profiles/gemm_block_choice.txt):
+//   too few tiles for the larger blocks, 16 bits 256^3:  14.7, 12.5, 6.9;  B=256 96x96x1024:  86, 56, 62;
+//     32 bits B=2 1000^3:  455, 239, 135;  8 bits 1024^3:  24.9, 22.3, 11.5;
+//     1 bit 64x64x65536:  526, 305, 116
+//   every unit busy, 16 bits on tiles, 4096x4096x512:  68, 89, 102
+//     on planar rows, of which a copy fetches half cache lines, B=157 192x604x3680:  747, 909, 1026
+//     32 bits (bound by the matrix cores at any shape), 4096x4096x512:  480, 495, 503
+//     8 bits on tiles, 4096x4096x512:  48, 48, 69
+//     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
+//       277, 288, 312
+// Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles of 8- and 1-bit input, and
 // a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
-//   With beta the epilogue first reads C, from all its registers' addresses at once, which costs
-// the larger tiles more (fp8 on planar rows, B=11 456x1542x192: 96, 85, 47 us).
-// The constants are fitted, for each type and operand layout, to times of all three shapes over
-// 30000 problems of random sizes, half of them on operands that no cache held
+// With beta the epilogue reads C first, which costs the larger tiles more (8 bits on planar
+// rows, B=11 456x1542x192: 96, 84, 46). Interleaved fp32 C behind tiles, which only the 256 x 128
+// block regroups through LDS, moves no line: where a smaller block is chosen the larger one is
+// slower by 0.95 to several times, 1.37 (128 x 128) and 2.9 (64 x 64) at the median.
+//   The constants are fitted, for each type and operand layout, to the times of all three shapes over
+// 30000 problems of random sizes, 40 % of them on operands that no cache held
 // (python -m ccglib_amd.tuning.block_choice times such problems): the choice is then on average
 // 0.2 % behind the fastest of the three shapes, and more than 8 % behind in 0.7 % of the problems.
 enum BlockShape { k256x128, k128x128, k64x64 };
@@ -2412,7 +2420,6 @@ hipError_t launch_gemm_mfma_int1(const GemmParams &p, hipStream_t stream) {
 // Which kernel launch_gemm_mfma starts for these parameters (the decisions of
 // launch_typed, in words).
 const char *describe_gemm_mfma(const GemmParams &p) {
-  const bool bits8 = p.type_in == kFloat8e4m3 || p.type_in == kFloat8e5m2;
   const bool bits16 = p.type_in == kFloat16 || p.type_in == kBfloat16;
   const bool int1 = p.type_in == kInt1;
   const size_t k_bytes = (size_t)p.k * bits_of(p.type_in) / 8;
