@@ -74,9 +74,10 @@ def test_c_rows_of_any_length_and_alignment(block_tile, tin, tout, axis, nx, off
 @pytest.mark.parametrize("tin,tout", [(VT.float16, VT.float16), (VT.bfloat16, VT.bfloat16),
                                       (VT.float16, VT.float32), (VT.float8e4m3, VT.float32)])
 def test_c_rows_behind_planar_and_interleaved_operands(block_tile, rows, tin, tout):
-    """The same for operands read in place: 256 x 128 blocks regroup a wave's 64 x 64 results through LDS
-    and store 16 bytes wherever a row starts (every first wave here lies inside C), the
-    smaller ones store from registers; with a complex alpha where C is offset."""
+    """The same for operands read in place. Blocks that regroup a wave's 64 x 64 results through LDS
+    (256 x 128 on interleaved rows, the two larger ones of 8-bit input) store 16 bytes wherever a row
+    starts (every first wave here lies inside C), the others store from registers; with a complex
+    alpha where C is offset."""
     B, ny, K = 2, 70, 64
     dtype = np.float32 if tout == VT.float32 else np.uint16
     for nx in (66, 129, 255):
