@@ -276,6 +276,7 @@ hipError_t launch_width(const TransposeParams &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+constexpr size_t kPairBytes = (size_t)128 << 20;
 template <int EB>
 bool try_launch_pair(const TransposeParams &p0, const TransposeParams &p1, hipStream_t stream,
                      hipError_t &result) {
@@ -287,9 +288,13 @@ bool try_launch_pair(const TransposeParams &p0, const TransposeParams &p1, hipSt
   // and tail: B=64, 512 and 4096 rows of 576 halfs take 0.231 ms together against
   // 0.234 ms one after the other). Two operands of similar size are 1-3 % faster as
   // two launches (fp8 B=16 4096 x 8192 twice: 0.753 against 0.775 ms; 1-bit words
-  // B=32 1024 x 2048 twice: 0.376 against 0.384 ms).
+  // B=32 1024 x 2048 twice: 0.376 against 0.384 ms), as long as that is more than the
+  // second launch costs (with what follows and goes before: 1-bit words B=3, 128 and 320
+  // rows of 101, 23.6 -> 20.1 us in one launch; fp8 B=13, 696 and 936 rows of 1917, 81 MB,
+  // 127.7 -> 118.9 us).
   const size_t small = p0.m < p1.m ? p0.m : p1.m, large = p0.m < p1.m ? p1.m : p0.m;
-  if (small * 4 > large) return false;
+  const size_t bytes = p0.batch * 2 * (p0.m + p1.m) * p0.n * EB;
+  if (small * 4 > large && bytes > kPairBytes) return false;
   const VecPlan<EB> v0 = plan_operand<EB>(p0), v1 = plan_operand<EB>(p1);
   if (!v0.out_vec_ok || !v1.out_vec_ok || v0.in_vec_ok != v1.in_vec_ok ||
       v0.y_blocks + v1.y_blocks > 65535) {
