@@ -156,6 +156,7 @@ struct ccglib_pipeline {
   // `unfused` is the pipeline with transposes that takes over for buffers that
   // are not 16-byte aligned, created by the first Run that meets such buffers
   bool fused = false;
+  bool ragged = false;   // (fused) rows of any length, read from any address
   std::atomic<ccglib_pipeline *> unfused{nullptr};   // (set once, under lazy_lock)
   std::mutex lazy_lock;
   ccglib_packing_t pack_a = nullptr, pack_b = nullptr;
@@ -196,6 +197,39 @@ void tiled_bytes(const ccglib_gemm *g, size_t *bytes_a, size_t *bytes_b) {
   const size_t kp = ceil_div(g->K, kc) * kc;
   *bytes_a = g->B * 2 * ceil_div(g->M, kTileRows) * kTileRows * kp * bits / 8;
   *bytes_b = g->B * 2 * ceil_div(g->N, kTileRows) * kTileRows * kp * bits / 8;
+}
+
+// Whether a GEMM that reads its operands where they lie is expected to be faster than one
+// on tiled copies with the transposes that make them. Reading in place costs the GEMM a
+// few per cent (and more where rows are ragged); the transposes cost two bandwidth-bound
+// passes over A and B and a launch or two. The GEMM's work grows with M N and the transposes'
+// with M + N, so reading in place is the smaller price while
+//   M N / (M + N)  <  T (1 + c / (B K (M + N)))
+// with the break-even T of large problems and c the launches' fixed cost in operand
+// elements. Measured (python -m ccglib_amd.tuning.pipeline_crossover):
+//   16-bit pairs    3800, c = 1e7 where the 192 x 256 kernel reads them (planar C, no beta,
+//                   M and N multiples of 64, K of 32), 2800 elsewhere
+//   8-bit pairs     2700, c = 1e7
+//   planar rows     1500, c = 6e6 (squares; long rectangles at small K would still gain up to
+//                   8 % from reading in place beyond it)
+//   ragged pairs, ragged planar rows, ragged 32-bit rows   800, 400, 700; c = 5e6, 6e6, 1e6. Over 205
+//                   random problems of each kind of route (B to 256, sizes to 8192) this choice
+//                   takes 0.77 of the time of tiled copies, the best one 0.76
+struct BreakEven {
+  double t, c;
+};
+bool rows_in_place_pay(size_t B, size_t M, size_t N, size_t K, BreakEven e) {
+  const double operand_elements = (double)B * (double)K * (double)(M + N);
+  return operand_elements > 0 &&
+         (double)M * (double)N / (double)(M + N) < e.t * (1.0 + e.c / operand_elements);
+}
+BreakEven break_even_planar(int bits, bool ragged) {
+  if (!ragged) return {1500.0, 6.0e6};
+  return bits == 32 ? BreakEven{700.0, 1.0e6} : BreakEven{400.0, 6.0e6};
+}
+BreakEven break_even_pairs(int bits, bool ragged, bool wide) {
+  if (ragged) return {800.0, 5.0e6};
+  return {bits == 8 ? 2700.0 : wide ? 3800.0 : 2800.0, 1.0e7};
 }
 
 // Gives a basic-variant GEMM the workspace for tiled copies of its operands.
@@ -381,11 +415,16 @@ int ccglib_gemm_get_dimensions(int type_in, int type_out, int variant, unsigned 
   return CCGLIB_OK;
 }
 
-int ccglib_gemm_create(ccglib_gemm_t *gemm, size_t B, size_t M, size_t N, size_t K, int device,
-                       void *stream, int type_in, int type_out, int variant,
-                       int c_complex_axis_location, int c_mem_order, int a_mem_order,
-                       int b_mem_order, float alpha_re, float alpha_im, float beta_re,
-                       float beta_im) {
+}  // extern "C"
+
+namespace {
+
+// rows_in_place: the caller (a pipeline) has decided that the basic variant reads its
+// rows where they are.
+int gemm_create(ccglib_gemm_t *gemm, size_t B, size_t M, size_t N, size_t K, int device,
+                void *stream, int type_in, int type_out, int variant, int c_complex_axis_location,
+                int c_mem_order, int a_mem_order, int b_mem_order, float alpha_re, float alpha_im,
+                float beta_re, float beta_im, bool rows_in_place) {
   if (!gemm) return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "null handle pointer");
   *gemm = nullptr;
   if (int rc = validate_gemm(B, M, N, K, type_in, type_out, variant, c_complex_axis_location,
@@ -400,19 +439,37 @@ int ccglib_gemm_create(ccglib_gemm_t *gemm, size_t B, size_t M, size_t N, size_t
   g->retile_allowed = g_options[CCGLIB_AMD_OPTION_BASIC_RETILE] != 0;
   g->int1_direct = g_options[CCGLIB_AMD_OPTION_INT1_POPCOUNT] == 0;
   g->block_tile = (int)g_options[CCGLIB_AMD_OPTION_GEMM_BLOCK_TILE];
-  // Planar rows that direct-to-LDS copies cannot fetch in whole chunks (for 1-bit
-  // input: rows of K / 32 words). Re-tiling them costs two bandwidth-bound passes
-  // and a copy of A and B; the kernel for the tiled layout then runs several
-  // times faster than the ones that load ragged rows through registers.
+  // Planar rows that are not whole 16-byte chunks (for 1-bit input: rows of K / 32 words).
+  // Re-tiling them costs two bandwidth-bound passes and a copy of A and B; the kernel for
+  // the tiled layout then runs faster than the one that reads them in place - and
+  // several times faster than those that load them through registers (1-bit input, and
+  // rows of less than 16 bytes).
   // (Operands that are not 16-byte aligned get the same workspace at their first Run.)
   const size_t row_bytes = type_in == kInt1 ? ceil_div(K, 32) * 4 : K * (size_t)bits_of(type_in) / 8;
+  const bool ragged = row_bytes % 16 != 0;
+  const bool copies_pay = type_in == kInt1 || row_bytes < 16 ||
+                          !rows_in_place_pay(B, M, N, K, break_even_planar(bits_of(type_in), true));
   if (variant == kBasic && B && M && N && K &&
-      (row_bytes % 16 != 0 || g_options[CCGLIB_AMD_OPTION_EXPECT_UNALIGNED] != 0) &&
-      (type_in != kInt1 || g->int1_direct)) {
+      (ragged ? copies_pay : g_options[CCGLIB_AMD_OPTION_EXPECT_UNALIGNED] != 0) &&
+      (type_in != kInt1 || g->int1_direct) && !rows_in_place) {
     make_retile_workspace(g);
   }
   *gemm = g;
   return CCGLIB_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int ccglib_gemm_create(ccglib_gemm_t *gemm, size_t B, size_t M, size_t N, size_t K, int device,
+                       void *stream, int type_in, int type_out, int variant,
+                       int c_complex_axis_location, int c_mem_order, int a_mem_order,
+                       int b_mem_order, float alpha_re, float alpha_im, float beta_re,
+                       float beta_im) {
+  return gemm_create(gemm, B, M, N, K, device, stream, type_in, type_out, variant,
+                     c_complex_axis_location, c_mem_order, a_mem_order, b_mem_order, alpha_re,
+                     alpha_im, beta_re, beta_im, false);
 }
 
 int ccglib_gemm_run(ccglib_gemm_t g, const void *d_a, const void *d_b, void *d_c) {
@@ -421,10 +478,6 @@ int ccglib_gemm_run(ccglib_gemm_t g, const void *d_a, const void *d_b, void *d_c
   if (!d_a || !d_b || !d_c) return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "null device pointer");
   GemmParams p;
   fill_gemm_params(g, d_a, d_b, d_c, &p);
-  if (g->input_interleaved && ((uintptr_t)d_a % 16 != 0 || (uintptr_t)d_b % 16 != 0)) {
-    return fail(CCGLIB_ERROR_INVALID_ARGUMENT,
-                "interleaved pipeline input must be 16-byte aligned");
-  }
   if (g->K == 0 && g->variant == kOpt) {
     return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "K = 0 has no tiled layout");
   }
@@ -440,7 +493,7 @@ int ccglib_gemm_run(ccglib_gemm_t g, const void *d_a, const void *d_b, void *d_c
   if (g->variant == kBasic && g->K && (g->type_in != kInt1 || g->int1_direct)) {
     const size_t row_bytes = g->type_in == kInt1 ? ceil_div(g->K, 32) * 4
                                                  : g->K * (size_t)bits_of(g->type_in) / 8;
-    const bool misaligned = (uintptr_t)d_a % 16 != 0 || (uintptr_t)d_b % 16 != 0;
+    const bool misaligned = row_bytes % 16 == 0 && ((uintptr_t)d_a % 16 != 0 || (uintptr_t)d_b % 16 != 0);
     // Planar operands that are not 16-byte aligned cannot be copied to LDS in
     // place either: the object gets its workspace at the first such Run (the one
     // allocation a Run may make) and keeps it - unless the stream is being
@@ -809,47 +862,32 @@ int pipeline_create(ccglib_pipeline_t *pipeline, size_t B, size_t M, size_t N, s
   p->beta_im = beta_im;
   int rc = CCGLIB_OK;
   const bool packing = (input_type == kInt1);   // src/pipeline/Pipeline.cpp:52
-  // Interleaved 8/16-bit input whose rows are whole 16-byte chunks is fed to the
-  // GEMM as it is (the kernel de-interleaves in its arithmetic), which saves the
-  // two transposes and their intermediate buffers for either variant.
+  // Interleaved 8/16-bit input is fed to the GEMM as it is (the kernel de-interleaves in its
+  // arithmetic) where that pays, which saves the two transposes and their
+  // intermediate buffers for either variant.
   const size_t in_bits = (size_t)bits_of(input_type);
-  // Reading rows in place costs the GEMM a few per cent against reading tiles; the
-  // transposes cost two bandwidth-bound passes over A and B and two more launches.
-  // The GEMM's work grows with M N and the transposes' with M + N, so reading in
-  // place is the smaller price while
-  //   M N / (M + N)  <  T (1 + c / (B K (M + N)))
-  // with the break-even T of large problems and c the launches' fixed cost in
-  // operand elements. Measured (python -m ccglib_amd.tuning.pipeline_crossover at
-  // K = 256, 1024, 4096): 16-bit interleaved rows T = 3800 where the 192 x 256 kernel
-  // reads them (planar C, no beta, alpha only with fp32 C, M and N multiples of 64, K of 32) and
-  // 2800 elsewhere, 8-bit interleaved rows T = 2700, c = 1e7 for both.
-  const double mn_over_sum = (M + N) ? (double)M * (double)N / (double)(M + N) : 0.0;
-  const double operand_elements = (double)B * (double)K * (double)(M + N);
   // (option PIPELINE_ROUTE: 1 in place wherever possible, 2 never for the opt variant)
   const size_t route = g_options[CCGLIB_AMD_OPTION_PIPELINE_ROUTE];
-  auto below = [&](double break_even, double fixed_cost) {
-    return route == 1 ||
-           (route == 0 && operand_elements > 0 &&
-            mn_over_sum < break_even * (1.0 + fixed_cost / operand_elements));
+  auto in_place = [&](BreakEven e) {
+    return route == 1 || (route == 0 && rows_in_place_pay(B, M, N, K, e));
   };
   const bool wide_rows = in_bits == 16 && output_complex_axis_location == kPlanar &&
                          beta_re == 0.f && beta_im == 0.f &&
                          M % 64 == 0 && N % 64 == 0 && K % 32 == 0 && K >= 64;
-  const bool fused = allow_fused && !packing && input_complex_axis_location == kInterleaved && K > 0 &&
-                     (in_bits == 8 || in_bits == 16) && (2 * K * in_bits / 8) % 16 == 0 &&
-                     (variant == kBasic ||
-                      below(in_bits == 8 ? 2700.0 : wide_rows ? 3800.0 : 2800.0, 1.0e7));
-  // Planar input of the opt variant whose rows are whole 16-byte chunks: the GEMM
-  // can read the rows in place as well (the basic variant's loader, same
-  // arithmetic and K order as on tiles). That costs the GEMM more (the tiled
-  // operands have the 192 x 256 kernel), so the break-even lies lower: T = 1500,
-  // c = 6e6 (measured on squares; long rectangles at small K would still gain up to
-  // 8 % from reading in place beyond it).
+  const size_t il_row_bytes = 2 * K * in_bits / 8, planar_row_bytes = K * in_bits / 8;
+  const bool il_ragged = il_row_bytes % 16 != 0, planar_ragged = planar_row_bytes % 16 != 0;
+  const bool fused = allow_fused && !packing && input_complex_axis_location == kInterleaved &&
+                     (in_bits == 8 || in_bits == 16) && il_row_bytes >= 16 &&
+                     ((variant == kBasic && !il_ragged) ||
+                      in_place(break_even_pairs((int)in_bits, il_ragged, wide_rows)));
+  // Planar input of the opt variant: the GEMM can read the rows in place as well (the basic
+  // variant's loader, same arithmetic and K order as on tiles). That costs the GEMM
+  // more (the tiled operands have the 192 x 256 kernel), so the break-even lies lower.
+  // (B=49 2984x256x5824 bf16 to (re, im) rows of C: 2567 us with transposes, 1290 without.)
   const bool planar_in_place = allow_fused && !packing && variant == kOpt &&
-                               input_complex_axis_location == kPlanar &&
-                               output_complex_axis_location == kPlanar && K > 0 &&
+                               input_complex_axis_location == kPlanar && planar_row_bytes >= 16 &&
                                (in_bits == 8 || in_bits == 16 || in_bits == 32) &&
-                               (K * in_bits / 8) % 16 == 0 && below(1500.0, 6.0e6);
+                               in_place(break_even_planar((int)in_bits, planar_ragged));
   // The reference transposes for the opt variant only (:53) and hands interleaved
   // input of the basic variant to a kernel that reads it as planar. Here such
   // input is always de-interleaved: in the GEMM's loader (fused) or, where that
@@ -947,16 +985,21 @@ int pipeline_create(ccglib_pipeline_t *pipeline, size_t B, size_t M, size_t N, s
         break;
       }
     }
-    rc = ccglib_gemm_create(&p->gemm, B, M, N, K, device, stream, input_type, output_type,
-                            (fused || basic_needs_tiles) ? (int)kOpt
-                            : planar_in_place            ? (int)kBasic
-                                                         : variant,
-                            output_complex_axis_location,
-                            c_mem_order, a_mem_order, b_mem_order, alpha_re, alpha_im, beta_re,
-                            beta_im);  // :102-105
-    if (rc == CCGLIB_OK) p->gemm->input_interleaved = fused;
-    p->fused = fused || planar_in_place;   // (both need 16-byte aligned rows at Run)
-    if (rc == CCGLIB_OK && p->fused && allow_fused &&
+    rc = gemm_create(&p->gemm, B, M, N, K, device, stream, input_type, output_type,
+                     (fused || basic_needs_tiles) ? (int)kOpt
+                     : planar_in_place            ? (int)kBasic
+                                                  : variant,
+                     planar_in_place ? (int)kPlanar : output_complex_axis_location, c_mem_order,
+                     a_mem_order, b_mem_order, alpha_re, alpha_im, beta_re, beta_im,
+                     planar_in_place);  // :102-105
+    if (rc == CCGLIB_OK) {
+      p->gemm->input_interleaved = fused;
+      // (the basic variant's own interface has planar C only, its kernels store either)
+      p->gemm->c_axis = output_complex_axis_location;
+    }
+    p->fused = fused || planar_in_place;
+    p->ragged = fused ? il_ragged : planar_ragged;
+    if (rc == CCGLIB_OK && p->fused && !p->ragged && allow_fused &&
         g_options[CCGLIB_AMD_OPTION_EXPECT_UNALIGNED] != 0) {
       // the pipeline with transposes that takes over for unaligned buffers, now
       // rather than at the first Run that meets them
@@ -1003,8 +1046,8 @@ int ccglib_pipeline_run(ccglib_pipeline_t p, const void *d_a, const void *d_b, v
   if (!p) return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "null pipeline handle");
   int rc;
   const void *a = d_a, *b = d_b;
-  if (p->fused && d_a && d_b && ((uintptr_t)d_a % 16 != 0 || (uintptr_t)d_b % 16 != 0)) {
-    // The GEMM's copies to LDS need 16-byte aligned rows; the transposes take any
+  if (p->fused && !p->ragged && d_a && d_b && ((uintptr_t)d_a % 16 != 0 || (uintptr_t)d_b % 16 != 0)) {
+    // Rows of whole chunks are copied to LDS from 16-byte aligned addresses only; the transposes take any
     // element-aligned address. The pipeline that runs them is created here, once
     // (the one allocation a device Run may make), and kept.
     ccglib_pipeline *stand_by = p->unfused.load(std::memory_order_acquire);

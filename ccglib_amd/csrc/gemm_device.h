@@ -13,7 +13,11 @@ typedef int int4_t __attribute__((ext_vector_type(4)));
 // load (global memory takes any alignment on this target).
 typedef int4_t int4_unaligned_t __attribute__((aligned(1)));
 
-enum Loader { kLoadTiled = 0, kLoadPlanarVec = 1, kLoadPlanarElem = 2, kLoadInterleavedVec = 3 };
+// (Ragged: rows of any length from 16 bytes on, at any address)
+enum Loader {
+  kLoadTiled = 0, kLoadPlanarVec = 1, kLoadPlanarElem = 2, kLoadInterleavedVec = 3,
+  kLoadPlanarRagged = 4, kLoadInterleavedRagged = 5
+};
 
 constexpr int kNumXcd = 8;
 

@@ -1566,11 +1566,13 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   static_assert(MS == 32 || DtypeTraits<DT>::kTilesPerMfma == 1,
                 "one K tile per iteration: fp8 input runs on the 32-row MFMA here");
   constexpr int KPM = 1;
-  static_assert(MS == 16 || LOADER != kLoadInterleavedVec || DtypeTraits<DT>::kElemBytes == 1,
-                "interleaved operands on the 32-row MFMAs: 8-bit input only");
   // interleaved operands: one plane of (re, im) rows
   // (their slots hold 128 bytes of every row, fetched as whole cache lines)
-  constexpr bool IL = (LOADER == kLoadInterleavedVec);
+  constexpr bool IL = (LOADER == kLoadInterleavedVec || LOADER == kLoadInterleavedRagged);
+  static_assert(MS == 16 || !IL || DtypeTraits<DT>::kElemBytes == 1,
+                "interleaved operands on the 32-row MFMAs: 8-bit input only");
+  // rows that are no whole aligned 16-byte chunks, see chunk_source and settle_row_ends
+  constexpr bool RAGGED = (LOADER == kLoadPlanarRagged || LOADER == kLoadInterleavedRagged);
   constexpr int PLANES = IL ? 1 : 2;
   constexpr int RB = IL ? 128 : kTileRowBytes;      // bytes of a row in one slot
   constexpr int RPB = 1024 / RB;                    // rows moved by one 1 KiB copy instruction
@@ -1716,6 +1718,21 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       }
     }
   };
+  // Where a lane's chunk of K tile kt comes from when it lies at `src` in K tile 0 of its row.
+  // Rows of whole chunks: it is either inside K or reads zeros. Ragged rows: the chunk
+  // that holds the end of the row is fetched as the last 16 bytes of the row instead
+  // (nothing outside the row is touched): its elements lie at the chunk's end and
+  // in front of them, once more, some that the chunk before holds, until
+  // settle_row_ends puts them right.
+  auto chunk_source = [&](const char *src, unsigned kt, int chunk) {
+    const unsigned end = kt * RB + chunk * 16 + 16;
+    if constexpr (RAGGED) {
+      const unsigned over = end > row_bytes ? end - row_bytes : 0;
+      return over < 16 ? src + (size_t)kt * RB - over : g_zero_tile + lane * 16;
+    } else {
+      return end <= row_bytes ? src + (size_t)kt * RB : g_zero_tile + lane * 16;
+    }
+  };
   // issue_*: straight-line code (it is placed between MFMAs, and a branch there
   // would let the compiler sink those MFMAs below it); advance_*: the
   // bookkeeping, with the branches of the tile change.
@@ -1726,12 +1743,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       if constexpr (LOADER == kLoadTiled) {
         load_1k_to_lds(x_src[i] + (size_t)xs.kt * kTileBytes + x_tile_off[i], lane_off_x, dst);
       } else {
-        // rows are whole 16-byte chunks: a chunk is either inside K or reads zeros
         const int q = i * NW + wave, rb = q % (BX / RPB);
-        const int chunk = XT ? xt_chunk : c_of(rb);
-        const bool inside = (xs.kt * RB + chunk * 16 + 16 <= row_bytes);
-        load_1k_to_lds_by_lane(inside ? x_lane_src[i] + (size_t)xs.kt * RB : g_zero_tile + lane * 16,
-                               dst);
+        load_1k_to_lds_by_lane(chunk_source(x_lane_src[i], xs.kt, XT ? xt_chunk : c_of(rb)), dst);
       }
     }
   };
@@ -1743,9 +1756,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         load_1k_to_lds(y_src[i] + (size_t)ys.kt * kTileBytes + y_tile_off[i], lane_off, dst);
       } else {
         const int q = i * NW + wave, rb = q % (BY / RPB);
-        const bool inside = (ys.kt * RB + c_of(rb) * 16 + 16 <= row_bytes);
-        load_1k_to_lds_by_lane(inside ? y_lane_src[i] + (size_t)ys.kt * RB : g_zero_tile + lane * 16,
-                               dst);
+        load_1k_to_lds_by_lane(chunk_source(y_lane_src[i], ys.kt, c_of(rb)), dst);
       }
     }
   };
@@ -1762,6 +1773,30 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       ys.tile += gridDim.x;
       point_y(ys.tile);
     }
+  };
+
+  // (RAGGED) Shifts the last elements of every row of both operands, which lie at the end of
+  // the row's last chunk, to its front and clears the rest: the slots then hold what the
+  // tiled layout holds. Once per C tile, between the barrier that says that its last K
+  // tile has landed and a second one.
+  auto settle_row_ends = [&](unsigned x_in, unsigned y_in) {
+    const unsigned shift = 8 * (16 - row_bytes % 16), chunk = row_bytes / 16 % CPR;
+    for (unsigned t = threadIdx.x; t < (unsigned)(PLANES * (BX + BY)); t += 64 * NW) {
+      const bool of_y = t >= (unsigned)(PLANES * BX);
+      const unsigned row = of_y ? t - PLANES * BX : t;   // (row of LDS; planes follow each other)
+      // the chunk's place: the swizzles of the copies above
+      const unsigned at = IL ? (MS == 32 ? (((row >> 3) & 1) << 2) | ((row >> 1) & 3) : row & 7)
+                          : XT && !of_y ? 3 * ((row >> 4) & 1)
+                          : MS == 32    ? (row >> 2) & 3
+                                        : (row >> 1) & 3;
+      typedef unsigned long long ulong2_t __attribute__((ext_vector_type(2)));
+      ulong2_t *p = reinterpret_cast<ulong2_t *>(lds + (of_y ? y_slot_off(y_in) : x_slot_off(x_in)) +
+                                                 row * RB + (chunk ^ at) * 16);
+      const ulong2_t v = *p;
+      *p = shift >= 64 ? ulong2_t{v[1] >> (shift - 64), 0ull}
+                       : ulong2_t{(v[0] >> shift) | (v[1] << (64 - shift)), v[1] >> shift};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
 
   const int frag_lane_off = swizzled_row_offset(lane & 15, lane >> 4);
@@ -1855,6 +1890,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         asm volatile("s_barrier" ::: "memory");
       } else {
         wait_vmcnt_then_barrier<kOutstandingOk>();
+      }
+      if constexpr (RAGGED) {
+        if (it + 1 == iters && row_bytes % 16 != 0) settle_row_ends(x_slot, y_slot);
       }
       // The slots of the previous iteration are free now: refill them with the
       // K tiles that are XLEAD / YLEAD iterations ahead (of this C tile or the
@@ -2262,9 +2300,19 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   const BlockShape shape = block_choice(p).shape;
   if (p.input_interleaved) {
     // raw (re, im) rows straight from the caller: the host side only takes this
-    // path for 8- and 16-bit input whose rows are whole aligned 16-byte chunks
+    // path for 8- and 16-bit input with rows of at least 16 bytes
+    const bool ragged = 2 * k_bytes % 16 != 0 || (uintptr_t)p.x % 16 != 0 || (uintptr_t)p.y % 16 != 0;
     if constexpr (DT == kFloat32) {
       return hipErrorInvalidValue;
+    } else if (ragged) {
+      if (2 * k_bytes < 16) return hipErrorInvalidValue;
+      constexpr int MS = KPM == 1 ? 16 : 32;
+      if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedRagged, MS>(p, stream);
+      if (shape == k128x128) {
+        return launch_dtl<DT, TOUT, 128, 128, 64, KPM == 1 ? 32 : 64, KPM == 1 ? 4 : 2, 2, kLoadInterleavedRagged,
+                          MS>(p, stream);
+      }
+      return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedRagged, MS>(p, stream);
     } else if constexpr (KPM == 1) {
       if constexpr (DtypeTraits<DT>::kElemBytes == 2) {
         if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT, true>(p, stream);
@@ -2336,6 +2384,15 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
                  ? launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>(p, stream)
                  : launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarVec, 32>(p, stream);
     }
+  }
+  if (k_bytes >= 16) {
+    constexpr int MS = KPM == 1 ? 16 : 32;
+    if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarRagged, MS>(p, stream);
+    if (shape == k128x128) {
+      return launch_dtl<DT, TOUT, 128, 128, 64, KPM == 1 ? 32 : 64, KPM == 1 ? 4 : 2, 2, kLoadPlanarRagged,
+                        MS>(p, stream);
+    }
+    return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarRagged, MS, KPM == 1>(p, stream);
   }
   // fp8 stages are twice as large (two K tiles per MFMA): one wave per SIMD
   // with the full register file
@@ -2433,6 +2490,11 @@ const char *describe_gemm_mfma(const GemmParams &p) {
     if (bits16 && wide_tiles_apply(p) && wide_tiles_pay(p)) {
       return "complex_gemm_mfma_wide, 192x256 block, one wave per SIMD, interleaved rows";
     }
+    if (2 * k_bytes % 16 != 0 || (uintptr_t)p.x % 16 != 0 || (uintptr_t)p.y % 16 != 0) {
+      return name("complex_gemm_mfma_dtl, 256x128 block, ragged interleaved rows",
+                  "complex_gemm_mfma_dtl, 128x128 block, ragged interleaved rows",
+                  "complex_gemm_mfma_dtl, 64x64 block, ragged interleaved rows");
+    }
     return name("complex_gemm_mfma_dtl, 256x128 block, interleaved rows",
                 "complex_gemm_mfma_dtl, 128x128 block, interleaved rows",
                 "complex_gemm_mfma_dtl, 64x64 block, interleaved rows");
@@ -2449,6 +2511,11 @@ const char *describe_gemm_mfma(const GemmParams &p) {
     return name("complex_gemm_mfma_dtl, 256x128 block, planar rows",
                 "complex_gemm_mfma_dtl, 128x128 block, planar rows",
                 "complex_gemm_mfma_dtl, 64x64 block, planar rows");
+  }
+  if (k_bytes >= 16) {
+    return name("complex_gemm_mfma_dtl, 256x128 block, ragged planar rows",
+                "complex_gemm_mfma_dtl, 128x128 block, ragged planar rows",
+                "complex_gemm_mfma_dtl, 64x64 block, ragged planar rows");
   }
   return "complex_gemm_mfma, 128x128 block, planar rows through registers";
 }

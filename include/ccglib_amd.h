@@ -76,10 +76,12 @@ CCGLIB_API const char *ccglib_version(void);
  *                    MFMA on +-1 values, exact); 1: XOR + population count on
  *                    the vector ALUs, which is otherwise only the fallback.
  *   BASIC_RETILE     1 (default): a basic-variant GEMM whose planar rows are not
- *                    whole 16-byte chunks, or whose operands are not 16-byte
- *                    aligned, owns a tiled copy of A and B and re-tiles into it
- *                    at every Run; 0: it reads such rows in place through
- *                    registers (several times slower, no extra memory).
+ *                    whole 16-byte chunks owns a tiled copy of A and B and
+ *                    re-tiles into it at every Run where that is faster than
+ *                    reading the rows in place; so does one whose rows are whole
+ *                    chunks and whose operands turn out not to be 16-byte
+ *                    aligned; 0: such rows are always read in place (no extra
+ *                    memory).
  *   HOST_CHUNK_BYTES 0 (default): ccglib_pipeline_run_host moves jobs of 8 MiB
  *                    or more in chunks of whole batches of about 32 MiB; any
  *                    other value: chunks of about that many bytes, whatever
@@ -106,7 +108,7 @@ CCGLIB_API const char *ccglib_version(void);
  *                    allocated when the object is created, and no device Run
  *                    allocates.
  *   PIPELINE_ROUTE   0 (default): an opt-variant pipeline whose input rows are
- *                    whole 16-byte chunks lets the GEMM read them in place
+ *                    16 bytes or longer lets the GEMM read them in place
  *                    where that is faster than transposing them into tiles
  *                    first (small M N / (M + N); the break-even points are
  *                    measured ones), and transposes otherwise; 1: in place
@@ -151,11 +153,12 @@ CCGLIB_API int ccglib_amd_get_option(int option, size_t *value);
  * integers (src/reference/GEMM.cpp:202-205).
  * C is read only when beta != 0.
  * K whose interleaved row (2 * K * bits / 8 bytes) does not fit 32 bits is
- * refused. Operands should be 16-byte aligned: basic-variant operands that are
- * not (or whose rows are not whole 16-byte chunks) are re-tiled into a
- * workspace the object owns (allocated at creation for such K, at the first
- * such Run for such pointers; see CCGLIB_AMD_OPTION_BASIC_RETILE); opt-variant
- * operands that are not are refused by Run.
+ * refused. Operands should be 16-byte aligned: basic-variant operands whose rows
+ * are whole 16-byte chunks and that are not aligned are re-tiled into a workspace
+ * the object owns (allocated at the first such Run). Rows that are not whole
+ * chunks are read in place from any address, or re-tiled likewise where that is
+ * faster (workspace allocated at creation; see CCGLIB_AMD_OPTION_BASIC_RETILE).
+ * Opt-variant operands that are not aligned are refused by Run.
  * ---------------------------------------------------------------------- */
 CCGLIB_API int ccglib_gemm_create(ccglib_gemm_t *gemm, size_t B, size_t M,
                                   size_t N, size_t K, int device, void *stream,

@@ -1,0 +1,132 @@
+"""GPU parity tests of GEMMs and pipelines that read rows of any length in place: rows that end
+inside a 16-byte chunk, at every remainder, from any address, against the bits of the tiled
+route (planar rows: same arithmetic) or the oracle ((re, im) rows)."""
+import numpy as np
+import pytest
+import torch
+
+import ccglib_amd as cc
+import oracle as orc
+from gpu_util import (ORC_TYPE, check_float, dequantize, quantize, stream, to_device, to_host,
+                      transpose_operand)
+
+pytestmark = pytest.mark.gpu
+VT = cc.ValueType
+PLANAR, INTERLEAVED = cc.ComplexAxisLocation.complex_planar, cc.ComplexAxisLocation.complex_interleaved
+ROW, COL = cc.MemOrder.row_major, cc.MemOrder.col_major
+
+# (type, K): the shortest rows, one K tile and one element less and more, several K tiles, all
+# remainders of a chunk among them
+PLANAR_K = [(VT.float16, k) for k in (9, 15, 31, 33, 61, 66, 100, 229)] + \
+           [(VT.bfloat16, 301), (VT.float32, 5), (VT.float32, 47), (VT.float32, 114)] + \
+           [(VT.float8e4m3, k) for k in (17, 31, 63, 65, 130, 135, 268)] + [(VT.float8e5m2, 201)]
+PAIRS_K = [(VT.float16, k) for k in (5, 31, 33, 62, 67, 97, 230)] + [(VT.bfloat16, 225)] + \
+          [(VT.float8e4m3, k) for k in (9, 63, 65, 130, 197)] + [(VT.float8e5m2, 332)]
+
+
+def operands(rng, B, M, N, K, tin, scale=1.0):
+    qa = quantize((scale * rng.uniform(-1, 1, B * 2 * M * K)).astype(np.float32), tin)
+    qb = quantize((scale * rng.uniform(-1, 1, B * 2 * N * K)).astype(np.float32), tin)
+    return qa, qb
+
+
+def pairs(q, B, rows, K):
+    return np.ascontiguousarray(q.reshape(B, 2, rows, K).transpose(0, 2, 3, 1)).reshape(-1)
+
+
+def at_offset(q, skew):
+    """A device buffer that ends with the data (whatever is read behind a row's end is not
+    there), which starts `skew` elements behind a 16-byte boundary."""
+    d = to_device(np.concatenate([np.zeros(skew, q.dtype), q]))
+    return d, d.data_ptr() + skew * q.dtype.itemsize
+
+
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("tin,K", PLANAR_K)
+def test_planar_rows(block_tile, tin, K):
+    B, M, N = 2, 150, 270
+    skew = K % 3
+    qa, qb = operands(np.random.default_rng(K), B, M, N, K, tin)
+    (d_a, p_a), (d_b, p_b) = at_offset(qa, skew), at_offset(qb, skew)
+    for order in (ROW, COL):
+        d_c = to_device(np.full(B * 2 * M * N, np.nan, dtype=np.float32))
+        with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.basic_retile, 0):
+            g = cc.GEMM(B, M, N, K, 0, stream(), cc.Precision(tin, VT.float32), cc.Variant.basic,
+                        PLANAR, order)
+        g.Run(p_a, p_b, d_c.data_ptr())
+        t_a, t_b = transpose_operand(qa, B, M, K, tin), transpose_operand(qb, B, N, K, tin)
+        want = to_device(np.full(B * 2 * M * N, np.nan, dtype=np.float32))
+        cc.GEMM(B, M, N, K, 0, stream(), cc.Precision(tin, VT.float32), cc.Variant.opt, PLANAR,
+                order).Run(t_a.data_ptr(), t_b.data_ptr(), want.data_ptr())
+        torch.cuda.synchronize()
+        assert torch.equal(d_c, want)
+
+
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("tin,K", PAIRS_K)
+def test_pairs(block_tile, tin, K):
+    B, M, N = 2, 150, 270
+    qa, qb = operands(np.random.default_rng(K), B, M, N, K, tin)
+    skew = 2 * (K % 3)
+    (d_a, p_a), (d_b, p_b) = at_offset(pairs(qa, B, M, K), skew), at_offset(pairs(qb, B, N, K), skew)
+    d_c = to_device(np.full(B * 2 * M * N, np.nan, dtype=np.float32))
+    with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.pipeline_route, 1):
+        p = cc.Pipeline(B, M, N, K, 0, stream(), INTERLEAVED, INTERLEAVED, ROW, COL, ROW, tin, VT.float32,
+                        cc.Variant.opt)
+    assert p.ReadsInPlace()
+    p.Run(p_a, p_b, d_c.data_ptr())
+    torch.cuda.synchronize()
+    got = to_host(d_c, np.float32).reshape(B, M, N, 2).transpose(0, 3, 1, 2)
+    check_float(got, orc.gemm(qa, qb, M, N, K, ORC_TYPE[tin], orc.FLOAT32),
+                orc.gemm_float64(qa, qb, M, N, K, ORC_TYPE[tin]), tin, VT.float32)
+
+
+@pytest.mark.parametrize("axis", [PLANAR, INTERLEAVED])
+def test_infinities_at_the_end_of_a_row(axis):
+    # The last elements of a row are fetched together with some before them, which must not
+    # count twice: neither in a sum nor as 0 times an infinity.
+    B, M, N, K, tin = 1, 70, 80, 45, VT.float16
+    qa, qb = operands(np.random.default_rng(1), B, M, N, K, tin)
+    a, b = qa.reshape(B, 2, M, K), qb.reshape(B, 2, N, K)
+    inf = np.float16(np.inf).view(np.uint16)
+    a[0, 0, 3, K - 7], a[0, 1, 66, K - 1], b[0, 0, 50, 37], b[0, 1, 79, 40] = inf, inf, inf, inf
+    d_a = to_device(pairs(qa, B, M, K) if axis == INTERLEAVED else qa)
+    d_b = to_device(pairs(qb, B, N, K) if axis == INTERLEAVED else qb)
+    d_c = to_device(np.zeros(B * 2 * M * N, dtype=np.float32))
+    with cc.option(cc.Option.pipeline_route, 1):
+        p = cc.Pipeline(B, M, N, K, 0, stream(), axis, PLANAR, ROW, COL, ROW, tin, VT.float32, cc.Variant.opt)
+    p.Run(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr())
+    torch.cuda.synchronize()
+    got = to_host(d_c, np.float32).reshape(2, M, N)
+    x = dequantize(a, tin).astype(np.float64)[0]
+    y = dequantize(b, tin).astype(np.float64)[0]
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(x[0][:, None] * y[0] - x[1][:, None] * y[1]).sum(2),
+                         (x[0][:, None] * y[1] + x[1][:, None] * y[0]).sum(2)])
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(got), kind(want))
+    finite = np.isfinite(want)
+    assert np.allclose(got[finite], want[finite], rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("tin,tout", [(VT.float16, VT.float32), (VT.float16, VT.float16),
+                                      (VT.float32, VT.float32), (VT.float8e4m3, VT.float32)])
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("K", [64, 77])
+def test_planar_rows_to_pairs(tin, tout, block_tile, K):
+    # planar rows read in place with (re, im) pairs in C: the bits of the tiled route
+    B, M, N = 2, 150, 270
+    qa, qb = operands(np.random.default_rng(K), B, M, N, K, tin)
+    d_a, d_b = to_device(qa), to_device(qb)
+    outs = []
+    for route in (1, 2):
+        with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.pipeline_route, route):
+            p = cc.Pipeline(B, M, N, K, 0, stream(), PLANAR, INTERLEAVED, ROW, COL, ROW, tin, tout,
+                            cc.Variant.opt, 0.5 + 2j, 0)
+        assert p.ReadsInPlace() == (route == 1)
+        d_c = torch.full((B * 2 * M * N,), -1, dtype=torch.float32 if tout == VT.float32 else torch.float16,
+                         device="cuda")
+        p.Run(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr())
+        outs.append(d_c)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
