@@ -152,7 +152,7 @@ struct ccglib_pipeline {
   // 1-bit input, one byte per sample, planar: expanded straight into the GEMM's
   // workspace (no packed or transposed intermediates)
   bool int1_direct = false;
-  // 8/16-bit interleaved input that the GEMM reads in place (no transposes);
+  // interleaved (or planar) input that the GEMM reads in place (no transposes);
   // `unfused` is the pipeline with transposes that takes over for buffers that
   // are not 16-byte aligned, created by the first Run that meets such buffers
   bool fused = false;
@@ -212,9 +212,10 @@ void tiled_bytes(const ccglib_gemm *g, size_t *bytes_a, size_t *bytes_b) {
 //   8-bit pairs     2700, c = 1e7
 //   planar rows     1500, c = 6e6 (squares; long rectangles at small K would still gain up to
 //                   8 % from reading in place beyond it)
-//   ragged pairs, ragged planar rows, ragged 32-bit rows   800, 400, 700; c = 5e6, 6e6, 1e6. Over 205
-//                   random problems of each kind of route (B to 256, sizes to 8192) this choice
-//                   takes 0.77 of the time of tiled copies, the best one 0.76
+//   ragged rows     800, c = 5e6 (pairs), 400, c = 6e6 (planar). Over 270 random problems (B to 256,
+//                   sizes to 8192) this choice takes 0.76 of the time of tiled copies, the best one 0.75
+//   32-bit rows     450, c = 8e6 (pairs; ragged 300, 4e6), 800, c = 1e7 (planar; ragged 600, 3e6).
+//                   Over 550 random problems 0.81 of the time of tiled copies, as the best one
 struct BreakEven {
   double t, c;
 };
@@ -224,10 +225,11 @@ bool rows_in_place_pay(size_t B, size_t M, size_t N, size_t K, BreakEven e) {
          (double)M * (double)N / (double)(M + N) < e.t * (1.0 + e.c / operand_elements);
 }
 BreakEven break_even_planar(int bits, bool ragged) {
-  if (!ragged) return {1500.0, 6.0e6};
-  return bits == 32 ? BreakEven{700.0, 1.0e6} : BreakEven{400.0, 6.0e6};
+  if (bits == 32) return ragged ? BreakEven{600.0, 3.0e6} : BreakEven{800.0, 1.0e7};
+  return ragged ? BreakEven{400.0, 6.0e6} : BreakEven{1500.0, 6.0e6};
 }
 BreakEven break_even_pairs(int bits, bool ragged, bool wide) {
+  if (bits == 32) return ragged ? BreakEven{300.0, 4.0e6} : BreakEven{450.0, 8.0e6};
   if (ragged) return {800.0, 5.0e6};
   return {bits == 8 ? 2700.0 : wide ? 3800.0 : 2800.0, 1.0e7};
 }
@@ -862,7 +864,7 @@ int pipeline_create(ccglib_pipeline_t *pipeline, size_t B, size_t M, size_t N, s
   p->beta_im = beta_im;
   int rc = CCGLIB_OK;
   const bool packing = (input_type == kInt1);   // src/pipeline/Pipeline.cpp:52
-  // Interleaved 8/16-bit input is fed to the GEMM as it is (the kernel de-interleaves in its
+  // Interleaved input is fed to the GEMM as it is (the kernel de-interleaves in its
   // arithmetic) where that pays, which saves the two transposes and their
   // intermediate buffers for either variant.
   const size_t in_bits = (size_t)bits_of(input_type);
@@ -877,7 +879,7 @@ int pipeline_create(ccglib_pipeline_t *pipeline, size_t B, size_t M, size_t N, s
   const size_t il_row_bytes = 2 * K * in_bits / 8, planar_row_bytes = K * in_bits / 8;
   const bool il_ragged = il_row_bytes % 16 != 0, planar_ragged = planar_row_bytes % 16 != 0;
   const bool fused = allow_fused && !packing && input_complex_axis_location == kInterleaved &&
-                     (in_bits == 8 || in_bits == 16) && il_row_bytes >= 16 &&
+                     (in_bits == 8 || in_bits == 16 || in_bits == 32) && il_row_bytes >= 16 &&
                      ((variant == kBasic && !il_ragged) ||
                       in_place(break_even_pairs((int)in_bits, il_ragged, wide_rows)));
   // Planar input of the opt variant: the GEMM can read the rows in place as well (the basic

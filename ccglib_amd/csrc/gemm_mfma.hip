@@ -19,7 +19,8 @@
 //  * LDS rows are 64 bytes with the 16-byte chunk index XORed by a function of
 //    the row that suits the fragment shape of the MFMA in use (measured free of
 //    bank conflicts; see complex_gemm_mfma_dtl).
-//  * 16-bit and 32-bit input: 16x16x32 (16x16x4 for fp32) MFMA; fp8: the
+//  * 16-bit input: 16x16x32 MFMA; 32-bit input: every value split into three
+//    bf16 for the 32x32x16 one (fp32 products to fp32 accuracy); fp8: the
 //    32x32x64 f8f6f4 MFMA, which runs at twice the rate of the legacy fp8
 //    instruction; 1-bit input: the same instruction on fp4 +-1 values expanded
 //    from the packed words in registers.
@@ -54,6 +55,16 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef int int8_t_ __attribute__((ext_vector_type(8)));
 typedef unsigned short ushort4_t __attribute__((ext_vector_type(4)));
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in this order.
+template <int... Is, class F>
+__device__ __forceinline__ void static_for_each(std::integer_sequence<int, Is...>, F &&f) {
+  (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_each(std::make_integer_sequence<int, N>{}, f);
+}
 
 // K tiles consumed by one MFMA: one for 16-bit input (16x16x32), two for fp8
 // (16x16x128: 32 bytes per lane, 16 from each of two K tiles).
@@ -927,6 +938,209 @@ __device__ __forceinline__ void mma_step32_interleaved_single(const char *slot, 
   }
 }
 
+// 32-bit input on the bf16 instruction. x = h + m + l, each of the three a bf16 (8 of the 24
+// significant bits; what rounding to nearest takes too much or too little the next
+// part gives back), and of the nine products of two such sums the six down to 2^-16 of
+// the largest are added up: what is left out lies below 2^-24 of the product, less than the
+// rounding of the sum. Six 32x32x16 instructions take the time of six sixteenths of the
+// fp32 ones they stand for (2.5 PFLOP/s dense against 0.157), and round the sum 6 times
+// per 16 products instead of up to 16 times. N(0, 1) operands, relative error of the result against 64
+// bits, fp32 instructions and these: K = 32 1.5e-7, 1.1e-7; K = 1000 8.0e-7, 7.0e-7; K = 8192
+// 2.3e-6, 2.1e-6. Times, tiles of both: 4096x4096x512 480 and 305 us; planar B=2 1000^3 134 and 112.
+//   Both operands are scaled by 2^24 first and the result by 2^-48, so that no part of a
+// small number falls below the range of a bf16: the split is exact for every finite
+// float. What the instructions cannot do is an infinity, a NaN (their parts are NaN) or a sum
+// beyond 2^80: the accumulators are then not finite, and the wave computes its tile
+// again with the fp32 instructions (recompute_f32).
+//   The splitting, 13 vector instructions for two elements, runs in every wave that reads an
+// element (split tiles would take half as much LDS again) and in the shadow of the matrix
+// instructions: those of a K tile are issued while the next one is split (see
+// mma_step32_split).
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
+struct SplitF32 {
+  int4_t h, m, l;
+};
+// Step s of 4 of the splitting of 8 values (x holds what is left to split). A step's
+// instructions are independent of each other but for pairs of them: a chain of 13 for one
+// pair of values after the other leaves the vector ALU waiting for its own results.
+__device__ __forceinline__ void split_step(float (&x)[8], SplitF32 &o, int s) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  auto pack = [&](int4_t &p) {   // (round to nearest even)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = __builtin_bit_cast(int, __builtin_convertvector((float2_t{x[2 * i], x[2 * i + 1]}), bf16x2_t));
+    }
+  };
+  auto subtract = [&](const int4_t &p) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned v = (unsigned)p[i];
+      x[2 * i] -= __builtin_bit_cast(float, v << 16);
+      x[2 * i + 1] -= __builtin_bit_cast(float, v & 0xffff0000u);
+    }
+  };
+  if (s == 0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] *= kSplitScale;
+    pack(o.h);
+  } else if (s == 1) {
+    subtract(o.h);
+  } else if (s == 2) {
+    pack(o.m);
+    subtract(o.m);
+  } else {
+    pack(o.l);
+  }
+}
+__device__ __forceinline__ SplitF32 negate(const SplitF32 &f) {
+  SplitF32 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r.h[i] = f.h[i] ^ (int)0x80008000u;
+    r.m[i] = f.m[i] ^ (int)0x80008000u;
+    r.l[i] = f.l[i] ^ (int)0x80008000u;
+  }
+  return r;
+}
+// product P of the six, smallest first
+template <int P>
+__device__ __forceinline__ float16_t_ mfma_split(const SplitF32 &x, const SplitF32 &y, float16_t_ acc) {
+  const int4_t &a = P == 0 ? x.l : P == 2 || P == 3 ? x.m : x.h;
+  const int4_t &b = P == 1 ? y.l : P == 2 || P == 4 ? y.m : y.h;
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
+}
+struct SplitPair {   // (re, im) fragments of 32 rows
+  SplitF32 re, im;
+};
+
+// The 24 instructions of one 32 x 32 tile and K tile, in turn for its two sums (one that adds
+// to the result of the one before waits for it); behind(n) is issued behind the n-th.
+template <class F>
+__device__ __forceinline__ void mma_split_tile(const SplitPair &x, const SplitPair &y, float16_t_ &acc_re,
+                                               float16_t_ &acc_im, F &&behind) {
+#define CCGLIB_PIN __builtin_amdgcn_sched_barrier(0)
+  static_for<6>([&](auto product) {
+    constexpr int P = decltype(product)::value;
+    acc_re = mfma_split<P>(x.re, y.re, acc_re);
+    behind(2 * P);
+    CCGLIB_PIN;
+    acc_im = mfma_split<P>(x.re, y.im, acc_im);
+    behind(2 * P + 1);
+    CCGLIB_PIN;
+  });
+  const SplitF32 minus = negate(x.im);
+  static_for<6>([&](auto product) {
+    constexpr int P = decltype(product)::value;
+    acc_im = mfma_split<P>(x.im, y.re, acc_im);
+    behind(12 + 2 * P);
+    CCGLIB_PIN;
+    acc_re = mfma_split<P>(minus, y.im, acc_re);
+    behind(13 + 2 * P);
+    CCGLIB_PIN;
+  });
+#undef CCGLIB_PIN
+}
+
+// What a wave carries from one K iteration to the next: the split fragments of the last K tile.
+template <int TX, int TY> struct SplitState {
+  SplitPair x[TX], y[TY];
+};
+
+// One K iteration of a wave with TX x TY tiles of 32 x 32 (1 x 1, 2 x 1, 2 x 2): reads the K tile
+// of `slot` and splits it, a fragment at a time, behind the instructions of one tile, those
+// of the K tile before among them (FIRST: there is none); its last tiles' instructions
+// follow in the next iteration, or in mma_split_last. With 2 x 2 tiles every fragment is
+// overwritten right behind its last use.
+// A lane's 8 values of a row are its two 16-byte chunks (of either plane), or every other
+// word of its four (IL: 128 bytes of pairs, off[2 h + u]).
+template <int BX, int BY, int TX, int TY, bool IL, bool FIRST, typename Mid>
+__device__ __forceinline__ void mma_step32_split(const char *slot, const int *x_off, const int *y_off,
+                                                 SplitState<TX, TY> &st, float16_t_ (&acc_re)[TY][TX],
+                                                 float16_t_ (&acc_im)[TY][TX], Mid &&mid) {
+  static_assert(TX >= TY && TX <= 2, "1 x 1, 2 x 1 or 2 x 2 tiles");
+  constexpr int ROW32 = 32 * (IL ? 128 : kTileRowBytes);
+  struct Raw {
+    float re[8], im[8];
+  };
+  auto rd = [&](const int *off, int extra, int plane_bytes) {
+    Raw r;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const char *p = slot + (IL ? off[u] : off[u & 1] + (u >> 1) * plane_bytes) + extra;
+      const float4_t v = *reinterpret_cast<const float4_t *>(p);
+      if constexpr (IL) {
+        r.re[2 * u] = v[0], r.re[2 * u + 1] = v[2], r.im[2 * u] = v[1], r.im[2 * u + 1] = v[3];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) (u < 2 ? r.re : r.im)[4 * (u & 1) + e] = v[e];
+      }
+    }
+    return r;
+  };
+  auto rd_x = [&](int i) { return rd(x_off, i * ROW32, BX * kTileRowBytes); };
+  auto rd_y = [&](int j) { return rd(y_off, j * ROW32, BY * kTileRowBytes); };
+  // step s of 8: the real part, then the imaginary one
+  auto split = [](Raw &r, SplitPair &o, int s) {
+    split_step(s < 4 ? r.re : r.im, s < 4 ? o.re : o.im, s & 3);
+  };
+  auto split_now = [&](Raw r, SplitPair &o) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) split(r, o, s);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the instructions of tile (i, j), and behind them the split of one fragment (whose raw
+  // values are there by the time of the fourth instruction after their read)
+  auto tile = [&](int i, int j, Raw raw, SplitPair &o, bool with_mid) {
+    __builtin_amdgcn_sched_barrier(0);
+    mma_split_tile(st.x[i], st.y[j], acc_re[j][i], acc_im[j][i], [&](int n) {
+      if (with_mid && n == 2) mid();
+      if (n >= 5 && n % 2 == 1 && n < 21) split(raw, o, (n - 5) / 2);
+    });
+  };
+  if constexpr (TY == 2) {
+    if constexpr (FIRST) {
+      split_now(rd_y(0), st.y[0]);
+      mid();
+      split_now(rd_x(0), st.x[0]);
+    } else {
+      tile(0, 1, rd_y(0), st.y[0], true);
+      tile(1, 1, rd_x(0), st.x[0], false);
+    }
+    tile(0, 0, rd_x(1), st.x[1], false);
+    tile(1, 0, rd_y(1), st.y[1], false);
+  } else {
+    SplitPair x_next, y_next;
+    Raw raw = rd_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FIRST) {
+      split_now(raw, x_next);
+      mid();
+      split_now(rd_y(0), y_next);
+    } else {
+      mma_split_tile(st.x[TX - 1], st.y[0], acc_re[0][TX - 1], acc_im[0][TX - 1], [&](int n) {
+        if (n == 2) mid();
+        if (n >= 4 && n < 12) split(raw, x_next, n - 4);
+        if (n == 12) raw = rd_y(0);
+        if (n >= 16 && n < 24) split(raw, y_next, n - 16);
+      });
+    }
+    st.x[0] = x_next;
+    st.y[0] = y_next;
+    if constexpr (TX == 2) tile(0, 0, rd_x(1), st.x[1], false);
+  }
+}
+template <int TX, int TY>
+__device__ __forceinline__ void mma_split_last(SplitState<TX, TY> &st, float16_t_ (&acc_re)[TY][TX],
+                                               float16_t_ (&acc_im)[TY][TX]) {
+  if constexpr (TY == 2) {
+    mma_split_tile(st.x[0], st.y[1], acc_re[1][0], acc_im[1][0], [](int) {});
+    mma_split_tile(st.x[1], st.y[1], acc_re[1][1], acc_im[1][1], [](int) {});
+  } else {
+    mma_split_tile(st.x[TX - 1], st.y[0], acc_re[0][TX - 1], acc_im[0][TX - 1], [](int) {});
+  }
+}
+
 // Wide accesses to C at an address that is aligned to its elements only: rows of any
 // length start anywhere, and global memory takes any alignment on this target. Element
 // by element, every store instruction touches 64 lines for 4 bytes each: B=16 255x128x256
@@ -1055,6 +1269,56 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
         }
       }
     }
+  }
+}
+
+// A wave's tile of 32-bit input on the fp32 instructions, straight from global memory, one
+// 32 x 32 tile at a time: for tiles whose split sums are not finite (mma_step32_split).
+template <int TOUT, int LOADER, int TX, int TY>
+__device__ __forceinline__ void recompute_f32(const KernelArgs &args, unsigned b, unsigned x_wave,
+                                              unsigned y_wave, int lane) {
+  constexpr bool IL = (LOADER == kLoadInterleavedVec || LOADER == kLoadInterleavedRagged);
+  constexpr int FROM = LOADER == kLoadTiled ? kLoadTiled : kLoadPlanarElem;
+  const OperandView xv{args.x + (size_t)b * args.x_batch_bytes, args.nx, args.x_tiles, 0};
+  const OperandView yv{args.y + (size_t)b * args.y_batch_bytes, args.ny, args.y_tiles, 0};
+  // the four values K = 16 kt + 4 c .. of a row
+  auto fetch = [&](const OperandView &v, unsigned row, unsigned kt, int c, float4_t &re, float4_t &im) {
+    if constexpr (IL) {
+      row = row < v.rows ? row : v.rows - 1;
+      const float *p = reinterpret_cast<const float *>(v.base + (size_t)row * 2 * args.row_stride_bytes);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned k = kt * 16 + c * 4 + e;
+        re[e] = k < args.k ? p[2 * (size_t)k] : 0.f;
+        im[e] = k < args.k ? p[2 * (size_t)k + 1] : 0.f;
+      }
+    } else {
+      re = __builtin_bit_cast(float4_t, load_chunk<4, FROM>(v, kt, args.k_tiles, args.k_bytes, 0, row, c));
+      im = __builtin_bit_cast(float4_t, load_chunk<4, FROM>(v, kt, args.k_tiles, args.k_bytes, 1, row, c));
+    }
+  };
+  const unsigned k_tiles = (args.k + 15) / 16;
+  for (int t = 0; t < TX * TY; ++t) {
+    const unsigned x0 = x_wave + 32 * (t % TX), y0 = y_wave + 32 * (t / TX);
+    float16_t_ re[1][1], im[1][1];
+    re[0][0] = 0.f;
+    im[0][0] = 0.f;
+    for (unsigned kt = 0; kt < k_tiles; ++kt) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        float4_t xr, xi, yr, yi;
+        fetch(xv, x0 + (lane & 31), kt, (lane >> 5) + 2 * s, xr, xi);
+        fetch(yv, y0 + (lane & 31), kt, (lane >> 5) + 2 * s, yr, yi);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          re[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[e], yr[e], re[0][0], 0, 0, 0);
+          im[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[e], yi[e], im[0][0], 0, 0, 0);
+          re[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xi[e], -yi[e], re[0][0], 0, 0, 0);
+          im[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xi[e], yr[e], im[0][0], 0, 0, 0);
+        }
+      }
+    }
+    store_wave_tile<TOUT, 1, 1, 32>(args, b, x0, y0, lane, re, im);
   }
 }
 
@@ -1569,8 +1833,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   // interleaved operands: one plane of (re, im) rows
   // (their slots hold 128 bytes of every row, fetched as whole cache lines)
   constexpr bool IL = (LOADER == kLoadInterleavedVec || LOADER == kLoadInterleavedRagged);
-  static_assert(MS == 16 || !IL || DtypeTraits<DT>::kElemBytes == 1,
-                "interleaved operands on the 32-row MFMAs: 8-bit input only");
+  static_assert(MS == 16 || !IL || DtypeTraits<DT>::kElemBytes != 2,
+                "interleaved operands on the 32-row MFMAs: 8- and 32-bit input");
   // rows that are no whole aligned 16-byte chunks, see chunk_source and settle_row_ends
   constexpr bool RAGGED = (LOADER == kLoadPlanarRagged || LOADER == kLoadInterleavedRagged);
   constexpr int PLANES = IL ? 1 : 2;
@@ -1661,7 +1925,12 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   unsigned x_tile_off[XL], y_tile_off[YL];   // wave-uniform: the row block inside its operand tile
   unsigned x_lds[XL], y_lds[YL];             // wave-uniform: LDS byte address inside slot 0 of the ring
   const char *x_src[XL], *y_src[YL];         // wave-uniform: K tile 0 of the operand tile (tiled layout)
-  const char *x_lane_src[XL], *y_lane_src[YL];   // planar layouts: this lane's chunk of K tile 0
+  // rows in place: this lane's chunk of K tile 0. The second half of a wave's row blocks are the
+  // imaginary planes of the first half's rows (x_plane, y_plane bytes away).
+  constexpr int XLS = IL || LOADER == kLoadTiled ? XL : XL / 2, YLS = IL || LOADER == kLoadTiled ? YL : YL / 2;
+  static_assert(IL || ((BX / RPB) % NW == 0 && (BY / RPB) % NW == 0), "planes split a wave's row blocks evenly");
+  const char *x_lane_src[XLS], *y_lane_src[YLS];
+  const size_t x_plane = (size_t)args.nx * row_stride, y_plane = (size_t)args.ny * row_stride;
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int q = i * NW + wave, plane = q / (BX / RPB), rb = q % (BX / RPB);
@@ -1680,8 +1949,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     const TileCoord tc = tile_coord(args, vt);
     const char *op = args.x + (size_t)tc.b * args.x_batch_bytes;
 #pragma unroll
-    for (int i = 0; i < XL; ++i) {
-      const int q = i * NW + wave, plane = q / (BX / RPB), rb = q % (BX / RPB);
+    for (int i = 0; i < XLS; ++i) {
+      const int q = i * NW + wave, rb = q % (BX / RPB);
       const unsigned row0 = tc.block_x * BX + rb * RPB;
       if constexpr (LOADER == kLoadTiled) {
         unsigned tile = row0 / kTileRows;
@@ -1692,8 +1961,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       } else {
         unsigned row = row0 + (XT ? xt_row : r);
         row = row < args.nx ? row : args.nx - 1;   // likewise
-        x_lane_src[i] = op + ((size_t)plane * args.nx + row) * row_stride +
-                        (XT ? xt_chunk : c_of(rb)) * 16;
+        x_lane_src[i] = op + (size_t)row * row_stride + (XT ? xt_chunk : c_of(rb)) * 16;
       }
     }
   };
@@ -1702,8 +1970,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     const TileCoord tc = tile_coord(args, vt);
     const char *op = args.y + (size_t)tc.b * args.y_batch_bytes;
 #pragma unroll
-    for (int i = 0; i < YL; ++i) {
-      const int q = i * NW + wave, plane = q / (BY / RPB), rb = q % (BY / RPB);
+    for (int i = 0; i < YLS; ++i) {
+      const int q = i * NW + wave, rb = q % (BY / RPB);
       const unsigned row0 = tc.block_y * BY + rb * RPB;
       if constexpr (LOADER == kLoadTiled) {
         unsigned tile = row0 / kTileRows;
@@ -1714,23 +1982,25 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       } else {
         unsigned row = row0 + r;
         row = row < args.ny ? row : args.ny - 1;
-        y_lane_src[i] = op + ((size_t)plane * args.ny + row) * row_stride + c_of(rb) * 16;
+        y_lane_src[i] = op + (size_t)row * row_stride + c_of(rb) * 16;
       }
     }
   };
-  // Where a lane's chunk of K tile kt comes from when it lies at `src` in K tile 0 of its row.
+  // Where a lane's chunk of K tile kt comes from when it lies at `src` in K tile 0 of its row
+  // (of the plane `plane` bytes away).
   // Rows of whole chunks: it is either inside K or reads zeros. Ragged rows: the chunk
   // that holds the end of the row is fetched as the last 16 bytes of the row instead
   // (nothing outside the row is touched): its elements lie at the chunk's end and
   // in front of them, once more, some that the chunk before holds, until
   // settle_row_ends puts them right.
-  auto chunk_source = [&](const char *src, unsigned kt, int chunk) {
+  auto chunk_source = [&](const char *src, unsigned kt, int chunk, size_t plane) {
     const unsigned end = kt * RB + chunk * 16 + 16;
+    plane += (size_t)kt * RB;
     if constexpr (RAGGED) {
       const unsigned over = end > row_bytes ? end - row_bytes : 0;
-      return over < 16 ? src + (size_t)kt * RB - over : g_zero_tile + lane * 16;
+      return over < 16 ? src + plane - over : g_zero_tile + lane * 16;
     } else {
-      return end <= row_bytes ? src + (size_t)kt * RB : g_zero_tile + lane * 16;
+      return end <= row_bytes ? src + plane : g_zero_tile + lane * 16;
     }
   };
   // issue_*: straight-line code (it is placed between MFMAs, and a branch there
@@ -1744,7 +2014,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         load_1k_to_lds(x_src[i] + (size_t)xs.kt * kTileBytes + x_tile_off[i], lane_off_x, dst);
       } else {
         const int q = i * NW + wave, rb = q % (BX / RPB);
-        load_1k_to_lds_by_lane(chunk_source(x_lane_src[i], xs.kt, XT ? xt_chunk : c_of(rb)), dst);
+        load_1k_to_lds_by_lane(
+            chunk_source(x_lane_src[i % XLS], xs.kt, XT ? xt_chunk : c_of(rb), i < XLS ? 0 : x_plane), dst);
       }
     }
   };
@@ -1756,7 +2027,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         load_1k_to_lds(y_src[i] + (size_t)ys.kt * kTileBytes + y_tile_off[i], lane_off, dst);
       } else {
         const int q = i * NW + wave, rb = q % (BY / RPB);
-        load_1k_to_lds_by_lane(chunk_source(y_lane_src[i], ys.kt, c_of(rb)), dst);
+        load_1k_to_lds_by_lane(chunk_source(y_lane_src[i % YLS], ys.kt, c_of(rb), i < YLS ? 0 : y_plane), dst);
       }
     }
   };
@@ -1866,6 +2137,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   const unsigned iters = k_tiles;
   for (unsigned vt = blockIdx.x; vt < total; vt += gridDim.x) {
     typename AccType<MS>::type acc_re[TY][TX], acc_im[TY][TX];
+    SplitState<DT == kFloat32 ? TX : 1, DT == kFloat32 ? TY : 1> split;   // (32-bit input)
     // (the hand-ordered step of the 16-row MFMAs starts its first iteration from zero itself)
     constexpr bool kStepClears = !IL && DT != kInt1 && MS == 16 && TX == 4 && TY == 4;
     static_assert(!SPLIT || kStepClears, "separate X and Y rings: hand-ordered 16-row step only");
@@ -1879,7 +2151,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       }
     }
-    for (unsigned it = 0; it < iters; ++it) {
+    // One K iteration; `first` says at compile time that it is a C tile's first one (32-bit input).
+    auto iteration = [&](unsigned it, auto first) __attribute__((always_inline)) {
       advance_y();
       advance_x();
       // After the first C tile, the K tiles of the first YLEAD iterations were
@@ -1929,7 +2202,12 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       } else {
         const char *slot_ptr = lds + x_slot_off(x_slot);
-        if constexpr (IL && MS == 32 && TX == 1 && TY == 1) {
+        if constexpr (DT == kFloat32) {
+          static_assert(MS == 32, "32-bit input: 32-row MFMA");
+          const int *x_off = IL ? xil32_off[0] : x32_off, *y_off = IL ? yil32_off[0] : y32_off;
+          mma_step32_split<BX, BY, TX, TY, IL, decltype(first)::value>(slot_ptr, x_off, y_off, split, acc_re,
+                                                                       acc_im, refill_slots);
+        } else if constexpr (IL && MS == 32 && TX == 1 && TY == 1) {
           mma_step32_interleaved_single<DT>(slot_ptr, xil32_off, yil32_off, acc_re, acc_im,
                                             refill_slots);
         } else if constexpr (IL && MS == 32) {
@@ -1960,7 +2238,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       }
       x_slot = x_next;
       y_slot = y_next;
-    }
+    };
+    unsigned it = 0;
+    if constexpr (DT == kFloat32) iteration(it++, std::true_type{});
+    for (; it < iters; ++it) iteration(it, std::false_type{});
     // The stores below are not waited for here: they drain while the next C
     // tile is being computed. The counter cannot tell loads from stores, so
     // the next tile's first K tiles, which are already on their way, are waited
@@ -1969,6 +2250,25 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const TileCoord tc = tile_coord(args, vt);
     const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
+    bool redo = false;   // (32-bit input) this wave's tile is computed again
+    if constexpr (DT == kFloat32) {
+      mma_split_last<TX, TY>(split, acc_re, acc_im);
+      float sum = 0.f;   // not finite as soon as one of the accumulators is not
+#pragma unroll
+      for (int j = 0; j < TY; ++j) {
+#pragma unroll
+        for (int i = 0; i < TX; ++i) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            sum = __builtin_fmaf(acc_re[j][i][e], 0.f, sum);
+            sum = __builtin_fmaf(acc_im[j][i][e], 0.f, sum);
+            acc_re[j][i][e] *= kSplitUnscale;
+            acc_im[j][i][e] *= kSplitUnscale;
+          }
+        }
+      }
+      redo = __any(sum != 0.f);
+    }
     bool staged = false;
     if constexpr (XT) {
       // the accumulators already hold whole row segments
@@ -2022,7 +2322,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         unsigned free_slot = y_slot + YLEAD;
         free_slot = free_slot >= SLOTS ? free_slot - SLOTS : free_slot;
         asm volatile("s_barrier" ::: "memory");
-        if (x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
+        if (!redo && x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
           store_wave_tile_staged32<TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane,
                                            lds + free_slot * SLOT_BYTES + wave * kStagePatch32Bytes,
                                            acc_re, acc_im);
@@ -2030,9 +2330,25 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       }
     }
+    if constexpr (DT == kFloat32) {
+      if (redo) {
+        recompute_f32<TOUT, LOADER, TX, TY>(args, tc.b, x_wave, y_wave, lane);
+        // (its loads and stores are not among those that the next tile's waits count)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        staged = true;
+      }
+    }
     if (!staged) {
       if constexpr (TOUT == kInt32) {
         store_wave_tile_int32<TX, TY, MS>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
+      } else if constexpr (DT == kFloat32) {
+        // (one MFMA tile after the other: the addresses of both at once do not fit the registers)
+#pragma unroll
+        for (int t = 0; t < TX * TY; ++t) {
+          const float16_t_ re[1][1] = {{acc_re[t / TX][t % TX]}}, im[1][1] = {{acc_im[t / TX][t % TX]}};
+          store_wave_tile<TOUT, 1, 1, MS>(args, tc.b, x_wave + 32 * (t % TX), y_wave + 32 * (t / TX), lane, re, im);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       } else {
         store_wave_tile<TOUT, TX, TY, MS>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
       }
@@ -2199,11 +2515,11 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // moves per flop. Times with 256 x 128, 128 x 128 and 64 x 64 blocks in us, on operands that no cache
 // held (profiles/gemm_block_choice.txt):
 //   too few tiles for the larger blocks, 16 bits 256^3:  14.7, 12.5, 6.9;  B=256 96x96x1024:  86, 56, 62;
-//     32 bits B=2 1000^3:  455, 239, 135;  8 bits 1024^3:  24.9, 22.3, 11.5;
+//     32 bits B=2 1000^3:  224, 147, 104;  8 bits 1024^3:  24.9, 22.3, 11.5;
 //     1 bit 64x64x65536:  526, 305, 116
 //   every unit busy, 16 bits on tiles, 4096x4096x512:  68, 89, 102
 //     on planar rows, of which a copy fetches half cache lines, B=157 192x604x3680:  747, 909, 1026
-//     32 bits (bound by the matrix cores at any shape), 4096x4096x512:  480, 495, 503
+//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  312, 358, 426
 //     8 bits on tiles, 4096x4096x512:  48, 48, 69
 //     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
 //       277, 288, 312
@@ -2230,7 +2546,9 @@ struct BlockCosts {
 };
 inline BlockCosts block_costs(const GemmParams &p) {
   if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0};
-  if (p.type_in == kFloat32) return {1.04, 1.04, 10.3, 10.9, 0.0, 0.0, 0.0, 0.0, 0.0};
+  // (32-bit pairs: the 128 x 128 block stands in for the 256 x 128 one)
+  if (p.type_in == kFloat32 && p.input_interleaved) return {1.13, 1.40, 6.0, 4.6, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (p.type_in == kFloat32) return {1.16, 1.52, 9.8, 8.5, 0.0, 0.0, 0.0, 0.0, 0.0};
   const bool planar = p.variant == kBasic && !p.input_interleaved;
   if (bits_of(p.type_in) == 8) {
     if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0};
@@ -2298,25 +2616,45 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   const bool planar_direct = (p.variant == kBasic) && (k_bytes >= 16) && (k_bytes % 16 == 0) &&
                              ((uintptr_t)p.x % 16 == 0) && ((uintptr_t)p.y % 16 == 0);
   const BlockShape shape = block_choice(p).shape;
-  if (p.input_interleaved) {
-    // raw (re, im) rows straight from the caller: the host side only takes this
-    // path for 8- and 16-bit input with rows of at least 16 bytes
-    const bool ragged = 2 * k_bytes % 16 != 0 || (uintptr_t)p.x % 16 != 0 || (uintptr_t)p.y % 16 != 0;
-    if constexpr (DT == kFloat32) {
-      return hipErrorInvalidValue;
-    } else if (ragged) {
+  constexpr bool BITS16 = DtypeTraits<DT>::kElemBytes == 2;
+  constexpr int MS = BITS16 ? 16 : 32;
+  if constexpr (DT == kFloat32) {
+    // 256 x 128 blocks of 8 waves of 64 x 64, 3-slot ring; 128 x 128 of 8 waves of 64 x 32, 4-slot
+    // ring; 64 x 64 of 4 waves of 32 x 32, 5-slot ring, two blocks a unit. The more a wave
+    // computes the fewer elements it splits per matrix instruction: 4096x4096x512 on tiles
+    // 305, 345, 413 us. (Rows of pairs: a wave of 64 x 64 spills 37 registers.)
+    auto launch = [&](auto loader) {
+      constexpr int L = decltype(loader)::value;
+      if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, L, 32>(p, stream);
+      if constexpr (L != kLoadInterleavedVec && L != kLoadInterleavedRagged) {
+        if (shape == k256x128) return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, L, 32>(p, stream);
+      }
+      return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, L, 32>(p, stream);
+    };
+    const bool aligned = (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 16 == 0;
+    if (p.input_interleaved) {
       if (2 * k_bytes < 16) return hipErrorInvalidValue;
-      constexpr int MS = KPM == 1 ? 16 : 32;
+      return aligned && 2 * k_bytes % 16 == 0 ? launch(std::integral_constant<int, kLoadInterleavedVec>{})
+                                              : launch(std::integral_constant<int, kLoadInterleavedRagged>{});
+    }
+    if (p.variant == kOpt) return launch(std::integral_constant<int, kLoadTiled>{});
+    if (planar_direct) return launch(std::integral_constant<int, kLoadPlanarVec>{});
+    if (k_bytes >= 16) return launch(std::integral_constant<int, kLoadPlanarRagged>{});
+  }
+  else if (p.input_interleaved) {
+    // raw (re, im) rows straight from the caller: the host side only takes this
+    // path for rows of at least 16 bytes
+    const bool ragged = 2 * k_bytes % 16 != 0 || (uintptr_t)p.x % 16 != 0 || (uintptr_t)p.y % 16 != 0;
+    if (ragged && 2 * k_bytes < 16) return hipErrorInvalidValue;
+    if (ragged) {
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedRagged, MS>(p, stream);
       if (shape == k128x128) {
-        return launch_dtl<DT, TOUT, 128, 128, 64, KPM == 1 ? 32 : 64, KPM == 1 ? 4 : 2, 2, kLoadInterleavedRagged,
+        return launch_dtl<DT, TOUT, 128, 128, 64, BITS16 ? 32 : 64, BITS16 ? 4 : 2, 2, kLoadInterleavedRagged,
                           MS>(p, stream);
       }
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedRagged, MS>(p, stream);
-    } else if constexpr (KPM == 1) {
-      if constexpr (DtypeTraits<DT>::kElemBytes == 2) {
-        if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT, true>(p, stream);
-      }
+    } else if constexpr (BITS16) {
+      if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT, true>(p, stream);
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec>(p, stream);
       if (shape == k128x128) {
         return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadInterleavedVec>(p, stream);
@@ -2332,14 +2670,14 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec, 32>(p, stream);
     }
   }
-  if (p.variant == kOpt || planar_direct) {
-    if constexpr (KPM == 1 && DtypeTraits<DT>::kElemBytes == 2) {
+  else if (p.variant == kOpt || planar_direct) {
+    if constexpr (BITS16) {
       // 16-bit input, tiled operands, planar C without beta: 192 x 256 block, 4 waves
       // of 192 x 64 (one per SIMD), where that pays
       if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT>(p, stream);
     }
-    if constexpr (KPM == 1) {
-      // 16- and 32-bit input: 256 x 128 block, 8 waves of 64 x 64 (two per SIMD), 3-slot ring.
+    if constexpr (BITS16) {
+      // 16-bit input: 256 x 128 block, 8 waves of 64 x 64 (two per SIMD), 3-slot ring.
       // Interleaved fp32 C: in the exchanged-roles layout a lane's (re, im) pairs of
       // a row lie 32 bytes apart, so every store instruction would write half
       // cache lines; the other layout regroups the tile through LDS into whole
@@ -2385,14 +2723,13 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
                  : launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarVec, 32>(p, stream);
     }
   }
-  if (k_bytes >= 16) {
-    constexpr int MS = KPM == 1 ? 16 : 32;
+  else if (k_bytes >= 16) {
     if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarRagged, MS>(p, stream);
     if (shape == k128x128) {
-      return launch_dtl<DT, TOUT, 128, 128, 64, KPM == 1 ? 32 : 64, KPM == 1 ? 4 : 2, 2, kLoadPlanarRagged,
+      return launch_dtl<DT, TOUT, 128, 128, 64, BITS16 ? 32 : 64, BITS16 ? 4 : 2, 2, kLoadPlanarRagged,
                         MS>(p, stream);
     }
-    return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarRagged, MS, KPM == 1>(p, stream);
+    return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarRagged, MS, BITS16>(p, stream);
   }
   // fp8 stages are twice as large (two K tiles per MFMA): one wave per SIMD
   // with the full register file

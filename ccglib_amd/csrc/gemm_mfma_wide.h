@@ -185,16 +185,6 @@ __device__ __forceinline__ WideTile wide_tile(const KernelArgs &args, unsigned i
 // four), so the chunk swizzles of that layout carry over.
 // ALPHA: the result is multiplied by the complex alpha of the arguments on its way
 // out (both parts of an element sit in the same lane, in acc_re and acc_im).
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in this order.
-template <int... Is, class F>
-__device__ __forceinline__ void static_for_each(std::integer_sequence<int, Is...>, F &&f) {
-  (f(std::integral_constant<int, Is>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F &&f) {
-  static_for_each(std::make_integer_sequence<int, N>{}, f);
-}
-
 // (the lambdas of the kernel: left to its cost estimate, the compiler keeps the larger
 // ones as functions in some instantiations, and the accumulators then live in memory)
 #define CCGLIB_INLINE __attribute__((always_inline))

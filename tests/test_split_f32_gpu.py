@@ -1,0 +1,106 @@
+"""GPU tests of 32-bit input, whose values the kernels split into three bf16: accuracy of fp32
+products over the whole range of the type, and infinities, NaN and sums beyond what the split
+sums hold, on every block shape and operand layout."""
+import numpy as np
+import pytest
+import torch
+
+import ccglib_amd as cc
+from gpu_util import stream, to_device, to_host, transpose_operand
+
+pytestmark = pytest.mark.gpu
+VT = cc.ValueType
+PLANAR, INTERLEAVED = cc.ComplexAxisLocation.complex_planar, cc.ComplexAxisLocation.complex_interleaved
+ROW, COL = cc.MemOrder.row_major, cc.MemOrder.col_major
+LAYOUTS = ["tiled", "planar", "pairs"]
+
+
+def product(layout, block_tile, a, b, beta=0, c=None):
+    """C of planar a [B][2][M][K] and b [B][2][N][K]."""
+    B, _, M, K = a.shape
+    N = b.shape[2]
+    d_c = to_device(np.full((B, 2, M, N), np.nan, np.float32) if c is None else c)
+    with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.pipeline_route, 1), \
+            cc.option(cc.Option.basic_retile, 0):
+        if layout == "pairs":
+            obj = cc.Pipeline(B, M, N, K, 0, stream(), INTERLEAVED, PLANAR, ROW, COL, ROW, VT.float32, VT.float32,
+                              cc.Variant.opt, 1, beta)
+            assert obj.ReadsInPlace()
+            d_a, d_b = (to_device(np.ascontiguousarray(x.transpose(0, 2, 3, 1))) for x in (a, b))
+        else:
+            variant = cc.Variant.opt if layout == "tiled" else cc.Variant.basic
+            obj = cc.GEMM(B, M, N, K, 0, stream(), cc.Precision(VT.float32, VT.float32), variant, beta=beta)
+            d_a, d_b = ((transpose_operand(x.reshape(-1), B, x.shape[2], K, VT.float32)
+                         if layout == "tiled" else to_device(x)) for x in (a, b))
+    obj.Run(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr())
+    torch.cuda.synchronize()
+    return to_host(d_c, np.float32).reshape(B, 2, M, N)
+
+
+def exact(a, b):
+    a, b = a.astype(np.float64), b.astype(np.float64).transpose(0, 1, 3, 2)
+    return np.stack([a[:, 0] @ b[:, 0] - a[:, 1] @ b[:, 1], a[:, 0] @ b[:, 1] + a[:, 1] @ b[:, 0]], 1)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("K", [4, 5, 16, 17, 32, 47, 96, 333])
+def test_accuracy(layout, block_tile, K):
+    B, M, N = 2, 150, 290
+    rng = np.random.default_rng(K)
+    a = rng.standard_normal((B, 2, M, K)).astype(np.float32)
+    b = rng.standard_normal((B, 2, N, K)).astype(np.float32)
+    got, want = product(layout, block_tile, a, b), exact(a, b)
+    # what is left out of a product lies below 2^-23 of it; a sum is rounded 12 times per 16
+    # values of K by up to 2^-24 of a partial sum, which never exceeds the sum of the moduli
+    scale = np.abs(a).astype(np.float64), np.abs(b).astype(np.float64).transpose(0, 1, 3, 2)
+    moduli = np.stack([scale[0][:, 0] @ scale[1][:, 0] + scale[0][:, 1] @ scale[1][:, 1],
+                       scale[0][:, 0] @ scale[1][:, 1] + scale[0][:, 1] @ scale[1][:, 0]], 1)
+    assert np.all(np.abs(got - want) <= moduli * (2.0 ** -23 + 2.0 ** -24 * (12 * (K // 16 + 1) + 1)))
+    # rounding errors of random sign: what fp32 products added up in fp32 show
+    assert np.linalg.norm(got - want) <= 2.0 ** -24 * (2 + 1.5 * np.sqrt(2 * K)) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("exponents", [(-126, 100), (100, -126), (-140, 120), (-60, -60), (39, 39)])
+def test_every_magnitude_is_split_exactly(layout, block_tile, exponents):
+    B, M, N, K = 1, 70, 90, 40
+    rng = np.random.default_rng(7)
+    a = np.ldexp(rng.standard_normal((B, 2, M, K)), exponents[0]).astype(np.float32)
+    b = np.ldexp(rng.standard_normal((B, 2, N, K)), exponents[1]).astype(np.float32)
+    got, want = product(layout, block_tile, a, b), exact(a, b)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [1, 2, 4])
+@pytest.mark.parametrize("beta", [0, 0.5 - 0.25j])
+def test_infinities_nan_and_large_sums(layout, block_tile, beta):
+    B, M, N, K = 2, 140, 270, 50
+    rng = np.random.default_rng(3)
+    a = rng.standard_normal((B, 2, M, K)).astype(np.float32)
+    b = rng.standard_normal((B, 2, N, K)).astype(np.float32)
+    c = rng.standard_normal((B, 2, M, N)).astype(np.float32)
+    a[0, 0, 3, 49], a[0, 1, 130, 0], b[0, 1, 200, 17] = np.inf, -np.inf, np.inf
+    a[1, 0, 70, 5] = np.nan
+    a[1, :, 20] *= np.float32(1e20)      # sums of 1e32, beyond those that the split sums hold
+    b[1, :, 7] *= np.float32(1e12)
+    a[0, 0, 64, 1], b[0, 0, 3, 1] = 3.3e38, 1.5      # overflows to infinity; rounds to infinity as bf16
+    got = product(layout, block_tile, a, b, beta=beta, c=c)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = exact(a, b)
+        if beta:
+            z = beta * (c[:, 0].astype(np.complex128) + 1j * c[:, 1])
+            want += np.stack([z.real, z.imag], 1)
+        want = want.astype(np.float32)
+    # (element a[0, 0, 64, 1] overflows where its product does: nothing but the sign is compared there)
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        same = kind(got) == kind(want)
+        same[0, :, 64] = True
+        assert np.all(same)
+    assert np.isposinf(got[0, 0, 64, 3])
+    finite = np.isfinite(want) & np.isfinite(got)
+    x, y = (np.abs(np.nan_to_num(v, posinf=0, neginf=0)).astype(np.float64) for v in (a, b))
+    bound = np.stack([x.sum(1) @ y.sum(1).transpose(0, 2, 1)] * 2, 1) + 2
+    assert np.all(np.abs(got[finite].astype(np.float64) - want[finite]) <= 2.0 ** -18 * bound[finite])
