@@ -179,6 +179,13 @@ struct ccglib_pipeline {
   hipStream_t lane_stream[kHostLanes] = {};
   void *lane_a[kHostLanes] = {}, *lane_b[kHostLanes] = {}, *lane_c[kHostLanes] = {};
   hipEvent_t caller_ready = nullptr;
+  // Host-pointer Run in one piece: device memory for A, B and C, allocated by the first such
+  // Run of at most kHostKeep bytes and kept. (A call of another thread that meets the lock
+  // taken allocates its own, as larger jobs do: three allocations and releases, and the
+  // wait that a release is, cost 60 us, a few per cent of moving more than that.)
+  static constexpr size_t kHostKeep = (size_t)64 << 20;
+  void *host_buffers = nullptr;
+  std::mutex host_lock;
 };
 
 namespace {
@@ -807,6 +814,7 @@ int ccglib_pipeline_destroy(ccglib_pipeline_t p) {
     if (p->d_b_packed) (void)hipFree(p->d_b_packed);
     if (p->d_a_trans) (void)hipFree(p->d_a_trans);
     if (p->d_b_trans) (void)hipFree(p->d_b_trans);
+    if (p->host_buffers) (void)hipFree(p->host_buffers);
   }
   destroy_host_lanes(p);
   ccglib_pipeline_destroy(p->unfused.load());
@@ -1221,16 +1229,24 @@ int ccglib_pipeline_run_host(ccglib_pipeline_t p, const void *h_a, const void *h
     return rc;
   }
 
-  void *d_a = nullptr, *d_b = nullptr, *d_c = nullptr;
-  e = hipMalloc(&d_a, bytes_a ? bytes_a : 16);
-  if (e == hipSuccess) e = hipMalloc(&d_b, bytes_b ? bytes_b : 16);
-  if (e == hipSuccess) e = hipMalloc(&d_c, bytes_c);
-  if (e == hipSuccess && bytes_a) e = hipMemcpyAsync(d_a, h_a, bytes_a, hipMemcpyHostToDevice, p->stream);
+  // A, B and C one after the other
+  const size_t at_b = ceil_div(bytes_a, 256) * 256, at_c = at_b + ceil_div(bytes_b, 256) * 256;
+  std::unique_lock<std::mutex> lock(p->host_lock, std::defer_lock);
+  const bool keep = at_c + bytes_c <= ccglib_pipeline::kHostKeep && lock.try_lock();
+  void *own = nullptr;
+  void *&buffers = keep ? p->host_buffers : own;
+  if (!buffers) e = hipMalloc(&buffers, at_c + bytes_c);
+  if (e != hipSuccess) {
+    buffers = nullptr;
+    return fail_hip(e, "pipeline host staging");
+  }
+  char *d_a = static_cast<char *>(buffers), *d_b = d_a + at_b, *d_c = d_a + at_c;
+  if (bytes_a) e = hipMemcpyAsync(d_a, h_a, bytes_a, hipMemcpyHostToDevice, p->stream);
   if (e == hipSuccess && bytes_b) e = hipMemcpyAsync(d_b, h_b, bytes_b, hipMemcpyHostToDevice, p->stream);
-  if (e == hipSuccess) {
-    // src/pipeline/Pipeline.cpp:168-172
-    e = p->need_copyin_c ? hipMemcpyAsync(d_c, h_c, bytes_c, hipMemcpyHostToDevice, p->stream)
-                         : hipMemsetAsync(d_c, 0, bytes_c, p->stream);
+  // (src/pipeline/Pipeline.cpp:168-172 clears C where it is not copied in; every kernel writes
+  // all of it then)
+  if (e == hipSuccess && p->need_copyin_c) {
+    e = hipMemcpyAsync(d_c, h_c, bytes_c, hipMemcpyHostToDevice, p->stream);
   }
   if (e != hipSuccess) rc = fail_hip(e, "pipeline host staging");
   if (rc == CCGLIB_OK) rc = ccglib_pipeline_run(p, d_a, d_b, d_c);
@@ -1241,9 +1257,7 @@ int ccglib_pipeline_run_host(ccglib_pipeline_t p, const void *h_a, const void *h
   } else {
     (void)hipStreamSynchronize(p->stream);
   }
-  if (d_a) (void)hipFree(d_a);
-  if (d_b) (void)hipFree(d_b);
-  if (d_c) (void)hipFree(d_c);
+  if (own) (void)hipFree(own);
   return rc;
 }
 
