@@ -642,39 +642,6 @@ __device__ __forceinline__ void mma_step32_bits(const char *slot, const int (&x_
 #undef CCGLIB_PIN
 }
 
-// The same for a wave with one 32 x 32 tile. Every word is expanded for a single tile
-// here, so the vector ALU has about as much to do as the matrix cores; the order of
-// the instructions is left to the compiler.
-template <int BX, int BY, typename Mid>
-__device__ __forceinline__ void mma_step32_bits_single(const char *slot, const int (&x_off)[2],
-                                                       const int (&y_off)[2],
-                                                       float16_t_ (&acc_re)[1][1],
-                                                       float16_t_ (&acc_im)[1][1], Mid &&mid) {
-  constexpr int XP = BX * kTileRowBytes, YP = BY * kTileRowBytes;
-  int4_t xr[2], xi[2], yr[2], yi[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    xr[u] = *reinterpret_cast<const int4_t *>(slot + x_off[u]);
-    yr[u] = *reinterpret_cast<const int4_t *>(slot + y_off[u]);
-    yi[u] = *reinterpret_cast<const int4_t *>(slot + y_off[u] + YP);
-    xi[u] = *reinterpret_cast<const int4_t *>(slot + x_off[u] + XP);
-  }
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    const int u = s >> 2, w = s & 3;
-    const int4_t x0 = expand_bits(xr[u][w]), x1 = expand_bits(xi[u][w]);
-    const int4_t y0 = expand_bits(yr[u][w]), y1 = expand_bits(yi[u][w]);
-    int4_t y1n;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y1n[e] = y1[e] ^ (int)0x88888888u;
-    acc_re[0][0] = mfma_fp4(x0, y0, acc_re[0][0]);
-    acc_im[0][0] = mfma_fp4(x0, y1, acc_im[0][0]);
-    acc_re[0][0] = mfma_fp4(x1, y1n, acc_re[0][0]);
-    acc_im[0][0] = mfma_fp4(x1, y0, acc_im[0][0]);
-    if (s == 0) mid();
-  }
-}
-
 // The same for interleaved operands (rows of (re, im) pairs, as the caller's
 // buffers hold them). With K running over the 2K real numbers of a row,
 //   Re = sum X~ . Y1,  Y1 = (yr, -yi, ...)   and   Im = sum X~ . Y2,  Y2 = (yi, yr, ...)
@@ -904,37 +871,122 @@ __device__ __forceinline__ void mma_step32_interleaved(const char *slot, const i
 #undef CCGLIB_PIN
 }
 
-// The same for a wave with one 32 x 32 tile, in the order of the sums above.
-template <int DT, typename Mid>
-__device__ __forceinline__ void mma_step32_interleaved_single(const char *slot, const int (&x_off)[2][2],
-                                                              const int (&y_off)[2][2],
-                                                              float16_t_ (&acc_re)[1][1],
-                                                              float16_t_ (&acc_im)[1][1], Mid &&mid) {
-  static_assert(DtypeTraits<DT>::kElemBytes == 1, "8-bit input");
-  Fragment32 x[2], raw[2];
+// The K tile of a wave of 32 x 32 in a 64 x 64 block (2 x 2 MFMA tiles of 16 x 16, or one of 32 x 32):
+// eight 16-byte fragments, read from the slot in one iteration and multiplied in the next, while
+// those of the next K tile are read. A lone wave of a SIMD, which is what a small problem
+// has, would otherwise wait for its reads in every iteration (bf16 planar rows, 256^3
+// 6.45 -> 6.27 us, B=4 48x64x1600 19.0 -> 17.9; the loop then runs at the rate at which the copies of
+// half cache lines are issued, and a deeper ring is slower: 9 slots 7.2 and 21.2 us).
+struct SmallTile {
+  int4_t x[4], y[4];
+};
+// x[2 i + p]: 16-row MFMA: fragment i, plane p (pairs: half p of the 128 bytes); 32-row MFMA: chunk i
+// of plane p (pairs: chunk i of half p). The same for y.
+__device__ __forceinline__ void read_small_tile(const char *slot, const int (&x_off)[2][2], const int (&y_off)[2][2],
+                                                SmallTile &t) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int i = 0; i < 2; ++i) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      x[h].v[u] = *reinterpret_cast<const int4_t *>(slot + x_off[h][u]);
-      raw[h].v[u] = *reinterpret_cast<const int4_t *>(slot + y_off[h][u]);
+    for (int p = 0; p < 2; ++p) {
+      t.x[2 * i + p] = *reinterpret_cast<const int4_t *>(slot + x_off[p][i]);
+      t.y[2 * i + p] = *reinterpret_cast<const int4_t *>(slot + y_off[p][i]);
     }
   }
+}
+// For every sum the order of the steps for larger wave tiles.
+template <int DT, bool IL, typename Mid>
+__device__ __forceinline__ void mma_small_tile(const SmallTile &t, float4_t (&acc_re)[2][2], float4_t (&acc_im)[2][2],
+                                               Mid &&mid) {
+  auto frag = [](const int4_t &v) {
+    Fragment<DT> f;
+    f.v[0] = v;
+    return f;
+  };
+  if constexpr (IL) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    Fragment32 ya, yb;
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        Fragment<DT> y1, y2;   // (yr, -yi, ...), (yi, yr, ...)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const unsigned v = (unsigned)t.y[2 * j + h][w];
+          y1.v[0][w] = (int)(v ^ 0x80000000u);
+          y2.v[0][w] = (int)__builtin_amdgcn_alignbit(v, v, 16);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc_re[j][i] = mfma<DT>(frag(t.x[2 * i + h]), y1, acc_re[j][i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc_im[j][i] = mfma<DT>(frag(t.x[2 * i + h]), y2, acc_im[j][i]);
+        if (h == 0 && j == 0) mid();
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const Fragment<DT> yr = frag(t.y[2 * j]), yi = frag(t.y[2 * j + 1]), yin = negate<DT>(yi);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc_re[j][i] = mfma<DT>(frag(t.x[2 * i]), yr, acc_re[j][i]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc_im[j][i] = mfma<DT>(frag(t.x[2 * i]), yi, acc_im[j][i]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc_re[j][i] = mfma<DT>(frag(t.x[2 * i + 1]), yin, acc_re[j][i]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc_im[j][i] = mfma<DT>(frag(t.x[2 * i + 1]), yr, acc_im[j][i]);
+      if (j == 0) mid();
+    }
+  }
+}
+template <int DT, bool IL, typename Mid>
+__device__ __forceinline__ void mma_small_tile(const SmallTile &t, float16_t_ (&acc_re)[1][1],
+                                               float16_t_ (&acc_im)[1][1], Mid &&mid) {
+  if constexpr (DT == kInt1) {
+    // (every word is expanded for a single tile: the vector ALU has about as much to do as the
+    // matrix cores)
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int u = 2 * (s >> 2), w = s & 3;
+      const int4_t x0 = expand_bits(t.x[u][w]), x1 = expand_bits(t.x[u + 1][w]);
+      const int4_t y0 = expand_bits(t.y[u][w]), y1 = expand_bits(t.y[u + 1][w]);
+      int4_t y1n;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y1n[e] = y1[e] ^ (int)0x88888888u;
+      acc_re[0][0] = mfma_fp4(x0, y0, acc_re[0][0]);
+      acc_im[0][0] = mfma_fp4(x0, y1, acc_im[0][0]);
+      acc_re[0][0] = mfma_fp4(x1, y1n, acc_re[0][0]);
+      acc_im[0][0] = mfma_fp4(x1, y0, acc_im[0][0]);
+      if (s == 0) mid();
+    }
+  } else if constexpr (IL) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      Fragment32 x{{t.x[h], t.x[2 + h]}}, ya, yb;   // (yr, -yi, ...), (yi, yr, ...)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const unsigned v = (unsigned)t.y[2 * u + h][w];
+          ya.v[u][w] = (int)(v ^ 0x80008000u);
+          yb.v[u][w] = (int)__builtin_amdgcn_perm(v, v, 0x02030001u);
+        }
+      }
+      acc_re[0][0] = mfma32<DT>(x, ya, acc_re[0][0]);
+      acc_im[0][0] = mfma32<DT>(x, yb, acc_im[0][0]);
+      if (h == 0) mid();
+    }
+  } else {
+    const Fragment32 xr{{t.x[0], t.x[2]}}, xi{{t.x[1], t.x[3]}}, yr{{t.y[0], t.y[2]}}, yi{{t.y[1], t.y[3]}};
+    Fragment32 yin;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const unsigned v = (unsigned)raw[h].v[u][w];
-        ya.v[u][w] = (int)(v ^ 0x80008000u);                               // (yr, -yi, ...)
-        yb.v[u][w] = (int)__builtin_amdgcn_perm(v, v, 0x02030001u);        // (yi, yr, ...)
-      }
+      for (int w = 0; w < 4; ++w) yin.v[u][w] = yi.v[u][w] ^ (int)DtypeTraits<DT>::kSignMask;
     }
-    acc_re[0][0] = mfma32<DT>(x[h], ya, acc_re[0][0]);
-    acc_im[0][0] = mfma32<DT>(x[h], yb, acc_im[0][0]);
-    if (h == 0) mid();
+    acc_re[0][0] = mfma32<DT>(xr, yr, acc_re[0][0]);
+    acc_im[0][0] = mfma32<DT>(xr, yi, acc_im[0][0]);
+    mid();
+    acc_re[0][0] = mfma32<DT>(xi, yin, acc_re[0][0]);
+    acc_im[0][0] = mfma32<DT>(xi, yr, acc_im[0][0]);
   }
 }
 
@@ -1769,9 +1821,12 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
 // ---------------------------------------------------------------------------
 __device__ __attribute__((aligned(256))) char g_zero_tile[kTileBytes];
 
-template <int N> __device__ __forceinline__ void wait_vmcnt_then_barrier() {
+// READS: the wave's reads of LDS are waited for as well (their slot is refilled behind the barrier).
+template <int N, bool READS = false> __device__ __forceinline__ void wait_vmcnt_then_barrier() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-  if constexpr (kAblateBarrier) {
+  if constexpr (READS) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  } else if constexpr (kAblateBarrier) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
@@ -1879,6 +1934,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     return SPLIT ? XSLOTS * X_BYTES + s * Y_BYTES : s * SLOT_BYTES + X_BYTES;
   };
 
+  constexpr bool SMALL = BX == 64 && BY == 64 && DT != kFloat32;   // (see SmallTile)
+  static_assert(!SMALL || TX * MS == 32, "waves of 32 x 32");
+
   extern __shared__ __attribute__((aligned(1024))) char lds[];
 
   const int lane = threadIdx.x & 63;
@@ -1943,10 +2001,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     y_tile_off[i] = plane * kTilePlaneBytes + ((rb * RPB) % kTileRows) * kTileRowBytes;
     y_lds[i] = lds_base + y_slot_off(0) + q * 1024;
   }
-  // Points one side of the copy at the operand tile of C tile vt.
-  auto point_x = [&](unsigned vt) {
-    if (vt >= total) return;
-    const TileCoord tc = tile_coord(args, vt);
+  // Points one side of the copy at the operand tile of a C tile.
+  auto point_x = [&](const TileCoord &tc) {
     const char *op = args.x + (size_t)tc.b * args.x_batch_bytes;
 #pragma unroll
     for (int i = 0; i < XLS; ++i) {
@@ -1965,9 +2021,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       }
     }
   };
-  auto point_y = [&](unsigned vt) {
-    if (vt >= total) return;
-    const TileCoord tc = tile_coord(args, vt);
+  auto point_y = [&](const TileCoord &tc) {
     const char *op = args.y + (size_t)tc.b * args.y_batch_bytes;
 #pragma unroll
     for (int i = 0; i < YLS; ++i) {
@@ -2035,14 +2089,31 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     if (++xs.kt == k_tiles) {
       xs.kt = 0;
       xs.tile += gridDim.x;
-      point_x(xs.tile);
+      if (xs.tile < total) point_x(tile_coord(args, xs.tile));
     }
   };
   auto advance_y = [&] {
     if (++ys.kt == k_tiles) {
       ys.kt = 0;
       ys.tile += gridDim.x;
-      point_y(ys.tile);
+      if (ys.tile < total) point_y(tile_coord(args, ys.tile));
+    }
+  };
+  // both, with one look at the coordinates (X and Y walk together unless their rings differ)
+  auto advance = [&] {
+    if constexpr (SPLIT) {
+      advance_y();
+      advance_x();
+    } else if (++xs.kt == k_tiles) {
+      xs.kt = ys.kt = 0;
+      xs.tile = ys.tile = xs.tile + gridDim.x;
+      if (xs.tile < total) {
+        const TileCoord tc = tile_coord(args, xs.tile);
+        point_y(tc);
+        point_x(tc);
+      }
+    } else {
+      ys.kt = xs.kt;
     }
   };
 
@@ -2110,24 +2181,50 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       yil32_off[h][u] = X_BYTES + (wy * WY) * 128 + off;
     }
   }
+  // (64 x 64 blocks) the lane's fragments, see SmallTile: [plane or half][fragment or chunk]
+  int small_x[2][2], small_y[2][2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      small_x[p][i] = IL ? (MS == 32 ? xil32_off[p][i] : xil_off[p] + i * 16 * 128)
+                         : (MS == 32 ? x32_off[i] : x_frag_off + i * 16 * kTileRowBytes) + p * BX * kTileRowBytes;
+      small_y[p][i] = IL ? (MS == 32 ? yil32_off[p][i] : yil_off[p] + i * 16 * 128)
+                         : (MS == 32 ? y32_off[i] : y_frag_off + i * 16 * kTileRowBytes) + p * BY * kTileRowBytes;
+    }
+  }
   // wide stores through LDS: no beta term (interleaved C only with the 16-row layout)
   const bool staged_ok = (MS == 16 || !args.c_interleaved) && !args.have_beta;
 
   // ---- pipeline ----------------------------------------------------------
-  point_x(xs.tile);
-  point_y(ys.tile);
-  // The bookkeeping of the copy (advance_*, which branches) is done at the top of
+  {
+    const TileCoord tc = tile_coord(args, blockIdx.x);
+    point_x(tc);
+    point_y(tc);
+  }
+  // The bookkeeping of the copy (advance, which branches) is done at the top of
   // an iteration for the copies issued inside it, so that nothing but
   // straight-line code follows the barrier. Before the first iteration: the
-  // requests that iterations -XLEAD .. -1 would have made, in their order.
+  // requests that iterations -XLEAD .. -1 would have made, in their order (as a loop: written
+  // out, they are most of the code that a block fetches on the way to its first product;
+  // with one look at the coordinates instead of two 64x64x32 4.66 -> 4.23 us, 256^3 7.05 -> 6.45).
+  if constexpr (SPLIT) {
 #pragma unroll
-  for (int t = -XLEAD; t < 0; ++t) {
-    if (t + YLEAD >= 0) {
-      if (t + YLEAD > 0) advance_y();
-      issue_y(t + YLEAD);
+    for (int t = -XLEAD; t < 0; ++t) {
+      if (t + YLEAD >= 0) {
+        if (t + YLEAD > 0) advance_y();
+        issue_y(t + YLEAD);
+      }
+      if (t + XLEAD > 0) advance_x();
+      issue_x(t + XLEAD);
     }
-    if (t + XLEAD > 0) advance_x();
-    issue_x(t + XLEAD);
+  } else {
+#pragma unroll 1
+    for (unsigned t = 0; t < (unsigned)XLEAD; ++t) {
+      if (t > 0) advance();
+      issue_y(t);
+      issue_x(t);
+    }
   }
   unsigned x_slot = 0, y_slot = 0;         // slots of the current iteration
   // (hand-ordered 16-row step) the lane's fragment addresses in the current slots
@@ -2138,6 +2235,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   for (unsigned vt = blockIdx.x; vt < total; vt += gridDim.x) {
     typename AccType<MS>::type acc_re[TY][TX], acc_im[TY][TX];
     SplitState<DT == kFloat32 ? TX : 1, DT == kFloat32 ? TY : 1> split;   // (32-bit input)
+    SmallTile small;                                                      // (64 x 64 blocks)
     // (the hand-ordered step of the 16-row MFMAs starts its first iteration from zero itself)
     constexpr bool kStepClears = !IL && DT != kInt1 && MS == 16 && TX == 4 && TY == 4;
     static_assert(!SPLIT || kStepClears, "separate X and Y rings: hand-ordered 16-row step only");
@@ -2151,18 +2249,22 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       }
     }
-    // One K iteration; `first` says at compile time that it is a C tile's first one (32-bit input).
+    // One K iteration; `first` says at compile time that it is a C tile's first one (kCarries:
+    // kernels that multiply a K tile while they read the next one).
     auto iteration = [&](unsigned it, auto first) __attribute__((always_inline)) {
-      advance_y();
-      advance_x();
+      advance();
       // After the first C tile, the K tiles of the first YLEAD iterations were
       // already waited for before the previous epilogue (see below), so these
       // iterations only need the barrier; waiting on the counter here would
       // wait for the previous tile's C stores, which are younger than them.
       if (vt != blockIdx.x && it < (unsigned)YLEAD) {
-        asm volatile("s_barrier" ::: "memory");
+        if constexpr (SMALL) {
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        } else {
+          asm volatile("s_barrier" ::: "memory");
+        }
       } else {
-        wait_vmcnt_then_barrier<kOutstandingOk>();
+        wait_vmcnt_then_barrier<kOutstandingOk, SMALL>();
       }
       if constexpr (RAGGED) {
         if (it + 1 == iters && row_bytes % 16 != 0) settle_row_ends(x_slot, y_slot);
@@ -2202,14 +2304,20 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       } else {
         const char *slot_ptr = lds + x_slot_off(x_slot);
-        if constexpr (DT == kFloat32) {
+        if constexpr (SMALL) {
+          SmallTile next;
+          read_small_tile(slot_ptr, small_x, small_y, next);
+          if constexpr (decltype(first)::value) {
+            refill_slots();
+          } else {
+            mma_small_tile<DT, IL>(small, acc_re, acc_im, refill_slots);
+          }
+          small = next;
+        } else if constexpr (DT == kFloat32) {
           static_assert(MS == 32, "32-bit input: 32-row MFMA");
           const int *x_off = IL ? xil32_off[0] : x32_off, *y_off = IL ? yil32_off[0] : y32_off;
           mma_step32_split<BX, BY, TX, TY, IL, decltype(first)::value>(slot_ptr, x_off, y_off, split, acc_re,
                                                                        acc_im, refill_slots);
-        } else if constexpr (IL && MS == 32 && TX == 1 && TY == 1) {
-          mma_step32_interleaved_single<DT>(slot_ptr, xil32_off, yil32_off, acc_re, acc_im,
-                                            refill_slots);
         } else if constexpr (IL && MS == 32) {
           static_assert(TX == 2 && TY == 2, "2 x 2 tiles of 32 x 32 per wave");
           mma_step32_interleaved<DT, BX, BY>(slot_ptr, xil32_off, yil32_off, acc_re, acc_im,
@@ -2222,9 +2330,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
                                                    refill_slots);
         } else {
           const char *tile[KPM] = {slot_ptr};
-          if constexpr (DT == kInt1 && TX == 1 && TY == 1) {
-            mma_step32_bits_single<BX, BY>(tile[0], x32_off, y32_off, acc_re, acc_im, refill_slots);
-          } else if constexpr (DT == kInt1) {
+          if constexpr (DT == kInt1) {
             static_assert(MS == 32 && TX == 2 && TY == 2, "2 x 2 tiles of 32 x 32 per wave");
             mma_step32_bits<BX, BY>(tile[0], x32_off, y32_off, acc_re, acc_im, refill_slots);
           } else if constexpr (MS == 32 && TX == 2 && TY == 2) {
@@ -2240,8 +2346,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       y_slot = y_next;
     };
     unsigned it = 0;
-    if constexpr (DT == kFloat32) iteration(it++, std::true_type{});
+    constexpr bool kCarries = SMALL || DT == kFloat32;
+    if constexpr (kCarries) iteration(it++, std::true_type{});
     for (; it < iters; ++it) iteration(it, std::false_type{});
+    if constexpr (SMALL) mma_small_tile<DT, IL>(small, acc_re, acc_im, [] {});
     // The stores below are not waited for here: they drain while the next C
     // tile is being computed. The counter cannot tell loads from stores, so
     // the next tile's first K tiles, which are already on their way, are waited
