@@ -2639,7 +2639,8 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // slower by 0.95 to several times, 1.37 (128 x 128) and 2.9 (64 x 64) at the median.
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
 // 30000 problems of random sizes, 40 % of them on operands that no cache held
-// (python -m ccglib_amd.tuning.block_choice times such problems): the choice is then on average
+// (python -m ccglib_amd.tuning.block_choice times such problems); those of 32-bit input, 8-bit tiles
+// and 16-bit pairs to 1900 further ones, timed since those kernels last changed. The choice is then on average
 // 0.2 % behind the fastest of the three shapes, and more than 8 % behind in 0.7 % of the problems.
 enum BlockShape { k256x128, k128x128, k64x64 };
 struct BlockChoice {
@@ -2661,9 +2662,9 @@ inline BlockCosts block_costs(const GemmParams &p) {
   if (bits_of(p.type_in) == 8) {
     if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0};
     if (planar) return {1.30, 2.54, 7.6, 7.9, 0.3, 0.1, 13.0, 10.0, 1.0};
-    return {1.05, 1.49, 9.2, 13.6, 0.3, 0.1, 13.0, 10.0, 1.0};
+    return {1.05, 1.61, 9.2, 9.4, 0.3, 0.11, 13.0, 10.0, 1.0};
   }
-  if (p.input_interleaved) return {1.19, 1.90, 11.7, 8.8, 0.0, 0.25, 12.0, 8.0, 6.0};
+  if (p.input_interleaved) return {1.19, 1.80, 11.7, 7.6, 0.0, 0.35, 12.0, 8.0, 6.0};
   if (planar) return {1.24, 2.58, 12.6, 6.8, 0.0, 0.25, 12.0, 8.0, 6.0};
   return {1.30, 1.71, 11.0, 10.1, 0.0, 0.25, 12.0, 8.0, 6.0};
 }
