@@ -2354,8 +2354,14 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     // tile is being computed. The counter cannot tell loads from stores, so
     // the next tile's first K tiles, which are already on their way, are waited
     // for now; the first wait that has to include the stores then comes YLEAD
-    // iterations into the next tile.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // iterations into the next tile. (64 x 64 blocks: the wave's reads of the last slot as well,
+    // which the compiler waits for no sooner than at its last matrix instructions, behind the
+    // epilogue's barrier if it moves those there; other waves write to that slot behind the barrier.)
+    if constexpr (SMALL) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
     const TileCoord tc = tile_coord(args, vt);
     const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     bool redo = false;   // (32-bit input) this wave's tile is computed again
