@@ -78,17 +78,16 @@ def _no_scratch_in_gemm_kernels(src, remarks):
     loop. The compiler's resource remarks say whether a kernel spills registers to scratch
     memory. The one-wave-per-SIMD kernels (complex_gemm_mfma_wide) run at the edge of the
     register file and must not spill at all: the build stops if one does. Of the others, the
-    1-bit 128 x 128 kernel and the 256 x 128 one of 32-bit planar rows spill values at set-up
-    (4 and up to 13) and reload them where a block moves to its next C tile (the compiler
-    waits for all memory operations there); anything beyond those few bytes stops the
-    build as well."""
+    1-bit 128 x 128 kernel spills four values at set-up and reloads them where a block moves
+    to its next C tile (the compiler waits for all memory operations there); anything beyond
+    those few bytes stops the build as well."""
     name = None
     for l in remarks:
         if "Function Name:" in l:
             name = l.split("Function Name:")[1].split("[")[0].strip()
         elif "ScratchSize [bytes/lane]:" in l and name and "complex_gemm_mfma" in name:
             size = int(l.split("ScratchSize [bytes/lane]:")[1].split("[")[0])
-            if size > (0 if "complex_gemm_mfma_wide" in name else 64):
+            if size > (0 if "complex_gemm_mfma_wide" in name else 32):
                 os.remove(os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o"))
                 raise RuntimeError("%s: kernel %s spills %d bytes per lane to scratch memory; its "
                                    "explicit vmcnt counts would not hold" % (src, name, size))

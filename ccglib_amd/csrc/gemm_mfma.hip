@@ -29,6 +29,7 @@
 //  * Workgroup ids are remapped so that consecutive tiles land on the same
 //    XCD (shared L2), in groups that reuse both operands.
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -992,18 +993,24 @@ __device__ __forceinline__ void mma_small_tile(const SmallTile &t, float16_t_ (&
 
 // 32-bit input on the bf16 instruction. x = h + m + l, each of the three a bf16 (8 of the 24
 // significant bits; what rounding to nearest takes too much or too little the next
-// part gives back), and of the nine products of two such sums the six down to 2^-16 of
-// the largest are added up: what is left out lies below 2^-24 of the product, less than the
-// rounding of the sum. Six 32x32x16 instructions take the time of six sixteenths of the
-// fp32 ones they stand for (2.5 PFLOP/s dense against 0.157), and round the sum 6 times
-// per 16 products instead of up to 16 times. N(0, 1) operands, relative error of the result against 64
-// bits, fp32 instructions and these: K = 32 1.5e-7, 1.1e-7; K = 1000 8.0e-7, 7.0e-7; K = 8192
-// 2.3e-6, 2.1e-6. Times, tiles of both: 4096x4096x512 480 and 305 us; planar B=2 1000^3 134 and 112.
+// part gives back), and of the nine products of two such sums all but l * l, which lies below
+// 2^-33 of the largest, are added up. The product h * h, which has 16 bits, goes into one
+// accumulator, the seven others into a second one, of 2^-8 of its size; the two are added when K is
+// through. So nothing of a single product is lost but in that last addition, as on the fp32
+// instructions, and the large sum is rounded twice per 16 values of K and part. (In one accumulator,
+// and with six products, every small product rounds the whole sum - and the instruction drops what of a
+// smaller sum lies below half a unit of its largest product: one product of two numbers was off by
+// up to 1.4 units in the last place.) N(0, 1) operands, relative error of the result against 64
+// bits, fp32 instructions and these: K = 1 3.1e-8, 2.6e-8; K = 32 1.4e-7, 4.9e-8; K = 1000
+// 8.0e-7, 2.7e-7; K = 8192 2.3e-6, 8.3e-7; a single product 0.5 units in the last place either way.
+// Eight 32x32x16 instructions take the time of half of the fp32 ones they stand for (2.5 PFLOP/s
+// dense against 0.157). Planar pipelines, fp32 instructions, these, and one accumulator with six products,
+// in us: 4096x4096x512 496, 421, 316; 8192x8192x1024 3740, 3250, 2400; B=2 1000^3 134, 128, 111.
 //   Both operands are scaled by 2^24 first and the result by 2^-48, so that no part of a
-// small number falls below the range of a bf16: the split is exact for every finite
-// float. What the instructions cannot do is an infinity, a NaN (their parts are NaN) or a sum
-// beyond 2^80: the accumulators are then not finite, and the wave computes its tile
-// again with the fp32 instructions (recompute_f32).
+// small number falls below the range of a bf16: the split is exact for every magnitude up to 2^104.
+// What the instructions cannot do is an infinity, a NaN or a larger number (their parts are
+// infinite or NaN) or a sum beyond 2^80: the accumulators are then not finite, and the wave computes
+// its tile again with the fp32 instructions (recompute_f32).
 //   The splitting, 13 vector instructions for two elements, runs in every wave that reads an
 // element (split tiles would take half as much LDS again) and in the shadow of the matrix
 // instructions: those of a K tile are issued while the next one is split (see
@@ -1044,78 +1051,83 @@ __device__ __forceinline__ void split_step(float (&x)[8], SplitF32 &o, int s) {
     pack(o.l);
   }
 }
-__device__ __forceinline__ SplitF32 negate(const SplitF32 &f) {
-  SplitF32 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    r.h[i] = f.h[i] ^ (int)0x80008000u;
-    r.m[i] = f.m[i] ^ (int)0x80008000u;
-    r.l[i] = f.l[i] ^ (int)0x80008000u;
-  }
-  return r;
+// products 0 to 7: l h, l m, m l, m m, m h, h l, h m, and h h, which goes into an accumulator of its own
+constexpr int kSplitProducts = 8;
+template <int P> __device__ __forceinline__ const int4_t &split_x(const SplitF32 &x) {
+  return P < 2 ? x.l : P < 5 ? x.m : x.h;
 }
-// product P of the six, smallest first
 template <int P>
-__device__ __forceinline__ float16_t_ mfma_split(const SplitF32 &x, const SplitF32 &y, float16_t_ acc) {
-  const int4_t &a = P == 0 ? x.l : P == 2 || P == 3 ? x.m : x.h;
-  const int4_t &b = P == 1 ? y.l : P == 2 || P == 4 ? y.m : y.h;
+__device__ __forceinline__ float16_t_ mfma_split(const int4_t &a, const SplitF32 &y, float16_t_ acc) {
+  const int4_t &b = P == 2 || P == 5 ? y.l : P == 1 || P == 3 || P == 6 ? y.m : y.h;
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                  __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
 }
 struct SplitPair {   // (re, im) fragments of 32 rows
   SplitF32 re, im;
 };
+struct SplitSum {    // of the products h h; of the others
+  float16_t_ large, small;
+};
 
-// The 24 instructions of one 32 x 32 tile and K tile, in turn for its two sums (one that adds
+// The 32 instructions of one 32 x 32 tile and K tile, in turn for its two parts (one that adds
 // to the result of the one before waits for it); behind(n) is issued behind the n-th.
 template <class F>
-__device__ __forceinline__ void mma_split_tile(const SplitPair &x, const SplitPair &y, float16_t_ &acc_re,
-                                               float16_t_ &acc_im, F &&behind) {
+__device__ __forceinline__ void mma_split_tile(const SplitPair &x, const SplitPair &y, SplitSum &re, SplitSum &im,
+                                               F &&behind) {
 #define CCGLIB_PIN __builtin_amdgcn_sched_barrier(0)
-  static_for<6>([&](auto product) {
+  auto sum = [](SplitSum &s, auto product) -> float16_t_ & {
+    return decltype(product)::value == kSplitProducts - 1 ? s.large : s.small;
+  };
+  static_for<kSplitProducts>([&](auto product) {
     constexpr int P = decltype(product)::value;
-    acc_re = mfma_split<P>(x.re, y.re, acc_re);
+    const int4_t &a = split_x<P>(x.re);
+    sum(re, product) = mfma_split<P>(a, y.re, sum(re, product));
     behind(2 * P);
     CCGLIB_PIN;
-    acc_im = mfma_split<P>(x.re, y.im, acc_im);
+    sum(im, product) = mfma_split<P>(a, y.im, sum(im, product));
     behind(2 * P + 1);
     CCGLIB_PIN;
   });
-  const SplitF32 minus = negate(x.im);
-  static_for<6>([&](auto product) {
-    constexpr int P = decltype(product)::value;
-    acc_im = mfma_split<P>(x.im, y.re, acc_im);
-    behind(12 + 2 * P);
+  int4_t minus;
+  static_for<kSplitProducts>([&](auto product) {
+    constexpr int P = decltype(product)::value, N = 2 * kSplitProducts;
+    const int4_t &a = split_x<P>(x.im);
+    if constexpr (P == 0 || P == 2 || P == 5) {   // (the first product of a part of x)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) minus[i] = a[i] ^ (int)0x80008000u;
+    }
+    sum(im, product) = mfma_split<P>(a, y.re, sum(im, product));
+    behind(N + 2 * P);
     CCGLIB_PIN;
-    acc_re = mfma_split<P>(minus, y.im, acc_re);
-    behind(13 + 2 * P);
+    sum(re, product) = mfma_split<P>(minus, y.im, sum(re, product));
+    behind(N + 2 * P + 1);
     CCGLIB_PIN;
   });
 #undef CCGLIB_PIN
 }
 
-// What a wave carries from one K iteration to the next: the split fragments of the last K tile.
-template <int TX, int TY> struct SplitState {
-  SplitPair x[TX], y[TY];
+// What a wave carries from one K iteration to the next: the split fragments of the last K
+// tile, and its sums.
+template <int TX> struct SplitState {
+  SplitPair x[TX], y;
+  SplitSum re[TX], im[TX];
 };
 
-// One K iteration of a wave with TX x TY tiles of 32 x 32 (1 x 1, 2 x 1, 2 x 2): reads the K tile
+// One K iteration of a wave with TX tiles of 32 x 32 side by side (1 or 2): reads the K tile
 // of `slot` and splits it, a fragment at a time, behind the instructions of one tile, those
-// of the K tile before among them (FIRST: there is none); its last tiles' instructions
-// follow in the next iteration, or in mma_split_last. With 2 x 2 tiles every fragment is
-// overwritten right behind its last use.
+// of the K tile before among them (FIRST: there is none); its last tile's instructions
+// follow in the next iteration, or in mma_split_last.
 // A lane's 8 values of a row are its two 16-byte chunks (of either plane), or every other
 // word of its four (IL: 128 bytes of pairs, off[2 h + u]).
-template <int BX, int BY, int TX, int TY, bool IL, bool FIRST, typename Mid>
-__device__ __forceinline__ void mma_step32_split(const char *slot, const int *x_off, const int *y_off,
-                                                 SplitState<TX, TY> &st, float16_t_ (&acc_re)[TY][TX],
-                                                 float16_t_ (&acc_im)[TY][TX], Mid &&mid) {
-  static_assert(TX >= TY && TX <= 2, "1 x 1, 2 x 1 or 2 x 2 tiles");
+template <int BX, int BY, int TX, bool IL, bool FIRST, typename Mid>
+__device__ __forceinline__ void mma_step32_split(const char *slot, const int (&x_off)[4], const int (&y_off)[4],
+                                                 SplitState<TX> &st, Mid &&mid) {
+  static_assert(TX == 1 || TX == 2, "1 x 1 or 2 x 1 tiles");
   constexpr int ROW32 = 32 * (IL ? 128 : kTileRowBytes);
   struct Raw {
     float re[8], im[8];
   };
-  auto rd = [&](const int *off, int extra, int plane_bytes) {
+  auto rd = [&](const int (&off)[4], int extra, int plane_bytes) {
     Raw r;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -1131,7 +1143,7 @@ __device__ __forceinline__ void mma_step32_split(const char *slot, const int *x_
     return r;
   };
   auto rd_x = [&](int i) { return rd(x_off, i * ROW32, BX * kTileRowBytes); };
-  auto rd_y = [&](int j) { return rd(y_off, j * ROW32, BY * kTileRowBytes); };
+  auto rd_y = [&] { return rd(y_off, 0, BY * kTileRowBytes); };
   // step s of 8: the real part, then the imaginary one
   auto split = [](Raw &r, SplitPair &o, int s) {
     split_step(s < 4 ? r.re : r.im, s < 4 ? o.re : o.im, s & 3);
@@ -1141,56 +1153,52 @@ __device__ __forceinline__ void mma_step32_split(const char *slot, const int *x_
     for (int s = 0; s < 8; ++s) split(r, o, s);
     __builtin_amdgcn_sched_barrier(0);
   };
-  // the instructions of tile (i, j), and behind them the split of one fragment (whose raw
-  // values are there by the time of the fourth instruction after their read)
-  auto tile = [&](int i, int j, Raw raw, SplitPair &o, bool with_mid) {
-    __builtin_amdgcn_sched_barrier(0);
-    mma_split_tile(st.x[i], st.y[j], acc_re[j][i], acc_im[j][i], [&](int n) {
-      if (with_mid && n == 2) mid();
-      if (n >= 5 && n % 2 == 1 && n < 21) split(raw, o, (n - 5) / 2);
-    });
+  // the split's eight steps behind instructions n0, n0 + 1, n0 + 3, n0 + 4, n0 + 6, ...
+  auto split_behind = [&](Raw &r, SplitPair &o, int n, int n0) {
+    if (n >= n0 && n < n0 + 12 && (n - n0) % 3 < 2) split(r, o, (n - n0) / 3 * 2 + (n - n0) % 3);
   };
-  if constexpr (TY == 2) {
-    if constexpr (FIRST) {
-      split_now(rd_y(0), st.y[0]);
-      mid();
-      split_now(rd_x(0), st.x[0]);
-    } else {
-      tile(0, 1, rd_y(0), st.y[0], true);
-      tile(1, 1, rd_x(0), st.x[0], false);
-    }
-    tile(0, 0, rd_x(1), st.x[1], false);
-    tile(1, 0, rd_y(1), st.y[1], false);
+  // (the raw values of a read are there by the time of the fourth instruction after it)
+  SplitPair x_next, y_next;
+  Raw raw = rd_x(0);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (FIRST) {
+    split_now(raw, x_next);
+    mid();
+    split_now(rd_y(), y_next);
   } else {
-    SplitPair x_next, y_next;
-    Raw raw = rd_x(0);
+    mma_split_tile(st.x[TX - 1], st.y, st.re[TX - 1], st.im[TX - 1], [&](int n) {
+      if (n == 2) mid();
+      split_behind(raw, x_next, n, 4);
+      if (n == 16) raw = rd_y();
+      split_behind(raw, y_next, n, 20);
+    });
+  }
+  st.x[0] = x_next;
+  st.y = y_next;
+  if constexpr (TX == 2) {
+    raw = rd_x(1);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (FIRST) {
-      split_now(raw, x_next);
-      mid();
-      split_now(rd_y(0), y_next);
-    } else {
-      mma_split_tile(st.x[TX - 1], st.y[0], acc_re[0][TX - 1], acc_im[0][TX - 1], [&](int n) {
-        if (n == 2) mid();
-        if (n >= 4 && n < 12) split(raw, x_next, n - 4);
-        if (n == 12) raw = rd_y(0);
-        if (n >= 16 && n < 24) split(raw, y_next, n - 16);
-      });
-    }
-    st.x[0] = x_next;
-    st.y[0] = y_next;
-    if constexpr (TX == 2) tile(0, 0, rd_x(1), st.x[1], false);
+    mma_split_tile(st.x[0], st.y, st.re[0], st.im[0], [&](int n) { split_behind(raw, st.x[1], n, 5); });
   }
 }
-template <int TX, int TY>
-__device__ __forceinline__ void mma_split_last(SplitState<TX, TY> &st, float16_t_ (&acc_re)[TY][TX],
-                                               float16_t_ (&acc_im)[TY][TX]) {
-  if constexpr (TY == 2) {
-    mma_split_tile(st.x[0], st.y[1], acc_re[1][0], acc_im[1][0], [](int) {});
-    mma_split_tile(st.x[1], st.y[1], acc_re[1][1], acc_im[1][1], [](int) {});
-  } else {
-    mma_split_tile(st.x[TX - 1], st.y[0], acc_re[0][TX - 1], acc_im[0][TX - 1], [](int) {});
+// What is left after the last K iteration, and the sums as they belong into C; false for
+// any that is not finite.
+template <int TX>
+__device__ __forceinline__ bool mma_split_last(SplitState<TX> &st, float16_t_ (&acc_re)[1][TX],
+                                               float16_t_ (&acc_im)[1][TX]) {
+  mma_split_tile(st.x[TX - 1], st.y, st.re[TX - 1], st.im[TX - 1], [](int) {});
+  float check = 0.f;   // not zero as soon as one of the sums is not finite
+#pragma unroll
+  for (int i = 0; i < TX; ++i) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      acc_re[0][i][e] = (st.re[i].large[e] + st.re[i].small[e]) * kSplitUnscale;
+      acc_im[0][i][e] = (st.im[i].large[e] + st.im[i].small[e]) * kSplitUnscale;
+      check = __builtin_fmaf(acc_re[0][i][e], 0.f, check);
+      check = __builtin_fmaf(acc_im[0][i][e], 0.f, check);
+    }
   }
+  return check == 0.f;
 }
 
 // Wide accesses to C at an address that is aligned to its elements only: rows of any
@@ -2193,6 +2201,11 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
                          : (MS == 32 ? y32_off[i] : y_frag_off + i * 16 * kTileRowBytes) + p * BY * kTileRowBytes;
     }
   }
+  // (32-bit input) the lane's four chunks, see mma_step32_split
+  const int x_split_off[4] = {IL ? xil32_off[0][0] : x32_off[0], IL ? xil32_off[0][1] : x32_off[1],
+                              xil32_off[1][0], xil32_off[1][1]};
+  const int y_split_off[4] = {IL ? yil32_off[0][0] : y32_off[0], IL ? yil32_off[0][1] : y32_off[1],
+                              yil32_off[1][0], yil32_off[1][1]};
   // wide stores through LDS: no beta term (interleaved C only with the 16-row layout)
   const bool staged_ok = (MS == 16 || !args.c_interleaved) && !args.have_beta;
 
@@ -2234,12 +2247,18 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   const unsigned iters = k_tiles;
   for (unsigned vt = blockIdx.x; vt < total; vt += gridDim.x) {
     typename AccType<MS>::type acc_re[TY][TX], acc_im[TY][TX];
-    SplitState<DT == kFloat32 ? TX : 1, DT == kFloat32 ? TY : 1> split;   // (32-bit input)
-    SmallTile small;                                                      // (64 x 64 blocks)
+    SplitState<DT == kFloat32 ? TX : 1> split;   // (32-bit input)
+    SmallTile small;                             // (64 x 64 blocks)
     // (the hand-ordered step of the 16-row MFMAs starts its first iteration from zero itself)
     constexpr bool kStepClears = !IL && DT != kInt1 && MS == 16 && TX == 4 && TY == 4;
     static_assert(!SPLIT || kStepClears, "separate X and Y rings: hand-ordered 16-row step only");
-    if constexpr (!kStepClears) {
+    if constexpr (DT == kFloat32) {
+#pragma unroll
+      for (int i = 0; i < TX; ++i) {
+        split.re[i] = SplitSum{0.f, 0.f};
+        split.im[i] = SplitSum{0.f, 0.f};
+      }
+    } else if constexpr (!kStepClears) {
 #pragma unroll
       for (int j = 0; j < TY; ++j) {
 #pragma unroll
@@ -2314,10 +2333,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
           }
           small = next;
         } else if constexpr (DT == kFloat32) {
-          static_assert(MS == 32, "32-bit input: 32-row MFMA");
-          const int *x_off = IL ? xil32_off[0] : x32_off, *y_off = IL ? yil32_off[0] : y32_off;
-          mma_step32_split<BX, BY, TX, TY, IL, decltype(first)::value>(slot_ptr, x_off, y_off, split, acc_re,
-                                                                       acc_im, refill_slots);
+          static_assert(MS == 32 && TY == 1, "32-bit input: 32-row MFMA, tiles side by side");
+          mma_step32_split<BX, BY, TX, IL, decltype(first)::value>(slot_ptr, x_split_off, y_split_off, split,
+                                                                   refill_slots);
         } else if constexpr (IL && MS == 32) {
           static_assert(TX == 2 && TY == 2, "2 x 2 tiles of 32 x 32 per wave");
           mma_step32_interleaved<DT, BX, BY>(slot_ptr, xil32_off, yil32_off, acc_re, acc_im,
@@ -2366,22 +2384,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     bool redo = false;   // (32-bit input) this wave's tile is computed again
     if constexpr (DT == kFloat32) {
-      mma_split_last<TX, TY>(split, acc_re, acc_im);
-      float sum = 0.f;   // not finite as soon as one of the accumulators is not
-#pragma unroll
-      for (int j = 0; j < TY; ++j) {
-#pragma unroll
-        for (int i = 0; i < TX; ++i) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            sum = __builtin_fmaf(acc_re[j][i][e], 0.f, sum);
-            sum = __builtin_fmaf(acc_im[j][i][e], 0.f, sum);
-            acc_re[j][i][e] *= kSplitUnscale;
-            acc_im[j][i][e] *= kSplitUnscale;
-          }
-        }
-      }
-      redo = __any(sum != 0.f);
+      redo = __any(!mma_split_last(split, acc_re, acc_im));
     }
     bool staged = false;
     if constexpr (XT) {
@@ -2629,11 +2632,11 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // moves per flop. Times with 256 x 128, 128 x 128 and 64 x 64 blocks in us, on operands that no cache
 // held (profiles/gemm_block_choice.txt):
 //   too few tiles for the larger blocks, 16 bits 256^3:  14.7, 12.5, 6.9;  B=256 96x96x1024:  86, 56, 62;
-//     32 bits B=2 1000^3:  224, 147, 104;  8 bits 1024^3:  24.9, 22.3, 11.5;
+//     32 bits B=2 1000^3:  (none), 176, 122;  8 bits 1024^3:  24.9, 22.3, 11.5;
 //     1 bit 64x64x65536:  526, 305, 116
 //   every unit busy, 16 bits on tiles, 4096x4096x512:  68, 89, 102
 //     on planar rows, of which a copy fetches half cache lines, B=157 192x604x3680:  747, 909, 1026
-//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  312, 358, 426
+//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  (none), 435, 502
 //     8 bits on tiles, 4096x4096x512:  48, 48, 69
 //     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
 //       277, 288, 312
@@ -2645,9 +2648,11 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // slower by 0.95 to several times, 1.37 (128 x 128) and 2.9 (64 x 64) at the median.
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
 // 30000 problems of random sizes, 40 % of them on operands that no cache held
-// (python -m ccglib_amd.tuning.block_choice times such problems); those of 32-bit input, 8-bit tiles
+// (python -m ccglib_amd.tuning.block_choice times such problems); those of 8-bit tiles
 // and 16-bit pairs to 1900 further ones, timed since those kernels last changed. The choice is then on average
 // 0.2 % behind the fastest of the three shapes, and more than 8 % behind in 0.7 % of the problems.
+// 32-bit input: 1200 problems, on average less than 0.1 % behind the faster of its two shapes, more than
+// 8 % in one.
 enum BlockShape { k256x128, k128x128, k64x64 };
 struct BlockChoice {
   BlockShape shape;
@@ -2661,9 +2666,8 @@ struct BlockCosts {
 };
 inline BlockCosts block_costs(const GemmParams &p) {
   if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0};
-  // (32-bit pairs: the 128 x 128 block stands in for the 256 x 128 one)
-  if (p.type_in == kFloat32 && p.input_interleaved) return {1.13, 1.40, 6.0, 4.6, 0.0, 0.0, 0.0, 0.0, 0.0};
-  if (p.type_in == kFloat32) return {1.16, 1.52, 9.8, 8.5, 0.0, 0.0, 0.0, 0.0, 0.0};
+  // (32-bit input has no 256 x 128 block: relative to 128 x 128)
+  if (p.type_in == kFloat32) return {1.0, 1.24, 6.0, 5.0, 0.0, 0.0, 0.0, 4.0, 2.0};
   const bool planar = p.variant == kBasic && !p.input_interleaved;
   if (bits_of(p.type_in) == 8) {
     if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0};
@@ -2686,11 +2690,12 @@ inline BlockChoice block_choice(const GemmParams &p) {
     return ((double)mine + (mine % 2 ? lone : 0.0)) * (double)(bx * by) * cost *
            (pieces + tile + (p.have_beta ? beta : 0.0)) / large;
   };
-  const double t256 = time(256, 128, 1.0, 10.0, 0.0, costs.beta_256);
+  const bool no_256 = p.type_in == kFloat32;
+  const double t256 = no_256 ? HUGE_VAL : time(256, 128, 1.0, 10.0, 0.0, costs.beta_256);
   const double t128 = time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
   const double t64 = time(64, 64, costs.cost_64, costs.tile_64, costs.lone_64, costs.beta_64);
-  if (p.block_tile == 1) return {k256x128, t256};
-  if (p.block_tile == 2) return {k128x128, t128};
+  if (p.block_tile == 1 && !no_256) return {k256x128, t256};
+  if (p.block_tile == 1 || p.block_tile == 2) return {k128x128, t128};
   if (p.block_tile == 4) return {k64x64, t64};
   if (t256 <= t128 && t256 <= t64) return {k256x128, t256};
   return t128 <= t64 ? BlockChoice{k128x128, t128} : BlockChoice{k64x64, t64};
@@ -2734,16 +2739,13 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   constexpr bool BITS16 = DtypeTraits<DT>::kElemBytes == 2;
   constexpr int MS = BITS16 ? 16 : 32;
   if constexpr (DT == kFloat32) {
-    // 256 x 128 blocks of 8 waves of 64 x 64, 3-slot ring; 128 x 128 of 8 waves of 64 x 32, 4-slot
-    // ring; 64 x 64 of 4 waves of 32 x 32, 5-slot ring, two blocks a unit. The more a wave
-    // computes the fewer elements it splits per matrix instruction: 4096x4096x512 on tiles
-    // 305, 345, 413 us. (Rows of pairs: a wave of 64 x 64 spills 37 registers.)
+    // 128 x 128 blocks of 8 waves of 64 x 32, 4-slot ring; 64 x 64 of 4 waves of 32 x 32, 5-slot
+    // ring, two blocks a unit. The more a wave computes the fewer elements it splits per matrix
+    // instruction: planar pipeline of 8192x8192x1024 3250 and 3900 us. (A wave of 64 x 64, which 256 x 128 blocks
+    // have, would need 256 registers for its sums alone.)
     auto launch = [&](auto loader) {
       constexpr int L = decltype(loader)::value;
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, L, 32>(p, stream);
-      if constexpr (L != kLoadInterleavedVec && L != kLoadInterleavedRagged) {
-        if (shape == k256x128) return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, L, 32>(p, stream);
-      }
       return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, L, 32>(p, stream);
     };
     const bool aligned = (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 16 == 0;

@@ -117,7 +117,7 @@ static const std::vector<Config> kConfigs = {
     {"f16 planar 64x64 w32x32 s5 m16", launch_dtl<kFloat16, kFloat32, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 16>, kFloat16, kFloat32, kLoadPlanarVec},
     {"f16 interleaved 64x64 w32x32 s5 m16", launch_dtl<kFloat16, kFloat32, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 16>, kFloat16, kFloat32, kLoadInterleavedVec},
     {"fp8 interleaved 64x64 w32x32 s5 m32", launch_dtl<kFloat8e4m3, kFloat32, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 32>, kFloat8e4m3, kFloat32, kLoadInterleavedVec},
-    {"f32 256x128 w64x64 s3 m32 split", launch_dtl<kFloat32, kFloat32, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>, kFloat32, kFloat32},
+    {"f32 128x128 w64x32 s4 m32 split", launch_dtl<kFloat32, kFloat32, 128, 128, 64, 32, 4, 2, kLoadTiled, 32>, kFloat32, kFloat32},
     {"fp8 256x128 w64x64 s3 m32", launch_dtl<kFloat8e4m3, kFloat32, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>, kFloat8e4m3, kFloat32},
     {"fp8 128x128 w64x64 s2 m32", launch_dtl<kFloat8e4m3, kFloat32, 128, 128, 64, 64, 2, 2, kLoadTiled, 32>, kFloat8e4m3, kFloat32},
     {"fp8 128x128 w64x32 s4 m32", launch_dtl<kFloat8e4m3, kFloat32, 128, 128, 64, 32, 4, 2, kLoadTiled, 32>, kFloat8e4m3, kFloat32},

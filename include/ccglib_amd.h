@@ -93,7 +93,8 @@ CCGLIB_API const char *ccglib_version(void);
  *                    192 x 256 ones (16-bit tiled input, planar C without
  *                    beta, M and N multiples of 64, K of more than 32) when
  *                    those fill the compute units well enough;
- *                    1: always 256 x 128; 2: always 128 x 128; 3: 192 x 256
+ *                    1: always 256 x 128 (32-bit input, which has no such
+ *                    block: 128 x 128); 2: always 128 x 128; 3: 192 x 256
  *                    wherever that kernel applies, else as 0; 4: always
  *                    64 x 64. The 192 x 256 block also serves 16-bit
  *                    interleaved rows read in place (the pipeline) when K is a

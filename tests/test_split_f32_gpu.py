@@ -51,14 +51,59 @@ def test_accuracy(layout, block_tile, K):
     a = rng.standard_normal((B, 2, M, K)).astype(np.float32)
     b = rng.standard_normal((B, 2, N, K)).astype(np.float32)
     got, want = product(layout, block_tile, a, b), exact(a, b)
-    # what is left out of a product lies below 2^-23 of it; a sum is rounded 12 times per 16
-    # values of K by up to 2^-24 of a partial sum, which never exceeds the sum of the moduli
+    # (wide enough for 12 roundings of the whole sum per 16 values of K, by up to 2^-24 of a partial
+    # sum, which never exceeds the sum of the moduli; the next two tests are closer)
     scale = np.abs(a).astype(np.float64), np.abs(b).astype(np.float64).transpose(0, 1, 3, 2)
     moduli = np.stack([scale[0][:, 0] @ scale[1][:, 0] + scale[0][:, 1] @ scale[1][:, 1],
                        scale[0][:, 0] @ scale[1][:, 1] + scale[0][:, 1] @ scale[1][:, 0]], 1)
     assert np.all(np.abs(got - want) <= moduli * (2.0 ** -23 + 2.0 ** -24 * (12 * (K // 16 + 1) + 1)))
     # rounding errors of random sign: what fp32 products added up in fp32 show
     assert np.linalg.norm(got - want) <= 2.0 ** -24 * (2 + 1.5 * np.sqrt(2 * K)) * np.linalg.norm(want)
+
+
+def fp32_sum_error(n):
+    """Relative error of n complex products added up in fp32: 2 n roundings of 0.42 * 2^-24 of the
+    partial sum each in the mean, and with random signs the squares of the partial sums grow evenly,
+    so together 0.42 * 2^-24 * sqrt((2 n + 1) / 2); a tenth more for the sample."""
+    return 2.0 ** -24 * 0.33 * np.sqrt(2 * n + 1)
+
+
+@pytest.mark.parametrize("block_tile", [2, 4])
+@pytest.mark.parametrize("layout,K", [(layout, K) for layout in LAYOUTS for K in (1, 2, 3, 4, 5, 16, 17, 333)
+                                      if (layout, K) != ("pairs", 1)])   # (rows of at least 16 bytes)
+def test_no_less_accurate_than_fp32_sums(layout, block_tile, K):
+    rng = np.random.default_rng(K)
+    a = rng.standard_normal((2, 2, 150, K)).astype(np.float32)
+    b = rng.standard_normal((2, 2, 290, K)).astype(np.float32)
+    got, want = product(layout, block_tile, a, b), exact(a, b)
+    assert np.linalg.norm(got - want) <= fp32_sum_error(K) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [2, 4])
+def test_two_products_a_row(layout, block_tile):
+    M, N = 150, 290
+    rng = np.random.default_rng(5)
+    a = np.zeros((1, 2, M, 2 * M), np.float32)
+    for first in (0, M):
+        a[0, :, np.arange(M), first + rng.permutation(M)] = rng.standard_normal((M, 2))
+    b = rng.standard_normal((1, 2, N, 2 * M)).astype(np.float32)
+    got, want = product(layout, block_tile, a, b), exact(a, b)
+    assert np.linalg.norm(got - want) <= fp32_sum_error(2) * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [2, 4])
+def test_single_products_are_rounded_once(layout, block_tile):
+    # a gain for every row: half a unit in the last place, and the seven small products' roundings,
+    # 2^-24 of a sum below 2^-7 of the product each
+    M, N = 150, 290
+    rng = np.random.default_rng(5)
+    a = np.zeros((1, 2, M, M), np.float32)
+    a[0, 0, np.arange(M), rng.permutation(M)] = rng.standard_normal(M)
+    b = rng.standard_normal((1, 2, N, M)).astype(np.float32)
+    got, want = product(layout, block_tile, a, b), exact(a, b)
+    assert np.all(np.abs(got - want) <= (0.5 + 7 * 2.0 ** -8) * np.spacing(np.abs(want).astype(np.float32)))
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
