@@ -1,15 +1,16 @@
 """How well the dispatch picks a block shape: GEMMs of random sizes, types, operand layouts and C
 layouts, timed with each shape forced (option GEMM_BLOCK_TILE = 1, 2, 4: 256 x 128, 128 x 128,
-64 x 64), and how far the shape that the default takes is behind the fastest of the three. The
+64 x 64; 32-bit input has no 256 x 128), and how far the shape that the default takes is behind the fastest. The
 constants of block_choice (../csrc/gemm_mfma.hip) are fitted to such times.
 
-    python -m ccglib_amd.tuning.block_choice [--problems 2000] [--seed 1] [--warm] [--csv FILE]
+    python -m ccglib_amd.tuning.block_choice [--problems 2000] [--seed 1] [--warm] [--csv FILE] [--input float32]
 
 One MI355X, N(0, 1) operands (fp8 scaled into range, random bits for 1-bit input). Every pass takes
 other buffers, out of pools larger than the last-level cache; with --warm the same ones. The three
 shapes take turns, five times about 2 ms each; the medians count. Sizes: B up to 256, M and N 16 to
 4096, K 64 to 4096 (1-bit: 512 to 32768), half of them multiples of 8 to 128, up to about 1.5 ms
-and 1536 tiles of 256 x 128.
+and 1536 tiles of 256 x 128. K is a multiple of 16 (1-bit: 128); a third of the problems on rows in place
+have any K ("ragged").
 """
 import argparse
 import collections
@@ -44,18 +45,24 @@ def extent(rng):
     return max(16, (n + step // 2) // step * step)
 
 
-def problem(rng):
+def problem(rng, pairs):
     """(tin, tout, layout, C axis, alpha, beta, B, M, N, K) and the bytes of A, B and C."""
     while True:
-        tin, tout = rng.choice(PAIRS)
+        tin, tout = rng.choice(pairs)
         layout = rng.choice(["tiled", "tiled", "planar", "interleaved"])
-        if layout == "interleaved" and tin in (VT.float32, VT.int1):
+        if layout == "interleaved" and tin == VT.int1:
             layout = "tiled"
-        c_axis = AX.complex_interleaved if layout != "planar" and rng.random() < 0.4 else AX.complex_planar
+        if layout != "tiled" and tin != VT.int1 and rng.random() < 0.33:
+            layout += " ragged"
+        c_axis = AX.complex_planar
+        if not layout.startswith("planar") and rng.random() < 0.4:
+            c_axis = AX.complex_interleaved
         alpha = 1 if rng.random() < 0.8 or tin == VT.int1 else 0.5 - 1.5j
         beta = 0 if rng.random() < 0.8 or tin == VT.int1 else 0.25 + 0.5j
         B, M, N = log_size(rng, 1, 256), extent(rng), extent(rng)
         K = (128 if tin == VT.int1 else 16) * log_size(rng, 4, 256)
+        if layout.endswith("ragged"):
+            K -= rng.randrange(1, 16)
         sizes = bytes_of(tin, tout, layout, B, M, N, K)
         if (8 * B * M * N * K / RATE[tin] <= 1.5e-3 and max(sizes) <= POOL_BYTES and
                 B * cc.ceildiv(M, 128) * cc.ceildiv(N, 256) <= 1536):
@@ -80,6 +87,7 @@ NAMED = [(VT.float16, VT.float32, "tiled", 0, 1, 4096, 4096, 512),
          (VT.float16, VT.float32, "planar", 0, 157, 192, 604, 3680),
          (VT.float32, VT.float32, "tiled", 0, 1, 4096, 4096, 512),
          (VT.float32, VT.float32, "tiled", 0, 2, 1000, 1000, 1000),
+         (VT.float32, VT.float32, "interleaved", 0, 2, 1000, 1000, 1000),
          (VT.float8e4m3, VT.float32, "tiled", 0, 1, 4096, 4096, 512),
          (VT.float8e4m3, VT.float32, "tiled", 0, 1, 1024, 1024, 1024),
          (VT.float8e4m3, VT.float32, "planar", 0.25 + 0.5j, 11, 456, 1542, 192),
@@ -109,9 +117,10 @@ def pool(tin, which):
 def make(case, block_tile):
     tin, tout, layout, c_axis, alpha, beta, B, M, N, K = case
     s = torch.cuda.current_stream().cuda_stream
-    variant = cc.Variant.basic if layout == "planar" else cc.Variant.opt
-    with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.pipeline_route, 1):
-        if layout == "interleaved":
+    variant = cc.Variant.basic if layout.startswith("planar") else cc.Variant.opt
+    with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.pipeline_route, 1), \
+            cc.option(cc.Option.basic_retile, 0):
+        if layout.startswith("interleaved"):
             pipe = cc.Pipeline(B, M, N, K, 0, s, AX.complex_interleaved, c_axis, MO.row_major, MO.col_major,
                                MO.row_major, tin, tout, variant, alpha, beta)
             assert pipe.ReadsInPlace()
@@ -125,7 +134,7 @@ def measure(case, sizes, warm):
     slots = 1 if warm else int(max(1, min(4096, FOOTPRINT // sum(steps), *(POOL_BYTES // v for v in steps))))
     base = [pool(case[0], "a"), pool(case[0], "b"), pool(None, "c")]
     where = [[p + i * v for p, v in zip(base, steps)] for i in range(slots)]
-    runs = {t: make(case, t) for t in (0, 1, 2, 4)}
+    runs = {t: make(case, t) for t in (0, 1, 2, 4) if t != 1 or case[0] != VT.float32}
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     at = 0
 
@@ -146,7 +155,9 @@ def measure(case, sizes, warm):
     for i in range(5):
         for t in (list(runs) if i % 2 else reversed(list(runs))):
             times[t].append(once(runs[t], n))
-    return {t: statistics.median(v) for t, v in times.items()}
+    medians = {t: statistics.median(v) for t, v in times.items()}
+    medians.setdefault(1, math.nan)
+    return medians
 
 
 def main():
@@ -155,9 +166,13 @@ def main():
     ap.add_argument("--seed", type=int, default=1)
     ap.add_argument("--warm", action="store_true")
     ap.add_argument("--csv")
+    ap.add_argument("--input", help="only problems of this input type")
     args = ap.parse_args()
+    pairs = [p for p in PAIRS if args.input in (None, p[0].name)]
     print("us: 256x128, 128x128, 64x64 on cold operands; on warm ones; default (warm)")
     for tin, tout, layout, beta, B, M, N, K in NAMED:
+        if args.input not in (None, tin.name):
+            continue
         case = (tin, tout, layout, AX.complex_planar, 1, beta, B, M, N, K)
         cold, warm = (measure(case, bytes_of(tin, tout, layout, B, M, N, K), w) for w in (False, True))
         print("%-52s %8.1f %8.1f %8.1f   %8.1f %8.1f %8.1f   %8.1f" % (
@@ -167,13 +182,13 @@ def main():
     groups, worst = collections.defaultdict(list), []
     csv = open(args.csv, "w") if args.csv else None
     for i in range(args.problems):
-        case, sizes = problem(rng)
+        case, sizes = problem(rng, pairs)
         t = measure(case, sizes, args.warm)
         tin, tout, layout, c_axis, alpha, beta, B, M, N, K = case
         text = "%s->%s %s%s%s B=%d %dx%dx%d" % (tin.name, tout.name, layout,
                                                 " interleaved C" if c_axis == AX.complex_interleaved else "",
                                                 " beta" if beta else "", B, M, N, K)
-        behind = t[0] / min(t[1], t[2], t[4])
+        behind = t[0] / min(v for v in (t[1], t[2], t[4]) if v == v)
         groups["%-12s %s" % (tin.name, layout)].append(behind)
         groups["all"].append(behind)
         worst.append((behind, text, t))
