@@ -2056,13 +2056,14 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   // in front of them, once more, some that the chunk before holds, until
   // settle_row_ends puts them right.
   auto chunk_source = [&](const char *src, unsigned kt, int chunk, size_t plane) {
-    const unsigned end = kt * RB + chunk * 16 + 16;
+    // (the end of a chunk may lie 4 GiB behind the row's start, and its 32-bit offset be 0)
+    const unsigned start = kt * RB + chunk * 16;
     plane += (size_t)kt * RB;
     if constexpr (RAGGED) {
-      const unsigned over = end > row_bytes ? end - row_bytes : 0;
-      return over < 16 ? src + plane - over : g_zero_tile + lane * 16;
+      const unsigned left = row_bytes - start;
+      return start < row_bytes ? src + plane - (left < 16 ? 16 - left : 0) : g_zero_tile + lane * 16;
     } else {
-      return end <= row_bytes ? src + plane : g_zero_tile + lane * 16;
+      return start < row_bytes ? src + plane : g_zero_tile + lane * 16;
     }
   };
   // issue_*: straight-line code (it is placed between MFMAs, and a branch there

@@ -130,3 +130,26 @@ def test_planar_rows_to_pairs(tin, tout, block_tile, K):
         outs.append(d_c)
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("K", [2 ** 31 - 1, 2 ** 31 - 8])
+def test_pairs_in_rows_of_4_gib(K):
+    # Rows that end less than a K tile below 4 GiB, inside a chunk and behind one: the offset of the last
+    # chunk's end has no 32 bits.
+    M, tin = 2, VT.float8e4m3
+    at = [0, 5, K - 9, K - 2, K - 1]
+    a = np.array([[3 - 2j, 1j, 2, 5, 1 + 4j], [1, 2, 3 + 1j, 4j, -6]])
+    b = np.array([2, 1 - 1j, 3 + 2j, 1j, 4 - 1j])
+    d_a, d_b = (torch.zeros(rows * 2 * K, dtype=torch.uint8, device="cuda") for rows in (M, 1))
+    for d, values in ((d_a, a), (d_b, b[None])):
+        for row, v in enumerate(values):
+            for k, z in zip(at, v):
+                pair = torch.tensor([z.real, z.imag]).to(torch.float8_e4m3fn).view(torch.uint8)
+                d[2 * (row * K + k):2 * (row * K + k) + 2] = pair.cuda()
+    d_c = torch.full((2, M), np.nan, device="cuda")
+    with cc.option(cc.Option.pipeline_route, 1):
+        p = cc.Pipeline(1, M, 1, K, 0, stream(), INTERLEAVED, PLANAR, ROW, COL, ROW, tin, VT.float32, cc.Variant.opt)
+    assert p.ReadsInPlace()
+    p.Run(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr())
+    got = d_c.cpu().numpy()
+    assert np.array_equal(got[0] + 1j * got[1], a @ b)
