@@ -1010,7 +1010,11 @@ __device__ __forceinline__ void mma_small_tile(const SmallTile &t, float16_t_ (&
 // small number falls below the range of a bf16: the split is exact for every magnitude up to 2^104.
 // What the instructions cannot do is an infinity, a NaN or a larger number (their parts are
 // infinite or NaN) or a sum beyond 2^80: the accumulators are then not finite, and the wave computes
-// its tile again with the fp32 instructions (recompute_f32).
+// its tile again with the fp32 instructions (recompute_f32) - unless those sums are NaN because of
+// a NaN in their rows, such as marks a flagged sample, for which it only looks through the rows
+// (only_nan_rows). Planar rows, 4096x4096x512 and B=2 1000^3, in us: finite 428, 124; a NaN in every row of X 531,
+// 151 (computed again 1029, 288); an infinity in every row 1015, 279; the fp32 instructions 498, 134 at
+// any values.
 //   The splitting, 13 vector instructions for two elements, runs in every wave that reads an
 // element (split tiles would take half as much LDS again) and in the shadow of the matrix
 // instructions: those of a K tile are issued while the next one is split (see
@@ -1181,8 +1185,8 @@ __device__ __forceinline__ void mma_step32_split(const char *slot, const int (&x
     mma_split_tile(st.x[0], st.y, st.re[0], st.im[0], [&](int n) { split_behind(raw, st.x[1], n, 5); });
   }
 }
-// What is left after the last K iteration, and the sums as they belong into C; false for
-// any that is not finite.
+// What is left after the last K iteration, and the sums as they belong into C; false where the
+// wave has one that is not finite.
 template <int TX>
 __device__ __forceinline__ bool mma_split_last(SplitState<TX> &st, float16_t_ (&acc_re)[1][TX],
                                                float16_t_ (&acc_im)[1][TX]) {
@@ -1198,7 +1202,17 @@ __device__ __forceinline__ bool mma_split_last(SplitState<TX> &st, float16_t_ (&
       check = __builtin_fmaf(acc_im[0][i][e], 0.f, check);
     }
   }
-  return check == 0.f;
+  if (__builtin_expect(!__any(check != 0.f), 1)) return true;
+  // (an infinity's small products are NaN, the large ones infinite as a rule)
+#pragma unroll
+  for (int i = 0; i < TX; ++i) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      if (__builtin_isinf(st.re[i].large[e])) acc_re[0][i][e] = st.re[i].large[e];
+      if (__builtin_isinf(st.im[i].large[e])) acc_im[0][i][e] = st.im[i].large[e];
+    }
+  }
+  return false;
 }
 
 // Wide accesses to C at an address that is aligned to its elements only: rows of any
@@ -1332,50 +1346,218 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
   }
 }
 
+// One row of a 32-bit operand in global memory, four values of K at a time.
+template <int LOADER> struct RowF32 {
+  static constexpr bool kPairs = (LOADER == kLoadInterleavedVec || LOADER == kLoadInterleavedRagged);
+  static constexpr unsigned kStep = LOADER == kLoadTiled ? kTileBytes : kPairs ? 128 : kTileRowBytes;
+  const char *p;    // K tile 0
+  size_t second;    // from the real values to the imaginary ones (pairs: to the second two)
+  unsigned k;       // values in whole K tiles, and all
+  unsigned k_all;
+
+  // `rows` of them from `base` on; one past the end is read as the last one
+  __device__ RowF32(const KernelArgs &args, const char *base, unsigned rows, unsigned row) {
+    if constexpr (LOADER == kLoadTiled) {
+      rows = (rows + kTileRows - 1) / kTileRows * kTileRows;
+    }
+    row = row < rows ? row : rows - 1;
+    k_all = args.k;
+    if constexpr (LOADER == kLoadTiled) {
+      p = base + (size_t)(row / kTileRows) * args.k_tiles * kTileBytes + row % kTileRows * kTileRowBytes;
+      second = kTilePlaneBytes;
+      k = k_all = args.k_tiles * 16;
+    } else {
+      p = base + (size_t)row * (kPairs ? 2 : 1) * args.row_stride_bytes;
+      second = kPairs ? 16 : (size_t)rows * args.row_stride_bytes;
+      k = k_all / 16 * 16;
+    }
+  }
+  // values 4 c ... of K tile kt, of which the row has all sixteen
+  __device__ void get(unsigned kt, int c, float4_t &re, float4_t &im) const {
+    const char *q = p + (size_t)kt * kStep + c * (kPairs ? 32 : 16);
+    const float4_t u = *reinterpret_cast<const float4_any_t *>(q);
+    const float4_t v = *reinterpret_cast<const float4_any_t *>(q + second);
+    if constexpr (kPairs) {
+      re = float4_t{u[0], u[2], v[0], v[2]};
+      im = float4_t{u[1], u[3], v[1], v[3]};
+    } else {
+      re = u;
+      im = v;
+    }
+  }
+  // ... and of the last K tile, which it has in part
+  __device__ void get_end(int c, float4_t &re, float4_t &im) const {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned at = k + 4 * c + e;
+      const float *q = reinterpret_cast<const float *>(p) + (kPairs ? 2 * (size_t)at : (size_t)at);
+      re[e] = at < k_all ? q[0] : 0.f;
+      im[e] = at < k_all ? q[kPairs ? 1 : second / 4] : 0.f;
+    }
+  }
+};
+
+// The lane, counted where this is called: what follows from it is then worked out there as well, and
+// not before the K loop, across which no register is left to keep it.
+__device__ __forceinline__ int lane_here() {
+  unsigned none = 0;
+  asm volatile("" : "+s"(none));
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none));
+}
+
+// Which of 16 rows of an operand from row0 on hold a NaN (a bit each), read by the wave until all of
+// `wanted` have been found to.
+template <int LOADER>
+__device__ __forceinline__ unsigned nan_rows(const KernelArgs &args, const char *base, unsigned rows, unsigned row0,
+                                             int lane, unsigned wanted) {
+  const RowF32<LOADER> row(args, base, rows, row0 + (lane >> 2));
+  const bool mine = (wanted >> (lane >> 2)) & 1;
+  bool nan = false;
+  float4_t re, im;
+  auto look = [&] {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) nan |= __builtin_isunordered(re[e], im[e]);
+  };
+  auto of_row = [&] { return ((__ballot(nan) >> (lane & ~3)) & 15) != 0; };
+  for (unsigned kt = 0; kt < row.k / 16 && __any(mine && !of_row()); kt += 8) {
+    float4_t r8[8], i8[8];   // (sixteen loads under way at a time)
+#pragma unroll
+    for (unsigned u = 0; u < 8; ++u) row.get(kt + u < row.k / 16 ? kt + u : kt, lane & 3, r8[u], i8[u]);
+#pragma unroll
+    for (unsigned u = 0; u < 8; ++u) {
+      re = r8[u];
+      im = i8[u];
+      look();
+    }
+  }
+  if (row.k < row.k_all) {
+    row.get_end(lane & 3, re, im);
+    look();
+  }
+  const unsigned long long found = __ballot(of_row());
+  unsigned bits = 0;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) bits |= (unsigned)((found >> (4 * r)) & 1) << r;
+  return bits;
+}
+
+// Whether all sums of a wave's tile (32-bit input, TX MFMA tiles side by side) that are not finite are
+// those of a row with a NaN. They are NaN then, in the split sums as on the fp32 instructions. (A sum that
+// is infinite is not, and the rows need no look.)
+template <int LOADER, int TX>
+__device__ __forceinline__ bool only_nan_rows(const KernelArgs &args, unsigned b, unsigned x_wave, unsigned y_wave,
+                                              int lane, const float16_t_ (&acc_re)[1][TX],
+                                              const float16_t_ (&acc_im)[1][TX]) {
+  const char *x = args.x + (size_t)b * args.x_batch_bytes, *y = args.y + (size_t)b * args.y_batch_bytes;
+  const bool y_inside = y_wave + (lane & 31) < args.ny;
+  unsigned bad[TX];   // bit e: element e of a tile (x = 8 (e / 4) + 4 (lane / 32) + e % 4) is not finite
+  bool infinite = false;
+#pragma unroll
+  for (int i = 0; i < TX; ++i) {
+    bad[i] = 0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const unsigned at = x_wave + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+      const float re = acc_re[0][i][e], im = acc_im[0][i][e];
+      const bool finite = __builtin_isfinite(re) && __builtin_isfinite(im), inside = y_inside && at < args.nx;
+      bad[i] |= (unsigned)(!finite && inside) << e;
+      infinite |= inside && (__builtin_isinf(re) || __builtin_isinf(im));
+    }
+  }
+  if (__any(infinite)) return false;
+  // rows of X without a finite sum
+#pragma unroll
+  for (int i = 0; i < TX; ++i) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!__any((bad[i] >> (8 * h)) & 0xff)) continue;
+      unsigned wanted = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const unsigned long long none = __ballot(((bad[i] >> (8 * h + e)) & 1) || !y_inside);
+        const int bit = 8 * (e >> 2) + (e & 3);
+        wanted |= (unsigned)((unsigned)none == ~0u) << bit | (unsigned)((unsigned)(none >> 32) == ~0u) << (bit + 4);
+      }
+      if (wanted == 0) continue;
+      const unsigned nan = nan_rows<LOADER>(args, x, args.nx, x_wave + 32 * i + 16 * h, lane, wanted);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const unsigned mine = (nan >> (8 * (e >> 2) + 4 * (lane >> 5) + (e & 3))) & 1;
+        bad[i] &= ~(mine << (8 * h + e));
+      }
+    }
+  }
+  auto left = [&] {
+    unsigned any = 0;
+#pragma unroll
+    for (int i = 0; i < TX; ++i) any |= bad[i];
+    return any != 0;
+  };
+  // rows of Y with one that is not explained yet
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const unsigned long long m = __ballot(left());
+    const unsigned wanted = ((unsigned)(m | (m >> 32)) >> (16 * h)) & 0xffff;
+    if (wanted == 0) continue;
+    const unsigned nan = nan_rows<LOADER>(args, y, args.ny, y_wave + 16 * h, lane, wanted);
+    if (((lane >> 4) & 1) == h && ((nan >> (lane & 15)) & 1)) {
+#pragma unroll
+      for (int i = 0; i < TX; ++i) bad[i] = 0;
+    }
+  }
+  return !__any(left());
+}
+
 // A wave's tile of 32-bit input on the fp32 instructions, straight from global memory, one
-// 32 x 32 tile at a time: for tiles whose split sums are not finite (mma_step32_split).
+// 32 x 32 tile at a time: for tiles whose split sums are not finite for another reason than a NaN
+// among the operands (mma_step32_split).
 template <int TOUT, int LOADER, int TX, int TY>
 __device__ __forceinline__ void recompute_f32(const KernelArgs &args, unsigned b, unsigned x_wave,
                                               unsigned y_wave, int lane) {
-  constexpr bool IL = (LOADER == kLoadInterleavedVec || LOADER == kLoadInterleavedRagged);
-  constexpr int FROM = LOADER == kLoadTiled ? kLoadTiled : kLoadPlanarElem;
-  const OperandView xv{args.x + (size_t)b * args.x_batch_bytes, args.nx, args.x_tiles, 0};
-  const OperandView yv{args.y + (size_t)b * args.y_batch_bytes, args.ny, args.y_tiles, 0};
-  // the four values K = 16 kt + 4 c .. of a row
-  auto fetch = [&](const OperandView &v, unsigned row, unsigned kt, int c, float4_t &re, float4_t &im) {
-    if constexpr (IL) {
-      row = row < v.rows ? row : v.rows - 1;
-      const float *p = reinterpret_cast<const float *>(v.base + (size_t)row * 2 * args.row_stride_bytes);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const unsigned k = kt * 16 + c * 4 + e;
-        re[e] = k < args.k ? p[2 * (size_t)k] : 0.f;
-        im[e] = k < args.k ? p[2 * (size_t)k + 1] : 0.f;
-      }
-    } else {
-      re = __builtin_bit_cast(float4_t, load_chunk<4, FROM>(v, kt, args.k_tiles, args.k_bytes, 0, row, c));
-      im = __builtin_bit_cast(float4_t, load_chunk<4, FROM>(v, kt, args.k_tiles, args.k_bytes, 1, row, c));
-    }
+  struct Four {
+    float4_t xr, xi, yr, yi;
   };
-  const unsigned k_tiles = (args.k + 15) / 16;
   for (int t = 0; t < TX * TY; ++t) {
     const unsigned x0 = x_wave + 32 * (t % TX), y0 = y_wave + 32 * (t / TX);
+    const RowF32<LOADER> x(args, args.x + (size_t)b * args.x_batch_bytes, args.nx, x0 + (lane & 31));
+    const RowF32<LOADER> y(args, args.y + (size_t)b * args.y_batch_bytes, args.ny, y0 + (lane & 31));
     float16_t_ re[1][1], im[1][1];
     re[0][0] = 0.f;
     im[0][0] = 0.f;
-    for (unsigned kt = 0; kt < k_tiles; ++kt) {
+    auto multiply = [&](const Four &f) {
 #pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        re[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.xr[e], f.yr[e], re[0][0], 0, 0, 0);
+        im[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.xr[e], f.yi[e], im[0][0], 0, 0, 0);
+        re[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.xi[e], -f.yi[e], re[0][0], 0, 0, 0);
+        im[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.xi[e], f.yr[e], im[0][0], 0, 0, 0);
+      }
+    };
+    // (half a K tile is read while the one before is multiplied)
+    auto get = [&](unsigned half) {
+      Four f;
+      x.get(half >> 1, (lane >> 5) + 2 * (half & 1), f.xr, f.xi);
+      y.get(half >> 1, (lane >> 5) + 2 * (half & 1), f.yr, f.yi);
+      return f;
+    };
+    const unsigned halves = x.k / 8;
+    if (halves != 0) {
+      Four now = get(0);
+#pragma unroll 1
+      for (unsigned n = 1; n < halves; ++n) {
+        const Four next = get(n);
+        multiply(now);
+        now = next;
+      }
+      multiply(now);
+    }
+    if (x.k < x.k_all) {
+#pragma unroll 1
       for (int s = 0; s < 2; ++s) {
-        float4_t xr, xi, yr, yi;
-        fetch(xv, x0 + (lane & 31), kt, (lane >> 5) + 2 * s, xr, xi);
-        fetch(yv, y0 + (lane & 31), kt, (lane >> 5) + 2 * s, yr, yi);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          re[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[e], yr[e], re[0][0], 0, 0, 0);
-          im[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xr[e], yi[e], im[0][0], 0, 0, 0);
-          re[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xi[e], -yi[e], re[0][0], 0, 0, 0);
-          im[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xi[e], yr[e], im[0][0], 0, 0, 0);
-        }
+        Four f;
+        x.get_end((lane >> 5) + 2 * s, f.xr, f.xi);
+        y.get_end((lane >> 5) + 2 * s, f.yr, f.yi);
+        multiply(f);
       }
     }
     store_wave_tile<TOUT, 1, 1, 32>(args, b, x0, y0, lane, re, im);
@@ -2385,7 +2567,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     bool redo = false;   // (32-bit input) this wave's tile is computed again
     if constexpr (DT == kFloat32) {
-      redo = __any(!mma_split_last(split, acc_re, acc_im));
+      redo = !mma_split_last(split, acc_re, acc_im);
+      if (__builtin_expect(redo, 0)) {
+        redo = !only_nan_rows<LOADER, TX>(args, tc.b, x_wave, y_wave, lane_here(), acc_re, acc_im);
+      }
     }
     bool staged = false;
     if constexpr (XT) {
@@ -2449,8 +2634,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
       }
     }
     if constexpr (DT == kFloat32) {
-      if (redo) {
-        recompute_f32<TOUT, LOADER, TX, TY>(args, tc.b, x_wave, y_wave, lane);
+      if (__builtin_expect(redo, 0)) {
+        recompute_f32<TOUT, LOADER, TX, TY>(args, tc.b, x_wave, y_wave, lane_here());
         // (its loads and stores are not among those that the next tile's waits count)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         staged = true;
@@ -2461,10 +2646,11 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         store_wave_tile_int32<TX, TY, MS>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
       } else if constexpr (DT == kFloat32) {
         // (one MFMA tile after the other: the addresses of both at once do not fit the registers)
+        const int at = lane_here();
 #pragma unroll
         for (int t = 0; t < TX * TY; ++t) {
           const float16_t_ re[1][1] = {{acc_re[t / TX][t % TX]}}, im[1][1] = {{acc_im[t / TX][t % TX]}};
-          store_wave_tile<TOUT, 1, 1, MS>(args, tc.b, x_wave + 32 * (t % TX), y_wave + 32 * (t / TX), lane, re, im);
+          store_wave_tile<TOUT, 1, 1, MS>(args, tc.b, x_wave + 32 * (t % TX), y_wave + 32 * (t / TX), at, re, im);
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {

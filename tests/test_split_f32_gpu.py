@@ -149,3 +149,94 @@ def test_infinities_nan_and_large_sums(layout, block_tile, beta):
     x, y = (np.abs(np.nan_to_num(v, posinf=0, neginf=0)).astype(np.float64) for v in (a, b))
     bound = np.stack([x.sum(1) @ y.sum(1).transpose(0, 2, 1)] * 2, 1) + 2
     assert np.all(np.abs(got[finite].astype(np.float64) - want[finite]) <= 2.0 ** -18 * bound[finite])
+
+
+def pipeline_product(layout, block_tile, a, b, c_axis=PLANAR, order=ROW, alpha=1, beta=0, tout=VT.float32, c=None):
+    """C as [B][2][M][N] of planar a [B][2][M][K] and b [B][2][N][K], by a pipeline that reads planar
+    rows or pairs in place or transposes them into tiles."""
+    B, _, M, K = a.shape
+    N = b.shape[2]
+    dtype = {VT.float32: torch.float32, VT.float16: torch.float16, VT.bfloat16: torch.bfloat16}[tout]
+    il = c_axis == INTERLEAVED
+    if c is None:
+        c = np.full((B, 2, M, N), np.nan, np.float32)
+    d_c = torch.from_numpy(c).cuda().to(dtype)
+    d_c = d_c.permute(0, 2, 3, 1) if il else d_c
+    if order == COL:
+        d_c = d_c.permute(0, 2, 1, 3) if il else d_c.permute(0, 1, 3, 2)
+    d_c = d_c.contiguous()
+    axis = INTERLEAVED if layout == "pairs" else PLANAR
+    d_a, d_b = (to_device(np.ascontiguousarray(x.transpose(0, 2, 3, 1)) if layout == "pairs" else x) for x in (a, b))
+    with cc.option(cc.Option.gemm_block_tile, block_tile), \
+            cc.option(cc.Option.pipeline_route, 2 if layout == "tiled" else 1):
+        p = cc.Pipeline(B, M, N, K, 0, stream(), axis, c_axis, ROW, COL, order, VT.float32, tout, cc.Variant.opt,
+                        alpha, beta)
+    assert p.ReadsInPlace() == (layout != "tiled")
+    p.Run(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr())
+    torch.cuda.synchronize()
+    if order == COL:
+        d_c = d_c.permute(0, 2, 1, 3) if il else d_c.permute(0, 1, 3, 2)
+    return (d_c.permute(0, 3, 1, 2) if il else d_c).float().cpu().numpy()
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [2, 4])
+@pytest.mark.parametrize("B,M,N,K", [(2, 150, 270, 16), (2, 150, 270, 333), (200, 150, 140, 45), (300, 33, 260, 7)])
+def test_nan_in_rows(layout, block_tile, B, M, N, K):
+    """NaN among the samples (no infinities): every sum of such a row is NaN, and all others have the bits
+    that they have without - also those that the same blocks compute next (the larger batches)."""
+    rng = np.random.default_rng(B + K)
+    a = rng.standard_normal((B, 2, M, K)).astype(np.float32)
+    b = rng.standard_normal((B, 2, N, K)).astype(np.float32)
+    clean = pipeline_product(layout, block_tile, a, b)
+    for x in (a, b):   # a few rows of most matrices, and every row of one
+        for i in range(0, B, 3 if x is a else 4):
+            for r in rng.integers(0, x.shape[2], 2):
+                x[i, rng.integers(2), r, rng.integers(K)] = np.nan
+    a[1, rng.integers(0, 2, M), np.arange(M), rng.integers(0, K, M)] = np.nan
+    a[0, 0, M - 1, K - 1] = b[0, 1, N - 1, K - 1] = np.nan
+    got = pipeline_product(layout, block_tile, a, b)
+    rows, cols = np.isnan(a).any(axis=(1, 3)), np.isnan(b).any(axis=(1, 3))
+    nan = (rows[:, :, None] | cols[:, None, :])[:, None] & np.ones((1, 2, 1, 1), bool)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan], clean[~nan])
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("block_tile", [2, 4])
+@pytest.mark.parametrize("c_axis,order,alpha,beta,tout", [(PLANAR, COL, 1, 0, VT.float32),
+                                                          (INTERLEAVED, ROW, 0.5 - 2j, 0, VT.float32),
+                                                          (INTERLEAVED, COL, 1, 0.5 + 1j, VT.float32),
+                                                          (PLANAR, ROW, 2, 0, VT.bfloat16),
+                                                          (INTERLEAVED, ROW, 1, 0.25, VT.float16)])
+def test_infinities_and_nan_before_further_tiles(layout, block_tile, c_axis, order, alpha, beta, tout):
+    """More tiles than blocks, with infinities and NaN in the same wave's rows, in all forms of C."""
+    B, M, N, K = 200, 150, 140, 37
+    rng = np.random.default_rng(4)
+    a = rng.standard_normal((B, 2, M, K)).astype(np.float32)
+    b = rng.standard_normal((B, 2, N, K)).astype(np.float32)
+    c = rng.integers(-8, 8, (B, 2, M, N)).astype(np.float32)
+    for i in range(0, B, 5):
+        a[i, 0, rng.integers(M), rng.integers(K)] = np.inf
+        b[i, 1, rng.integers(N), rng.integers(K)] = -np.inf
+        a[i, 1, rng.integers(M), rng.integers(K)] = np.nan
+    got = pipeline_product(layout, block_tile, a, b, c_axis, order, alpha, beta, tout, c)
+    # (no square of a sum overflows: where both parts are finite so is the result)
+    with np.errstate(invalid="ignore"):
+        re, im = exact(a, b).transpose(1, 0, 2, 3)
+        # (alpha and beta part by part: in numpy's complex product an infinite part spoils the other)
+        z, w = complex(alpha), complex(beta)
+        want = np.stack([z.real * re - z.imag * im + w.real * c[:, 0] - w.imag * c[:, 1] if z.imag else
+                         z.real * re + w.real * c[:, 0] - w.imag * c[:, 1],
+                         z.imag * re + z.real * im + w.imag * c[:, 0] + w.real * c[:, 1] if z.imag else
+                         z.real * im + w.imag * c[:, 0] + w.real * c[:, 1]], 1)
+    finite = np.isfinite(want).all(axis=1, keepdims=True) & np.ones((1, 2, 1, 1), bool)
+    assert not np.isfinite(got[~finite]).all(axis=None) and np.isfinite(got[finite]).all()
+    if alpha == 1:   # (otherwise 0 times an infinity comes in)
+        for kind in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(kind(got), kind(want))
+    # 2 K roundings by half a unit of partial sums below 40 (five standard deviations), times alpha, and one to
+    # the type of C
+    unit = {VT.float32: 0.0, VT.float16: 2.0 ** -11, VT.bfloat16: 2.0 ** -8}[tout]
+    difference = np.abs(got[finite] - want[finite])
+    assert np.all(difference <= 2 * K * 2.0 ** -23 * 40 + 2 * unit * np.abs(want[finite]) + 1e-6)
