@@ -1867,6 +1867,78 @@ __device__ __forceinline__ void store_wave_tile_staged32(const KernelArgs &args,
   }
 }
 
+// The same for 32-bit input, whose blocks have 4 KiB of a slot for each wave: no padding, the 16-byte
+// chunks of the patch's 128-byte rows are XORed with the row (both ways free of bank conflicts). Planar C: a 32 x 32
+// tile at a time; (re, im) pairs: half of one. A store instruction writes eight whole lines instead of
+// 32 pieces of 32 or 64 bytes, us before and after: one K tile to planar C, 4096x4096x16 40.0, 37.5 (planar rows 41.2,
+// 37.9); rows of C that start anywhere, 4001x3999x16 to pairs 46.3, 39.8, x64 81, 75. (Whole lines of
+// pairs at longer K: between 2 % faster and 5 % slower, B=64 512x512x64 70.2, 74.5.)
+constexpr int kStagePatchF32Bytes = 32 * 128;
+
+template <int TX>
+__device__ __forceinline__ void store_wave_tile_staged_f32(const KernelArgs &args, unsigned b, unsigned x_wave,
+                                                           unsigned y_wave, int lane, char *patch,
+                                                           const float16_t_ (&acc_re)[1][TX],
+                                                           const float16_t_ (&acc_im)[1][TX]) {
+  const unsigned nx = args.nx, ny = args.ny;
+  const bool have_alpha = args.have_alpha;
+  const float ar = args.alpha_re, ai = args.alpha_im;
+  float *cbase = reinterpret_cast<float *>(args.c) + (size_t)b * 2 * nx * ny;
+  auto write = [&](int chunk, float4_t v) {   // (row lane % 32 of the tile)
+    *reinterpret_cast<float4_t *>(patch + (lane & 31) * 128 + (chunk ^ (lane & 7)) * 16) = v;
+  };
+  // rows lane / 8 + 8 q
+  const char *rd = patch + (lane >> 3) * 128 + ((lane & 7) ^ (lane >> 3)) * 16;
+  auto store = [&](float *out, size_t stride) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4_t v = *reinterpret_cast<const float4_t *>(rd + q * 8 * 128);
+      *reinterpret_cast<float4_any_t *>(out + (size_t)(q * 8) * stride) = v;
+    }
+  };
+  auto re_of = [&](int i, int e) {
+    const float re = acc_re[0][i][e], im = acc_im[0][i][e];
+    return have_alpha ? alpha_times_re(ar, ai, re, im) : re;
+  };
+  auto im_of = [&](int i, int e) {
+    const float re = acc_re[0][i][e], im = acc_im[0][i][e];
+    return have_alpha ? alpha_times_im(ar, ai, re, im) : im;
+  };
+  const size_t row = (size_t)(y_wave + (lane >> 3)) * nx + x_wave;
+  if (args.c_interleaved) {
+    float *out = cbase + 2 * row + (lane & 7) * 4;
+#pragma unroll
+    for (int i = 0; i < TX; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int e = 8 * h + 4 * k, chunk = 4 * k + 2 * (lane >> 5);
+          write(chunk, float4_t{re_of(i, e), im_of(i, e), re_of(i, e + 1), im_of(i, e + 1)});
+          write(chunk + 1, float4_t{re_of(i, e + 2), im_of(i, e + 2), re_of(i, e + 3), im_of(i, e + 3)});
+        }
+        store(out + 2 * (32 * i + 16 * h), 2 * (size_t)nx);
+      }
+    }
+  } else {
+    float *out = cbase + row + (lane & 7) * 4;
+#pragma unroll
+    for (int plane = 0; plane < 2; ++plane) {
+#pragma unroll
+      for (int i = 0; i < TX; ++i) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = plane == 0 ? re_of(i, 4 * k + e) : im_of(i, 4 * k + e);
+          write(2 * k + (lane >> 5), v);
+        }
+        store(out + (size_t)plane * nx * ny + 32 * i, nx);
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Register-staged kernel: global -> registers -> LDS, two LDS stages. Used for
 // planar (basic) input whose rows are not whole aligned 16-byte chunks: its
@@ -2618,14 +2690,26 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       }
     }
-    if constexpr (MS == 32 && (TOUT == kFloat32 || TOUT == kInt32) &&
-                  !SPLIT && NW * kStagePatch32Bytes <= SLOT_BYTES) {
+    if constexpr (DT == kFloat32 && TOUT == kFloat32) {
+      static_assert(!SPLIT && NW * kStagePatchF32Bytes <= SLOT_BYTES, "a patch for each wave in one slot");
+      if (!args.have_beta) {
+        unsigned free_slot = y_slot + YLEAD;
+        free_slot = free_slot >= SLOTS ? free_slot - SLOTS : free_slot;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (!redo && x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
+          store_wave_tile_staged_f32<TX>(args, tc.b, x_wave, y_wave, lane_here(),
+                                         lds + free_slot * SLOT_BYTES + wave * kStagePatchF32Bytes, acc_re, acc_im);
+          staged = true;
+        }
+      }
+    } else if constexpr (MS == 32 && (TOUT == kFloat32 || TOUT == kInt32) &&
+                         !SPLIT && NW * kStagePatch32Bytes <= SLOT_BYTES) {
       if (staged_ok) {
         // ([X | Y] slots here: the rings are one)
         unsigned free_slot = y_slot + YLEAD;
         free_slot = free_slot >= SLOTS ? free_slot - SLOTS : free_slot;
         asm volatile("s_barrier" ::: "memory");
-        if (!redo && x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
+        if (x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
           store_wave_tile_staged32<TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane,
                                            lds + free_slot * SLOT_BYTES + wave * kStagePatch32Bytes,
                                            acc_re, acc_im);
