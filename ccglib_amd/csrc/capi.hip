@@ -5,6 +5,7 @@
 // src/pipeline/Pipeline.cpp.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -219,25 +220,36 @@ void tiled_bytes(const ccglib_gemm *g, size_t *bytes_a, size_t *bytes_b) {
 //   8-bit pairs     2700, c = 1e7
 //   planar rows     1500, c = 6e6 (squares; long rectangles at small K would still gain up to
 //                   8 % from reading in place beyond it)
-//   ragged rows     800, c = 5e6 (pairs), 400, c = 6e6 (planar). Over 270 random problems (B to 256,
-//                   sizes to 8192) this choice takes 0.76 of the time of tiled copies, the best one 0.75
-//   32-bit rows     450, c = 8e6 (pairs; ragged 300, 4e6), 800, c = 1e7 (planar; ragged 600, 3e6).
-//                   Over 550 random problems 0.81 of the time of tiled copies, as the best one
+//   ragged 8- and 16-bit rows  700, c = 3e6 (pairs), 350, c = 4e6 (planar), by tiles (`by_tiles`): a block takes longer
+//                   for a ragged K tile, which counts in full where there are few blocks, and the transposes write
+//                   whole tiles of rows. fp16 planar rows, in place and with tiles, us: 64x320x6598 147, 71; B=2 192x128x5116
+//                   117, 59; B=55 32x16x7026 93, 150. By M N and M + N alone (800, 5e6; 400, 6e6) the choice was more than
+//                   8 % behind the better one in 3.5 % (pairs) and 9 % (planar) of the problems, up to 2.35 times;
+//                   now in 1.3 % and 2.9 %, up to 1.3 times
+//   32-bit rows     1200, c = 3e6 (pairs; ragged 600, 1e6), 800, c = 1e7 (planar; ragged 500, 1e6): more than
+//                   8 % behind in one problem of 1000. Beyond its break-even, reading pairs in place takes 0.97 to 1.03 times as long
+// The last two over 1130 random problems of each type and layout (the same program, --random).
 struct BreakEven {
   double t, c;
+  bool by_tiles = false;
 };
 bool rows_in_place_pay(size_t B, size_t M, size_t N, size_t K, BreakEven e) {
-  const double operand_elements = (double)B * (double)K * (double)(M + N);
-  return operand_elements > 0 &&
-         (double)M * (double)N / (double)(M + N) < e.t * (1.0 + e.c / operand_elements);
+  double products = (double)B * (double)M * (double)N, rows = (double)M + (double)N;
+  if (e.by_tiles) {   // (two blocks of 64 x 64 a unit, 128 rows a tile)
+    const double blocks = (double)B * (double)ceil_div(M, 64) * (double)ceil_div(N, 64);
+    products = std::max(products, std::ceil(blocks / 512.0) * 512.0 * 64 * 64);
+    rows = (rows + (double)(ceil_div(M, kTileRows) + ceil_div(N, kTileRows)) * kTileRows) / 2;
+  }
+  const double operand_elements = (double)B * (double)K * rows;
+  return operand_elements > 0 && products * (double)K < e.t * (operand_elements + e.c);
 }
 BreakEven break_even_planar(int bits, bool ragged) {
-  if (bits == 32) return ragged ? BreakEven{600.0, 3.0e6} : BreakEven{800.0, 1.0e7};
-  return ragged ? BreakEven{400.0, 6.0e6} : BreakEven{1500.0, 6.0e6};
+  if (bits == 32) return ragged ? BreakEven{500.0, 1.0e6} : BreakEven{800.0, 1.0e7};
+  return ragged ? BreakEven{350.0, 4.0e6, true} : BreakEven{1500.0, 6.0e6};
 }
 BreakEven break_even_pairs(int bits, bool ragged, bool wide) {
-  if (bits == 32) return ragged ? BreakEven{300.0, 4.0e6} : BreakEven{450.0, 8.0e6};
-  if (ragged) return {800.0, 5.0e6};
+  if (bits == 32) return ragged ? BreakEven{600.0, 1.0e6} : BreakEven{1200.0, 3.0e6};
+  if (ragged) return {700.0, 3.0e6, true};
   return {bits == 8 ? 2700.0 : wide ? 3800.0 : 2800.0, 1.0e7};
 }
 
@@ -503,12 +515,11 @@ int ccglib_gemm_run(ccglib_gemm_t g, const void *d_a, const void *d_b, void *d_c
     const size_t row_bytes = g->type_in == kInt1 ? ceil_div(g->K, 32) * 4
                                                  : g->K * (size_t)bits_of(g->type_in) / 8;
     const bool misaligned = row_bytes % 16 == 0 && ((uintptr_t)d_a % 16 != 0 || (uintptr_t)d_b % 16 != 0);
-    // Planar operands that are not 16-byte aligned cannot be copied to LDS in
-    // place either: the object gets its workspace at the first such Run (the one
+    // Planar rows of whole chunks that are not 16-byte aligned are read faster from
+    // tiles: the object gets its workspace at the first such Run (the one
     // allocation a Run may make) and keeps it - unless the stream is being
-    // captured into a graph, where the kernel that reads such rows through
-    // registers runs instead (the option EXPECT_UNALIGNED makes the object
-    // allocate at construction).
+    // captured into a graph, where they are read in place as ragged rows
+    // instead (the option EXPECT_UNALIGNED makes the object allocate at construction).
     if (misaligned && !g->retile.load(std::memory_order_acquire) && !stream_is_capturing(g->stream)) {
       // (two threads may Run one object: only one of them allocates)
       std::lock_guard<std::mutex> lock(g->lazy_lock);
@@ -888,7 +899,7 @@ int pipeline_create(ccglib_pipeline_t *pipeline, size_t B, size_t M, size_t N, s
   const bool il_ragged = il_row_bytes % 16 != 0, planar_ragged = planar_row_bytes % 16 != 0;
   const bool fused = allow_fused && !packing && input_complex_axis_location == kInterleaved &&
                      (in_bits == 8 || in_bits == 16 || in_bits == 32) && il_row_bytes >= 16 &&
-                     ((variant == kBasic && !il_ragged) ||
+                     ((variant == kBasic && !il_ragged && in_bits != 32) ||
                       in_place(break_even_pairs((int)in_bits, il_ragged, wide_rows)));
   // Planar input of the opt variant: the GEMM can read the rows in place as well (the basic
   // variant's loader, same arithmetic and K order as on tiles). That costs the GEMM

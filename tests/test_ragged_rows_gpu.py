@@ -81,6 +81,42 @@ def test_pairs(block_tile, tin, K):
                 orc.gemm_float64(qa, qb, M, N, K, ORC_TYPE[tin]), tin, VT.float32)
 
 
+@pytest.mark.parametrize("block_tile,B,M,N", [(4, 70, 180, 190), (2, 256, 140, 130), (1, 300, 150, 200)])
+@pytest.mark.parametrize("axis,tin,K", [(PLANAR, VT.float16, 13), (PLANAR, VT.float16, 77), (PLANAR, VT.bfloat16, 205),
+                                        (PLANAR, VT.float32, 7), (PLANAR, VT.float32, 45),
+                                        (PLANAR, VT.float8e4m3, 29), (PLANAR, VT.float8e5m2, 333),
+                                        (INTERLEAVED, VT.float16, 9), (INTERLEAVED, VT.float16, 141),
+                                        (INTERLEAVED, VT.float32, 3), (INTERLEAVED, VT.float32, 37),
+                                        (INTERLEAVED, VT.float8e4m3, 61), (INTERLEAVED, VT.float8e4m3, 259)])
+def test_more_tiles_than_blocks(block_tile, B, M, N, axis, tin, K):
+    """Blocks that go on to further C tiles: K of one K tile and of several, the row ends of the one put
+    right while the copies of the next are under way. Planar rows: the bits of the tiled route."""
+    qa, qb = operands(np.random.default_rng(K), B, M, N, K, tin)
+    if axis == INTERLEAVED:
+        qa, qb = pairs(qa, B, M, K), pairs(qb, B, N, K)
+    d_a, d_b = to_device(qa), to_device(qb)
+    outs = []
+    for route in (1, 2):
+        with cc.option(cc.Option.gemm_block_tile, block_tile), cc.option(cc.Option.pipeline_route, route):
+            p = cc.Pipeline(B, M, N, K, 0, stream(), axis, PLANAR, ROW, COL, ROW, tin, VT.float32, cc.Variant.opt)
+        assert p.ReadsInPlace() == (route == 1)
+        d_c = torch.full((B, 2, M, N), np.nan, device="cuda")
+        p.Run(d_a.data_ptr(), d_b.data_ptr(), d_c.data_ptr())
+        outs.append(d_c)
+    torch.cuda.synchronize()
+    if axis == PLANAR:
+        assert torch.equal(outs[0], outs[1])
+    else:
+        # two orders of the same products. fp32 sums: 2 K roundings each, of partial sums that never exceed the
+        # sum of the moduli, 2 K here; 8-bit ones: each within 6e-5 of the product in 64 bits
+        # (test_64x64_blocks_on_interleaved_bytes)
+        difference = (outs[0] - outs[1]).double()
+        if tin == VT.float8e4m3:
+            assert difference.norm() <= 2 * 6e-5 * outs[1].double().norm()
+        else:
+            assert difference.abs().max() <= 2 * 2.0 ** -24 * (2 * K) ** 2
+
+
 @pytest.mark.parametrize("axis", [PLANAR, INTERLEAVED])
 def test_infinities_at_the_end_of_a_row(axis):
     # The last elements of a row are fetched together with some before them, which must not
