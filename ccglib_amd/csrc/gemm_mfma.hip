@@ -11,11 +11,11 @@
 //  * One persistent block owns a sequence of BX x BY patches of C and walks K in
 //    tiles of 64 bytes per row. Tiles go global -> LDS directly
 //    (global_load_lds_dwordx4) through a ring of LDS slots, two iterations ahead
-//    of the math: for the tiled (opt) layout, for planar (basic) rows that are
-//    whole aligned 16-byte chunks, and for the pipeline's interleaved rows. Only
-//    planar rows that are neither (and have no tiled copy) are staged through
-//    registers by a second kernel, whose element-wise loads do their bounds
-//    checks and zero fill.
+//    of the math: for the tiled (opt) layout, for planar (basic) rows and for the
+//    pipeline's interleaved rows, of any length from 16 bytes on and at any address.
+//    Only shorter planar rows, and 1-bit ones that are not whole aligned 16-byte
+//    chunks (both without a tiled copy), are staged through registers by kernels
+//    whose element-wise loads do their bounds checks and zero fill.
 //  * LDS rows are 64 bytes with the 16-byte chunk index XORed by a function of
 //    the row that suits the fragment shape of the MFMA in use (measured free of
 //    bank conflicts; see complex_gemm_mfma_dtl).
@@ -1941,8 +1941,8 @@ __device__ __forceinline__ void store_wave_tile_staged_f32(const KernelArgs &arg
 
 // ---------------------------------------------------------------------------
 // Register-staged kernel: global -> registers -> LDS, two LDS stages. Used for
-// planar (basic) input whose rows are not whole aligned 16-byte chunks: its
-// element-wise loads do the bounds checks and the zero fill.
+// planar (basic) input whose rows are shorter than 16 bytes: its element-wise
+// loads do the bounds checks and the zero fill.
 // ---------------------------------------------------------------------------
 template <int DT, int TOUT, int BX, int BY, int WX, int WY, int KT, int LOADER, int WAVES_PER_EU>
 __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void complex_gemm_mfma(
@@ -2627,14 +2627,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     // tile is being computed. The counter cannot tell loads from stores, so
     // the next tile's first K tiles, which are already on their way, are waited
     // for now; the first wait that has to include the stores then comes YLEAD
-    // iterations into the next tile. (64 x 64 blocks: the wave's reads of the last slot as well,
-    // which the compiler waits for no sooner than at its last matrix instructions, behind the
-    // epilogue's barrier if it moves those there; other waves write to that slot behind the barrier.)
-    if constexpr (SMALL) {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    // iterations into the next tile. (64 x 64 blocks: the wave's reads of the last slot may still be
+    // under way; the next tile's first barrier, behind which the slot is refilled, waits for them,
+    // and no epilogue of theirs uses LDS.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const TileCoord tc = tile_coord(args, vt);
     const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     bool redo = false;   // (32-bit input) this wave's tile is computed again
@@ -2914,7 +2910,7 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles of 8- and 1-bit input, and
 // a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
 // With beta the epilogue reads C first, which costs the larger tiles more (8 bits on planar
-// rows, B=11 456x1542x192: 96, 84, 46). Interleaved fp32 C behind tiles, which only the 256 x 128
+// rows, B=11 456x1542x192: 96, 84, 46). Interleaved fp32 C of 16-bit tiles, which only the 256 x 128
 // block regroups through LDS, moves no line: where a smaller block is chosen the larger one is
 // slower by 0.95 to several times, 1.37 (128 x 128) and 2.9 (64 x 64) at the median.
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
@@ -3002,8 +2998,9 @@ template <int DT, int TOUT>
 hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   constexpr int KPM = DtypeTraits<DT>::kTilesPerMfma;
   const size_t k_bytes = (size_t)p.k * bits_of(p.type_in) / 8;
-  // planar rows made of whole, aligned 16-byte chunks can be copied straight
-  // into LDS as well; anything else goes through the register-staged kernel
+  // planar rows made of whole, aligned 16-byte chunks are copied straight into LDS,
+  // other rows from 16 bytes on by the ragged loader; what is left goes through the
+  // register-staged kernel
   const bool planar_direct = (p.variant == kBasic) && (k_bytes >= 16) && (k_bytes % 16 == 0) &&
                              ((uintptr_t)p.x % 16 == 0) && ((uintptr_t)p.y % 16 == 0);
   const BlockShape shape = block_choice(p).shape;

@@ -315,8 +315,8 @@ hipError_t launch_transpose(const TransposeParams &p, hipStream_t stream) {
   }
 }
 
-// Both operands of one GEMM. One launch when they take the same vector kernel and
-// one of them is at most a quarter of the other, otherwise one launch each.
+// Both operands of one GEMM. One launch when they take the same vector kernel and one
+// of them is at most a quarter of the other, or both are small (try_launch_pair), otherwise one launch each.
 hipError_t launch_transpose_pair(const TransposeParams &p0, const TransposeParams &p1,
                                  hipStream_t stream) {
   hipError_t e = hipSuccess;
