@@ -35,20 +35,8 @@
 
 #include "gemm_device.h"
 
-// Timing-only builds for the kernel-configuration sweep (never for the library):
-// a bit mask of parts of the kernels to leave out, which gives wrong numbers and
-// shows what each part costs. 1: the C stores (of the register-direct epilogues of
-// 16-bit input); 2: the matrix instructions (16-row shapes); 4: the global -> LDS
-// copies; 8: the barrier of the K loop.
-#ifndef CCGLIB_ABLATE
-#define CCGLIB_ABLATE 0
-#endif
-
 namespace ccglib_amd {
 namespace {
-
-constexpr bool kAblateStores = (CCGLIB_ABLATE & 1) != 0, kAblateMfma = (CCGLIB_ABLATE & 2) != 0,
-               kAblateCopies = (CCGLIB_ABLATE & 4) != 0, kAblateBarrier = (CCGLIB_ABLATE & 8) != 0;
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -86,11 +74,6 @@ template <int DT> struct Fragment {
 template <int DT>
 __device__ __forceinline__ float4_t mfma(const Fragment<DT> &a, const Fragment<DT> &b,
                                          float4_t acc) {
-  if constexpr (kAblateMfma) {
-    // (timing-only build: the operands are still fetched)
-    asm volatile("" : "+v"(acc) : "v"(a.v[0]), "v"(b.v[0]));
-    return acc;
-  }
   if constexpr (DT == kFloat16) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(
         __builtin_bit_cast(half8_t, a.v[0]), __builtin_bit_cast(half8_t, b.v[0]), acc, 0, 0, 0);
@@ -1672,9 +1655,7 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
                             : (have_alpha ? alpha_times_im(ar, ai, re, im) : im);
         }
         Tout *p = out + (size_t)plane * nx * ny + (size_t)(j * 16 + e) * nx;
-        if constexpr (kAblateStores) {
-          if (v[0] == 12345.678f) *p = (Tout)v[1];   // (timing-only build)
-        } else if constexpr (TOUT == kFloat32) {
+        if constexpr (TOUT == kFloat32) {
           *reinterpret_cast<float4_any_t *>(p) = float4_t{v[0], v[1], v[2], v[3]};
         } else {
           Tout t[4] = {(Tout)v[0], (Tout)v[1], (Tout)v[2], (Tout)v[3]};
@@ -2088,8 +2069,6 @@ template <int N, bool READS = false> __device__ __forceinline__ void wait_vmcnt_
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
   if constexpr (READS) {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-  } else if constexpr (kAblateBarrier) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
   } else {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
   }
@@ -2109,7 +2088,6 @@ template <int N, bool READS = false> __device__ __forceinline__ void wait_vmcnt_
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_1k_to_lds(const char *base, unsigned lane_offset,
                                                unsigned lds_address) {
-  if constexpr (kAblateCopies) return;
   unsigned long long base_here;
   asm volatile(
       "s_mov_b64 %0, %3\n\t"
@@ -2125,7 +2103,6 @@ __device__ __forceinline__ void load_1k_to_lds(const char *base, unsigned lane_o
 // are not contiguous in memory).
 __device__ __forceinline__ void load_1k_to_lds_by_lane(const char *lane_address,
                                                        unsigned lds_address) {
-  if constexpr (kAblateCopies) return;
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
       "s_nop 0\n\t"

@@ -70,15 +70,6 @@ constexpr int kWideShortBX = 128;       // columns of a short tile: the first ei
 // ZERO: the sum starts from zero (first K tile of a C tile).
 template <int DT, bool ACC_IN_AGPR, bool ZERO>
 __device__ __forceinline__ void mfma16_asm(float4_t &acc, const int4_t &a, const int4_t &b) {
-  if constexpr (kAblateMfma) {
-    // (timing-only build: the accumulator and the operands stay where they are)
-    if constexpr (ACC_IN_AGPR) {
-      asm volatile("" : "+a"(acc) : "v"(a), "v"(b));
-    } else {
-      asm volatile("" : "+v"(acc) : "v"(a), "v"(b));
-    }
-    return;
-  }
 #define CCGLIB_MFMA_ASM(OPCODE)                                                                    \
   if constexpr (ACC_IN_AGPR) {                                                                     \
     if constexpr (ZERO) {                                                                          \
@@ -445,7 +436,7 @@ __global__ __launch_bounds__(256, 1) void complex_gemm_mfma_wide(const KernelArg
     yr[j] = rd(yo + j * TILE16);
     yi[j] = rd(yo + Y2ND + j * TILE16);
   }
-  if constexpr (!kAblateBarrier) asm volatile("s_barrier" ::: "memory");
+  asm volatile("s_barrier" ::: "memory");
   xr[0] = rd(xo[0]);
   xi[0] = rd(xo[0] + X2ND);
   if constexpr (IL) {
@@ -560,9 +551,7 @@ __global__ __launch_bounds__(256, 1) void complex_gemm_mfma_wide(const KernelArg
     }
     char *p = target.base + plane * plane_bytes +
               ((size_t)(j * 16 + e) * args.nx + g * 64) * sizeof(Tout) + lane_store_off;
-    if constexpr (kAblateStores) {
-      if (v[0] == 12345.678f) *reinterpret_cast<Tout *>(p) = (Tout)v[1];   // (timing-only build)
-    } else if constexpr (TOUT == kFloat32) {
+    if constexpr (TOUT == kFloat32) {
       // (C is written once and not read again by this kernel: stores marked
       // non-temporal measured 0.4 % faster at B=64 512x4096x576)
       __builtin_nontemporal_store(float4_t{v[0], v[1], v[2], v[3]}, reinterpret_cast<float4_t *>(p));
@@ -702,7 +691,7 @@ __global__ __launch_bounds__(256, 1) void complex_gemm_mfma_wide(const KernelArg
           }
           // every wave's part of the next X tile has landed, and nobody reads the
           // current X slot any more
-          if constexpr (!kAblateBarrier) asm volatile("s_barrier" ::: "memory");
+          asm volatile("s_barrier" ::: "memory");
           xr[0] = rd(xo[0] + xa_next);
           xi[0] = rd(xo[0] + xa_next + X2ND);
           CCGLIB_PIN;

@@ -19,7 +19,6 @@
 // --fill=legacy: the fill of earlier sweeps (a 2 MiB pattern of numbers with three
 //   exponents; fp8 without sign bit), kept for comparison with their files.
 // --fill=zero: all-zero operands (no power limit).
-// `make ABLATE=n` builds timing-only variants (see CCGLIB_ABLATE in gemm_mfma.hip).
 //
 //   ./tune_gemm --probe=mfma|mix|fill|l2read [--fill=...]
 // Small probes of the machine that the kernels' floors are argued from: the rate
@@ -525,9 +524,8 @@ int main(int argc, char **argv) {
   hipEvent_t e0, e1;
   CHECK(hipEventCreate(&e0));
   CHECK(hipEventCreate(&e1));
-  std::printf("%-44s %10s %12s %10s   (B=%u M=%u N=%u K=%u, %s operands%s)\n", "configuration", "ms", "TFLOP/s",
-              "of peak", B, M, N, K, fill.c_str(), CCGLIB_ABLATE ? ", TIMING-ONLY BUILD" : "");
-  if (CCGLIB_ABLATE) std::printf("CCGLIB_ABLATE = %d: parts of the kernels are left out, C is wrong\n", CCGLIB_ABLATE);
+  std::printf("%-44s %10s %12s %10s   (B=%u M=%u N=%u K=%u, %s operands)\n", "configuration", "ms", "TFLOP/s",
+              "of peak", B, M, N, K, fill.c_str());
   for (const Config &c : kConfigs) {
     if (filter && !std::strstr(c.name, filter)) continue;
     GemmParams p;

@@ -109,7 +109,8 @@ CCGLIB_API const char *ccglib_version(void);
  *                    allocated when the object is created, and no device Run
  *                    allocates.
  *   PIPELINE_ROUTE   0 (default): an opt-variant pipeline whose input rows are
- *                    16 bytes or longer lets the GEMM read them in place
+ *                    16 bytes or longer (of the basic variant: ragged and 32-bit
+ *                    interleaved rows) lets the GEMM read them in place
  *                    where that is faster than transposing them into tiles
  *                    first (small M N / (M + N); the break-even points are
  *                    measured ones), and transposes otherwise; 1: in place
