@@ -2875,28 +2875,27 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // problem fills and the less it computes beyond the edges of C, but the more bytes it
 // moves per flop. Times with 256 x 128, 128 x 128 and 64 x 64 blocks in us, on operands that no cache
 // held (profiles/gemm_block_choice.txt):
-//   too few tiles for the larger blocks, 16 bits 256^3:  14.7, 12.5, 6.9;  B=256 96x96x1024:  86, 56, 62;
-//     32 bits B=2 1000^3:  (none), 176, 122;  8 bits 1024^3:  24.9, 22.3, 11.5;
-//     1 bit 64x64x65536:  526, 305, 116
-//   every unit busy, 16 bits on tiles, 4096x4096x512:  68, 89, 102
-//     on planar rows, of which a copy fetches half cache lines, B=157 192x604x3680:  747, 909, 1026
-//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  (none), 435, 502
-//     8 bits on tiles, 4096x4096x512:  48, 48, 69
+//   too few tiles for the larger blocks, 16 bits 256^3:  14.4, 12.2, 6.5;  B=256 96x96x1024:  87, 57, 63;
+//     32 bits B=2 1000^3:  (none), 186, 129;  8 bits 1024^3:  24.3, 21.8, 10.8;
+//     1 bit 64x64x65536:  529, 308, 115
+//   every unit busy, 16 bits on tiles, 4096x4096x512:  73, 92, 106
+//     on planar rows, of which a copy fetches half cache lines, B=157 192x604x3680:  762, 908, 1057
+//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  (none), 453, 523
+//     8 bits on tiles, 4096x4096x512:  52, 51, 69
 //     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
-//       277, 288, 312
+//       308, 317, 339
 // Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles of 8- and 1-bit input, and
 // a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
 // With beta the epilogue reads C first, which costs the larger tiles more (8 bits on planar
-// rows, B=11 456x1542x192: 96, 84, 46). Interleaved fp32 C of 16-bit tiles, which only the 256 x 128
+// rows, B=11 456x1542x192: 97, 84, 47). Interleaved fp32 C of 16-bit tiles, which only the 256 x 128
 // block regroups through LDS, moves no line: where a smaller block is chosen the larger one is
 // slower by 0.95 to several times, 1.37 (128 x 128) and 2.9 (64 x 64) at the median.
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
 // 30000 problems of random sizes, 40 % of them on operands that no cache held
 // (python -m ccglib_amd.tuning.block_choice times such problems); those of 8-bit tiles
-// and 16-bit pairs to 1900 further ones, timed since those kernels last changed. The choice is then on average
-// 0.2 % behind the fastest of the three shapes, and more than 8 % behind in 0.7 % of the problems.
-// 32-bit input: 1200 problems, on average less than 0.1 % behind the faster of its two shapes, more than
-// 8 % in one.
+// and 16-bit pairs to 1900, of 32-bit input to 1200 further ones, timed since those kernels last changed. On 8000
+// others, ragged rows among them, the choice is on average 0.1 % behind the fastest of the three shapes, and more
+// than 8 % behind in 1.2 % of the problems.
 enum BlockShape { k256x128, k128x128, k64x64 };
 struct BlockChoice {
   BlockShape shape;
