@@ -19,6 +19,7 @@ SOURCES = ["capi.hip", "gemm_mfma_f16.hip", "gemm_mfma_bf16.hip", "gemm_mfma_f32
            "transpose.hip", "packing.hip"]
 HEADERS = [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_device.h"),
            os.path.join(CSRC, "gemm_mfma.hip"), os.path.join(CSRC, "gemm_mfma_wide.h"),
+           os.path.join(CSRC, "gemm_mfma_wave.h"),
            os.path.join(os.path.dirname(HERE), "include", "ccglib_amd.h")]
 
 # Packed-fp32 instruction selection is switched off for all device code.

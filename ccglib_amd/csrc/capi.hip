@@ -398,8 +398,8 @@ int ccglib_amd_set_option(int option, size_t value) {
   if (option < 0 || option >= CCGLIB_AMD_OPTION_COUNT) {
     return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "unknown option %d", option);
   }
-  if (option == CCGLIB_AMD_OPTION_GEMM_BLOCK_TILE && value > 4) {
-    return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "GEMM_BLOCK_TILE is 0, 1, 2, 3 or 4 (got %zu)", value);
+  if (option == CCGLIB_AMD_OPTION_GEMM_BLOCK_TILE && value > 7) {
+    return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "GEMM_BLOCK_TILE is 0 to 7 (got %zu)", value);
   }
   if (option == CCGLIB_AMD_OPTION_PIPELINE_ROUTE && value > 2) {
     return fail(CCGLIB_ERROR_INVALID_ARGUMENT, "PIPELINE_ROUTE is 0, 1 or 2 (got %zu)", value);

@@ -162,13 +162,14 @@ __device__ __forceinline__ unsigned small_div(unsigned n, unsigned d, unsigned *
 }
 
 // Splits the logical tile id into (batch, block_x, block_y). Inside a batch,
-// tiles are walked in groups of 4 block rows with y fastest, so the 32
-// consecutive tiles that one XCD works on touch 4 Y panels and 8 X panels.
+// tiles are walked in groups of GROUP block rows with y fastest, so the 32
+// consecutive tiles that one XCD works on touch 4 Y panels and 8 X panels (GROUP = 4).
 // (Persistent blocks call this once per C tile, between two K iterations: with
 // fewer than 2^20 tiles in all it takes the short divisions above.)
 struct TileCoord {
   unsigned b, block_x, block_y;
 };
+template <unsigned GROUP = 4>
 __device__ __forceinline__ TileCoord tile_coord(const KernelArgs &args, unsigned wg) {
   const unsigned per_batch = args.blocks_x * args.blocks_y;
   const unsigned total = per_batch * args.batch;
@@ -182,7 +183,6 @@ __device__ __forceinline__ TileCoord tile_coord(const KernelArgs &args, unsigned
     tc.b = logical / per_batch;
     t = logical % per_batch;
   }
-  constexpr unsigned GROUP = 4;
   const unsigned group_size = GROUP * args.blocks_x;
   unsigned in_group;
   const unsigned g = small ? small_div(t, group_size, &in_group) : t / group_size;

@@ -28,6 +28,7 @@
 //    sign of Re -= Xi*Yi is a sign-bit flip of the Yi fragment registers.
 //  * Workgroup ids are remapped so that consecutive tiles land on the same
 //    XCD (shared L2), in groups that reuse both operands.
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <type_traits>
@@ -2721,6 +2722,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+#include "gemm_mfma_wave.h"
+
 inline hipError_t check_grid(size_t total) {
   return total > 0x7fffffffu ? hipErrorInvalidValue : hipSuccess;
 }
@@ -2792,6 +2795,17 @@ hipError_t launch_dtl(const GemmParams &p, hipStream_t stream) {
   const size_t resident = (size_t)compute_units() * BLOCKS_PER_CU / kNumXcd * kNumXcd;
   const unsigned grid = (unsigned)(total < resident ? total : resident);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(NTHREADS), LDS_BYTES, stream, a);
+  return hipGetLastError();
+}
+
+template <int DT, int TOUT, int LOADER, int TX, int TY>
+hipError_t launch_wave(const GemmParams &p, hipStream_t stream) {
+  const KernelArgs a = make_kernel_args(p, 16 * TX, 16 * TY);
+  const size_t total = (size_t)a.blocks_x * a.blocks_y * p.batch;
+  if (total == 0) return hipSuccess;
+  if (hipError_t e = check_grid(total)) return e;
+  hipLaunchKernelGGL((complex_gemm_mfma_wave<DT, TOUT, LOADER, TX, TY>), dim3((unsigned)total), dim3(64), kWaveLdsBytes,
+                     stream, a);
   return hipGetLastError();
 }
 
@@ -2941,7 +2955,7 @@ inline BlockChoice block_choice(const GemmParams &p) {
   const double t64 = time(64, 64, costs.cost_64, costs.tile_64, costs.lone_64, costs.beta_64);
   if (p.block_tile == 1 && !no_256) return {k256x128, t256};
   if (p.block_tile == 1 || p.block_tile == 2) return {k128x128, t128};
-  if (p.block_tile == 4) return {k64x64, t64};
+  if (p.block_tile >= 4) return {k64x64, t64};   // (5 to 7: waves, where there are such kernels)
   if (t256 <= t128 && t256 <= t64) return {k256x128, t256};
   return t128 <= t64 ? BlockChoice{k128x128, t128} : BlockChoice{k64x64, t64};
 }
@@ -2972,8 +2986,103 @@ inline bool wide_tiles_pay(const GemmParams &p) {
   return wide_tiling(p).rounds * (kWideBX * kWideBY) < 1.075 * block_choice(p).time;
 }
 
+// Which tile the waves of complex_gemm_mfma_wave take, if that kernel is the faster one: the least of
+//   fixed + max(K tiles * alone, K tiles * crowded * n / 256) + tile * n / 256   in us
+// over 64 x 64 blocks and the wave tiles, with n blocks or waves on 256 units: `alone` is what a K tile takes
+// with a unit to itself, `crowded` with others next to it, `tile` what a tile costs besides. The constants are
+// fitted, for each type and operand layout, to the times of all shapes on 1600 problems of up to 1024 blocks of
+// 64 x 64 (450 of 1-bit input), 60 % of them on operands that no cache held, a fifth on ragged rows.
+// There the choice is 2 to 3 % (16 bits) and 1 % (8 and 1 bits) behind the fastest shape on average, and in front of
+// 64 x 64 blocks by 1.41 times (16 bits), 1.20 (8 bits), 1.15 (1 bit); it is more than 5 % slower than those
+// in 22 of 1644. More waves than fit the units at once are left to the blocks, which walk their tiles
+// without gaps (93 batches of 32x448x1584: 58 us, 85 with 1302 waves of 32 x 32).
+enum WaveShape { kNoWaves, kWaves32x32, kWaves32x16, kWaves16x16 };
+struct WaveCosts {
+  double fixed, alone, crowded, tile;
+};
+inline const WaveCosts *wave_costs(const GemmParams &p) {   // 64 x 64 blocks, then as WaveShape
+  static constexpr WaveCosts none = {0.0, 0.0, 0.0, 0.0};
+  static constexpr WaveCosts bits16_tiled[] = {{3.80, 0.286, 0.367, 1.48}, {2.92, 0.240, 0.139, 0.49},
+                                               {3.09, 0.141, 0.081, 0.13}, {3.24, 0.086, 0.058, 0.01}};
+  static constexpr WaveCosts bits16_planar[] = {{4.12, 0.438, 0.524, 1.36}, {3.35, 0.257, 0.253, 0.31},
+                                                {3.23, 0.165, 0.168, 0.00}, {3.24, 0.092, 0.102, 0.03}};
+  static constexpr WaveCosts bits16_pairs[] = {{4.13, 0.356, 0.423, 1.58}, {3.13, 0.295, 0.180, 0.51},
+                                               {3.05, 0.184, 0.099, 0.22}, {3.14, 0.110, 0.066, 0.08}};
+  static constexpr WaveCosts bits8_tiled[] = {{3.95, 0.265, 0.415, 1.65}, {3.38, 0.161, 0.129, 0.51}, none, none};
+  static constexpr WaveCosts bits8_planar[] = {{4.55, 0.349, 0.556, 1.92}, {4.08, 0.157, 0.249, 0.17}, none, none};
+  static constexpr WaveCosts bits8_pairs[] = {{4.54, 0.413, 0.433, 1.79}, {3.23, 0.238, 0.206, 0.84}, none, none};
+  static constexpr WaveCosts int1_tiled[] = {{4.08, 0.871, 1.041, 1.61}, {3.20, 0.735, 0.282, 0.50}, none, none};
+  static constexpr WaveCosts int1_planar[] = {{4.45, 0.840, 1.023, 1.77}, {3.31, 0.746, 0.359, 0.82}, none, none};
+  const bool tiled = p.variant == kOpt && !p.input_interleaved;
+  if (p.type_in == kInt1) return tiled ? int1_tiled : int1_planar;
+  if (bits_of(p.type_in) == 8) return p.input_interleaved ? bits8_pairs : tiled ? bits8_tiled : bits8_planar;
+  return p.input_interleaved ? bits16_pairs : tiled ? bits16_tiled : bits16_planar;
+}
+inline WaveShape wave_choice(const GemmParams &p) {
+  const bool bits16 = bits_of(p.type_in) == 16;
+  if (p.type_in == kFloat32 || (p.block_tile != 0 && p.block_tile < 5)) return kNoWaves;
+  if (p.variant != kOpt || p.input_interleaved) {
+    // rows in place: a lane's place among 32 rows is a 32-bit number, and its chunk never longer than the row
+    const size_t k_mem = p.k_in_memory ? p.k_in_memory : p.k, planes = p.input_interleaved ? 2 : 1;
+    if (planes * k_mem * bits_of(p.type_in) / 8 >= ((size_t)1 << 26) ||
+        planes * p.k * bits_of(p.type_in) / 8 < 16) {
+      return kNoWaves;
+    }
+  }
+  if (p.block_tile >= 5) return p.block_tile == 5 || !bits16 ? kWaves32x32 : p.block_tile == 6 ? kWaves32x16 : kWaves16x16;
+  if (block_choice(p).shape != k64x64) return kNoWaves;
+  const WaveCosts *costs = wave_costs(p);
+  const double k_tiles = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
+  const double units = (double)compute_units();
+  // Ragged rows of many K tiles go through the transposes (rows_in_place_pay), with waves on the tiles behind
+  // them; which route such rows take is fixed by a test, so that waves on the rows as they lie, which
+  // would be faster still (fp16 64x320x6598 22.5 us, transposes and waves 30.6, and 68 before
+  // there were waves), stay with the shorter ones.
+  const bool ragged = (p.variant != kOpt || p.input_interleaved) && p.type_in != kInt1 &&
+                      (p.input_interleaved ? 2 : 1) * (size_t)p.k * bits_of(p.type_in) / 8 % 16 != 0;
+  if (ragged && k_tiles > 64.0) return kNoWaves;
+  auto time = [&](int shape, unsigned x, unsigned y) {
+    const WaveCosts &c = costs[shape];
+    const double n = (double)p.batch * (double)ceil_div(p.nx, x) * (double)ceil_div(p.ny, y) / units;
+    if (shape != 0 && n > kWavesPerUnit) return HUGE_VAL;
+    return c.fixed + k_tiles * std::max(c.alone, c.crowded * n) + c.tile * n;
+  };
+  double best = time(0, 64, 64);
+  WaveShape shape = kNoWaves;
+  auto try_shape = [&](WaveShape s, unsigned x, unsigned y) {
+    const double t = time(s, x, y);
+    if (t < best) best = t, shape = s;
+  };
+  try_shape(kWaves32x32, 32, 32);
+  if (bits16) {
+    try_shape(kWaves32x16, 32, 16);
+    try_shape(kWaves16x16, 16, 16);
+  }
+  return shape;
+}
+template <int DT, int TOUT>
+hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream) {
+  auto launch = [&](auto loader) {
+    constexpr int L = decltype(loader)::value;
+    if constexpr (DT == kFloat16 || DT == kBfloat16) {
+      if (shape == kWaves16x16) return launch_wave<DT, TOUT, L, 1, 1>(p, stream);
+      if (shape == kWaves32x16) return launch_wave<DT, TOUT, L, 2, 1>(p, stream);
+    }
+    return launch_wave<DT, TOUT, L, 2, 2>(p, stream);
+  };
+  if constexpr (DT != kInt1) {
+    if (p.input_interleaved) return launch(std::integral_constant<int, kLoadInterleavedRagged>{});
+  }
+  if (p.variant == kOpt) return launch(std::integral_constant<int, kLoadTiled>{});
+  return launch(std::integral_constant<int, kLoadPlanarRagged>{});
+}
+
 template <int DT, int TOUT>
 hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
+  if constexpr (DT != kFloat32) {
+    const WaveShape waves = wave_choice(p);
+    if (waves != kNoWaves) return launch_waves<DT, TOUT>(p, waves, stream);
+  }
   constexpr int KPM = DtypeTraits<DT>::kTilesPerMfma;
   const size_t k_bytes = (size_t)p.k * bits_of(p.type_in) / 8;
   // planar rows made of whole, aligned 16-byte chunks are copied straight into LDS,
@@ -3156,6 +3265,8 @@ hipError_t launch_gemm_mfma_int1(const GemmParams &p, hipStream_t stream) {
   // packed 1-bit samples expanded in registers; the caller has checked that
   // planar rows are whole aligned 16-byte chunks and that K fits fp32 sums
   if (p.type_out != kInt32 || p.input_interleaved) return hipErrorInvalidValue;
+  const WaveShape waves = wave_choice(p);
+  if (waves != kNoWaves) return launch_waves<kInt1, kInt32>(p, waves, stream);
   const BlockShape shape = block_choice(p).shape;
   if (shape == k64x64) {
     return p.variant == kOpt
@@ -3183,6 +3294,25 @@ const char *describe_gemm_mfma(const GemmParams &p) {
   const bool planar_direct = (p.variant == kBasic) && (k_bytes >= 16) && (k_bytes % 16 == 0) &&
                              ((uintptr_t)p.x % 16 == 0) && ((uintptr_t)p.y % 16 == 0);
   const BlockShape shape = block_choice(p).shape;
+  const WaveShape waves = wave_choice(p);
+  if (waves != kNoWaves) {
+    // (a wave's tile, and the region of C whose waves are numbered consecutively)
+    const bool pairs = p.input_interleaved, tiled = p.variant == kOpt && !pairs;
+    auto by_layout = [&](const char *t, const char *i, const char *r) { return tiled ? t : pairs ? i : r; };
+    if (waves == kWaves16x16) {
+      return by_layout("complex_gemm_mfma_wave, 16x16 a wave, 16 waves to 64x64, tiled operands",
+                       "complex_gemm_mfma_wave, 16x16 a wave, 16 waves to 64x64, interleaved rows",
+                       "complex_gemm_mfma_wave, 16x16 a wave, 16 waves to 64x64, planar rows");
+    }
+    if (waves == kWaves32x16) {
+      return by_layout("complex_gemm_mfma_wave, 32x16 a wave, 8 waves to 64x64, tiled operands",
+                       "complex_gemm_mfma_wave, 32x16 a wave, 8 waves to 64x64, interleaved rows",
+                       "complex_gemm_mfma_wave, 32x16 a wave, 8 waves to 64x64, planar rows");
+    }
+    return by_layout("complex_gemm_mfma_wave, 32x32 a wave, 4 waves to 64x64, tiled operands",
+                     "complex_gemm_mfma_wave, 32x32 a wave, 4 waves to 64x64, interleaved rows",
+                     "complex_gemm_mfma_wave, 32x32 a wave, 4 waves to 64x64, planar rows");
+  }
   auto name = [&](const char *large, const char *middle, const char *small) {
     return shape == k256x128 ? large : shape == k128x128 ? middle : small;
   };

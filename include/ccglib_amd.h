@@ -96,7 +96,10 @@ CCGLIB_API const char *ccglib_version(void);
  *                    1: always 256 x 128 (32-bit input, which has no such
  *                    block: 128 x 128); 2: always 128 x 128; 3: 192 x 256
  *                    wherever that kernel applies, else as 0; 4: always
- *                    64 x 64. The 192 x 256 block also serves 16-bit
+ *                    64 x 64; 5, 6, 7: waves of 32 x 32, 32 x 16, 16 x 16 that
+ *                    share nothing, which 0 takes where 64 x 64 blocks leave
+ *                    units idle too (8- and 1-bit input: 32 x 32 only; where no
+ *                    such kernel applies, 32-bit input among that, as 4). The 192 x 256 block also serves 16-bit
  *                    interleaved rows read in place (the pipeline) when K is a
  *                    multiple of 32.
  *   EXPECT_UNALIGNED 0 (default): a basic-variant GEMM that meets operands that
