@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(HERE, "libccglib_amd.so")
 # (gemm_mfma.hip is compiled in parts, one per input type, so that they build in parallel)
 SOURCES = ["capi.hip", "gemm_mfma_f16.hip", "gemm_mfma_bf16.hip", "gemm_mfma_f32.hip",
            "gemm_mfma_fp8.hip", "gemm_mfma_int1.hip", "gemm_mfma_dispatch.hip", "gemm_int1.hip",
-           "transpose.hip", "packing.hip"]
+           "transpose.hip", "packing.hip", "host_copy.hip"]
 HEADERS = [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_device.h"),
            os.path.join(CSRC, "gemm_mfma.hip"), os.path.join(CSRC, "gemm_mfma_wide.h"),
            os.path.join(CSRC, "gemm_mfma_wave.h"),

@@ -1179,6 +1179,29 @@ int make_host_lanes(ccglib_pipeline *p, size_t chunk, size_t bytes_a, size_t byt
   return CCGLIB_OK;
 }
 
+// Where the GPU finds `bytes` bytes of host memory from `host` on, if all of them are one page-locked allocation
+// of this GPU's; null for any other memory.
+void *device_view(const void *host, size_t bytes, int device) {
+  hipPointerAttribute_t at = {};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (!bytes || hipPointerGetAttributes(&at, host) != hipSuccess || at.type != hipMemoryTypeHost ||
+      at.device != device || !at.devicePointer ||
+      hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)at.devicePointer) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const uintptr_t first = (uintptr_t)at.devicePointer, start = (uintptr_t)base;
+  return first >= start && first - start <= size && bytes <= size - (first - start) ? at.devicePointer : nullptr;
+}
+
+// Host Run in one piece on page-locked memory: up to these sizes one kernel fetches what goes in, and the GEMM stores
+// C where the caller wants it. A copy by the DMA engines costs about 10 us whatever its size, but moves 56 GB/s
+// where the kernel reads 50 and the GEMM writes 48 to 52: the call with copies and like this, in us, 32 KiB in
+// and out 29.0, 20.3; 0.5 MiB in, 0.14 out 51, 31; 1 MiB in, 4 out 132, 113; 3.4 MiB in, 4 out 181, 166;
+// 1.3 MiB in, 32 out 657, 684 (16 out 350, 345).
+constexpr size_t kHostCopyBytes = (size_t)4 << 20, kHostStoreBytes = (size_t)8 << 20;
+
 }  // namespace
 
 extern "C" {
@@ -1252,17 +1275,36 @@ int ccglib_pipeline_run_host(ccglib_pipeline_t p, const void *h_a, const void *h
     return fail_hip(e, "pipeline host staging");
   }
   char *d_a = static_cast<char *>(buffers), *d_b = d_a + at_b, *d_c = d_a + at_c;
-  if (bytes_a) e = hipMemcpyAsync(d_a, h_a, bytes_a, hipMemcpyHostToDevice, p->stream);
-  if (e == hipSuccess && bytes_b) e = hipMemcpyAsync(d_b, h_b, bytes_b, hipMemcpyHostToDevice, p->stream);
   // (src/pipeline/Pipeline.cpp:168-172 clears C where it is not copied in; every kernel writes
   // all of it then)
-  if (e == hipSuccess && p->need_copyin_c) {
-    e = hipMemcpyAsync(d_c, h_c, bytes_c, hipMemcpyHostToDevice, p->stream);
+  HostCopies in = {};
+  in.src[0] = device_view(h_a, bytes_a, p->device);
+  in.src[1] = device_view(h_b, bytes_b, p->device);
+  in.src[2] = p->need_copyin_c ? device_view(h_c, bytes_c, p->device) : nullptr;
+  in.dst[0] = d_a;
+  in.dst[1] = d_b;
+  in.dst[2] = d_c;
+  in.bytes[0] = bytes_a;
+  in.bytes[1] = bytes_b;
+  in.bytes[2] = p->need_copyin_c ? bytes_c : 0;
+  const size_t bytes_in = in.bytes[0] + in.bytes[1] + in.bytes[2];
+  if (bytes_in <= kHostCopyBytes && (!bytes_a || in.src[0]) && (!bytes_b || in.src[1]) &&
+      (!p->need_copyin_c || in.src[2])) {
+    e = launch_copy_from_host(in, p->stream);
+  } else {
+    if (bytes_a) e = hipMemcpyAsync(d_a, h_a, bytes_a, hipMemcpyHostToDevice, p->stream);
+    if (e == hipSuccess && bytes_b) e = hipMemcpyAsync(d_b, h_b, bytes_b, hipMemcpyHostToDevice, p->stream);
+    if (e == hipSuccess && p->need_copyin_c) {
+      e = hipMemcpyAsync(d_c, h_c, bytes_c, hipMemcpyHostToDevice, p->stream);
+    }
   }
   if (e != hipSuccess) rc = fail_hip(e, "pipeline host staging");
-  if (rc == CCGLIB_OK) rc = ccglib_pipeline_run(p, d_a, d_b, d_c);
+  const bool whole_elements = (uintptr_t)h_c % ((size_t)bits_of(p->type_out) / 8) == 0;
+  void *c_there = nullptr;
+  if (!p->need_copyin_c && whole_elements && bytes_c <= kHostStoreBytes) c_there = device_view(h_c, bytes_c, p->device);
+  if (rc == CCGLIB_OK) rc = ccglib_pipeline_run(p, d_a, d_b, c_there ? c_there : d_c);
   if (rc == CCGLIB_OK) {
-    e = hipMemcpyAsync(h_c, d_c, bytes_c, hipMemcpyDeviceToHost, p->stream);
+    if (!c_there) e = hipMemcpyAsync(h_c, d_c, bytes_c, hipMemcpyDeviceToHost, p->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
     if (e != hipSuccess) rc = fail_hip(e, "pipeline copy back");
   } else {

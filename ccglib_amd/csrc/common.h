@@ -123,5 +123,15 @@ hipError_t launch_pack_bits(const unsigned char *in, unsigned *out, size_t n,
 hipError_t launch_unpack_bits(const unsigned *in, unsigned char *out, size_t n,
                               hipStream_t stream);
 
+// Copies of page-locked host memory (as the device sees it) into device memory, up to three in
+// one launch; dst 16-byte aligned, `first` is the launcher's.
+struct HostCopies {
+  const void *src[3];
+  void *dst[3];
+  size_t bytes[3];
+  unsigned first[3];
+};
+hipError_t launch_copy_from_host(HostCopies c, hipStream_t stream);
+
 }  // namespace ccglib_amd
 #endif  // CCGLIB_AMD_COMMON_H_
