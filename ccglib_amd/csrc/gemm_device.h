@@ -108,6 +108,8 @@ struct KernelArgs {
   size_t x_batch_bytes, y_batch_bytes;
   float alpha_re, alpha_im, beta_re, beta_im;
   int have_alpha, have_beta, c_interleaved;
+  // planar C of 32 bits in rows of whole cache lines, more than the caches hold: stored past them
+  int c_past_caches;
   // 1-bit samples on the MFMA: what the zero bits past K add to every imaginary sum
   unsigned im_excess;
 };
@@ -208,6 +210,10 @@ __device__ __forceinline__ TileCoord tile_coord(const KernelArgs &args, unsigned
   return tc;
 }
 
+// From how many bytes on a planar C of 32-bit elements in whole lines is stored past the caches, by the epilogues that
+// write whole lines at once.
+constexpr size_t kPastCachesBytes = (size_t)128 << 20;
+
 // Fills the kernel argument block from the launch parameters for a BX x BY
 // block tile.
 inline KernelArgs make_kernel_args(const GemmParams &p, int bx, int by) {
@@ -247,6 +253,8 @@ inline KernelArgs make_kernel_args(const GemmParams &p, int bx, int by) {
   a.have_alpha = p.have_alpha;
   a.have_beta = p.have_beta;
   a.c_interleaved = p.c_interleaved;
+  a.c_past_caches = bits_of(p.type_out) == 32 && !p.c_interleaved && p.nx % 32 == 0 && (uintptr_t)p.c % 128 == 0 &&
+                    (size_t)8 * p.batch * p.nx * p.ny >= kPastCachesBytes;
   a.im_excess = (p.type_in == kInt1) ? 2u * (p.k_tiles * (unsigned)k_per_tile(kInt1) - p.k) : 0u;
   return a;
 }
