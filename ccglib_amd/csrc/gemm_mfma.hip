@@ -2819,14 +2819,16 @@ hipError_t launch_dtl(const GemmParams &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int DT, int TOUT, int LOADER, int TX, int TY>
+template <int DT, int TOUT, int LOADER, int TX, int TY, int SPLIT = 1>
 hipError_t launch_wave(const GemmParams &p, hipStream_t stream) {
   const KernelArgs a = make_kernel_args(p, 16 * TX, 16 * TY);
   const size_t total = (size_t)a.blocks_x * a.blocks_y * p.batch;
   if (total == 0) return hipSuccess;
   if (hipError_t e = check_grid(total)) return e;
-  hipLaunchKernelGGL((complex_gemm_mfma_wave<DT, TOUT, LOADER, TX, TY>), dim3((unsigned)total), dim3(64), kWaveLdsBytes,
-                     stream, a);
+  auto kernel = complex_gemm_mfma_wave<DT, TOUT, LOADER, TX, TY, SPLIT>;
+  static std::atomic<bool> lds_allowed[kMaxDevices];
+  if (hipError_t e = allow_lds(kernel, SPLIT * kWaveLdsBytes, lds_allowed)) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(64 * SPLIT), SPLIT * kWaveLdsBytes, stream, a);
   return hipGetLastError();
 }
 
@@ -3088,6 +3090,19 @@ hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream
     if constexpr (DT == kFloat16 || DT == kBfloat16) {
       if (shape == kWaves16x16) return launch_wave<DT, TOUT, L, 1, 1>(p, stream);
       if (shape == kWaves32x16) return launch_wave<DT, TOUT, L, 2, 1>(p, stream);
+    }
+    if constexpr (DT == kInt1) {
+      // The four SIMDs of a unit share the K tiles of one tile of C, a unit's tiles one after the other, or every wave has
+      // its own, all at once: 32x32 elements a wave, us on 64 x 64 blocks, single waves, four together:
+      //   512x512 (a tile a unit)  K=2048 7.8, 6.6, 4.9;  K=32768 59.7, 50.9, 19.2
+      //   B=20 128x128 (some two)  K=2048 8.0, 6.8, 8.0;  K=8192 18.4, 15.7, 13.9;  K=32768 60.3, 51.1, 33.7
+      //   1024x1024 (four)         K=32768 61.5, 57.3, 65.1
+      // which these times of the two (in us, as in wave_choice) follow.
+      const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 32) * ceil_div(p.ny, 32);
+      const size_t units = (size_t)compute_units();
+      const double together = (double)ceil_div(tiles, units) * (3.3 + 0.735 * (double)ceil_div(p.k_tiles, 4));
+      const double alone = 3.2 + p.k_tiles * std::max(0.735, 0.282 * (double)tiles / (double)units);
+      if (p.k_tiles > 1 && tiles <= 3 * units && together < alone) return launch_wave<DT, TOUT, L, 2, 2, 4>(p, stream);
     }
     return launch_wave<DT, TOUT, L, 2, 2>(p, stream);
   };

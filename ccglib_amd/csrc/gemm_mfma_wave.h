@@ -125,8 +125,11 @@ constexpr int kWaveLdsBytes = 32 * 1024, kWavesPerUnit = 160 * 1024 / kWaveLdsBy
 constexpr int wave_ring(int tx, int ty) { return kWaveLdsBytes / (2048 * (tx + ty)); }   // K tiles of the ring
 
 // (LOADER: tiled, or rows in place of any length from 16 bytes on, at any address)
-template <int DT, int TOUT, int LOADER, int TX, int TY>
-__global__ __launch_bounds__(64, 1) void complex_gemm_mfma_wave(const KernelArgs args) {
+// SPLIT > 1 (1-bit input, whose sums are exact in any order): a block is SPLIT waves, which share the K tiles of one tile of
+// C out among them, one after the other, and add their sums up in LDS.
+template <int DT, int TOUT, int LOADER, int TX, int TY, int SPLIT = 1>
+__global__ __launch_bounds__(64 * SPLIT, 1) void complex_gemm_mfma_wave(const KernelArgs args) {
+  static_assert(SPLIT == 1 || DT == kInt1, "sums in another order: whole numbers only");
   static_assert(LOADER == kLoadTiled || LOADER == kLoadPlanarRagged || LOADER == kLoadInterleavedRagged, "");
   constexpr bool IL = LOADER == kLoadInterleavedRagged, TILED = LOADER == kLoadTiled;
   constexpr bool BITS16 = DT == kFloat16 || DT == kBfloat16;
@@ -141,8 +144,10 @@ __global__ __launch_bounds__(64, 1) void complex_gemm_mfma_wave(const KernelArgs
   constexpr int XC = X_BYTES / 1024, COPIES = SLOT_BYTES / 1024;   // copy instructions of X, of a K tile
   static_assert(SLOT_BYTES * RING <= kWaveLdsBytes && COPIES * (RING - 1) < 64, "ring, vmcnt range");
 
-  extern __shared__ __attribute__((aligned(1024))) char lds[];
-  const int lane = threadIdx.x;
+  extern __shared__ __attribute__((aligned(1024))) char block_lds[];
+  const int lane = threadIdx.x & 63;
+  const unsigned part = SPLIT == 1 ? 0 : (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  char *lds = block_lds + part * kWaveLdsBytes;
   // (the waves of a 64 x 64 region of C have consecutive numbers, so that they share an L2)
   const TileCoord tc = tile_coord<64 / WY>(args, blockIdx.x);
   const unsigned x0 = tc.block_x * WX, y0 = tc.block_y * WY;
@@ -151,8 +156,10 @@ __global__ __launch_bounds__(64, 1) void complex_gemm_mfma_wave(const KernelArgs
   const unsigned row_bytes = IL ? 2 * args.k_bytes : args.k_bytes;
   const unsigned row_stride = TILED ? kTileRowBytes : (IL ? 2 : 1) * args.row_stride_bytes;
   const unsigned k_step = TILED ? kTileBytes : RB;
-  const unsigned k_tiles = TILED ? args.k_tiles : (row_bytes + RB - 1) / RB;
-  const bool partial = !TILED && row_bytes % RB != 0;
+  const unsigned all_k_tiles = TILED ? args.k_tiles : (row_bytes + RB - 1) / RB;
+  // this wave's K tiles: part, part + SPLIT, ...
+  const unsigned k_tiles = SPLIT == 1 ? all_k_tiles : part < all_k_tiles ? (all_k_tiles - part + SPLIT - 1) / SPLIT : 0;
+  const bool partial = !TILED && row_bytes % RB != 0 && (SPLIT == 1 || (all_k_tiles - 1) % SPLIT == part);
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)lds;
   const int r = lane / CPR;
   // chunk that this lane fetches of row RPB * rb + r (see the swizzles of complex_gemm_mfma_dtl)
@@ -184,17 +191,17 @@ __global__ __launch_bounds__(64, 1) void complex_gemm_mfma_wave(const KernelArgs
       const unsigned row = (want < most ? want : most) * row_stride;
       at[n] = row + chunk_of(rb) * 16;
       if constexpr (!TILED) {
-        const unsigned start = (k_tiles - 1) * RB + chunk_of(rb) * 16;
+        const unsigned start = (all_k_tiles - 1) * RB + chunk_of(rb) * 16;
         last[n] = row + (start < row_bytes - 16 ? start : row_bytes - 16);
       }
     }
   }
-  // K tile kt into slot `slot`, instruction n of COPIES. The chunks of a row's last, partial K tile (`end`)
+  // The wave's K tile kt into slot `slot`, instruction n of COPIES. The chunks of a row's last, partial K tile (`end`)
   // come as the 16 bytes that end with them or with the row, whichever comes first (nothing outside
   // the row is read).
   auto copy_one = [&](unsigned kt, unsigned slot, int n, auto end) {
     const int side = n >= XC, q = side ? n - XC : n, plane = q / ((side ? WY : WX) / RPB);
-    load_1k_to_lds(decltype(end)::value ? base[side][plane] : base[side][plane] + (size_t)kt * k_step,
+    load_1k_to_lds(decltype(end)::value ? base[side][plane] : base[side][plane] + (size_t)(kt * SPLIT + part) * k_step,
                    decltype(end)::value ? last[n] : at[n], lds_base + slot * SLOT_BYTES + n * 1024);
   };
   auto copy = [&](unsigned kt, unsigned slot, auto end) {
@@ -227,7 +234,7 @@ __global__ __launch_bounds__(64, 1) void complex_gemm_mfma_wave(const KernelArgs
   auto settle = [&](Tile &t) {
     typedef unsigned long long ulong2_t __attribute__((ext_vector_type(2)));
     auto shifted = [&](int4_t &v, int n) {
-      const unsigned start = (k_tiles - 1) * RB + frag_chunk(n / 2, n % 2) * 16;
+      const unsigned start = (all_k_tiles - 1) * RB + frag_chunk(n / 2, n % 2) * 16;
       const unsigned shift = start < row_bytes - 16 ? 0 : (start - (row_bytes - 16)) * 8;
       const ulong2_t u = __builtin_bit_cast(ulong2_t, v);
       ulong2_t o = u;
@@ -324,6 +331,29 @@ __global__ __launch_bounds__(64, 1) void complex_gemm_mfma_wave(const KernelArgs
         mma_wave_tile<DT, IL>(now, acc_re, acc_im, [](int) {});
       }
     });
+  }
+  if constexpr (SPLIT > 1) {
+    // The first wave's registers take the sums of the others, through the LDS of their rings (whose reads
+    // have landed: their last products are in the sums).
+    float *sums = reinterpret_cast<float *>(lds);
+    if (part > 0) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        sums[e * 64 + lane] = acc_re[0][0][e];
+        sums[(16 + e) * 64 + lane] = acc_im[0][0][e];
+      }
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int s = 1; s < SPLIT; ++s) {
+      const float *other = reinterpret_cast<const float *>(block_lds + s * kWaveLdsBytes);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        acc_re[0][0][e] += other[e * 64 + lane];
+        acc_im[0][0][e] += other[(16 + e) * 64 + lane];
+      }
+    }
   }
   if constexpr (TOUT == kInt32) {
     store_wave_tile_int32<NX, NY, MS>(args, tc.b, x0, y0, lane, acc_re, acc_im);
