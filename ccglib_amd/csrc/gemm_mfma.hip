@@ -2502,6 +2502,13 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   for (int i = 0; i < 4; ++i) xa[i] = lds_base + x_slot_off(0) + xo[i];
   const unsigned iters = k_tiles;
   for (unsigned vt = blockIdx.x; vt < total; vt += gridDim.x) {
+    const TileCoord tc = tile_coord(args, vt);
+    const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
+    // A wave whose part of the block lies beyond C leaves the matrix cores to the wave next to it on the SIMD (a block of
+    // 128 rows of which 64 exist has one of each two): B=16 300x3001x577 fp16 pairs 113.8 -> 108.6 us, B=247
+    // 456x299x1552 595 -> 567. (8- and 1-bit input: B=16 4096x4096x8192, where no wave is idle, 0.8 % slower.)
+    constexpr bool kMaySkip = BX * BY > 64 * 64 && DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1;
+    const bool inside = !kMaySkip || (x_wave < args.nx && y_wave < args.ny);
     typename AccType<MS>::type acc_re[TY][TX], acc_im[TY][TX];
     SplitState<DT == kFloat32 ? TX : 1> split;   // (32-bit input)
     SmallTile small;                             // (64 x 64 blocks)
@@ -2526,7 +2533,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     }
     // One K iteration; `first` says at compile time that it is a C tile's first one (kCarries:
     // kernels that multiply a K tile while they read the next one).
-    auto iteration = [&](unsigned it, auto first) __attribute__((always_inline)) {
+    // (math: whether the wave has elements of C to compute)
+    auto iteration = [&](unsigned it, auto first, auto math) __attribute__((always_inline)) {
       advance();
       // After the first C tile, the K tiles of the first YLEAD iterations were
       // already waited for before the previous epilogue (see below), so these
@@ -2570,7 +2578,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
           for (int i = 0; i < 4; ++i) xa[i] = lds_base + x_slot_off(x_next) + xo[i];
           ya = lds_base + y_slot_off(y_next) + (y_frag_off - X_BYTES);
         };
-        if (it == 0) {
+        if constexpr (!decltype(math)::value) {
+          refill_slots();
+          next_addresses();
+        } else if (it == 0) {
           mma_step_ordered<DT, BX, BY, XT, true>(xa, ya, acc_re, acc_im, refill_slots,
                                                  next_addresses);
         } else {
@@ -2579,7 +2590,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         }
       } else {
         const char *slot_ptr = lds + x_slot_off(x_slot);
-        if constexpr (SMALL) {
+        if constexpr (!decltype(math)::value) {
+          refill_slots();
+        } else if constexpr (SMALL) {
           SmallTile next;
           read_small_tile(slot_ptr, small_x, small_y, next);
           if constexpr (decltype(first)::value) {
@@ -2621,8 +2634,15 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     };
     unsigned it = 0;
     constexpr bool kCarries = SMALL || DT == kFloat32;
-    if constexpr (kCarries) iteration(it++, std::true_type{});
-    for (; it < iters; ++it) iteration(it, std::false_type{});
+    const std::true_type yes{};
+    const std::false_type no{};
+    if constexpr (kCarries) iteration(it++, yes, yes);
+    if (inside) {
+      for (; it < iters; ++it) iteration(it, no, yes);
+    } else {
+#pragma unroll 1
+      for (; it < iters; ++it) iteration(it, no, no);
+    }
     if constexpr (SMALL) mma_small_tile<DT, IL>(small, acc_re, acc_im, [] {});
     // The stores below are not waited for here: they drain while the next C
     // tile is being computed. The counter cannot tell loads from stores, so
@@ -2632,8 +2652,6 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     // under way; the next tile's first barrier, behind which the slot is refilled, waits for them,
     // and no epilogue of theirs uses LDS.)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const TileCoord tc = tile_coord(args, vt);
-    const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     bool redo = false;   // (32-bit input) this wave's tile is computed again
     if constexpr (DT == kFloat32) {
       redo = !mma_split_last(split, acc_re, acc_im);
