@@ -1226,12 +1226,43 @@ __device__ __forceinline__ void store_c(void *at, const Value &v, bool past_cach
   }
 }
 
+// The whole pieces of C of a wave tile, read before the sums are there (store_wave_tile): four real and four imaginary
+// elements of planar C, eight as they lie of interleaved C.
+struct NoPieces {};
+template <int TOUT, int TX, int TY, int MS> struct CPieces {
+  static constexpr int kPerRow = MS == 32 ? TX * 4 : TX;
+  typename OutType<TOUT>::type v[TY][kPerRow][8];
+
+  __device__ __forceinline__ void load(const KernelArgs &args, unsigned b, unsigned x_wave, unsigned y_wave, int lane) {
+    using Tout = typename OutType<TOUT>::type;
+    typedef Tout Vec4 __attribute__((ext_vector_type(4)));
+    typedef Vec4 Piece __attribute__((aligned(sizeof(Tout))));
+    const unsigned nx = args.nx, ny = args.ny;
+    const Tout *cbase = reinterpret_cast<const Tout *>(args.c) + (size_t)b * 2 * nx * ny;
+#pragma unroll
+    for (int j = 0; j < TY; ++j) {
+#pragma unroll
+      for (int i = 0; i < kPerRow; ++i) {
+        const unsigned y = y_wave + piece_y<MS>(j, i, lane), x = x_wave + piece_x<MS>(i, lane);
+        if (y >= ny || x + 4 > nx) continue;
+        const Tout *first = args.c_interleaved ? cbase + ((size_t)y * nx + x) * 2 : cbase + (size_t)y * nx + x;
+        const Tout *second = args.c_interleaved ? first + 4 : first + (size_t)nx * ny;
+        const Piece p = *reinterpret_cast<const Piece *>(first), q = *reinterpret_cast<const Piece *>(second);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][i][e] = p[e], v[j][i][4 + e] = q[e];
+      }
+    }
+  }
+};
+
 // Epilogue of one wave: alpha * acc + beta * C, conversion, bounds-checked
 // store, piece by piece (four consecutive elements of the contiguous C axis).
-template <int TOUT, int TX, int TY, int MS = 16, int TILE0 = 0, typename Acc>
+// pieces: the whole pieces of C if they have been read already (CPieces).
+template <int TOUT, int TX, int TY, int MS = 16, int TILE0 = 0, typename Acc, typename Pieces = NoPieces>
 __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned b, unsigned x_wave,
                                                 unsigned y_wave, int lane, const Acc &acc_re,
-                                                const Acc &acc_im) {
+                                                const Acc &acc_im, const Pieces &pieces = {}) {
+  constexpr bool READ = !std::is_same<Pieces, NoPieces>::value;
   // TX, TY count MFMA tiles; pieces per tile row: 1 (MS 16) or 4 (MS 32)
   constexpr int NPX = MS == 32 ? TX * 4 : TX;
   using Tout = typename OutType<TOUT>::type;
@@ -1264,7 +1295,13 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
         if (have_beta) {
           // (whole pieces: C comes in with one wide load per plane)
           Tout cr4[4], ci4[4];
-          if (full) {
+          if constexpr (READ) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              cr4[e] = pieces.v[j][i][e];
+              ci4[e] = pieces.v[j][i][4 + e];
+            }
+          } else if (full) {
             typedef Tout Vec __attribute__((ext_vector_type(4)));
             typedef Vec Piece __attribute__((aligned(sizeof(Tout))));
             const Piece vr = *reinterpret_cast<const Piece *>(pr), vi = *reinterpret_cast<const Piece *>(pi);
@@ -1307,7 +1344,10 @@ __device__ __forceinline__ void store_wave_tile(const KernelArgs &args, unsigned
         Tout *p = cbase + ((size_t)y * nx + x) * 2;
         if (have_beta) {
           Tout c8[8];
-          if (full) {
+          if constexpr (READ) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c8[e] = pieces.v[j][i][e];
+          } else if (full) {
             typedef Tout Vec __attribute__((ext_vector_type(8)));
             typedef Vec Piece __attribute__((aligned(sizeof(Tout))));
             const Piece v = *reinterpret_cast<const Piece *>(p);
