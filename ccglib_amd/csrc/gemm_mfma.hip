@@ -2975,24 +2975,20 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 //   too few tiles for the larger blocks, 16 bits 256^3:  14.4, 12.2, 6.5;  B=256 96x96x1024:  87, 57, 63;
 //     32 bits B=2 1000^3:  (none), 186, 129;  8 bits 1024^3:  24.3, 21.8, 10.8;
 //     1 bit 64x64x65536:  529, 308, 115
-//   every unit busy, 16 bits on tiles, 4096x4096x512:  73, 92, 106
-//     on planar rows, of which a copy fetches half cache lines, B=157 192x604x3680:  762, 908, 1057
+//   every unit busy, 16 bits on planar rows, B=64 512x4096x576:  613, 655, 962; B=300 512x512x128:  163, 158, 259
 //     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  (none), 453, 523
 //     8 bits on tiles, 4096x4096x512:  52, 51, 69
 //     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
 //       308, 317, 339
-// Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles of 8- and 1-bit input, and
+// Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles (of 16-bit input: from more tiles than units on), and
 // a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
 // With beta the epilogue reads C first, which costs the larger tiles more (8 bits on planar
-// rows, B=11 456x1542x192: 97, 84, 47). Interleaved fp32 C of 16-bit tiles, which only the 256 x 128
-// block regroups through LDS, moves no line: where a smaller block is chosen the larger one is
-// slower by 0.95 to several times, 1.37 (128 x 128) and 2.9 (64 x 64) at the median.
+// rows, B=11 456x1542x192: 97, 84, 47).
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
 // 30000 problems of random sizes, 40 % of them on operands that no cache held
 // (python -m ccglib_amd.tuning.block_choice times such problems); those of 8-bit tiles
-// and 16-bit pairs to 1900, of 32-bit input to 1200 further ones, timed since those kernels last changed. On 8000
-// others, ragged rows among them, the choice is on average 0.1 % behind the fastest of the three shapes, and more
-// than 8 % behind in 1.2 % of the problems.
+// to 1900, of 32-bit input to 1200, of all 16-bit layouts to 2100 further ones, timed since those kernels last changed, on
+// which (16 bits) the choice is 0.9 % behind the fastest of the three shapes on average and more than 8 % in 3.7 %.
 enum BlockShape { k256x128, k128x128, k64x64 };
 struct BlockChoice {
   BlockShape shape;
@@ -3003,24 +2999,25 @@ struct BlockCosts {
   double tile_128, tile_64;   // what a tile costs besides its K loop, in pieces of K
   double lone_128, lone_64;   // what a tile without a neighbour costs more, of a tile
   double beta_256, beta_128, beta_64;   // added to the tile's cost with beta
+  double cost_few, tile_few;  // (16 bits) 128 x 128 blocks with a unit each, see launch_128x128
 };
 inline BlockCosts block_costs(const GemmParams &p) {
-  if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0};
+  if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   // (32-bit input has no 256 x 128 block: relative to 128 x 128)
-  if (p.type_in == kFloat32) return {1.0, 1.24, 6.0, 5.0, 0.0, 0.0, 0.0, 4.0, 2.0};
+  if (p.type_in == kFloat32) return {1.0, 1.24, 6.0, 5.0, 0.0, 0.0, 0.0, 4.0, 2.0, 0.0, 0.0};
   const bool planar = p.variant == kBasic && !p.input_interleaved;
   if (bits_of(p.type_in) == 8) {
-    if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0};
-    if (planar) return {1.30, 2.54, 7.6, 7.9, 0.3, 0.1, 13.0, 10.0, 1.0};
-    return {1.05, 1.61, 9.2, 9.4, 0.3, 0.11, 13.0, 10.0, 1.0};
+    if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0, 0.0, 0.0};
+    if (planar) return {1.30, 2.54, 7.6, 7.9, 0.3, 0.1, 13.0, 10.0, 1.0, 0.0, 0.0};
+    return {1.05, 1.61, 9.2, 9.4, 0.3, 0.11, 13.0, 10.0, 1.0, 0.0, 0.0};
   }
-  if (p.input_interleaved) return {1.19, 1.80, 11.7, 7.6, 0.0, 0.35, 12.0, 8.0, 6.0};
-  if (planar) return {1.24, 2.58, 12.6, 6.8, 0.0, 0.25, 12.0, 8.0, 6.0};
-  return {1.30, 1.71, 11.0, 10.1, 0.0, 0.25, 12.0, 8.0, 6.0};
+  if (p.input_interleaved) return {1.10, 2.05, 8.74, 11.27, 0.29, 0.63, 8.56, 7.10, 5.17, 1.38, 10.0};
+  if (planar) return {1.14, 2.10, 7.99, 9.25, 0.28, 0.45, 13.57, 12.23, 2.60, 1.24, 8.29};
+  return {1.08, 1.69, 8.77, 9.34, 0.25, 0.63, 10.33, 9.22, 3.35, 0.87, 10.95};
 }
 inline BlockChoice block_choice(const GemmParams &p) {
   const size_t units = (size_t)compute_units();
-  const BlockCosts costs = block_costs(p);
+  BlockCosts costs = block_costs(p);
   // (pieces of a plane's row: an interleaved row holds both planes)
   const double pieces = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
   const double large = pieces + 10.0 + (p.have_beta ? costs.beta_256 : 0.0);
@@ -3032,7 +3029,16 @@ inline BlockChoice block_choice(const GemmParams &p) {
   };
   const bool no_256 = p.type_in == kFloat32;
   const double t256 = no_256 ? HUGE_VAL : time(256, 128, 1.0, 10.0, 0.0, costs.beta_256);
-  const double t128 = time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
+  const bool few = bits_of(p.type_in) == 16 &&
+                   (size_t)p.batch * ceil_div(p.nx, 128) * ceil_div(p.ny, 128) <= units;
+  // (a large C whose rows share cache lines, which the narrower blocks write in more parts: B=173 1728x1656x64 fp16
+  // 1030 us on 256 x 128 blocks, 1357 on these)
+  const size_t c_bytes = (size_t)2 * p.batch * p.nx * p.ny * bits_of(p.type_out) / 8;
+  const bool shared_lines = bits_of(p.type_in) == 16 && c_bytes >= ((size_t)256 << 20) &&
+                            (size_t)p.nx * (p.c_interleaved ? 2 : 1) * bits_of(p.type_out) / 8 % 128 != 0;
+  if (shared_lines) costs.tile_128 += 4.0;
+  const double t128 = few ? time(128, 128, costs.cost_few, costs.tile_few, 0.0, costs.beta_128)
+                          : time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
   const double t64 = time(64, 64, costs.cost_64, costs.tile_64, costs.lone_64, costs.beta_64);
   if (p.block_tile == 1 && !no_256) return {k256x128, t256};
   if (p.block_tile == 1 || p.block_tile == 2) return {k128x128, t128};
@@ -3075,8 +3081,8 @@ inline bool wide_tiles_pay(const GemmParams &p) {
 // 64 x 64 (450 of 1-bit input), 60 % of them on operands that no cache held, a fifth on ragged rows.
 // There the choice is 2 to 3 % (16 bits) and 1 % (8 and 1 bits) behind the fastest shape on average, and in front of
 // 64 x 64 blocks by 1.41 times (16 bits), 1.20 (8 bits), 1.15 (1 bit); it is more than 5 % slower than those
-// in 22 of 1644. More waves than fit the units at once are left to the blocks, which walk their tiles
-// without gaps (93 batches of 32x448x1584: 58 us, 85 with 1302 waves of 32 x 32).
+// in 22 of 1644. More waves than there are SIMDs are left to the blocks: the fifth wave of a unit has to share one
+// (B=213 32x192x3184 on planar rows, 1278 waves: 179 us on blocks, 261 on waves; B=93 32x448x1584 58, 85).
 enum WaveShape { kNoWaves, kWaves32x32, kWaves32x16, kWaves16x16 };
 struct WaveCosts {
   double fixed, alone, crowded, tile;
@@ -3171,6 +3177,27 @@ hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream
   return launch(std::integral_constant<int, kLoadPlanarRagged>{});
 }
 
+// 128 x 128 blocks. 16-bit input: while every block has a unit to itself, 8 waves of 64 x 32 and a ring of four slots, which
+// keeps more on its way (B=256 96x96x1024 pairs 48 us, 52 with the other); beyond, 4 waves of 64 x 64 and two slots, of which two
+// share a unit: one stores C or waits while the other multiplies, the fragments are read once for twice as many
+// products, and C is stored in whole row segments. In us, planar rows unless said, 8 and 4 waves (256 x 128 blocks):
+// B=67 384x3136x328 445, 329 (337); B=300 512x512x128 217, 158 (163); B=12 640x1328x512 57, 50 (54); B=100
+// 320x320x256 pairs 45, 40 (50); 2x3000x1500x256 37.5, 30.4 (35.8); B=64 512x4096x576 822, 655 (613).
+template <int DT, int TOUT, int LOADER>
+hipError_t launch_128x128(const GemmParams &p, hipStream_t stream) {
+  if constexpr (DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1) {
+    const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 128) * ceil_div(p.ny, 128);
+    if (tiles <= (size_t)compute_units()) return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, LOADER, 16>(p, stream);
+    if constexpr (LOADER != kLoadInterleavedVec && LOADER != kLoadInterleavedRagged) {
+      // (exchanged roles for planar C; pairs are regrouped through LDS)
+      if (!p.c_interleaved) return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16, true>(p, stream);
+    }
+    return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16>(p, stream);
+  } else {
+    return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 32>(p, stream);
+  }
+}
+
 template <int DT, int TOUT>
 hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   if constexpr (DT != kFloat32) {
@@ -3214,25 +3241,18 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
     if (ragged && 2 * k_bytes < 16) return hipErrorInvalidValue;
     if (ragged) {
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedRagged, MS>(p, stream);
-      if (shape == k128x128) {
-        return launch_dtl<DT, TOUT, 128, 128, 64, BITS16 ? 32 : 64, BITS16 ? 4 : 2, 2, kLoadInterleavedRagged,
-                          MS>(p, stream);
-      }
+      if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadInterleavedRagged>(p, stream);
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedRagged, MS>(p, stream);
     } else if constexpr (BITS16) {
       if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT, true>(p, stream);
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec>(p, stream);
-      if (shape == k128x128) {
-        return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadInterleavedVec>(p, stream);
-      }
+      if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadInterleavedVec>(p, stream);
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec>(p, stream);
     } else {
       if (shape == k64x64) {
         return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 32>(p, stream);
       }
-      if (shape == k128x128) {
-        return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadInterleavedVec, 32>(p, stream);
-      }
+      if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadInterleavedVec>(p, stream);
       return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec, 32>(p, stream);
     }
   }
@@ -3262,9 +3282,8 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
                    : launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 16>(p, stream);
       }
       if (shape == k128x128) {
-        return p.variant == kOpt
-                   ? launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadTiled, 16>(p, stream)
-                   : launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, kLoadPlanarVec, 16>(p, stream);
+        return p.variant == kOpt ? launch_128x128<DT, TOUT, kLoadTiled>(p, stream)
+                                 : launch_128x128<DT, TOUT, kLoadPlanarVec>(p, stream);
       }
       return p.variant == kOpt
                  ? launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 16, true>(p, stream)
@@ -3280,9 +3299,8 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
                    : launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarVec, 32>(p, stream);
       }
       if (shape == k128x128) {
-        return p.variant == kOpt
-                   ? launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadTiled, 32>(p, stream)
-                   : launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, kLoadPlanarVec, 32>(p, stream);
+        return p.variant == kOpt ? launch_128x128<DT, TOUT, kLoadTiled>(p, stream)
+                                 : launch_128x128<DT, TOUT, kLoadPlanarVec>(p, stream);
       }
       return p.variant == kOpt
                  ? launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>(p, stream)
@@ -3291,10 +3309,7 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
   }
   else if (k_bytes >= 16) {
     if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarRagged, MS>(p, stream);
-    if (shape == k128x128) {
-      return launch_dtl<DT, TOUT, 128, 128, 64, BITS16 ? 32 : 64, BITS16 ? 4 : 2, 2, kLoadPlanarRagged,
-                        MS>(p, stream);
-    }
+    if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadPlanarRagged>(p, stream);
     return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarRagged, MS, BITS16>(p, stream);
   }
   // fp8 stages are twice as large (two K tiles per MFMA): one wave per SIMD

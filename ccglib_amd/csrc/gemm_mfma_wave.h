@@ -120,8 +120,8 @@ __device__ __forceinline__ void mma_wave_tile(const WaveTile<2, 2> &t, float16_t
 #undef CCGLIB_PIN
 
 // LDS of a wave: seven K tiles of 16 x 16 or three of 32 x 32 are on their way while one is
-// multiplied, and five waves fit a unit.
-constexpr int kWaveLdsBytes = 32 * 1024, kWavesPerUnit = 160 * 1024 / kWaveLdsBytes;
+// multiplied, and the waves of four SIMDs fit a unit.
+constexpr int kWaveLdsBytes = 32 * 1024, kWavesPerUnit = 4;
 constexpr int wave_ring(int tx, int ty) { return kWaveLdsBytes / (2048 * (tx + ty)); }   // K tiles of the ring
 
 // (LOADER: tiled, or rows in place of any length from 16 bytes on, at any address)
