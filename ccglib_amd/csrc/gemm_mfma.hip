@@ -3079,9 +3079,8 @@ inline bool wide_tiles_pay(const GemmParams &p) {
 // with a unit to itself, `crowded` with others next to it, `tile` what a tile costs besides. The constants are
 // fitted, for each type and operand layout, to the times of all shapes on 1600 problems of up to 1024 blocks of
 // 64 x 64 (450 of 1-bit input), 60 % of them on operands that no cache held, a fifth on ragged rows.
-// There the choice is 2 to 3 % (16 bits) and 1 % (8 and 1 bits) behind the fastest shape on average, and in front of
-// 64 x 64 blocks by 1.41 times (16 bits), 1.20 (8 bits), 1.15 (1 bit); it is more than 5 % slower than those
-// in 22 of 1644. More waves than there are SIMDs are left to the blocks: the fifth wave of a unit has to share one
+// There the choice by these times was 2 to 3 % (16 bits) and 1 % (8 bits) behind the fastest shape on average, and in front of
+// 64 x 64 blocks by 1.41 times (16 bits) and 1.20 (8 bits), 1-bit input, whose waves share K, by 1.5. More waves than there are SIMDs are left to the blocks: the fifth wave of a unit has to share one
 // (B=213 32x192x3184 on planar rows, 1278 waves: 179 us on blocks, 261 on waves; B=93 32x448x1584 58, 85).
 enum WaveShape { kNoWaves, kWaves32x32, kWaves32x16, kWaves16x16 };
 struct WaveCosts {
@@ -3128,11 +3127,26 @@ inline WaveShape wave_choice(const GemmParams &p) {
   const bool ragged = (p.variant != kOpt || p.input_interleaved) && p.type_in != kInt1 &&
                       (p.input_interleaved ? 2 : 1) * (size_t)p.k * bits_of(p.type_in) / 8 % 16 != 0;
   if (ragged && k_tiles > 64.0) return kNoWaves;
+  if (p.type_in == kInt1) {
+    // The four SIMDs of a unit share the K tiles of one tile of C, a unit's tiles one after the other: us on 64 x 64 blocks and
+    // like this, 512x512 (a tile a unit) K=2048 7.8, 4.9; K=32768 59.7, 19.2; B=20 128x128 (some units two) K=8192
+    // 18.4, 13.9; K=32768 60.3, 33.7; 768x1024 (three) K=8192 19.0, 20.2; K=32768 60.9, 49.4.
+    const double tiles = (double)p.batch * (double)ceil_div(p.nx, 32) * (double)ceil_div(p.ny, 32);
+    const double n64 = (double)p.batch * (double)ceil_div(p.nx, 64) * (double)ceil_div(p.ny, 64) / units;
+    const double rounds = std::ceil(tiles / units);
+    const double blocks = costs[0].fixed + k_tiles * std::max(costs[0].alone, costs[0].crowded * n64) + costs[0].tile * n64;
+    return rounds <= 3.0 && rounds * (3.3 + costs[1].alone * std::ceil(k_tiles / 4.0)) < blocks ? kWaves32x32 : kNoWaves;
+  }
   auto time = [&](int shape, unsigned x, unsigned y) {
     const WaveCosts &c = costs[shape];
     const double n = (double)p.batch * (double)ceil_div(p.nx, x) * (double)ceil_div(p.ny, y) / units;
     if (shape != 0 && n > kWavesPerUnit) return HUGE_VAL;
-    return c.fixed + k_tiles * std::max(c.alone, c.crowded * n) + c.tile * n;
+    // (more than one wave a unit: which SIMDs they get depends on what the kernel before left, and two on one are
+    // slower: B=2 640x512x2048 e4m3 on waves 9.9 us behind itself, 15.8 behind another kernel, 15.1 on blocks)
+    const double alone = shape != 0 && n > 1.0 ? 1.35 * c.alone : c.alone;
+    // (blocks only request C with beta behind the last product)
+    const double beta = shape == 0 && p.have_beta ? 1.5 : 0.0;
+    return c.fixed + beta + k_tiles * std::max(alone, c.crowded * n) + c.tile * n;
   };
   double best = time(0, 64, 64);
   WaveShape shape = kNoWaves;
@@ -3156,17 +3170,9 @@ hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream
       if (shape == kWaves32x16) return launch_wave<DT, TOUT, L, 2, 1>(p, stream);
     }
     if constexpr (DT == kInt1) {
-      // The four SIMDs of a unit share the K tiles of one tile of C, a unit's tiles one after the other, or every wave has
-      // its own, all at once: 32x32 elements a wave, us on 64 x 64 blocks, single waves, four together:
-      //   512x512 (a tile a unit)  K=2048 7.8, 6.6, 4.9;  K=32768 59.7, 50.9, 19.2
-      //   B=20 128x128 (some two)  K=2048 8.0, 6.8, 8.0;  K=8192 18.4, 15.7, 13.9;  K=32768 60.3, 51.1, 33.7
-      //   1024x1024 (four)         K=32768 61.5, 57.3, 65.1
-      // which these times of the two (in us, as in wave_choice) follow.
+      // (see wave_choice; a single K tile is not shared out)
       const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 32) * ceil_div(p.ny, 32);
-      const size_t units = (size_t)compute_units();
-      const double together = (double)ceil_div(tiles, units) * (3.3 + 0.735 * (double)ceil_div(p.k_tiles, 4));
-      const double alone = 3.2 + p.k_tiles * std::max(0.735, 0.282 * (double)tiles / (double)units);
-      if (p.k_tiles > 1 && tiles <= 3 * units && together < alone) return launch_wave<DT, TOUT, L, 2, 2, 4>(p, stream);
+      if (p.k_tiles > 1 && tiles <= 3 * (size_t)compute_units()) return launch_wave<DT, TOUT, L, 2, 2, 4>(p, stream);
     }
     return launch_wave<DT, TOUT, L, 2, 2>(p, stream);
   };

@@ -35,7 +35,7 @@ def test_against_the_oracle(block_tile, variant, tin, tout):
                                      (1, 40, 20, 16384), (5, 256, 250, 16256), (9, 250, 256, 2688)])
 def test_int1(variant, B, M, N, K):
     """One K tile; three to nine and 32 of them, which four waves share out unevenly, the last one partial; more tiles of C
-    (320) than units, two of them one after the other; so many (576) that every wave has its own."""
+    (320, 576) than units, two or three of them one after the other."""
     with cc.option(cc.Option.gemm_block_tile, 5):
         int1_case(B, M, N, K, variant, seed=1)
         int1_case(B, M, N, K, variant, c_order=COL, alpha=2 - 1j, beta=1 + 3j, seed=2)
