@@ -197,7 +197,7 @@ def main():
         if i % 200 == 199:
             print("%d problems" % (i + 1), flush=True)
     print("\n%s operands; the default against the fastest of 256x128, 128x128, 64x64"
-          "\n(the default may also take 192x256 blocks, and two runs of one kernel differ by a few %%)" %
+          "\n(the default may also take 192x256 blocks or waves of their own, and is then in front; two runs of one kernel differ by a few %%)" %
           ("warm" if args.warm else "cold"))
     print("%-30s %8s %14s %10s %10s" % ("input, layout", "problems", "mean behind %", "> 8 % in", "> 20 % in"))
     for name in sorted(groups):
