@@ -2542,13 +2542,15 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   for (int i = 0; i < 4; ++i) xa[i] = lds_base + x_slot_off(0) + xo[i];
   const unsigned iters = k_tiles;
   for (unsigned vt = blockIdx.x; vt < total; vt += gridDim.x) {
-    const TileCoord tc = tile_coord(args, vt);
-    const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     // A wave whose part of the block lies beyond C leaves the matrix cores to the wave next to it on the SIMD (a block of
     // 128 rows of which 64 exist has one of each two): B=16 300x3001x577 fp16 pairs 113.8 -> 108.6 us, B=247
     // 456x299x1552 595 -> 567. (8- and 1-bit input: B=16 4096x4096x8192, where no wave is idle, 0.8 % slower.)
     constexpr bool kMaySkip = BX * BY > 64 * 64 && DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1;
-    const bool inside = !kMaySkip || (x_wave < args.nx && y_wave < args.ny);
+    bool inside = true;
+    if constexpr (kMaySkip) {
+      const TileCoord tc = tile_coord(args, vt);
+      inside = tc.block_x * BX + wx * WX < args.nx && tc.block_y * BY + wy * WY < args.ny;
+    }
     typename AccType<MS>::type acc_re[TY][TX], acc_im[TY][TX];
     SplitState<DT == kFloat32 ? TX : 1> split;   // (32-bit input)
     SmallTile small;                             // (64 x 64 blocks)
@@ -2692,6 +2694,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     // under way; the next tile's first barrier, behind which the slot is refilled, waits for them,
     // and no epilogue of theirs uses LDS.)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const TileCoord tc = tile_coord(args, vt);
+    const unsigned x_wave = tc.block_x * BX + wx * WX, y_wave = tc.block_y * BY + wy * WY;
     bool redo = false;   // (32-bit input) this wave's tile is computed again
     if constexpr (DT == kFloat32) {
       redo = !mma_split_last(split, acc_re, acc_im);
@@ -3037,6 +3041,8 @@ inline BlockChoice block_choice(const GemmParams &p) {
   const bool shared_lines = bits_of(p.type_in) == 16 && c_bytes >= ((size_t)256 << 20) &&
                             (size_t)p.nx * (p.c_interleaved ? 2 : 1) * bits_of(p.type_out) / 8 % 128 != 0;
   if (shared_lines) costs.tile_128 += 4.0;
+  // (pairs of C with beta are read and stored piece by piece: B=53 673x176x208 bf16 pairs 51 us, 38 on 64 x 64 blocks)
+  if (bits_of(p.type_in) == 16 && p.c_interleaved) costs.beta_128 += 12.0;
   const double t128 = few ? time(128, 128, costs.cost_few, costs.tile_few, 0.0, costs.beta_128)
                           : time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
   const double t64 = time(64, 64, costs.cost_64, costs.tile_64, costs.lone_64, costs.beta_64);
