@@ -156,3 +156,31 @@ def test_64x64_blocks_on_interleaved_bytes(B, M, N, K, tin):
     rms = np.sqrt(np.mean(np.abs(want) ** 2))
     assert np.linalg.norm(got - want) <= 6e-5 * np.linalg.norm(want)
     assert (np.abs(got - want) <= 3.5e-4 * np.maximum(rms, np.abs(want))).all()
+
+
+@pytest.mark.parametrize("tin,tout", TYPES[:3])
+@pytest.mark.parametrize("c_axis", [PLANAR, INTERLEAVED])
+@pytest.mark.parametrize("layout", ["tiled", "planar", "pairs"])
+@pytest.mark.parametrize("M,N,K,beta", [(128, 128, 64, 0), (70, 200, 40, 0), (129, 65, 96, 0.5 - 1j)])
+def test_128x128_blocks_of_four_waves(tin, tout, c_axis, layout, M, N, K, beta):
+    """More 128 x 128 tiles than units, with waves that lie beyond C: the same bits as 64 x 64 blocks."""
+    import torch
+    B = 300
+    if layout == "planar" and c_axis == INTERLEAVED:
+        return   # (the basic variant has planar C only)
+    types = {VT.float16: torch.float16, VT.bfloat16: torch.bfloat16, VT.float32: torch.float32}
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    a, b = (torch.randn(B * 2 * rows * K, device="cuda", generator=gen).to(types[tin]) for rows in (M, N))
+    start = torch.randn(B * 2 * M * N, device="cuda", generator=gen).to(types[tout])
+    axis = INTERLEAVED if layout == "pairs" else PLANAR
+    results = []
+    for block_tile in (2, 4):
+        with cc.option(cc.Option.gemm_block_tile, block_tile), \
+                cc.option(cc.Option.pipeline_route, 2 if layout == "tiled" else 1):
+            pipe = cc.Pipeline(B, M, N, K, 0, stream(), axis, c_axis, ROW, COL, ROW, tin, tout, cc.Variant.opt, 1.5j, beta)
+        c = start.clone()
+        pipe.Run(a.data_ptr(), b.data_ptr(), c.data_ptr())
+        torch.cuda.synchronize()
+        results.append(c)
+    assert not torch.equal(results[0], start)
+    assert torch.equal(results[0], results[1])
