@@ -108,7 +108,9 @@ struct KernelArgs {
   size_t x_batch_bytes, y_batch_bytes;
   float alpha_re, alpha_im, beta_re, beta_im;
   int have_alpha, have_beta, c_interleaved;
-  // planar C of 32 bits in rows of whole cache lines, more than the caches hold: stored past them
+  // planar C of 32 bits in rows of whole cache lines, as much as the last-level cache holds or more: stored past the
+  // caches by store_wave_tile_rows, _staged and _staged32, which write whole lines at once (whole wave tiles without
+  // beta; not the 192 x 256 and 64 x 64 blocks, the waves and 32-bit input)
   int c_past_caches;
   // 1-bit samples on the MFMA: what the zero bits past K add to every imaginary sum
   unsigned im_excess;
@@ -210,9 +212,12 @@ __device__ __forceinline__ TileCoord tile_coord(const KernelArgs &args, unsigned
   return tc;
 }
 
-// From how many bytes on a planar C of 32-bit elements in whole lines is stored past the caches, by the epilogues that
-// write whole lines at once.
-constexpr size_t kPastCachesBytes = (size_t)128 << 20;
+// From how many bytes on a planar C of 32-bit elements in whole lines is stored past the caches: what the last-level cache
+// holds, since a kernel that reads C next still finds a smaller one there. Us of the product, and of a maximum over
+// C behind it, kept and past the caches: 128 MiB (B=8 2048x1024x128 bf16) 37.6 + 33.7, 31.7 + 47.1; 192 MiB (B=24 1024x1024x256 bf16)
+// 69.8 + 42.6, 69.1 + 63.8; 256 MiB (B=32 1024x1024x512 e4m3 pairs) 101.8 + 77.5, 83.6 + 78.8; 512 MiB (B=64 1024x1024x512
+// fp16) 309 + 153, 259 + 192.
+constexpr size_t kPastCachesBytes = (size_t)256 << 20;
 
 // Fills the kernel argument block from the launch parameters for a BX x BY
 // block tile.

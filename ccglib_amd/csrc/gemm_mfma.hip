@@ -1209,11 +1209,10 @@ typedef float4_t float4_any_t __attribute__((aligned(4)));
 typedef int4_t int4_any_t __attribute__((aligned(2)));
 typedef ushort4_t ushort4_any_t __attribute__((aligned(2)));
 // A piece of C in an epilogue that writes whole cache lines at once. past_caches (KernelArgs::c_past_caches): a C of
-// 128 MiB or more is not kept: what the caches would make room for by and by, whole lines in some other order,
-// goes out as it comes. Us without and with it: B=16 1024x1024x256 bf16 53.0, 47.2, the same in
-// e4m3 pairs 39.4, 34.0; B=16 2048x2048x1024 e4m3 282, 255; B=64 1024x1024x512 fp16 304, 295; with K = 8192 nothing.
-// Of a C that the last-level cache holds (B=200 160x96x96 e4m3 11.9, 17.2) or rows that share lines (B=176
-// 629x4330x512 e4m3 1626, 3044) it only costs.
+// 256 MiB or more is not kept: what the caches would make room for by and by, whole lines in some other order,
+// goes out as it comes. Us without and with it: B=16 2048x2048x1024 e4m3 282, 259; B=64 1024x1024x512 fp16 309, 259; B=32
+// 1024x1024x512 e4m3 pairs 102, 84; with K = 8192 nothing. Of a smaller C the next kernel loses more than this one gains
+// (kPastCachesBytes), and rows that share lines (B=176 629x4330x512 e4m3 1626, 3044) only cost.
 template <typename Piece, typename Value>
 __device__ __forceinline__ void store_c(void *at, const Value &v, bool past_caches) {
   if (past_caches) {
