@@ -2177,7 +2177,7 @@ __device__ __forceinline__ void load_1k_to_lds_by_lane(const char *lane_address,
 #include "gemm_mfma_wide.h"
 
 template <int DT, int TOUT, int BX, int BY, int WX, int WY, int SLOTS, int WAVES_PER_EU, int LOADER,
-          int MS, bool XT, int XSLOTS>
+          int MS, bool XT, int XSLOTS, bool SKIP>
 __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void complex_gemm_mfma_dtl(
     const KernelArgs args) {
   constexpr int NWX = BX / WX, NWY = BY / WY, NW = NWX * NWY;
@@ -2541,12 +2541,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
   for (int i = 0; i < 4; ++i) xa[i] = lds_base + x_slot_off(0) + xo[i];
   const unsigned iters = k_tiles;
   for (unsigned vt = blockIdx.x; vt < total; vt += gridDim.x) {
-    // A wave whose part of the block lies beyond C leaves the matrix cores to the wave next to it on the SIMD (a block of
-    // 128 rows of which 64 exist has one of each two): B=16 300x3001x577 fp16 pairs 113.8 -> 108.6 us, B=247
-    // 456x299x1552 595 -> 567. (8- and 1-bit input: B=16 4096x4096x8192, where no wave is idle, 0.8 % slower.)
-    constexpr bool kMaySkip = BX * BY > 64 * 64 && DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1;
+    // (SKIP) A wave whose part of the block lies beyond C leaves the matrix cores to the wave next to it on the SIMD (a
+    // block of 128 rows of which 64 exist has one of each two); idle_waves_pay says when.
     bool inside = true;
-    if constexpr (kMaySkip) {
+    if constexpr (SKIP) {
       const TileCoord tc = tile_coord(args, vt);
       inside = tc.block_x * BX + wx * WX < args.nx && tc.block_y * BY + wy * WY < args.ny;
     }
@@ -2678,9 +2676,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     const std::true_type yes{};
     const std::false_type no{};
     if constexpr (kCarries) iteration(it++, yes, yes);
-    if (inside) {
+    if (!SKIP || inside) {
       for (; it < iters; ++it) iteration(it, no, yes);
-    } else {
+    } else if constexpr (SKIP) {
 #pragma unroll 1
       for (; it < iters; ++it) iteration(it, no, no);
     }
@@ -2856,7 +2854,7 @@ inline int compute_units() {
 }
 
 template <int DT, int TOUT, int BX, int BY, int WX, int WY, int SLOTS, int WPE,
-          int LOADER = kLoadTiled, int MS = 16, bool XT = false, int XSLOTS = SLOTS>
+          int LOADER = kLoadTiled, int MS = 16, bool XT = false, int XSLOTS = SLOTS, bool SKIP = false>
 hipError_t launch_dtl(const GemmParams &p, hipStream_t stream) {
   constexpr int NTHREADS = 64 * (BX / WX) * (BY / WY);
   constexpr int LDS_BYTES = 2 * (XSLOTS * BX + SLOTS * BY) * kTileRowBytes;
@@ -2869,7 +2867,7 @@ hipError_t launch_dtl(const GemmParams &p, hipStream_t stream) {
   const size_t total = (size_t)a.blocks_x * a.blocks_y * p.batch;
   if (total == 0) return hipSuccess;
   if (hipError_t e = check_grid(total)) return e;
-  auto kernel = complex_gemm_mfma_dtl<DT, TOUT, BX, BY, WX, WY, SLOTS, WPE, LOADER, MS, XT, XSLOTS>;
+  auto kernel = complex_gemm_mfma_dtl<DT, TOUT, BX, BY, WX, WY, SLOTS, WPE, LOADER, MS, XT, XSLOTS, SKIP>;
   static std::atomic<bool> lds_allowed[kMaxDevices];
   if (hipError_t e = allow_lds(kernel, LDS_BYTES, lds_allowed)) return e;
   // persistent blocks: as many as are resident at once, each walking C tiles
@@ -2878,6 +2876,38 @@ hipError_t launch_dtl(const GemmParams &p, hipStream_t stream) {
   const unsigned grid = (unsigned)(total < resident ? total : resident);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(NTHREADS), LDS_BYTES, stream, a);
   return hipGetLastError();
+}
+
+// Whether waves that have nothing of C to compute should leave their products out (SKIP of complex_gemm_mfma_dtl; 16-bit
+// input on 256 x 128 and 128 x 128 blocks). Looking for them takes every wave about 0.25 us a tile, and the loop on (re, im)
+// pairs 2 to 4 % besides, so it pays where the units that finish last have such waves and a tile is long enough. Time without
+// and with it, 2500 problems that have some (geometric means):
+//   a unit each, all blocks          up to 4 pieces of K 0.94 to 0.98 (pairs the least), 5 to 8 1.01 to 1.05 (pairs 1.00), from 33 on 1.08 to 1.11
+//   a unit each, some of the blocks  0.94 to 0.96 up to 4 pieces, 0.95 (pairs) to 1.01 beyond
+//   more blocks than units           fewer than 0.3 of them 0.97 to 1.00; beyond, up to 4 pieces 0.95 to 0.99, then on planar rows and
+//                                    tiles 1.01 to 1.08 (all of them: to 1.16), pairs 0.99 at 0.3 * 8 pieces, 1.02 at 0.3 * 32 and 0.8 * 4
+// (8- and 1-bit input: B=16 4096x4096x8192, where no wave is idle, 0.8 % slower with the test in the kernel.)
+template <int BX, int BY, int WX, int WY>
+bool idle_waves_pay(const GemmParams &p) {
+  const double pieces = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
+  const size_t across = ceil_div(p.nx, BX), down = ceil_div(p.ny, BY);
+  if (!across || !down) return false;
+  const bool idle_x = (p.nx - 1) % BX + 1 <= BX - WX, idle_y = (p.ny - 1) % BY + 1 <= BY - WY;
+  // share of the blocks that have idle waves
+  const double share = 1.0 - (1.0 - (idle_x ? 1.0 / (double)across : 0.0)) * (1.0 - (idle_y ? 1.0 / (double)down : 0.0));
+  if ((size_t)p.batch * across * down <= (size_t)compute_units()) {
+    return share == 1.0 && pieces >= (p.input_interleaved ? 8.0 : 5.0);
+  }
+  return pieces >= 5.0 && share >= 0.3 && share * pieces >= (p.input_interleaved ? 5.0 : 1.5);
+}
+template <int DT, int TOUT, int BX, int BY, int WX, int WY, int SLOTS, int WPE, int LOADER, int MS = 16, bool XT = false>
+hipError_t launch_block(const GemmParams &p, hipStream_t stream) {
+  if constexpr (DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1 && BX * BY > 64 * 64) {
+    if (idle_waves_pay<BX, BY, WX, WY>(p)) {
+      return launch_dtl<DT, TOUT, BX, BY, WX, WY, SLOTS, WPE, LOADER, MS, XT, SLOTS, true>(p, stream);
+    }
+  }
+  return launch_dtl<DT, TOUT, BX, BY, WX, WY, SLOTS, WPE, LOADER, MS, XT>(p, stream);
 }
 
 template <int DT, int TOUT, int LOADER, int TX, int TY, int SPLIT = 1>
@@ -3198,14 +3228,14 @@ template <int DT, int TOUT, int LOADER>
 hipError_t launch_128x128(const GemmParams &p, hipStream_t stream) {
   if constexpr (DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1) {
     const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 128) * ceil_div(p.ny, 128);
-    if (tiles <= (size_t)compute_units()) return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, LOADER, 16>(p, stream);
+    if (tiles <= (size_t)compute_units()) return launch_block<DT, TOUT, 128, 128, 64, 32, 4, 2, LOADER, 16>(p, stream);
     if constexpr (LOADER != kLoadInterleavedVec && LOADER != kLoadInterleavedRagged) {
       // (exchanged roles for planar C; pairs are regrouped through LDS)
-      if (!p.c_interleaved) return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16, true>(p, stream);
+      if (!p.c_interleaved) return launch_block<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16, true>(p, stream);
     }
-    return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16>(p, stream);
+    return launch_block<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16>(p, stream);
   } else {
-    return launch_dtl<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 32>(p, stream);
+    return launch_block<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 32>(p, stream);
   }
 }
 
@@ -3233,7 +3263,7 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
     auto launch = [&](auto loader) {
       constexpr int L = decltype(loader)::value;
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, L, 32>(p, stream);
-      return launch_dtl<DT, TOUT, 128, 128, 64, 32, 4, 2, L, 32>(p, stream);
+      return launch_block<DT, TOUT, 128, 128, 64, 32, 4, 2, L, 32>(p, stream);
     };
     const bool aligned = (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 16 == 0;
     if (p.input_interleaved) {
@@ -3253,18 +3283,18 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
     if (ragged) {
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedRagged, MS>(p, stream);
       if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadInterleavedRagged>(p, stream);
-      return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedRagged, MS>(p, stream);
+      return launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedRagged, MS>(p, stream);
     } else if constexpr (BITS16) {
       if (wide_tiles_apply(p) && wide_tiles_pay(p)) return launch_wide<DT, TOUT, true>(p, stream);
       if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec>(p, stream);
       if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadInterleavedVec>(p, stream);
-      return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec>(p, stream);
+      return launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec>(p, stream);
     } else {
       if (shape == k64x64) {
         return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadInterleavedVec, 32>(p, stream);
       }
       if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadInterleavedVec>(p, stream);
-      return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec, 32>(p, stream);
+      return launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadInterleavedVec, 32>(p, stream);
     }
   }
   else if (p.variant == kOpt || planar_direct) {
@@ -3281,7 +3311,7 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
       // rows of pairs (measured 5 % faster at B=64 512x4096x576).
       if constexpr (TOUT == kFloat32) {
         if (p.variant == kOpt && p.c_interleaved && shape == k256x128) {
-          return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 16, false>(p, stream);
+          return launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 16, false>(p, stream);
         }
       }
       // problems too small to give every compute unit a 256 x 128 tile: 128 x 128
@@ -3297,8 +3327,8 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
                                  : launch_128x128<DT, TOUT, kLoadPlanarVec>(p, stream);
       }
       return p.variant == kOpt
-                 ? launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 16, true>(p, stream)
-                 : launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarVec, 16, true>(p, stream);
+                 ? launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 16, true>(p, stream)
+                 : launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarVec, 16, true>(p, stream);
     } else {
       // fp8: the 32x32x64 MFMA takes one K tile per instruction, which lets the
       // same block shape and ring as for 16-bit input fit into LDS
@@ -3314,14 +3344,14 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
                                  : launch_128x128<DT, TOUT, kLoadPlanarVec>(p, stream);
       }
       return p.variant == kOpt
-                 ? launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>(p, stream)
-                 : launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarVec, 32>(p, stream);
+                 ? launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadTiled, 32>(p, stream)
+                 : launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarVec, 32>(p, stream);
     }
   }
   else if (k_bytes >= 16) {
     if (shape == k64x64) return launch_dtl<DT, TOUT, 64, 64, 32, 32, 5, 2, kLoadPlanarRagged, MS>(p, stream);
     if (shape == k128x128) return launch_128x128<DT, TOUT, kLoadPlanarRagged>(p, stream);
-    return launch_dtl<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarRagged, MS, BITS16>(p, stream);
+    return launch_block<DT, TOUT, 256, 128, 64, 64, 3, 2, kLoadPlanarRagged, MS, BITS16>(p, stream);
   }
   // fp8 stages are twice as large (two K tiles per MFMA): one wave per SIMD
   // with the full register file
