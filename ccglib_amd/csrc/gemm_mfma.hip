@@ -3013,46 +3013,66 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 //     8 bits on tiles, 4096x4096x512:  52, 51, 69
 //     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
 //       308, 317, 339
-// Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles (of 16-bit input: from more tiles than units on), and
+// Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles (of 16-bit input: those of four waves), and
 // a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
 // With beta the epilogue reads C first, which costs the larger tiles more (8 bits on planar
-// rows, B=11 456x1542x192: 97, 84, 47).
+// rows, B=11 456x1542x192: 97, 84, 47), and pairs of C with beta are read and stored piece by piece by all of them (B=43 144x1024x32
+// fp16 pairs 40.2, 36.3, 27.3).
+//   128 x 128 blocks of 16-bit input have eight waves and a ring of four slots while every block has a unit to itself, which
+// keeps more on its way (B=256 96x96x1024 pairs 48 us, 52 with the other); beyond, four waves of 64 x 64 and two slots, of which
+// two share a unit: one stores C or waits while the other multiplies, the fragments are read once for twice as many
+// products, and C is stored in whole row segments. In us, planar rows unless said, 8 and 4 waves (256 x 128 blocks):
+// B=67 384x3136x328 445, 329 (337); B=300 512x512x128 217, 158 (163); B=100 320x320x256 pairs 45, 40 (50). With beta, which
+// takes the four waves' registers while C is read, eight may be the faster ones there too (B=60 1536x128x80 fp16 planar 41.8, 51.3;
+// 750 such problems 0.97 times on planar rows of K up to 300, 1.03 to 1.12 elsewhere), which have constants of their own for it.
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
 // 30000 problems of random sizes, 40 % of them on operands that no cache held
 // (python -m ccglib_amd.tuning.block_choice times such problems); those of 8-bit tiles
-// to 1900, of 32-bit input to 1200, of all 16-bit layouts to 2100 further ones, timed since those kernels last changed, on
-// which (16 bits) the choice is 0.9 % behind the fastest of the three shapes on average and more than 8 % in 3.7 %.
+// to 1900, of 32-bit input to 1200 further ones, timed since those kernels last changed. Those of 16-bit input: to the choice among the
+// shapes in 8600 problems on cold operands, 40 % of them of K up to 128 (the least sum of what a choice loses against the fastest shape
+// and, counted twice, against the choice from before there were blocks of four waves). On a third kept out of the fit it is
+// 0.4 % (tiles), 0.7 % (planar rows) and 0.6 % (pairs) behind the fastest of the shapes on average.
 enum BlockShape { k256x128, k128x128, k64x64 };
 struct BlockChoice {
   BlockShape shape;
   double time;   // in units of one element of C in a 256 x 128 tile
+  bool eight_waves;   // (16-bit input, 128 x 128)
 };
 struct BlockCosts {
   double cost_128, cost_64;   // per element of C and piece of K, of 256 x 128's
   double tile_128, tile_64;   // what a tile costs besides its K loop, in pieces of K
   double lone_128, lone_64;   // what a tile without a neighbour costs more, of a tile
   double beta_256, beta_128, beta_64;   // added to the tile's cost with beta
-  double cost_few, tile_few;  // (16 bits) 128 x 128 blocks with a unit each, see launch_128x128
+  // 16-bit input: the same of 128 x 128 blocks of eight waves, and what beta adds if C holds pairs (256 x 128 and four waves; eight)
+  double cost_8w = 0.0, tile_8w = 0.0, beta_8w = 0.0, pairs_beta = 0.0, pairs_beta_8w = 0.0;
 };
 inline BlockCosts block_costs(const GemmParams &p) {
-  if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (p.type_in == kInt1) return {1.04, 1.44, 8.8, 9.0, 0.11, 0.0, 0.0, 0.0, 0.0};
   // (32-bit input has no 256 x 128 block: relative to 128 x 128)
-  if (p.type_in == kFloat32) return {1.0, 1.24, 6.0, 5.0, 0.0, 0.0, 0.0, 4.0, 2.0, 0.0, 0.0};
+  if (p.type_in == kFloat32) return {1.0, 1.24, 6.0, 5.0, 0.0, 0.0, 0.0, 4.0, 2.0};
   const bool planar = p.variant == kBasic && !p.input_interleaved;
   if (bits_of(p.type_in) == 8) {
-    if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0, 0.0, 0.0};
-    if (planar) return {1.30, 2.54, 7.6, 7.9, 0.3, 0.1, 13.0, 10.0, 1.0, 0.0, 0.0};
-    return {1.05, 1.61, 9.2, 9.4, 0.3, 0.11, 13.0, 10.0, 1.0, 0.0, 0.0};
+    if (p.input_interleaved) return {1.04, 1.87, 9.3, 7.0, 0.3, 0.1, 13.0, 10.0, 1.0};
+    if (planar) return {1.30, 2.54, 7.6, 7.9, 0.3, 0.1, 13.0, 10.0, 1.0};
+    return {1.05, 1.61, 9.2, 9.4, 0.3, 0.11, 13.0, 10.0, 1.0};
   }
-  if (p.input_interleaved) return {1.10, 2.05, 8.74, 11.27, 0.29, 0.63, 8.56, 7.10, 5.17, 1.38, 10.0};
-  if (planar) return {1.14, 2.10, 7.99, 9.25, 0.28, 0.45, 13.57, 12.23, 2.60, 1.24, 8.29};
-  return {1.08, 1.69, 8.77, 9.34, 0.25, 0.63, 10.33, 9.22, 3.35, 0.87, 10.95};
+  if (p.input_interleaved) {
+    return {1.06, 1.85, 9.07, 8.55, 0.34, 0.43, 19.94, 18.45, 10.0, 1.27, 11.81, 12.36, 3.44, 1.27};
+  }
+  if (planar) return {1.16, 2.51, 7.86, 6.97, 0.48, 0.26, 10.09, 11.93, 2.61, 1.29, 11.73, 3.88, 4.3, 1.6};
+  return {1.08, 1.85, 8.72, 8.86, 0.44, 0.60, 15.85, 15.28, 6.62, 1.30, 7.48, 12.97, 5.24, 1.91};
 }
 inline BlockChoice block_choice(const GemmParams &p) {
   const size_t units = (size_t)compute_units();
   BlockCosts costs = block_costs(p);
+  const bool bits16 = bits_of(p.type_in) == 16;
   // (pieces of a plane's row: an interleaved row holds both planes)
   const double pieces = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
+  if (p.c_interleaved) {
+    costs.beta_256 += costs.pairs_beta;
+    costs.beta_128 += costs.pairs_beta;
+    costs.beta_8w += costs.pairs_beta_8w;
+  }
   const double large = pieces + 10.0 + (p.have_beta ? costs.beta_256 : 0.0);
   auto time = [&](size_t bx, size_t by, double cost, double tile, double lone, double beta) {
     const size_t tiles = (size_t)p.batch * ceil_div((size_t)p.nx, bx) * ceil_div((size_t)p.ny, by);
@@ -3062,24 +3082,25 @@ inline BlockChoice block_choice(const GemmParams &p) {
   };
   const bool no_256 = p.type_in == kFloat32;
   const double t256 = no_256 ? HUGE_VAL : time(256, 128, 1.0, 10.0, 0.0, costs.beta_256);
-  const bool few = bits_of(p.type_in) == 16 &&
-                   (size_t)p.batch * ceil_div(p.nx, 128) * ceil_div(p.ny, 128) <= units;
   // (a large C whose rows share cache lines, which the narrower blocks write in more parts: B=173 1728x1656x64 fp16
   // 1030 us on 256 x 128 blocks, 1357 on these)
   const size_t c_bytes = (size_t)2 * p.batch * p.nx * p.ny * bits_of(p.type_out) / 8;
-  const bool shared_lines = bits_of(p.type_in) == 16 && c_bytes >= ((size_t)256 << 20) &&
+  const bool shared_lines = bits16 && c_bytes >= ((size_t)256 << 20) &&
                             (size_t)p.nx * (p.c_interleaved ? 2 : 1) * bits_of(p.type_out) / 8 % 128 != 0;
   if (shared_lines) costs.tile_128 += 4.0;
-  // (pairs of C with beta are read and stored piece by piece: B=53 673x176x208 bf16 pairs 51 us, 38 on 64 x 64 blocks)
-  if (bits_of(p.type_in) == 16 && p.c_interleaved) costs.beta_128 += 12.0;
-  const double t128 = few ? time(128, 128, costs.cost_few, costs.tile_few, 0.0, costs.beta_128)
-                          : time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
+  const bool few = (size_t)p.batch * ceil_div(p.nx, 128) * ceil_div(p.ny, 128) <= units;
+  const double t4w = bits16 && few ? HUGE_VAL
+                                   : time(128, 128, costs.cost_128, costs.tile_128, costs.lone_128, costs.beta_128);
+  const double t8w = bits16 && (few || p.have_beta) ? time(128, 128, costs.cost_8w, costs.tile_8w, 0.0, costs.beta_8w)
+                                                    : HUGE_VAL;
+  const bool eight = t8w < t4w;
+  const double t128 = eight ? t8w : t4w;
   const double t64 = time(64, 64, costs.cost_64, costs.tile_64, costs.lone_64, costs.beta_64);
-  if (p.block_tile == 1 && !no_256) return {k256x128, t256};
-  if (p.block_tile == 1 || p.block_tile == 2) return {k128x128, t128};
-  if (p.block_tile >= 4) return {k64x64, t64};   // (5 to 7: waves, where there are such kernels)
-  if (t256 <= t128 && t256 <= t64) return {k256x128, t256};
-  return t128 <= t64 ? BlockChoice{k128x128, t128} : BlockChoice{k64x64, t64};
+  if (p.block_tile == 1 && !no_256) return {k256x128, t256, false};
+  if (p.block_tile == 1 || p.block_tile == 2) return {k128x128, t128, eight};
+  if (p.block_tile >= 4) return {k64x64, t64, false};   // (5 to 7: waves, where there are such kernels)
+  if (t256 <= t128 && t256 <= t64) return {k256x128, t256, false};
+  return t128 <= t64 ? BlockChoice{k128x128, t128, eight} : BlockChoice{k64x64, t64, false};
 }
 
 // Whether the 192 x 256 block of gemm_mfma_wide.h can compute this problem (what
@@ -3218,17 +3239,11 @@ hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream
   return launch(std::integral_constant<int, kLoadPlanarRagged>{});
 }
 
-// 128 x 128 blocks. 16-bit input: while every block has a unit to itself, 8 waves of 64 x 32 and a ring of four slots, which
-// keeps more on its way (B=256 96x96x1024 pairs 48 us, 52 with the other); beyond, 4 waves of 64 x 64 and two slots, of which two
-// share a unit: one stores C or waits while the other multiplies, the fragments are read once for twice as many
-// products, and C is stored in whole row segments. In us, planar rows unless said, 8 and 4 waves (256 x 128 blocks):
-// B=67 384x3136x328 445, 329 (337); B=300 512x512x128 217, 158 (163); B=12 640x1328x512 57, 50 (54); B=100
-// 320x320x256 pairs 45, 40 (50); 2x3000x1500x256 37.5, 30.4 (35.8); B=64 512x4096x576 822, 655 (613).
+// 128 x 128 blocks (16-bit input: of eight or four waves, see block_choice).
 template <int DT, int TOUT, int LOADER>
 hipError_t launch_128x128(const GemmParams &p, hipStream_t stream) {
   if constexpr (DtypeTraits<DT>::kElemBytes == 2 && DT != kInt1) {
-    const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 128) * ceil_div(p.ny, 128);
-    if (tiles <= (size_t)compute_units()) return launch_block<DT, TOUT, 128, 128, 64, 32, 4, 2, LOADER, 16>(p, stream);
+    if (block_choice(p).eight_waves) return launch_block<DT, TOUT, 128, 128, 64, 32, 4, 2, LOADER, 16>(p, stream);
     if constexpr (LOADER != kLoadInterleavedVec && LOADER != kLoadInterleavedRagged) {
       // (exchanged roles for planar C; pairs are regrouped through LDS)
       if (!p.c_interleaved) return launch_block<DT, TOUT, 128, 128, 64, 64, 2, 2, LOADER, 16, true>(p, stream);
@@ -3315,7 +3330,7 @@ hipError_t launch_typed(const GemmParams &p, hipStream_t stream) {
         }
       }
       // problems too small to give every compute unit a 256 x 128 tile: 128 x 128
-      // blocks, 8 waves of 64 x 32, 4-slot ring, or 64 x 64 blocks, 4 waves of 32 x 32,
+      // blocks (launch_128x128), or 64 x 64 blocks, 4 waves of 32 x 32,
       // 5-slot ring, two blocks a unit
       if (shape == k64x64) {
         return p.variant == kOpt
