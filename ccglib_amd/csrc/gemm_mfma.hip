@@ -3129,32 +3129,48 @@ inline bool wide_tiles_pay(const GemmParams &p) {
   return wide_tiling(p).rounds * (kWideBX * kWideBY) < 1.075 * block_choice(p).time;
 }
 
-// Which tile the waves of complex_gemm_mfma_wave take, if that kernel is the faster one: the least of
-//   fixed + max(K tiles * alone, K tiles * crowded * n / 256) + tile * n / 256   in us
-// over 64 x 64 blocks and the wave tiles, with n blocks or waves on 256 units: `alone` is what a K tile takes
-// with a unit to itself, `crowded` with others next to it, `tile` what a tile costs besides. The constants are
-// fitted, for each type and operand layout, to the times of all shapes on 1600 problems of up to 1024 blocks of
-// 64 x 64 (450 of 1-bit input), 60 % of them on operands that no cache held, a fifth on ragged rows.
-// There the choice by these times was 2 to 3 % (16 bits) and 1 % (8 bits) behind the fastest shape on average, and in front of
-// 64 x 64 blocks by 1.41 times (16 bits) and 1.20 (8 bits), 1-bit input, whose waves share K, by 1.5. More waves than there are SIMDs are left to the blocks: the fifth wave of a unit has to share one
-// (B=213 32x192x3184 on planar rows, 1278 waves: 179 us on blocks, 261 on waves; B=93 32x448x1584 58, 85).
+// Which tile the waves of complex_gemm_mfma_wave take, if that kernel is the faster one: the least of, in us,
+//   fixed + max(K tiles * alone, K tiles * crowded * n / units, operand MB * bytes) + tile * n / units
+// over 64 x 64 blocks and the wave tiles, with n blocks or waves: `alone` is what a K tile takes
+// with a unit to itself, `crowded` with others next to it, `tile` what a tile costs besides. Waves: `alone` grows by `second` for every
+// further wave of the busiest unit (330 waves on 256 units take as long as 512 where the copies of one wave do not fill the time; a
+// wave keeps 32 KiB on its way where a block keeps 80, so that operands that no cache holds come in more slowly: B=197 24x49x2992
+// planar fp16 62 us on waves, 46 on blocks). The constants are
+// fitted, for each type and operand layout, to the choice among the shapes (what it loses against the fastest one, and three times
+// against 64 x 64 blocks alone): 7700 problems of 16 bits, 2130 of 8, 1890 of 1 bit that have 64 x 64 blocks by block_choice, on cold operands.
+// On a third kept out of the fit the choice was behind the fastest shape by 0.3 % (tiles), 0.6 % (pairs) and 1.2 %
+// (planar rows) for 16 bits, 0.4 to 0.8 % for 8, 3 to 4 % for 1 bit (waves that do not share K would serve more rounds), and in front of 64 x 64
+// blocks by 1.29 to 1.33 times (16 bits), 1.14 to 1.17 (8 bits), 1.21 to 1.31 (1 bit). More waves than there are SIMDs are left to the
+// blocks: the fifth wave of a unit has to share one (B=213 32x192x3184 on planar rows, 1278 waves: 179 us on blocks, 261 on waves).
 enum WaveShape { kNoWaves, kWaves32x32, kWaves32x16, kWaves16x16 };
 struct WaveCosts {
   double fixed, alone, crowded, tile;
 };
-inline const WaveCosts *wave_costs(const GemmParams &p) {   // 64 x 64 blocks, then as WaveShape
+struct WaveTable {
+  WaveCosts shape[4];   // 64 x 64 blocks, then as WaveShape
+  double second;        // waves: what every further one of the busiest unit adds to `alone`, of it
+  double beta;          // blocks: they only request C behind the last product
+  double block_bytes, wave_bytes;   // us per MB of A and B
+};
+inline const WaveTable &wave_costs(const GemmParams &p) {
   static constexpr WaveCosts none = {0.0, 0.0, 0.0, 0.0};
-  static constexpr WaveCosts bits16_tiled[] = {{3.80, 0.286, 0.367, 1.48}, {2.92, 0.240, 0.139, 0.49},
-                                               {3.09, 0.141, 0.081, 0.13}, {3.24, 0.086, 0.058, 0.01}};
-  static constexpr WaveCosts bits16_planar[] = {{4.12, 0.438, 0.524, 1.36}, {3.35, 0.257, 0.253, 0.31},
-                                                {3.23, 0.165, 0.168, 0.00}, {3.24, 0.092, 0.102, 0.03}};
-  static constexpr WaveCosts bits16_pairs[] = {{4.13, 0.356, 0.423, 1.58}, {3.13, 0.295, 0.180, 0.51},
-                                               {3.05, 0.184, 0.099, 0.22}, {3.14, 0.110, 0.066, 0.08}};
-  static constexpr WaveCosts bits8_tiled[] = {{3.95, 0.265, 0.415, 1.65}, {3.38, 0.161, 0.129, 0.51}, none, none};
-  static constexpr WaveCosts bits8_planar[] = {{4.55, 0.349, 0.556, 1.92}, {4.08, 0.157, 0.249, 0.17}, none, none};
-  static constexpr WaveCosts bits8_pairs[] = {{4.54, 0.413, 0.433, 1.79}, {3.23, 0.238, 0.206, 0.84}, none, none};
-  static constexpr WaveCosts int1_tiled[] = {{4.08, 0.871, 1.041, 1.61}, {3.20, 0.735, 0.282, 0.50}, none, none};
-  static constexpr WaveCosts int1_planar[] = {{4.45, 0.840, 1.023, 1.77}, {3.31, 0.746, 0.359, 0.82}, none, none};
+  static constexpr WaveTable bits16_tiled = {{{4.836, 0.427, 0.499, 1.107}, {3.070, 0.291, 0.105, 0.661},
+                                              {2.887, 0.222, 0.052, 0.189}, {2.405, 0.067, 0.094, 0.057}}, 0.286, 0.229, 0.145, 0.130};
+  static constexpr WaveTable bits16_planar = {{{4.737, 0.386, 0.474, 1.487}, {4.274, 0.256, 0.200, 0.251},
+                                               {3.058, 0.261, 0.189, 0.008}, {2.544, 0.179, 0.137, 0.024}}, 0.521, 0.317, 0.229, 0.277};
+  static constexpr WaveTable bits16_pairs = {{{5.172, 0.489, 0.551, 1.398}, {4.188, 0.384, 0.148, 0.478},
+                                              {2.579, 0.305, 0.165, 0.316}, {2.440, 0.161, 0.125, 0.053}}, 0.247, 1.206, 0.148, 0.087};
+  static constexpr WaveTable bits8_tiled = {{{3.762, 0.313, 0.405, 2.345}, {3.118, 0.221, 0.141, 0.495}, none, none},
+                                            0.236, 1.409, 0.150, 0.175};
+  static constexpr WaveTable bits8_planar = {{{3.816, 0.537, 0.670, 2.406}, {3.484, 0.271, 0.221, 0.351}, none, none},
+                                             0.809, 2.391, 0.269, 0.372};
+  static constexpr WaveTable bits8_pairs = {{{4.495, 0.359, 0.461, 1.901}, {3.511, 0.252, 0.117, 0.569}, none, none},
+                                            0.474, 1.997, 0.275, 0.309};
+  // (1 bit: `fixed` and `alone` of a tile shared by four waves, see wave_choice; `second`: of a launch)
+  static constexpr WaveTable int1_tiled = {{{3.738, 1.079, 1.353, 1.857}, {4.653, 1.026, 0.0, 0.0}, none, none},
+                                           -1.454, 0.0, 0.212, 0.271};
+  static constexpr WaveTable int1_planar = {{{6.040, 0.947, 0.938, 1.252}, {3.101, 1.079, 0.0, 0.0}, none, none},
+                                            2.437, 0.0, 0.268, 0.214};
   const bool tiled = p.variant == kOpt && !p.input_interleaved;
   if (p.type_in == kInt1) return tiled ? int1_tiled : int1_planar;
   if (bits_of(p.type_in) == 8) return p.input_interleaved ? bits8_pairs : tiled ? bits8_tiled : bits8_planar;
@@ -3173,7 +3189,8 @@ inline WaveShape wave_choice(const GemmParams &p) {
   }
   if (p.block_tile >= 5) return p.block_tile == 5 || !bits16 ? kWaves32x32 : p.block_tile == 6 ? kWaves32x16 : kWaves16x16;
   if (block_choice(p).shape != k64x64) return kNoWaves;
-  const WaveCosts *costs = wave_costs(p);
+  const WaveTable &table = wave_costs(p);
+  const WaveCosts *costs = table.shape;
   const double k_tiles = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
   const double units = (double)compute_units();
   // Ragged rows of many K tiles go through the transposes (rows_in_place_pay), with waves on the tiles behind
@@ -3183,27 +3200,25 @@ inline WaveShape wave_choice(const GemmParams &p) {
   const bool ragged = (p.variant != kOpt || p.input_interleaved) && p.type_in != kInt1 &&
                       (p.input_interleaved ? 2 : 1) * (size_t)p.k * bits_of(p.type_in) / 8 % 16 != 0;
   if (ragged && k_tiles > 64.0) return kNoWaves;
-  if (p.type_in == kInt1) {
-    // The four SIMDs of a unit share the K tiles of one tile of C, a unit's tiles one after the other: us on 64 x 64 blocks and
-    // like this, 512x512 (a tile a unit) K=2048 7.8, 4.9; K=32768 59.7, 19.2; B=20 128x128 (some units two) K=8192
-    // 18.4, 13.9; K=32768 60.3, 33.7; 768x1024 (three) K=8192 19.0, 20.2; K=32768 60.9, 49.4.
-    const double tiles = (double)p.batch * (double)ceil_div(p.nx, 32) * (double)ceil_div(p.ny, 32);
-    const double n64 = (double)p.batch * (double)ceil_div(p.nx, 64) * (double)ceil_div(p.ny, 64) / units;
-    const double rounds = std::ceil(tiles / units);
-    const double blocks = costs[0].fixed + k_tiles * std::max(costs[0].alone, costs[0].crowded * n64) + costs[0].tile * n64;
-    return rounds <= 3.0 && rounds * (3.3 + costs[1].alone * std::ceil(k_tiles / 4.0)) < blocks ? kWaves32x32 : kNoWaves;
-  }
+  const double operand_mb = 1e-6 * 2.0 * (double)p.batch * ((double)p.nx + (double)p.ny) * (double)p.k * bits_of(p.type_in) / 8;
   auto time = [&](int shape, unsigned x, unsigned y) {
     const WaveCosts &c = costs[shape];
     const double n = (double)p.batch * (double)ceil_div(p.nx, x) * (double)ceil_div(p.ny, y) / units;
     if (shape != 0 && n > kWavesPerUnit) return HUGE_VAL;
-    // (more than one wave a unit: which SIMDs they get depends on what the kernel before left, and two on one are
-    // slower: B=2 640x512x2048 e4m3 on waves 9.9 us behind itself, 15.8 behind another kernel, 15.1 on blocks)
-    const double alone = shape != 0 && n > 1.0 ? 1.35 * c.alone : c.alone;
-    // (blocks only request C with beta behind the last product)
-    const double beta = shape == 0 && p.have_beta ? 1.5 : 0.0;
-    return c.fixed + beta + k_tiles * std::max(alone, c.crowded * n) + c.tile * n;
+    const double alone = shape != 0 ? c.alone * (1.0 + table.second * (std::ceil(n) - 1.0)) : c.alone;
+    const double beta = shape == 0 && p.have_beta ? table.beta : 0.0;
+    const double bytes = operand_mb * (shape != 0 ? table.wave_bytes : table.block_bytes);
+    return c.fixed + beta + std::max(bytes, k_tiles * std::max(alone, c.crowded * n)) + c.tile * n;
   };
+  if (p.type_in == kInt1) {
+    // The four SIMDs of a unit share the K tiles of one tile of C, a unit's tiles one after the other: us on 64 x 64 blocks and
+    // like this, 512x512 (a tile a unit) K=2048 7.8, 4.9; K=32768 59.7, 19.2; B=20 128x128 (some units two) K=8192
+    // 18.4, 13.9; K=32768 60.3, 33.7; 768x1024 (three) K=8192 19.0, 20.2; K=32768 60.9, 49.4; B=5 1064x128 (three) K=9600 planar 23.8, 30.1.
+    const double rounds = std::ceil((double)p.batch * (double)ceil_div(p.nx, 32) * (double)ceil_div(p.ny, 32) / units);
+    const double waves = table.second + std::max(rounds * (costs[1].fixed + costs[1].alone * std::ceil(k_tiles / 4.0)),
+                                                 operand_mb * table.wave_bytes);
+    return rounds <= 3.0 && waves < time(0, 64, 64) ? kWaves32x32 : kNoWaves;
+  }
   double best = time(0, 64, 64);
   WaveShape shape = kNoWaves;
   auto try_shape = [&](WaveShape s, unsigned x, unsigned y) {
