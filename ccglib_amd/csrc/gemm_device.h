@@ -108,10 +108,6 @@ struct KernelArgs {
   size_t x_batch_bytes, y_batch_bytes;
   float alpha_re, alpha_im, beta_re, beta_im;
   int have_alpha, have_beta, c_interleaved;
-  // planar C of 32 bits in rows of whole cache lines, as much as the last-level cache holds or more: stored past the
-  // caches by store_wave_tile_rows, _staged and _staged32, which write whole lines at once (whole wave tiles without
-  // beta; not the 192 x 256 and 64 x 64 blocks, the waves and 32-bit input)
-  int c_past_caches;
   // 1-bit samples on the MFMA: what the zero bits past K add to every imaginary sum
   unsigned im_excess;
 };
@@ -218,6 +214,13 @@ __device__ __forceinline__ TileCoord tile_coord(const KernelArgs &args, unsigned
 // 69.8 + 42.6, 69.1 + 63.8; 256 MiB (B=32 1024x1024x512 e4m3 pairs) 101.8 + 77.5, 83.6 + 78.8; 512 MiB (B=64 1024x1024x512
 // fp16) 309 + 153, 259 + 192.
 constexpr size_t kPastCachesBytes = (size_t)256 << 20;
+// Planar C of 32 bits in rows of whole cache lines, as much as the last-level cache holds or more: stored past the
+// caches by store_wave_tile_rows, _staged and _staged32, which write whole lines at once (whole wave tiles without
+// beta; not the 192 x 256 and 64 x 64 blocks, the waves and 32-bit input). Worked out where it is needed: a flag among the arguments is
+// a scalar register more that is kept, or spilled, through the K loop.
+__device__ __forceinline__ bool past_caches(const KernelArgs &args) {
+  return args.nx % 32 == 0 && (uintptr_t)args.c % 128 == 0 && (size_t)8 * args.batch * args.nx * args.ny >= kPastCachesBytes;
+}
 
 // Fills the kernel argument block from the launch parameters for a BX x BY
 // block tile.
@@ -258,8 +261,6 @@ inline KernelArgs make_kernel_args(const GemmParams &p, int bx, int by) {
   a.have_alpha = p.have_alpha;
   a.have_beta = p.have_beta;
   a.c_interleaved = p.c_interleaved;
-  a.c_past_caches = bits_of(p.type_out) == 32 && !p.c_interleaved && p.nx % 32 == 0 && (uintptr_t)p.c % 128 == 0 &&
-                    (size_t)8 * p.batch * p.nx * p.ny >= kPastCachesBytes;
   a.im_excess = (p.type_in == kInt1) ? 2u * (p.k_tiles * (unsigned)k_per_tile(kInt1) - p.k) : 0u;
   return a;
 }

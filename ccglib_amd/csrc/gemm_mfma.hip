@@ -1208,18 +1208,16 @@ __device__ __forceinline__ bool mma_split_last(SplitState<TX> &st, float16_t_ (&
 typedef float4_t float4_any_t __attribute__((aligned(4)));
 typedef int4_t int4_any_t __attribute__((aligned(2)));
 typedef ushort4_t ushort4_any_t __attribute__((aligned(2)));
-// A piece of C in an epilogue that writes whole cache lines at once. past_caches (KernelArgs::c_past_caches): a C of
+// A piece of C in an epilogue that writes whole cache lines at once. PAST (past_caches): a C of
 // 256 MiB or more is not kept: what the caches would make room for by and by, whole lines in some other order,
 // goes out as it comes. Us without and with it: B=16 2048x2048x1024 e4m3 282, 259; B=64 1024x1024x512 fp16 309, 259; B=32
 // 1024x1024x512 e4m3 pairs 102, 84; with K = 8192 nothing. Of a smaller C the next kernel loses more than this one gains
 // (kPastCachesBytes), and rows that share lines (B=176 629x4330x512 e4m3 1626, 3044) only cost.
-template <typename Piece, typename Value>
-__device__ __forceinline__ void store_c(void *at, const Value &v, bool past_caches) {
-  if (past_caches) {
-    // (the empty statements keep the compiler from making one ordinary store of the two)
-    asm volatile("");
+// (An epilogue each: with the choice at every store planar C of 8 bits, which never takes it below 256 MiB, was 1 to 2 % slower.)
+template <typename Piece, bool PAST, typename Value>
+__device__ __forceinline__ void store_c(void *at, const Value &v) {
+  if constexpr (PAST) {
     __builtin_nontemporal_store((Piece)v, reinterpret_cast<Piece *>(at));
-    asm volatile("");
   } else {
     *reinterpret_cast<Piece *>(at) = v;
   }
@@ -1687,14 +1685,13 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
 // the four tiles of a tile row are four consecutive x, so a lane writes 16 bytes
 // (8 for fp16 / bf16 C) and a store instruction four whole 256-byte row segments,
 // straight from the accumulators.
-template <int TOUT, int TY>
+template <bool PAST, int TOUT, int TY>
 __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, unsigned b,
                                                      unsigned x_wave, unsigned y_wave, int lane,
                                                      float4_t (&acc_re)[TY][4],
                                                      float4_t (&acc_im)[TY][4]) {
   using Tout = typename OutType<TOUT>::type;
   const unsigned nx = args.nx, ny = args.ny;
-  const bool past_caches = args.c_past_caches;
   const bool have_alpha = args.have_alpha;
   const float ar = args.alpha_re, ai = args.alpha_im;
   Tout *out = reinterpret_cast<Tout *>(args.c) + (size_t)b * 2 * nx * ny +
@@ -1714,7 +1711,7 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
         }
         Tout *p = out + (size_t)plane * nx * ny + (size_t)(j * 16 + e) * nx;
         if constexpr (TOUT == kFloat32) {
-          store_c<float4_any_t>(p, float4_t{v[0], v[1], v[2], v[3]}, past_caches);
+          store_c<float4_any_t, PAST>(p, float4_t{v[0], v[1], v[2], v[3]});
         } else {
           Tout t[4] = {(Tout)v[0], (Tout)v[1], (Tout)v[2], (Tout)v[3]};
           *reinterpret_cast<ushort4_any_t *>(p) = __builtin_bit_cast(ushort4_t, t);
@@ -1732,14 +1729,13 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
 // the column-wise writes and the row-wise reads free of bank conflicts).
 constexpr int kStagePatchBytes = 16 * 272;
 
-template <int TX, int TY>
+template <bool PAST, int TX, int TY>
 __device__ __forceinline__ void store_wave_tile_staged(const KernelArgs &args, unsigned b,
                                                        unsigned x_wave, unsigned y_wave, int lane,
                                                        char *patch, float4_t (&acc_re)[TY][TX],
                                                        float4_t (&acc_im)[TY][TX]) {
   static_assert(TX == 4, "patch rows hold 64 columns");
   const unsigned nx = args.nx, ny = args.ny;
-  const bool past_caches = args.c_past_caches;
   const bool have_alpha = args.have_alpha;
   const float ar = args.alpha_re, ai = args.alpha_im;
   float *cbase = reinterpret_cast<float *>(args.c) + (size_t)b * 2 * nx * ny;
@@ -1764,7 +1760,7 @@ __device__ __forceinline__ void store_wave_tile_staged(const KernelArgs &args, u
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float4_t v = *reinterpret_cast<const float4_t *>(rd + r * 4 * 272);
-        store_c<float4_any_t>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 4) * nx, v, past_caches);
+        store_c<float4_any_t, PAST>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 4) * nx, v);
       }
     }
   }
@@ -1860,13 +1856,12 @@ __device__ __forceinline__ void store_wave_tile_staged_il(const KernelArgs &args
 // instruction writes eight whole 128-byte row segments.
 constexpr int kStagePatch32Bytes = 32 * 144;
 
-template <int TX, int TY, bool INT = false>
+template <bool PAST, int TX, int TY, bool INT = false>
 __device__ __forceinline__ void store_wave_tile_staged32(const KernelArgs &args, unsigned b,
                                                          unsigned x_wave, unsigned y_wave, int lane,
                                                          char *patch, float16_t_ (&acc_re)[TY][TX],
                                                          float16_t_ (&acc_im)[TY][TX]) {
   const unsigned nx = args.nx, ny = args.ny;
-  const bool past_caches = args.c_past_caches;
   const bool have_alpha = args.have_alpha;
   const float ar = args.alpha_re, ai = args.alpha_im;
   float *cbase = reinterpret_cast<float *>(args.c) + (size_t)b * 2 * nx * ny;
@@ -1901,8 +1896,8 @@ __device__ __forceinline__ void store_wave_tile_staged32(const KernelArgs &args,
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const float4_t v = *reinterpret_cast<const float4_t *>(rd + q * 8 * 144);
-          store_c<float4_any_t>(out + (size_t)plane * nx * ny +
-                                        (size_t)(j * 32 + q * 8) * nx + i * 32, v, past_caches);
+          store_c<float4_any_t, PAST>(out + (size_t)plane * nx * ny +
+                                        (size_t)(j * 32 + q * 8) * nx + i * 32, v);
         }
       }
     }
@@ -2704,7 +2699,11 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     if constexpr (XT) {
       // the accumulators already hold whole row segments
       if (staged_ok && !args.c_interleaved && x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
-        store_wave_tile_rows<TOUT, TY>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
+        if (TOUT == kFloat32 && past_caches(args)) {
+          store_wave_tile_rows<TOUT == kFloat32, TOUT, TY>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
+        } else {
+          store_wave_tile_rows<false, TOUT, TY>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
+        }
       } else {
         store_wave_tile<TOUT, TX, TY, kAcc16T>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
       }
@@ -2724,8 +2723,10 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
           char *patch = lds + free_slot * SLOT_BYTES + wave * kStagePatchBytes;
           if (args.c_interleaved) {
             store_wave_tile_staged_il<TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
+          } else if (past_caches(args)) {
+            store_wave_tile_staged<true, TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
           } else {
-            store_wave_tile_staged<TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
+            store_wave_tile_staged<false, TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
           }
           staged = true;
         }
@@ -2766,9 +2767,12 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         free_slot = free_slot >= SLOTS ? free_slot - SLOTS : free_slot;
         asm volatile("s_barrier" ::: "memory");
         if (x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
-          store_wave_tile_staged32<TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane,
-                                           lds + free_slot * SLOT_BYTES + wave * kStagePatch32Bytes,
-                                           acc_re, acc_im);
+          char *patch = lds + free_slot * SLOT_BYTES + wave * kStagePatch32Bytes;
+          if (past_caches(args)) {
+            store_wave_tile_staged32<true, TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
+          } else {
+            store_wave_tile_staged32<false, TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
+          }
           staged = true;
         }
       }
