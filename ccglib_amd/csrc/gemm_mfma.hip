@@ -3236,6 +3236,11 @@ inline WaveShape wave_choice(const GemmParams &p) {
   }
   return shape;
 }
+// Whether four waves share the K tiles of a tile of C (1-bit input, see wave_choice; a single K tile is not shared out).
+inline bool waves_share_k(const GemmParams &p) {
+  const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 32) * ceil_div(p.ny, 32);
+  return p.type_in == kInt1 && p.k_tiles > 1 && tiles <= 3 * (size_t)compute_units();
+}
 template <int DT, int TOUT>
 hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream) {
   auto launch = [&](auto loader) {
@@ -3245,9 +3250,7 @@ hipError_t launch_waves(const GemmParams &p, WaveShape shape, hipStream_t stream
       if (shape == kWaves32x16) return launch_wave<DT, TOUT, L, 2, 1>(p, stream);
     }
     if constexpr (DT == kInt1) {
-      // (see wave_choice; a single K tile is not shared out)
-      const size_t tiles = (size_t)p.batch * ceil_div(p.nx, 32) * ceil_div(p.ny, 32);
-      if (p.k_tiles > 1 && tiles <= 3 * (size_t)compute_units()) return launch_wave<DT, TOUT, L, 2, 2, 4>(p, stream);
+      if (waves_share_k(p)) return launch_wave<DT, TOUT, L, 2, 2, 4>(p, stream);
     }
     return launch_wave<DT, TOUT, L, 2, 2>(p, stream);
   };
@@ -3477,7 +3480,8 @@ const char *describe_gemm_mfma(const GemmParams &p) {
   const size_t k_bytes = (size_t)p.k * bits_of(p.type_in) / 8;
   const bool planar_direct = (p.variant == kBasic) && (k_bytes >= 16) && (k_bytes % 16 == 0) &&
                              ((uintptr_t)p.x % 16 == 0) && ((uintptr_t)p.y % 16 == 0);
-  const BlockShape shape = block_choice(p).shape;
+  const BlockChoice choice = block_choice(p);
+  const BlockShape shape = choice.shape;
   const WaveShape waves = wave_choice(p);
   if (waves != kNoWaves) {
     // (a wave's tile, and the region of C whose waves are numbered consecutively)
@@ -3493,12 +3497,16 @@ const char *describe_gemm_mfma(const GemmParams &p) {
                        "complex_gemm_mfma_wave, 32x16 a wave, 8 waves to 64x64, interleaved rows",
                        "complex_gemm_mfma_wave, 32x16 a wave, 8 waves to 64x64, planar rows");
     }
+    if (waves_share_k(p)) {
+      return tiled ? "complex_gemm_mfma_wave, 32x32 by four waves along K, 4 tiles to 64x64, tiled operands"
+                   : "complex_gemm_mfma_wave, 32x32 by four waves along K, 4 tiles to 64x64, planar rows";
+    }
     return by_layout("complex_gemm_mfma_wave, 32x32 a wave, 4 waves to 64x64, tiled operands",
                      "complex_gemm_mfma_wave, 32x32 a wave, 4 waves to 64x64, interleaved rows",
                      "complex_gemm_mfma_wave, 32x32 a wave, 4 waves to 64x64, planar rows");
   }
-  auto name = [&](const char *large, const char *middle, const char *small) {
-    return shape == k256x128 ? large : shape == k128x128 ? middle : small;
+  auto name = [&](const char *large, const char *middle, const char *eight, const char *small) {
+    return shape == k256x128 ? large : shape == k64x64 ? small : choice.eight_waves ? eight : middle;
   };
   if (p.input_interleaved) {
     if (bits16 && wide_tiles_apply(p) && wide_tiles_pay(p)) {
@@ -3507,10 +3515,12 @@ const char *describe_gemm_mfma(const GemmParams &p) {
     if (2 * k_bytes % 16 != 0 || (uintptr_t)p.x % 16 != 0 || (uintptr_t)p.y % 16 != 0) {
       return name("complex_gemm_mfma_dtl, 256x128 block, ragged interleaved rows",
                   "complex_gemm_mfma_dtl, 128x128 block, ragged interleaved rows",
+                  "complex_gemm_mfma_dtl, 128x128 block of eight waves, ragged interleaved rows",
                   "complex_gemm_mfma_dtl, 64x64 block, ragged interleaved rows");
     }
     return name("complex_gemm_mfma_dtl, 256x128 block, interleaved rows",
                 "complex_gemm_mfma_dtl, 128x128 block, interleaved rows",
+                "complex_gemm_mfma_dtl, 128x128 block of eight waves, interleaved rows",
                 "complex_gemm_mfma_dtl, 64x64 block, interleaved rows");
   }
   if (p.variant == kOpt || planar_direct || int1) {
@@ -3520,15 +3530,18 @@ const char *describe_gemm_mfma(const GemmParams &p) {
     if (p.variant == kOpt) {
       return name("complex_gemm_mfma_dtl, 256x128 block, tiled operands",
                   "complex_gemm_mfma_dtl, 128x128 block, tiled operands",
+                  "complex_gemm_mfma_dtl, 128x128 block of eight waves, tiled operands",
                   "complex_gemm_mfma_dtl, 64x64 block, tiled operands");
     }
     return name("complex_gemm_mfma_dtl, 256x128 block, planar rows",
                 "complex_gemm_mfma_dtl, 128x128 block, planar rows",
+                "complex_gemm_mfma_dtl, 128x128 block of eight waves, planar rows",
                 "complex_gemm_mfma_dtl, 64x64 block, planar rows");
   }
   if (k_bytes >= 16) {
     return name("complex_gemm_mfma_dtl, 256x128 block, ragged planar rows",
                 "complex_gemm_mfma_dtl, 128x128 block, ragged planar rows",
+                "complex_gemm_mfma_dtl, 128x128 block of eight waves, ragged planar rows",
                 "complex_gemm_mfma_dtl, 64x64 block, ragged planar rows");
   }
   return "complex_gemm_mfma, 128x128 block, planar rows through registers";
