@@ -125,6 +125,8 @@ struct ccglib_gemm {
   // keeps it on the vector ALUs was set when the object was created)
   int int1_direct = 1;
   int block_tile = 0;
+  // Set by the pipeline: whether the rows would be read in place by rows_in_place_pay as well
+  int in_place_pays = 1;
 };
 
 struct ccglib_transpose {
@@ -322,6 +324,7 @@ void fill_gemm_params(const ccglib_gemm *g, const void *d_a, const void *d_b, vo
   p.workspace_bytes = g->workspace_bytes;
   p.int1_direct = g->int1_direct;
   p.block_tile = g->block_tile;
+  p.in_place_pays = g->in_place_pays;
 }
 
 }  // namespace
@@ -1015,6 +1018,11 @@ int pipeline_create(ccglib_pipeline_t *pipeline, size_t B, size_t M, size_t N, s
                      planar_in_place);  // :102-105
     if (rc == CCGLIB_OK) {
       p->gemm->input_interleaved = fused;
+      if (fused && il_ragged) {
+        p->gemm->in_place_pays = rows_in_place_pay(B, M, N, K, break_even_pairs((int)in_bits, il_ragged, wide_rows));
+      } else if (planar_in_place && planar_ragged) {
+        p->gemm->in_place_pays = rows_in_place_pay(B, M, N, K, break_even_planar((int)in_bits, planar_ragged));
+      }
       // (the basic variant's own interface has planar C only, its kernels store either)
       p->gemm->c_axis = output_complex_axis_location;
     }

@@ -84,6 +84,8 @@ struct GemmParams {
   // 1-bit GEMM only: the MFMA kernel may multiply the packed words (0: the
   // vector-ALU kernel runs whatever the layout)
   int int1_direct = 1;
+  // 0: rows that are read in place although the transposes and tiles would be faster (a pipeline whose route an option forces)
+  int in_place_pays = 1;
   int block_tile = 0;      // 0: chosen per problem; 1: 256 x 128 blocks; 2: 128 x 128; 3: 192 x 256; 4: 64 x 64
 };
 

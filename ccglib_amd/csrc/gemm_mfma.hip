@@ -3197,13 +3197,13 @@ inline WaveShape wave_choice(const GemmParams &p) {
   const WaveCosts *costs = table.shape;
   const double k_tiles = (double)(p.input_interleaved ? (p.k_tiles + 1) / 2 : p.k_tiles);
   const double units = (double)compute_units();
-  // Ragged rows of many K tiles go through the transposes (rows_in_place_pay), with waves on the tiles behind
-  // them; which route such rows take is fixed by a test, so that waves on the rows as they lie, which
-  // would be faster still (fp16 64x320x6598 22.5 us, transposes and waves 30.6, and 68 before
-  // there were waves), stay with the shorter ones.
+  // Ragged rows of many K tiles that go through the transposes by default have their waves on the tiles behind them. Where an
+  // option has them read in place nevertheless they stay on blocks, with which the break-even points of rows_in_place_pay were
+  // measured and which its tests hold it to (fp16 64x320x6598: transposes and waves 30.6 us, in place on blocks 68, on
+  // waves 22.5). Rows that are read in place by default: fp16 planar B=55 32x16x7026 93 us on blocks, 24 on waves.
   const bool ragged = (p.variant != kOpt || p.input_interleaved) && p.type_in != kInt1 &&
                       (p.input_interleaved ? 2 : 1) * (size_t)p.k * bits_of(p.type_in) / 8 % 16 != 0;
-  if (ragged && k_tiles > 64.0) return kNoWaves;
+  if (ragged && k_tiles > 64.0 && !p.in_place_pays) return kNoWaves;
   const double operand_mb = 1e-6 * 2.0 * (double)p.batch * ((double)p.nx + (double)p.ny) * (double)p.k * bits_of(p.type_in) / 8;
   auto time = [&](int shape, unsigned x, unsigned y) {
     const WaveCosts &c = costs[shape];
