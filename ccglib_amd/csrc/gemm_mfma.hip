@@ -1217,7 +1217,10 @@ typedef ushort4_t ushort4_any_t __attribute__((aligned(2)));
 template <typename Piece, bool PAST, typename Value>
 __device__ __forceinline__ void store_c(void *at, const Value &v) {
   if constexpr (PAST) {
+    // (the empty statements keep the compiler from making one ordinary store of those of the two epilogues)
+    asm volatile("");
     __builtin_nontemporal_store((Piece)v, reinterpret_cast<Piece *>(at));
+    asm volatile("");
   } else {
     *reinterpret_cast<Piece *>(at) = v;
   }

@@ -1,12 +1,14 @@
 """How well the dispatch picks a block shape: GEMMs of random sizes, types, operand layouts and C
 layouts, timed with each shape forced (option GEMM_BLOCK_TILE = 1, 2, 4: 256 x 128, 128 x 128,
-64 x 64; 32-bit input has no 256 x 128), and how far the shape that the default takes is behind the fastest. The
-constants of block_choice (../csrc/gemm_mfma.hip) are fitted to such times.
+64 x 64; 32-bit input has no 256 x 128; 5, 6, 7: waves of their own, where there are at most 2048 blocks of 64 x 64), and how far the
+default is behind the fastest. One table for the problems whose default is a block (whichever forced shape the default's time is
+closest to), against the three block shapes; one for those on waves, against 64 x 64 blocks and all shapes. The
+constants of block_choice and wave_choice (../csrc/gemm_mfma.hip) are fitted to such times.
 
     python -m ccglib_amd.tuning.block_choice [--problems 2000] [--seed 1] [--warm] [--csv FILE] [--input float32]
 
 One MI355X, N(0, 1) operands (fp8 scaled into range, random bits for 1-bit input). Every pass takes
-other buffers, out of pools larger than the last-level cache; with --warm the same ones. The three
+other buffers, out of pools larger than the last-level cache; with --warm the same ones. The
 shapes take turns, five times about 2 ms each; the medians count. Sizes: B up to 256, M and N 16 to
 4096, K 64 to 4096 (1-bit: 512 to 32768), half of them multiples of 8 to 128, up to about 1.5 ms
 and 1536 tiles of 256 x 128. K is a multiple of 16 (1-bit: 128); a third of the problems on rows in place
@@ -17,6 +19,7 @@ import collections
 import math
 import random
 import statistics
+import sys
 
 import torch
 
@@ -134,7 +137,10 @@ def measure(case, sizes, warm):
     slots = 1 if warm else int(max(1, min(4096, FOOTPRINT // sum(steps), *(POOL_BYTES // v for v in steps))))
     base = [pool(case[0], "a"), pool(case[0], "b"), pool(None, "c")]
     where = [[p + i * v for p, v in zip(base, steps)] for i in range(slots)]
-    runs = {t: make(case, t) for t in (0, 1, 2, 4) if t != 1 or case[0] != VT.float32}
+    tiles = [0, 2, 4] if case[0] == VT.float32 else [0, 1, 2, 4]
+    if case[0] != VT.float32 and case[6] * cc.ceildiv(case[7], 64) * cc.ceildiv(case[8], 64) <= 2048:
+        tiles += [5, 6, 7] if BITS[case[0]] == 16 else [5]
+    runs = {t: make(case, t) for t in tiles}
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     at = 0
 
@@ -188,25 +194,32 @@ def main():
         text = "%s->%s %s%s%s B=%d %dx%dx%d" % (tin.name, tout.name, layout,
                                                 " interleaved C" if c_axis == AX.complex_interleaved else "",
                                                 " beta" if beta else "", B, M, N, K)
-        behind = t[0] / min(v for v in (t[1], t[2], t[4]) if v == v)
-        groups["%-12s %s" % (tin.name, layout)].append(behind)
-        groups["all"].append(behind)
+        times = {k: v for k, v in t.items() if k and v == v}
+        waves = min(times, key=lambda k: abs(times[k] - t[0])) >= 5
+        behind = t[0] / min(v for k, v in times.items() if waves or k < 5)
+        for name in ("all", "%-12s %s" % (tin.name, layout)):
+            groups[waves, name].append((behind, times[4] / t[0]))
         worst.append((behind, text, t))
         if csv:
-            csv.write("%s,%.2f,%.2f,%.2f,%.2f\n" % (text, t[0], t[1], t[2], t[4]))
+            csv.write("%s,%s\n" % (text, ",".join("%d:%.2f" % kv for kv in sorted(t.items()))))
         if i % 200 == 199:
-            print("%d problems" % (i + 1), flush=True)
-    print("\n%s operands; the default against the fastest of 256x128, 128x128, 64x64"
-          "\n(the default may also take 192x256 blocks or waves of their own, and is then in front; two runs of one kernel differ by a few %%)" %
-          ("warm" if args.warm else "cold"))
-    print("%-30s %8s %14s %10s %10s" % ("input, layout", "problems", "mean behind %", "> 8 % in", "> 20 % in"))
-    for name in sorted(groups):
-        v = groups[name]
-        print("%-30s %8d %14.2f %10d %10d" % (name, len(v), 100 * (statistics.mean(v) - 1),
-                                              sum(x > 1.08 for x in v), sum(x > 1.2 for x in v)))
-    print("\nfarthest behind (us: default, 256x128, 128x128, 64x64)")
+            print("%d problems" % (i + 1), file=sys.stderr, flush=True)
+    for waves in (False, True):
+        print("\n%s operands, default on %s" % (
+            "warm" if args.warm else "cold",
+            "waves: behind the fastest of blocks and waves, and 64x64 blocks over the default" if waves else
+            "blocks: behind the fastest of 256x128, 128x128, 64x64 (192x256 blocks are then in front)"))
+        print("%-30s %8s %14s %10s %10s%s" % ("input, layout", "problems", "mean behind %", "> 8 % in", "> 20 % in",
+                                             "  64x64 / default" if waves else ""))
+        for name in sorted(n for w, n in groups if w == waves):
+            v = [x for x, _ in groups[waves, name]]
+            over = [x for _, x in groups[waves, name]]
+            print("%-30s %8d %14.2f %10d %10d%s" % (name, len(v), 100 * (statistics.mean(v) - 1),
+                                                   sum(x > 1.08 for x in v), sum(x > 1.2 for x in v),
+                                                   "%17.2f" % statistics.geometric_mean(over) if waves else ""))
+    print("\nfarthest behind (us: default; 256x128, 128x128, 64x64; waves of 32x32, 32x16, 16x16)")
     for behind, text, t in sorted(worst, key=lambda w: -w[0])[:12]:
-        print("%5.2f  %-66s %8.1f %8.1f %8.1f %8.1f" % (behind, text, t[0], t[1], t[2], t[4]))
+        print("%5.2f  %-66s %s" % (behind, text, " ".join("%8.1f" % t.get(k, math.nan) for k in (0, 1, 2, 4, 5, 6, 7))))
 
 
 if __name__ == "__main__":
