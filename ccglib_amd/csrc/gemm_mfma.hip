@@ -1213,16 +1213,24 @@ typedef ushort4_t ushort4_any_t __attribute__((aligned(2)));
 // goes out as it comes. Us without and with it: B=16 2048x2048x1024 e4m3 282, 259; B=64 1024x1024x512 fp16 309, 259; B=32
 // 1024x1024x512 e4m3 pairs 102, 84; with K = 8192 nothing. Of a smaller C the next kernel loses more than this one gains
 // (kPastCachesBytes), and rows that share lines (B=176 629x4330x512 e4m3 1626, 3044) only cost.
-// (An epilogue each: with the choice at every store planar C of 8 bits, which never takes it below 256 MiB, was 1 to 2 % slower.)
+// Four stores at a time: with the choice at every store planar C of 8 bits that does not take it was 1 to 2 %
+// slower; with an epilogue each the 1-bit kernels spill.
 template <typename Piece, bool PAST, typename Value>
 __device__ __forceinline__ void store_c(void *at, const Value &v) {
   if constexpr (PAST) {
-    // (the empty statements keep the compiler from making one ordinary store of those of the two epilogues)
+    // (the empty statements keep the compiler from making one ordinary store of the two)
     asm volatile("");
     __builtin_nontemporal_store((Piece)v, reinterpret_cast<Piece *>(at));
     asm volatile("");
   } else {
     *reinterpret_cast<Piece *>(at) = v;
+  }
+}
+template <typename Store> __device__ __forceinline__ void store_four(bool past, Store &&store) {
+  if (past) {
+    static_for<4>([&](auto n) { store(n, std::true_type{}); });
+  } else {
+    static_for<4>([&](auto n) { store(n, std::false_type{}); });
   }
 }
 
@@ -1688,13 +1696,14 @@ __device__ __forceinline__ void store_wave_tile_int32(const KernelArgs &args, un
 // the four tiles of a tile row are four consecutive x, so a lane writes 16 bytes
 // (8 for fp16 / bf16 C) and a store instruction four whole 256-byte row segments,
 // straight from the accumulators.
-template <bool PAST, int TOUT, int TY>
+template <int TOUT, int TY>
 __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, unsigned b,
                                                      unsigned x_wave, unsigned y_wave, int lane,
                                                      float4_t (&acc_re)[TY][4],
                                                      float4_t (&acc_im)[TY][4]) {
   using Tout = typename OutType<TOUT>::type;
   const unsigned nx = args.nx, ny = args.ny;
+  const bool past = TOUT == kFloat32 && past_caches(args);
   const bool have_alpha = args.have_alpha;
   const float ar = args.alpha_re, ai = args.alpha_im;
   Tout *out = reinterpret_cast<Tout *>(args.c) + (size_t)b * 2 * nx * ny +
@@ -1703,8 +1712,8 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
   for (int plane = 0; plane < 2; ++plane) {
 #pragma unroll
     for (int j = 0; j < TY; ++j) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
+      store_four(past, [&](auto n, auto past_them) {
+        constexpr int e = n;
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -1714,12 +1723,12 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
         }
         Tout *p = out + (size_t)plane * nx * ny + (size_t)(j * 16 + e) * nx;
         if constexpr (TOUT == kFloat32) {
-          store_c<float4_any_t, PAST>(p, float4_t{v[0], v[1], v[2], v[3]});
+          store_c<float4_any_t, decltype(past_them)::value>(p, float4_t{v[0], v[1], v[2], v[3]});
         } else {
           Tout t[4] = {(Tout)v[0], (Tout)v[1], (Tout)v[2], (Tout)v[3]};
           *reinterpret_cast<ushort4_any_t *>(p) = __builtin_bit_cast(ushort4_t, t);
         }
-      }
+      });
     }
   }
 }
@@ -1732,13 +1741,14 @@ __device__ __forceinline__ void store_wave_tile_rows(const KernelArgs &args, uns
 // the column-wise writes and the row-wise reads free of bank conflicts).
 constexpr int kStagePatchBytes = 16 * 272;
 
-template <bool PAST, int TX, int TY>
+template <int TX, int TY>
 __device__ __forceinline__ void store_wave_tile_staged(const KernelArgs &args, unsigned b,
                                                        unsigned x_wave, unsigned y_wave, int lane,
                                                        char *patch, float4_t (&acc_re)[TY][TX],
                                                        float4_t (&acc_im)[TY][TX]) {
   static_assert(TX == 4, "patch rows hold 64 columns");
   const unsigned nx = args.nx, ny = args.ny;
+  const bool past = past_caches(args);
   const bool have_alpha = args.have_alpha;
   const float ar = args.alpha_re, ai = args.alpha_im;
   float *cbase = reinterpret_cast<float *>(args.c) + (size_t)b * 2 * nx * ny;
@@ -1760,11 +1770,12 @@ __device__ __forceinline__ void store_wave_tile_staged(const KernelArgs &args, u
         }
         *reinterpret_cast<float4_t *>(wr + i * 64) = v;
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
+      store_four(past, [&](auto n, auto past_them) {
+        constexpr int r = n;
         const float4_t v = *reinterpret_cast<const float4_t *>(rd + r * 4 * 272);
-        store_c<float4_any_t, PAST>(out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 4) * nx, v);
-      }
+        store_c<float4_any_t, decltype(past_them)::value>(
+            out + (size_t)plane * nx * ny + (size_t)(j * 16 + r * 4) * nx, v);
+      });
     }
   }
 }
@@ -1859,12 +1870,13 @@ __device__ __forceinline__ void store_wave_tile_staged_il(const KernelArgs &args
 // instruction writes eight whole 128-byte row segments.
 constexpr int kStagePatch32Bytes = 32 * 144;
 
-template <bool PAST, int TX, int TY, bool INT = false>
+template <int TX, int TY, bool INT = false>
 __device__ __forceinline__ void store_wave_tile_staged32(const KernelArgs &args, unsigned b,
                                                          unsigned x_wave, unsigned y_wave, int lane,
                                                          char *patch, float16_t_ (&acc_re)[TY][TX],
                                                          float16_t_ (&acc_im)[TY][TX]) {
   const unsigned nx = args.nx, ny = args.ny;
+  const bool past = past_caches(args);
   const bool have_alpha = args.have_alpha;
   const float ar = args.alpha_re, ai = args.alpha_im;
   float *cbase = reinterpret_cast<float *>(args.c) + (size_t)b * 2 * nx * ny;
@@ -1896,12 +1908,12 @@ __device__ __forceinline__ void store_wave_tile_staged32(const KernelArgs &args,
           }
           *reinterpret_cast<float4_t *>(wr + k * 32) = v;
         }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        store_four(past, [&](auto n, auto past_them) {
+          constexpr int q = n;
           const float4_t v = *reinterpret_cast<const float4_t *>(rd + q * 8 * 144);
-          store_c<float4_any_t, PAST>(out + (size_t)plane * nx * ny +
-                                        (size_t)(j * 32 + q * 8) * nx + i * 32, v);
-        }
+          store_c<float4_any_t, decltype(past_them)::value>(
+              out + (size_t)plane * nx * ny + (size_t)(j * 32 + q * 8) * nx + i * 32, v);
+        });
       }
     }
   }
@@ -2702,11 +2714,7 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
     if constexpr (XT) {
       // the accumulators already hold whole row segments
       if (staged_ok && !args.c_interleaved && x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
-        if (TOUT == kFloat32 && past_caches(args)) {
-          store_wave_tile_rows<TOUT == kFloat32, TOUT, TY>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
-        } else {
-          store_wave_tile_rows<false, TOUT, TY>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
-        }
+        store_wave_tile_rows<TOUT, TY>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
       } else {
         store_wave_tile<TOUT, TX, TY, kAcc16T>(args, tc.b, x_wave, y_wave, lane, acc_re, acc_im);
       }
@@ -2726,10 +2734,8 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
           char *patch = lds + free_slot * SLOT_BYTES + wave * kStagePatchBytes;
           if (args.c_interleaved) {
             store_wave_tile_staged_il<TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
-          } else if (past_caches(args)) {
-            store_wave_tile_staged<true, TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
           } else {
-            store_wave_tile_staged<false, TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
+            store_wave_tile_staged<TX, TY>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
           }
           staged = true;
         }
@@ -2770,12 +2776,9 @@ __global__ __launch_bounds__(64 * (BX / WX) * (BY / WY), WAVES_PER_EU) void comp
         free_slot = free_slot >= SLOTS ? free_slot - SLOTS : free_slot;
         asm volatile("s_barrier" ::: "memory");
         if (x_wave + WX <= args.nx && y_wave + WY <= args.ny) {
-          char *patch = lds + free_slot * SLOT_BYTES + wave * kStagePatch32Bytes;
-          if (past_caches(args)) {
-            store_wave_tile_staged32<true, TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
-          } else {
-            store_wave_tile_staged32<false, TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane, patch, acc_re, acc_im);
-          }
+          store_wave_tile_staged32<TX, TY, TOUT == kInt32>(args, tc.b, x_wave, y_wave, lane,
+                                           lds + free_slot * SLOT_BYTES + wave * kStagePatch32Bytes,
+                                           acc_re, acc_im);
           staged = true;
         }
       }
