@@ -3146,41 +3146,42 @@ inline bool wide_tiles_pay(const GemmParams &p) {
 // further wave of the busiest unit (330 waves on 256 units take as long as 512 where the copies of one wave do not fill the time; a
 // wave keeps 32 KiB on its way where a block keeps 80, so that operands that no cache holds come in more slowly: B=197 24x49x2992
 // planar fp16 62 us on waves, 46 on blocks). The constants are
-// fitted, for each type and operand layout, to the choice among the shapes (what it loses against the fastest one, and three times
-// against 64 x 64 blocks alone): 7700 problems of 16 bits, 2130 of 8, 1890 of 1 bit that have 64 x 64 blocks by block_choice, on cold operands.
-// On a third kept out of the fit the choice was behind the fastest shape by 0.3 % (tiles), 0.6 % (pairs) and 1.2 %
-// (planar rows) for 16 bits, 0.4 to 0.8 % for 8, 3 to 4 % for 1 bit (waves that do not share K would serve more rounds), and in front of 64 x 64
-// blocks by 1.29 to 1.33 times (16 bits), 1.14 to 1.17 (8 bits), 1.21 to 1.31 (1 bit). More waves than there are SIMDs are left to the
+// fitted, for each type and operand layout, to the choice among the shapes (what it loses against the fastest one, twice what it loses
+// against 64 x 64 blocks alone, and a little of the errors of the times themselves): 10700 problems of 16 bits and 4100 of 8, a fifth of
+// them on operands that the caches hold, 1890 of 1 bit, all of which have 64 x 64 blocks by block_choice.
+// On those kept out of the fit the choice was behind the fastest shape by 0.3 % (tiles), 0.5 % (pairs) and 1.0 % (planar rows; 1.9 % with the
+// constants before) for 16 bits, 0.1 to 0.4 % for 8, 3 to 4 % for 1 bit (waves that do not share K would serve more rounds), and in front of 64 x 64
+// blocks by 1.33 to 1.50 times (16 bits), 1.15 to 1.23 (8 bits), 1.21 to 1.31 (1 bit). More waves than there are SIMDs are left to the
 // blocks: the fifth wave of a unit has to share one (B=213 32x192x3184 on planar rows, 1278 waves: 179 us on blocks, 261 on waves).
 enum WaveShape { kNoWaves, kWaves32x32, kWaves32x16, kWaves16x16 };
 struct WaveCosts {
-  double fixed, alone, crowded, tile;
+  double fixed, alone, crowded, tile, second;
 };
 struct WaveTable {
   WaveCosts shape[4];   // 64 x 64 blocks, then as WaveShape
-  double second;        // waves: what every further one of the busiest unit adds to `alone`, of it
   double beta;          // blocks: they only request C behind the last product
-  double block_bytes, wave_bytes;   // us per MB of A and B
+  double block_bytes, wave_bytes;   // us per MB of A and B ...
+  double cached_mb = 0.0;           // ... beyond these, which the caches may hold
 };
 inline const WaveTable &wave_costs(const GemmParams &p) {
-  static constexpr WaveCosts none = {0.0, 0.0, 0.0, 0.0};
-  static constexpr WaveTable bits16_tiled = {{{4.836, 0.427, 0.499, 1.107}, {3.070, 0.291, 0.105, 0.661},
-                                              {2.887, 0.222, 0.052, 0.189}, {2.405, 0.067, 0.094, 0.057}}, 0.286, 0.229, 0.145, 0.130};
-  static constexpr WaveTable bits16_planar = {{{4.737, 0.386, 0.474, 1.487}, {4.274, 0.256, 0.200, 0.251},
-                                               {3.058, 0.261, 0.189, 0.008}, {2.544, 0.179, 0.137, 0.024}}, 0.521, 0.317, 0.229, 0.277};
-  static constexpr WaveTable bits16_pairs = {{{5.172, 0.489, 0.551, 1.398}, {4.188, 0.384, 0.148, 0.478},
-                                              {2.579, 0.305, 0.165, 0.316}, {2.440, 0.161, 0.125, 0.053}}, 0.247, 1.206, 0.148, 0.087};
-  static constexpr WaveTable bits8_tiled = {{{3.762, 0.313, 0.405, 2.345}, {3.118, 0.221, 0.141, 0.495}, none, none},
-                                            0.236, 1.409, 0.150, 0.175};
-  static constexpr WaveTable bits8_planar = {{{3.816, 0.537, 0.670, 2.406}, {3.484, 0.271, 0.221, 0.351}, none, none},
-                                             0.809, 2.391, 0.269, 0.372};
-  static constexpr WaveTable bits8_pairs = {{{4.495, 0.359, 0.461, 1.901}, {3.511, 0.252, 0.117, 0.569}, none, none},
-                                            0.474, 1.997, 0.275, 0.309};
-  // (1 bit: `fixed` and `alone` of a tile shared by four waves, see wave_choice; `second`: of a launch)
-  static constexpr WaveTable int1_tiled = {{{3.738, 1.079, 1.353, 1.857}, {4.653, 1.026, 0.0, 0.0}, none, none},
-                                           -1.454, 0.0, 0.212, 0.271};
-  static constexpr WaveTable int1_planar = {{{6.040, 0.947, 0.938, 1.252}, {3.101, 1.079, 0.0, 0.0}, none, none},
-                                            2.437, 0.0, 0.268, 0.214};
+  static constexpr WaveCosts none = {0.0, 0.0, 0.0, 0.0, 0.0};
+  static constexpr WaveTable bits16_tiled = {{{4.016, 0.295, 0.376, 1.653, 0.000}, {3.304, 0.200, 0.070, 0.437, 0.338},
+      {3.316, 0.147, 0.079, 0.009, 0.356}, {2.493, 0.097, 0.060, 0.062, 0.393}}, 1.114, 0.133, 0.090, 32.0};
+  static constexpr WaveTable bits16_planar = {{{4.059, 0.432, 0.470, 2.137, 0.000}, {3.899, 0.226, 0.223, 0.293, 0.660},
+      {2.865, 0.200, 0.180, 0.093, 0.411}, {2.660, 0.127, 0.097, 0.077, 0.268}}, 0.845, 0.316, 0.453, 32.0};
+  static constexpr WaveTable bits16_pairs = {{{4.010, 0.359, 0.476, 2.376, 0.000}, {3.246, 0.288, 0.182, 0.369, 0.253},
+      {3.060, 0.187, 0.106, 0.025, 0.381}, {2.581, 0.111, 0.085, 0.015, 0.445}}, 1.766, 0.195, 0.129, 32.0};
+  static constexpr WaveTable bits8_tiled = {{{3.670, 0.306, 0.387, 2.100, 0.000}, {3.195, 0.202, 0.136, 0.410, 0.229}, none, none},
+      1.888, 0.146, 0.166};
+  static constexpr WaveTable bits8_planar = {{{3.851, 0.504, 0.709, 2.196, 0.000}, {3.569, 0.236, 0.266, 0.127, 0.825}, none, none},
+      2.029, 0.236, 0.336};
+  static constexpr WaveTable bits8_pairs = {{{4.097, 0.391, 0.431, 1.849, 0.000}, {4.204, 0.240, 0.189, 0.043, 0.578}, none, none},
+      1.750, 0.285, 0.308};
+  // (1 bit: `fixed` and `alone` of a tile shared by four waves, `tile` of a launch, see wave_choice)
+  static constexpr WaveTable int1_tiled = {{{3.738, 1.079, 1.353, 1.857, 0.0}, {4.653, 1.026, 0.0, -1.454, 0.0}, none, none},
+      0.0, 0.212, 0.271};
+  static constexpr WaveTable int1_planar = {{{6.040, 0.947, 0.938, 1.252, 0.0}, {3.101, 1.079, 0.0, 2.437, 0.0}, none, none},
+      0.0, 0.268, 0.214};
   const bool tiled = p.variant == kOpt && !p.input_interleaved;
   if (p.type_in == kInt1) return tiled ? int1_tiled : int1_planar;
   if (bits_of(p.type_in) == 8) return p.input_interleaved ? bits8_pairs : tiled ? bits8_tiled : bits8_planar;
@@ -3210,12 +3211,13 @@ inline WaveShape wave_choice(const GemmParams &p) {
   const bool ragged = (p.variant != kOpt || p.input_interleaved) && p.type_in != kInt1 &&
                       (p.input_interleaved ? 2 : 1) * (size_t)p.k * bits_of(p.type_in) / 8 % 16 != 0;
   if (ragged && k_tiles > 64.0 && !p.in_place_pays) return kNoWaves;
-  const double operand_mb = 1e-6 * 2.0 * (double)p.batch * ((double)p.nx + (double)p.ny) * (double)p.k * bits_of(p.type_in) / 8;
+  const double operand_mb = std::max(0.0, 1e-6 * 2.0 * (double)p.batch * ((double)p.nx + (double)p.ny) * (double)p.k *
+                                                  bits_of(p.type_in) / 8 - table.cached_mb);
   auto time = [&](int shape, unsigned x, unsigned y) {
     const WaveCosts &c = costs[shape];
     const double n = (double)p.batch * (double)ceil_div(p.nx, x) * (double)ceil_div(p.ny, y) / units;
     if (shape != 0 && n > kWavesPerUnit) return HUGE_VAL;
-    const double alone = shape != 0 ? c.alone * (1.0 + table.second * (std::ceil(n) - 1.0)) : c.alone;
+    const double alone = c.alone * (1.0 + c.second * (std::ceil(n) - 1.0));
     const double beta = shape == 0 && p.have_beta ? table.beta : 0.0;
     const double bytes = operand_mb * (shape != 0 ? table.wave_bytes : table.block_bytes);
     return c.fixed + beta + std::max(bytes, k_tiles * std::max(alone, c.crowded * n)) + c.tile * n;
@@ -3225,7 +3227,7 @@ inline WaveShape wave_choice(const GemmParams &p) {
     // like this, 512x512 (a tile a unit) K=2048 7.8, 4.9; K=32768 59.7, 19.2; B=20 128x128 (some units two) K=8192
     // 18.4, 13.9; K=32768 60.3, 33.7; 768x1024 (three) K=8192 19.0, 20.2; K=32768 60.9, 49.4; B=5 1064x128 (three) K=9600 planar 23.8, 30.1.
     const double rounds = std::ceil((double)p.batch * (double)ceil_div(p.nx, 32) * (double)ceil_div(p.ny, 32) / units);
-    const double waves = table.second + std::max(rounds * (costs[1].fixed + costs[1].alone * std::ceil(k_tiles / 4.0)),
+    const double waves = costs[1].tile + std::max(rounds * (costs[1].fixed + costs[1].alone * std::ceil(k_tiles / 4.0)),
                                                  operand_mb * table.wave_bytes);
     return rounds <= 3.0 && waves < time(0, 64, 64) ? kWaves32x32 : kNoWaves;
   }
