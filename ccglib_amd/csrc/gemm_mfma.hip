@@ -3015,24 +3015,23 @@ hipError_t launch_wide(const GemmParams &p, hipStream_t stream) {
 // problem fills and the less it computes beyond the edges of C, but the more bytes it
 // moves per flop. Times with 256 x 128, 128 x 128 and 64 x 64 blocks in us, on operands that no cache
 // held (profiles/gemm_block_choice.txt):
-//   too few tiles for the larger blocks, 16 bits 256^3:  14.4, 12.2, 6.5;  B=256 96x96x1024:  87, 57, 63;
-//     32 bits B=2 1000^3:  (none), 186, 129;  8 bits 1024^3:  24.3, 21.8, 10.8;
-//     1 bit 64x64x65536:  529, 308, 115
-//   every unit busy, 16 bits on planar rows, B=64 512x4096x576:  613, 655, 962; B=300 512x512x128:  163, 158, 259
-//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  (none), 453, 523
-//     8 bits on tiles, 4096x4096x512:  52, 51, 69
+//   too few tiles for the larger blocks, 16 bits on tiles 256^3:  14.8, 12.2, 6.4;  32 bits B=2 1000^3:  (none), 166, 117;
+//     8 bits 1024^3:  24.2, 21.7, 10.5;  1 bit 64x64x65536:  526, 308, 115
+//   every unit busy, 16 bits on planar rows, B=157 192x604x3680:  735, 757, 1021; B=167 800x184x2064:  553, 642, 863
+//     32 bits, which a smaller wave tile splits more often, 4096x4096x512:  (none), 416, 480
+//     8 bits on tiles, 4096x4096x512:  46, 45, 65
 //     1 bit, whose words a wave with one tile expands for half as many products, 3452x1504x32256:
-//       308, 317, 339
+//       271, 288, 313
 // Two blocks share a unit with 64 x 64 tiles and with 128 x 128 tiles (of 16-bit input: those of four waves), and
 // a last tile that has the unit to itself leaves it idle for a part of the time: `lone` of a tile.
 // With beta the epilogue reads C first, which costs the larger tiles more (8 bits on planar
 // rows, B=11 456x1542x192: 97, 84, 47), and pairs of C with beta are read and stored piece by piece by all of them (B=43 144x1024x32
 // fp16 pairs 40.2, 36.3, 27.3).
 //   128 x 128 blocks of 16-bit input have eight waves and a ring of four slots while every block has a unit to itself, which
-// keeps more on its way (B=256 96x96x1024 pairs 48 us, 52 with the other); beyond, four waves of 64 x 64 and two slots, of which
+// keeps more on its way; beyond, four waves of 64 x 64 and two slots, of which
 // two share a unit: one stores C or waits while the other multiplies, the fragments are read once for twice as many
 // products, and C is stored in whole row segments. In us, planar rows unless said, 8 and 4 waves (256 x 128 blocks):
-// B=67 384x3136x328 445, 329 (337); B=300 512x512x128 217, 158 (163); B=100 320x320x256 pairs 45, 40 (50). With beta, which
+// B=67 384x3136x328 439, 330 (328); B=300 512x512x128 211, 126 (137); B=100 320x320x256 pairs 47, 41 (51). With beta, which
 // takes the four waves' registers while C is read, eight may be the faster ones there too (B=60 1536x128x80 fp16 planar 41.8, 51.3;
 // 750 such problems 0.97 times on planar rows of K up to 300, 1.03 to 1.12 elsewhere), which have constants of their own for it.
 //   The constants are fitted, for each type and operand layout, to the times of all three shapes over
