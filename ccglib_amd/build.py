@@ -79,7 +79,8 @@ def _no_scratch_in_gemm_kernels(src, remarks):
     loop. The compiler's resource remarks say whether a kernel spills registers to scratch
     memory. The one-wave-per-SIMD kernels (complex_gemm_mfma_wide) run at the edge of the
     register file and must not spill at all: the build stops if one does. Of the others, the
-    1-bit 128 x 128 kernel spills four values at set-up and reloads them where a block moves
+    1-bit 256 x 128 and 128 x 128 kernels spill four to eight values at set-up and in the epilogue, the four-wave 128 x 128
+    ones of ragged 16-bit pairs two or three, and reload them where a block moves
     to its next C tile (the compiler waits for all memory operations there), and those of 32-bit pairs
     to 16-bit C one address while they look for NaN behind the K loop; anything beyond
     those few bytes stops the build as well."""
